@@ -520,6 +520,19 @@ ZD void node_basics(const Pos &p, Node0 &B) {
   B.cmask = cm;
 }
 
+// Is the side to move's king (on square k of bitboard kb, kb = 0 for no king)
+// attacked?  One position per lane, the same k in every lane: the checkers of
+// node_basics without the check mask.
+ZD bool king_attacked(const Pos &p, int k, u64 kb) {
+  const u64 occ = p.b1 | p.b2 | p.b3;
+  const u64 opp = p.stm ? (p.b0 ^ occ) : p.b0;
+  const u64 rq = p.b3 & (p.b1 ^ p.b2), bq = p.b3 & ~p.b1;
+  u64 a = (rook_sq(k, occ) & rq) | (bishop_sq(k, occ) & bq);
+  a |= knight_att(kb) & ~p.b1 & p.b2 & ~p.b3;
+  a |= pawn_att(kb, p.stm) & p.b1 & ~p.b2 & ~p.b3;
+  return kb && (a & opp);
+}
+
 // is sq attacked by the opponent, the own king taken off the board?
 ZD bool attacked_nk(const Node0 &B, int sq) {
   const u64 b = bit(sq);

@@ -105,6 +105,43 @@ ZD int32_t eval_bishop_pair(const Pos &p) {
   return (popc((p.b0 ^ occ) & bishops) == 2 ? 25 : 0) - (popc(p.b0 & bishops) == 2 ? 25 : 0);
 }
 
+// The pawn terms of eval_square summed over the board, white minus black, set
+// by set: blocked by an opponent's piece in front (-15), defended by an own
+// pawn (+10 for each side), own pawns behind on the file (-30 each, so -30 for
+// every pair on a file).  Equal to the per-square terms when no pawn stands on
+// the first or the last rank (the reference's ranges there wrap).
+ZD int32_t pawn_terms(u64 pawns, u64 white, u64 black) {
+  const u64 w = pawns & white, b = pawns & black;
+  const int block = popc((w << 8) & black) - popc((b >> 8) & white);
+  const int chain = popc(w & (w << 7) & NOTH) + popc(w & (w << 9) & NOTA) - popc(b & (b >> 7) & NOTA) -
+                    popc(b & (b >> 9) & NOTH);
+  int pairs = 0;
+#pragma unroll
+  for (int k = 8; k <= 40; k += 8) pairs += popc(w & (w << k)) - popc(b & (b << k));
+  return 10 * chain - 15 * block - 30 * pairs;
+}
+
+// material + piece-square + square control of a coloured piece, white positive
+ZD int32_t eval_piece(u32 pc, int sq) {
+  const int v = EVAL_SQ.v[((pc >> 1) & 7) * 64 + ((pc & 1) ? sq : (sq ^ 56))];
+  return (pc & 1) ? -v : v;
+}
+
+// How a move changes the sum of eval_piece over the board (the castle rook
+// included).
+ZD int32_t eval_move_delta(u32 m) {
+  const int f = (int)mv_from(m), t = (int)mv_to(m);
+  const u32 pf = mv_pfrom(m), pc = mv_pcpt(m);
+  int32_t d = eval_piece(mv_pto(m), t) - eval_piece(pf, f);
+  if (((pc >> 1) & 7) != PNONE) d -= eval_piece(pc, (int)mv_cpt(m));
+  if (((pf >> 1) & 7) == KING && (f - t == 2 || t - f == 2)) {
+    const u32 rook = (ROOK << 1) | (pf & 1);
+    d += f - t == 2 ? eval_piece(rook, (t + 1) & 63) - eval_piece(rook, (f - 4) & 63)
+                    : eval_piece(rook, (t - 1) & 63) - eval_piece(rook, (f + 3) & 63);
+  }
+  return d;
+}
+
 // Move-ordering score of the reference picker (src/zeta.cl:2059-2071):
 // captures MVV-LVA (16*V[captured] - V[mover]), quiet moves by the change of
 // material + piece-square + control value.

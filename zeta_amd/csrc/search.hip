@@ -55,6 +55,8 @@ constexpr s32 KILLER_SCORE = 1400;
 constexpr s32 COUNTER_SCORE = 1300;
 constexpr int NCOUNTER = 64 * 64;  // counter-move table entries per worker (LDS)
 constexpr u32 DEFERRED = 0x80000000u;  // move-stack flag: deferred by ABDADA (move codes use bits 0-29)
+constexpr u32 REFUTED = 0x40000000u;   // move-stack flag: the child's stand pat refutes the move (mark_refuted)
+constexpr u32 MOVE_BITS = 0x3FFFFFFFu;
 constexpr int ABDADA_MIN_DEPTH = 2;  // default split depth (zeta_search_opts.split_depth)
 constexpr int POLL_EVERY = 64;
 
@@ -160,7 +162,8 @@ enum { C_TT_PROBE = 0, C_TT_HIT, C_TT_CUT, C_TT_STORE, C_DEFER, C_MAXPLY, C_MLP_
 // a parent board is recovered with undo() when a child returns.
 struct Ply {
   u64 cr, hash, phash;
-  s32 alpha, beta, depth;
+  s32 alpha, beta;
+  int16_t depth, ralpha;
   u32 move, best, lastmove;
   u16 mbeg, mcnt;
   u8 stm, hmc, qs, kic, iter, ndefer, busy, searched;
@@ -216,6 +219,7 @@ struct Node {  // the current node (wave-uniform)
   bool qs, kic;
   int iter, ndefer, searched;
   bool busy;
+  s32 ralpha;  // the alpha that the REFUTED flags of the move list were set for
 };
 
 __device__ __forceinline__ void save(Ply &y, const Node &n) {
@@ -224,7 +228,8 @@ __device__ __forceinline__ void save(Ply &y, const Node &n) {
   y.phash = n.phash;
   y.alpha = n.alpha;
   y.beta = n.beta;
-  y.depth = n.depth;
+  y.depth = (int16_t)n.depth;
+  y.ralpha = (int16_t)n.ralpha;
   y.move = n.move;
   y.best = n.best;
   y.lastmove = n.lastmove;
@@ -245,7 +250,8 @@ __device__ __forceinline__ void restore(const Ply &y, const Pos &child, Node &n)
   n.phash = uf(y.phash);
   n.alpha = uf(y.alpha);
   n.beta = uf(y.beta);
-  n.depth = uf(y.depth);
+  n.depth = uf((s32)y.depth);
+  n.ralpha = uf((s32)y.ralpha);
   n.move = uf(y.move);
   n.best = uf(y.best);
   n.lastmove = uf(y.lastmove);
@@ -498,7 +504,7 @@ __device__ void log_pairs(const SearchArgs &a, const Node &n, int lane, const u3
     bool neg = false;
     u32 m = 0;
     if (k < n.mcnt) {
-      m = mmove[n.mbeg + k] & ~DEFERRED;
+      m = mmove[n.mbeg + k] & MOVE_BITS;
       neg = m != n.move && m != ttm;
     }
     const u64 mask = __ballot(neg);
@@ -766,6 +772,37 @@ __device__ void serve_leave(const SearchArgs &a, int r, u64 tk, bool aborted, bo
   }
 }
 
+// The moves of a node whose children are quiescence nodes (depth <= 1) that
+// the child's stand pat refutes: the child is not in check, is not extended,
+// is no draw, and its static evaluation is at or above its beta (-alpha here),
+// so searching it returns that evaluation and changes nothing at this node but
+// the node count.  Lane = move: 64 children are made and evaluated together
+// (the piece-square sum by the move's change of it, the pawn terms and the
+// check test set by set), where each alone costs the wavefront a pass through
+// ENTER and RETURN.  alpha only rises while a node is searched, so a flag set
+// for one alpha holds for every later one; after a rise the rest is tested
+// again.  The flagged moves are counted off in move order by NEXT.
+__device__ void mark_refuted(const Node &n, int lane, u32 *mmove, const int16_t *mscore) {
+  const u64 occ = n.p.b1 | n.p.b2 | n.p.b3;
+  const u64 kings = n.p.b1 & n.p.b2 & ~n.p.b3;
+  const u64 kb = kings & (n.p.stm ? (n.p.b0 ^ occ) : n.p.b0);  // the opponent's king, to move in every child
+  const int k2 = kb ? lsb(kb) : 0;
+  const u32 pc = piece_at(n.p, lane);
+  const s32 base = wave_sum_i(((pc >> 1) & 7) != PNONE ? eval_piece(pc, lane) : 0);
+  const s32 limit = -n.alpha;  // the children's beta
+  for (int k = lane; k < n.mcnt; k += 64) {
+    const u32 mf = mmove[n.mbeg + k];
+    if (mscore[n.mbeg + k] == (int16_t)USED || (mf & (DEFERRED | REFUTED))) continue;
+    const Pos c = apply(n.p, mf, false);
+    const u64 cocc = c.b1 | c.b2 | c.b3;
+    const s32 e = base + eval_move_delta(mf) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ cocc, c.b0) + eval_bishop_pair(c);
+    const s32 ev = n.p.stm ? e : -e;  // for the side to move in the child
+    const bool ext = !n.qs && is_promo(mf);
+    if (ev >= limit && !ext && child_hmc(n.hmc, mf) < 100 && popc(cocc) > 2 && !king_attacked(c, k2, kb))
+      mmove[n.mbeg + k] = mf | REFUTED;
+  }
+}
+
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_search(SearchArgs a) {
   __shared__ Ply ply[MAXPLY + 2];
   __shared__ u32 mmove[MSTACK];
@@ -879,6 +916,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       n.iter = 1;
       n.ndefer = 0;
       n.searched = 0;
+      n.ralpha = -INF;
       int sd = 1;
       bool parent_qs = false;
       s32 rootscore = 0;  // DRAWSCORE until a root move raises alpha (src/zeta.cl:986)
@@ -944,6 +982,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.iter = 1;
           n.ndefer = 0;
           n.searched = 0;
+          n.ralpha = -INF;
           n.mcnt = 0;
           s32 ev0 = 0;
           bool have_ev = false;
@@ -1138,17 +1177,69 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 
         if (state == S_NEXT) {
           // ---------------- NEXT: pick the best remaining move (wave arg-max)
-          u32 bestkey = 0;
+          // a node whose children are quiescence nodes: first flag the moves
+          // that a child's stand pat refutes (the pawn sums want no pawn on
+          // the outer ranks; a child at MAXPLY is counted, so made)
+          const bool leafward = n.depth <= 1 && sd + 1 < MAXPLY;
+          if (leafward && n.alpha > n.ralpha && !(n.p.b1 & ~n.p.b2 & ~n.p.b3 & 0xFF000000000000FFULL)) {
+            mark_refuted(n, lane, mmove, mscore);
+            n.ralpha = n.alpha;
+          }
+          u32 bestkey = 0, topkey = 0;  // the best move to search, the best of all (flagged ones included)
           for (int k = lane; k < n.mcnt; k += 64) {
             const s32 sc = mscore[n.mbeg + k];
-            const bool fl = (mmove[n.mbeg + k] & DEFERRED) != 0u;
+            const u32 mf = mmove[n.mbeg + k];
+            const bool fl = (mf & DEFERRED) != 0u;
             const bool ok = sc != USED && (n.iter == 1 ? !fl : fl);
             if (ok) {
               const u32 key = ((u32)(sc + 32768) << 16) | (0xFFFFu - (u32)k);
-              bestkey = key > bestkey ? key : bestkey;
+              topkey = key > topkey ? key : topkey;
+              if (!(mf & REFUTED)) bestkey = key > bestkey ? key : bestkey;
             }
           }
           bestkey = wave_max_u32(bestkey);
+          if (leafward) {
+            // flagged moves ahead of the best: visited here, as their order
+            // has it, by counting them
+            int c = 0;
+            for (int k0 = 0; k0 < n.mcnt; k0 += 64) {
+              const int k = k0 + lane;
+              bool ahead = false;
+              if (k < n.mcnt) {
+                const s32 sc = mscore[n.mbeg + k];
+                ahead = sc != USED && (mmove[n.mbeg + k] & REFUTED) &&
+                        (((u32)(sc + 32768) << 16) | (0xFFFFu - (u32)k)) > bestkey;
+              }
+              c += popc(__ballot(ahead));
+            }
+            if (c) {
+              u32 upto = bestkey;
+              if (poll + c >= POLL_EVERY) {
+                // a poll falls among them: one at a time up to it, and the
+                // child whose turn it is is entered as any other
+                topkey = wave_max_u32(topkey);
+                if (poll + 1 >= POLL_EVERY) {
+                  bestkey = topkey;
+                  c = 0;
+                } else {
+                  upto = topkey - 1;
+                  c = 1;
+                }
+              }
+              if (c) {
+                for (int k = lane; k < n.mcnt; k += 64) {
+                  const s32 sc = mscore[n.mbeg + k];
+                  if (sc != USED && (mmove[n.mbeg + k] & REFUTED) &&
+                      (((u32)(sc + 32768) << 16) | (0xFFFFu - (u32)k)) > upto)
+                    mscore[n.mbeg + k] = (int16_t)USED;
+                }
+                poll += c;
+                nodes += (u64)c;
+                n.searched += c;
+                if (upto != bestkey) continue;
+              }
+            }
+          }
           if (bestkey == 0) {
             if (n.iter == 1 && n.ndefer > 0) {
               n.iter = 2;
@@ -1160,7 +1251,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             continue;
           }
           const int k = n.mbeg + (int)(0xFFFFu - (bestkey & 0xFFFFu));
-          const u32 m = uf(mmove[k]) & ~DEFERRED;
+          const u32 m = uf(mmove[k]) & MOVE_BITS;
           const s32 sk = (s32)(bestkey >> 16) - 32768;
           wsync();
           if (lane == 0) mscore[k] = (int16_t)USED;
@@ -1224,6 +1315,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           cn.iter = 1;
           cn.ndefer = 0;
           cn.searched = 0;
+          cn.ralpha = -INF;
           n = cn;
           sd++;
           wsync();
