@@ -15,16 +15,18 @@ extern "C" void hs_child(const uint64_t *b, int stm, uint32_t m, int32_t *out) {
   int32_t base = 0;
   for (int sq = 0; sq < 64; sq++) {
     const u32 pc = piece_at(p, sq);
-    if (((pc >> 1) & 7) != PNONE) base += eval_piece(pc, sq);
+    if (((pc >> 1) & 7) != PNONE) base += eval_piece(EVAL_SQ.v, pc, sq);
   }
   const Pos c = apply(p, m, false);
   const u64 occ = c.b1 | c.b2 | c.b3;
-  out[0] = base + eval_move_delta(m) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ occ, c.b0) + eval_bishop_pair(c);
+  out[0] = base + eval_move_delta(EVAL_SQ.v, m) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ occ, c.b0) + eval_bishop_pair(c);
   out[1] = eval_bishop_pair(c);
   for (int sq = 0; sq < 64; sq++) out[1] += eval_square(c, sq);
   const u64 kb = c.b1 & c.b2 & ~c.b3 & (c.stm ? c.b0 : (c.b0 ^ occ));
-  out[2] = king_attacked(c, kb ? lsb(kb) : 0, kb) ? 1 : 0;
+  out[2] = king_attacked(c, sq_lines(kb ? lsb(kb) : 0), kb, c.stm ^ 1u) ? 1 : 0;
   Node0 B;
   node_basics(c, B);
   out[3] = B.checkers ? 1 : 0;
 }
+extern "C" int32_t hs_piece_value(int type) { return piece_value((u32)type); }
+extern "C" int32_t hs_piece_value_table(int type) { return EVAL_VALUE[type]; }

@@ -46,4 +46,5 @@ def _check(H, p):
 
 def test_child_evaluation_and_check(H):
     pos = np.concatenate([R.setboard(f) for f in FENS] + [R.gen_playouts(3, 300, 20, 60), R.gen_playouts(2, 100, 4, 30)])
+    assert [H.hs_piece_value(t) for t in range(7)] == [H.hs_piece_value_table(t) for t in range(7)]
     assert sum(_check(H, pos[i:i + 1]) for i in range(len(pos))) > 100

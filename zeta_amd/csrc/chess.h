@@ -520,17 +520,35 @@ ZD void node_basics(const Pos &p, Node0 &B) {
   B.cmask = cm;
 }
 
-// Is the side to move's king (on square k of bitboard kb, kb = 0 for no king)
-// attacked?  One position per lane, the same k in every lane: the checkers of
+// The lines through a square (the square itself taken out), its bit and the
+// reversed bit: what the slider attacks of one square need besides the
+// occupancy.  The search holds the set of its lane's square in registers.
+struct SqLines {
+  u64 b, rb, rank, file, diag, anti;
+};
+ZD SqLines sq_lines(int sq) {
+  const u64 b = bit(sq);
+  return SqLines{b, rev64(b), rank_line(sq) ^ b, file_line(sq) ^ b, diag_line(sq) ^ b, anti_line(sq) ^ b};
+}
+ZD u64 line_att(const SqLines &q, u64 occ, u64 mask) {  // mask: one of q's lines
+  const u64 o = occ & mask;
+  return ((o - q.b) ^ rev64(rev64(o) - q.rb)) & mask;
+}
+ZD u64 rook_sq(const SqLines &q, u64 occ) { return line_att(q, occ, q.rank) | line_att(q, occ, q.file); }
+ZD u64 bishop_sq(const SqLines &q, u64 occ) { return line_att(q, occ, q.diag) | line_att(q, occ, q.anti); }
+
+// Does the side `by` attack the king of the other side?  kb = the king's
+// bitboard (0 for no king: never), q = the lines of its square.
+// One position per lane, the same king square in every lane: the checkers of
 // node_basics without the check mask.
-ZD bool king_attacked(const Pos &p, int k, u64 kb) {
+ZD bool king_attacked(const Pos &p, const SqLines &q, u64 kb, u32 by) {
   const u64 occ = p.b1 | p.b2 | p.b3;
-  const u64 opp = p.stm ? (p.b0 ^ occ) : p.b0;
+  const u64 them = by ? p.b0 : (p.b0 ^ occ);
   const u64 rq = p.b3 & (p.b1 ^ p.b2), bq = p.b3 & ~p.b1;
-  u64 a = (rook_sq(k, occ) & rq) | (bishop_sq(k, occ) & bq);
+  u64 a = (rook_sq(q, occ) & rq) | (bishop_sq(q, occ) & bq);
   a |= knight_att(kb) & ~p.b1 & p.b2 & ~p.b3;
-  a |= pawn_att(kb, p.stm) & p.b1 & ~p.b2 & ~p.b3;
-  return kb && (a & opp);
+  a |= pawn_att(kb, by ^ 1u) & p.b1 & ~p.b2 & ~p.b3;
+  return kb && (a & them);
 }
 
 // is sq attacked by the opponent, the own king taken off the board?
@@ -671,6 +689,21 @@ ZD Pos apply(const Pos &p, u32 m, bool rook_flag) {
   cr |= RANKS45;
   if (dbl) cr &= ~bit(t);
   c.cr = cr;
+  c.stm = p.stm ^ 1u;
+  return c;
+}
+
+// apply() of a capture (e.p. and promotions included, no castling): the
+// planes and the side to move; the moved flags are the parent's.
+ZD Pos apply_capture(const Pos &p, u32 m) {
+  Pos c = p;
+  const u64 t = bit((int)mv_to(m));
+  const u64 keep = ~(bit((int)mv_from(m)) | bit((int)mv_cpt(m)) | t);
+  const u32 pt = mv_pto(m);
+  c.b0 = (p.b0 & keep) | sel(pt & 1, t);
+  c.b1 = (p.b1 & keep) | sel((pt >> 1) & 1, t);
+  c.b2 = (p.b2 & keep) | sel((pt >> 2) & 1, t);
+  c.b3 = (p.b3 & keep) | sel((pt >> 3) & 1, t);
   c.stm = p.stm ^ 1u;
   return c;
 }

@@ -121,37 +121,43 @@ ZD int32_t pawn_terms(u64 pawns, u64 white, u64 black) {
   return 10 * chain - 15 * block - 30 * pairs;
 }
 
-// material + piece-square + square control of a coloured piece, white positive
-ZD int32_t eval_piece(u32 pc, int sq) {
-  const int v = EVAL_SQ.v[((pc >> 1) & 7) * 64 + ((pc & 1) ? sq : (sq ^ 56))];
+// material + piece-square + square control of a coloured piece, white
+// positive, from a table in EVAL_SQ's layout (the search keeps one in LDS)
+template <class T>
+ZD int32_t eval_piece(const T *tab, u32 pc, int sq) {
+  const int v = (int)tab[((pc >> 1) & 7) * 64 + ((pc & 1) ? sq : (sq ^ 56))];
   return (pc & 1) ? -v : v;
 }
 
 // How a move changes the sum of eval_piece over the board (the castle rook
 // included).
-ZD int32_t eval_move_delta(u32 m) {
+template <class T>
+ZD int32_t eval_move_delta(const T *tab, u32 m) {
   const int f = (int)mv_from(m), t = (int)mv_to(m);
   const u32 pf = mv_pfrom(m), pc = mv_pcpt(m);
-  int32_t d = eval_piece(mv_pto(m), t) - eval_piece(pf, f);
-  if (((pc >> 1) & 7) != PNONE) d -= eval_piece(pc, (int)mv_cpt(m));
+  int32_t d = eval_piece(tab, mv_pto(m), t) - eval_piece(tab, pf, f);
+  d -= eval_piece(tab, pc, (int)mv_cpt(m));  // no piece: the table's first 64 entries are 0
   if (((pf >> 1) & 7) == KING && (f - t == 2 || t - f == 2)) {
     const u32 rook = (ROOK << 1) | (pf & 1);
-    d += f - t == 2 ? eval_piece(rook, (t + 1) & 63) - eval_piece(rook, (f - 4) & 63)
-                    : eval_piece(rook, (t - 1) & 63) - eval_piece(rook, (f + 3) & 63);
+    d += f - t == 2 ? eval_piece(tab, rook, (t + 1) & 63) - eval_piece(tab, rook, (f - 4) & 63)
+                    : eval_piece(tab, rook, (t - 1) & 63) - eval_piece(tab, rook, (f + 3) & 63);
   }
   return d;
 }
 
+// EVAL_VALUE / 100 of the seven piece types as nibbles of a constant: no load
+ZD int32_t piece_value(u32 type) { return (int32_t)((0xC640410u >> (4 * type)) & 15u) * 100; }
+
 // Move-ordering score of the reference picker (src/zeta.cl:2059-2071):
 // captures MVV-LVA (16*V[captured] - V[mover]), quiet moves by the change of
 // material + piece-square + control value.
-ZD int32_t order_score(u32 stm, u32 m) {
-  const int from = (int)mv_from(m), to = (int)mv_to(m);
-  const int tf = (int)((mv_pto(m) >> 1) & 7), ff = (int)((mv_pfrom(m) >> 1) & 7), cf = (int)((mv_pcpt(m) >> 1) & 7);
-  if (cf != PNONE) return EVAL_VALUE[cf] * 16 - EVAL_VALUE[tf];
-  const int t = stm ? to : (to ^ 56), f = stm ? from : (from ^ 56);
-  return EVAL_VALUE[tf] + EVAL_PST[tf * 64 + t] + EVAL_CONTROL[t] - EVAL_VALUE[ff] - EVAL_PST[ff * 64 + f] -
-         EVAL_CONTROL[f];
+// tab: a table in EVAL_SQ's layout, whose constant part cancels.
+template <class T>
+ZD int32_t order_score(const T *tab, u32 stm, u32 m) {
+  const u32 tf = (mv_pto(m) >> 1) & 7, ff = (mv_pfrom(m) >> 1) & 7, cf = (mv_pcpt(m) >> 1) & 7;
+  if (cf != PNONE) return piece_value(cf) * 16 - piece_value(tf);
+  const u32 flip = stm ? 0 : 56;
+  return (int32_t)tab[tf * 64 + (mv_to(m) ^ flip)] - (int32_t)tab[ff * 64 + (mv_from(m) ^ flip)];
 }
 
 }  // namespace zc

@@ -46,7 +46,14 @@ constexpr int MAXPLY = 64;  // src/types.h:76
 constexpr s32 INF = 32000;
 constexpr s32 MATESCORE = 30000;
 constexpr int MSTACK = 1024;  // move-stack slots per worker (LDS)
-constexpr s32 USED = -32768;  // 16-bit move-ordering scores
+constexpr int MPAD = 48;      // slots past them for captures not yet tested for legality
+// A move-list entry is a move code and a key: the ordering score + 32768 in the
+// upper half (0: the move was searched), in the lower half what is known of
+// the child, if it is a quiescence node: KEY_CHECK, KEY_OPEN, or its static
+// evaluation for the side to move + 32768.
+constexpr u32 KEY_CHECK = 0;  // in check
+constexpr u32 KEY_OPEN = 1;   // nothing known
+__device__ __forceinline__ u32 move_key(s32 score, u32 child) { return ((u32)(score + 32768) << 16) | child; }
 constexpr s32 TTMOVE_SCORE = 32000;  // above every other score (src/zeta.cl:2101)
 constexpr s32 HINT_SCORE = 32100;    // the hint table's move, above the TT move
 // the killer (one per ply) and the counter move (indexed by the previous
@@ -55,7 +62,6 @@ constexpr s32 KILLER_SCORE = 1400;
 constexpr s32 COUNTER_SCORE = 1300;
 constexpr int NCOUNTER = 64 * 64;  // counter-move table entries per worker (LDS)
 constexpr u32 DEFERRED = 0x80000000u;  // move-stack flag: deferred by ABDADA (move codes use bits 0-29)
-constexpr u32 REFUTED = 0x40000000u;   // move-stack flag: the child's stand pat refutes the move (mark_refuted)
 constexpr u32 MOVE_BITS = 0x3FFFFFFFu;
 constexpr int ABDADA_MIN_DEPTH = 2;  // default split depth (zeta_search_opts.split_depth)
 constexpr int POLL_EVERY = 64;
@@ -153,6 +159,25 @@ struct SearchArgs {
   u64 watchdog_ticks; // wall-clock ticks without a heartbeat before the grid exits (0 = never)
 };
 
+// The kernel's arguments, read from the kernarg segment where they are used:
+// held in registers through the search they take 120 of the 102 scalar
+// registers a wavefront has, and the compiler then keeps them in vector lanes
+// (270 spilled registers in k_search, a v_readlane at every use).  The empty
+// asm hides where the pointer comes from, so that a load stays behind it.
+typedef const __attribute__((address_space(4))) SearchArgs *Args;
+__device__ __forceinline__ Args args() {
+  Args p = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// a pointer read from the arguments, known to point to device memory (an
+// address the compiler cannot place costs the slower flat access)
+template <class T>
+__device__ __forceinline__ T *glob(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)p;
+}
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -163,7 +188,8 @@ enum { C_TT_PROBE = 0, C_TT_HIT, C_TT_CUT, C_TT_STORE, C_DEFER, C_MAXPLY, C_MLP_
 struct Ply {
   u64 cr, hash, phash;
   s32 alpha, beta;
-  int16_t depth, ralpha;
+  int16_t depth;
+  u16 keyed;
   u32 move, best, lastmove;
   u16 mbeg, mcnt;
   u8 stm, hmc, qs, kic, iter, ndefer, busy, searched;
@@ -219,7 +245,7 @@ struct Node {  // the current node (wave-uniform)
   bool qs, kic;
   int iter, ndefer, searched;
   bool busy;
-  s32 ralpha;  // the alpha that the REFUTED flags of the move list were set for
+  bool keyed;  // the move keys hold what is known of the children (key_children)
 };
 
 __device__ __forceinline__ void save(Ply &y, const Node &n) {
@@ -229,7 +255,7 @@ __device__ __forceinline__ void save(Ply &y, const Node &n) {
   y.alpha = n.alpha;
   y.beta = n.beta;
   y.depth = (int16_t)n.depth;
-  y.ralpha = (int16_t)n.ralpha;
+  y.keyed = n.keyed;
   y.move = n.move;
   y.best = n.best;
   y.lastmove = n.lastmove;
@@ -251,7 +277,7 @@ __device__ __forceinline__ void restore(const Ply &y, const Pos &child, Node &n)
   n.alpha = uf(y.alpha);
   n.beta = uf(y.beta);
   n.depth = uf((s32)y.depth);
-  n.ralpha = uf((s32)y.ralpha);
+  n.keyed = uf((u32)y.keyed) != 0;
   n.move = uf(y.move);
   n.best = uf(y.best);
   n.lastmove = uf(y.lastmove);
@@ -297,7 +323,7 @@ __device__ __forceinline__ u32 child_hmc(u32 hmc, u32 m) {
   return (hmc + 1) & 0xFF;
 }
 
-enum { S_ENTER = 0, S_NEXT = 1, S_RETURN = 2 };
+enum { S_ENTER = 0, S_NEXT = 1, S_RETURN = 2, S_QS = 3 };
 
 // TT store when a full-width node returns: with a move that raised alpha, a
 // lower bound of the node's value and that move; with none (every move
@@ -306,8 +332,8 @@ enum { S_ENTER = 0, S_NEXT = 1, S_RETURN = 2 };
 // depth-limited subtree, which a node with a zero half-move clock cannot see
 // depend on the path above it: entries are used at the same depth and clock
 // only, so no root value depends on them.
-__device__ __forceinline__ u32 tt_store(const SearchArgs &a, const Node &n, int sd, int lane) {
-  if (!a.ttmask || n.qs || n.depth < 1) return 0;
+__device__ __forceinline__ u32 tt_store(Args a, const Node &n, int sd, int lane) {
+  if (!a->ttmask || n.qs || n.depth < 1) return 0;
   s32 s = n.alpha;
   const int plyn = sd - 1;
   if (is_mate(s) && s > 0) s += plyn;
@@ -322,7 +348,7 @@ __device__ __forceinline__ u32 tt_store(const SearchArgs &a, const Node &n, int 
     e.y = (u32)(w0 >> 32);
     e.z = (u32)w1;
     e.w = (u32)(w1 >> 32);
-    *(u32x4 *)(a.tt + 2 * (key & a.ttmask)) = e;  // one 16-byte vector store
+    *glob((u32x4 *)(a->tt + 2 * (key & a->ttmask))) = e;  // one 16-byte vector store
   }
   return 1;
 }
@@ -335,35 +361,35 @@ __device__ __forceinline__ u32 tt_store(const SearchArgs &a, const Node &n, int 
 __device__ __forceinline__ u16 counter_code(u32 m) { return (u16)((m & 0xFFFu) | (mv_pfrom(m) << 12)); }
 __device__ __forceinline__ int counter_index(u32 prev) { return (int)(mv_from(prev) * 64 + mv_to(prev)); }
 
-__device__ __forceinline__ void busy_release(const SearchArgs &a, u64 hash, u64 cr, int lane) {
-  const u32 bidx = (u32)(tt_key(hash, cr) >> 40) & a.busymask;
-  if (lane == 0) atomicSub(&a.busy[bidx], 1u);
+__device__ __forceinline__ void busy_release(Args a, u64 hash, u64 cr, int lane) {
+  const u32 bidx = (u32)(tt_key(hash, cr) >> 40) & a->busymask;
+  if (lane == 0) atomicSub(&a->busy[bidx], 1u);
 }
 
 // next root for this worker: the queue first, then the unfinished root with
-// the fewest workers (ABDADA helper), at most a.workers per root
+// the fewest workers (ABDADA helper), at most a->workers per root
 // A worker takes the next unstarted root; once all have started it joins,
 // as an ABDADA helper below the per-root limit, the unfinished root with the
 // fewest completed iterations (the most work left: an iteration costs
 // several times the one before it), then the fewest workers.  The wave's
 // lanes scan the roots together and agree on the minimum.
-__device__ int pick_root(const SearchArgs &a, int hstart, int lane) {
+__device__ int pick_root(Args a, int hstart, int lane) {
   int r = 0;
-  if (lane == 0) r = atomicAdd(a.queue, 1);
+  if (lane == 0) r = atomicAdd(a->queue, 1);
   r = uf(r);
-  if (r < a.nroots) {
-    if (lane == 0) atomicAdd(&a.nworkers[r], 1);
+  if (r < a->nroots) {
+    if (lane == 0) atomicAdd(&a->nworkers[r], 1);
     return r;
   }
-  if (a.workers <= 1) return -1;
+  if (a->workers <= 1) return -1;
   for (int attempt = 0; attempt < 8; attempt++) {
     u64 best = ~0ULL;  // (iterations done << 48) | (workers << 32) | root
-    for (int k = lane; k < a.nroots; k += 64) {
-      const int rr = (hstart + k) % a.nroots;
-      if (__atomic_load_n(&a.done[rr], __ATOMIC_RELAXED)) continue;
-      const int w = __atomic_load_n(&a.nworkers[rr], __ATOMIC_RELAXED);
-      if (w >= a.workers) continue;
-      const int dd = __atomic_load_n(&a.depth_done[rr], __ATOMIC_RELAXED);
+    for (int k = lane; k < a->nroots; k += 64) {
+      const int rr = (hstart + k) % a->nroots;
+      if (__atomic_load_n(&a->done[rr], __ATOMIC_RELAXED)) continue;
+      const int w = __atomic_load_n(&a->nworkers[rr], __ATOMIC_RELAXED);
+      if (w >= a->workers) continue;
+      const int dd = __atomic_load_n(&a->depth_done[rr], __ATOMIC_RELAXED);
       const u64 key = ((u64)(dd < 0 ? 0 : (dd > 255 ? 255 : dd)) << 48) | ((u64)(u32)w << 32) | (u32)rr;
       best = key < best ? key : best;
     }
@@ -378,8 +404,8 @@ __device__ int pick_root(const SearchArgs &a, int hstart, int lane) {
     const int pick = (int)(u32)best;
     int got = 0;
     if (lane == 0) {
-      got = atomicAdd(&a.nworkers[pick], 1) < a.workers ? 1 : 0;
-      if (!got) atomicSub(&a.nworkers[pick], 1);
+      got = atomicAdd(&a->nworkers[pick], 1) < a->workers ? 1 : 0;
+      if (!got) atomicSub(&a->nworkers[pick], 1);
     }
     if (uf(got)) return pick;
   }
@@ -397,22 +423,23 @@ __device__ __forceinline__ void add_row(float x[8], const u16 *row) {
 }
 
 // Learned ordering: network score of every move of the node (moves
-// [mbeg, mbeg+total) in LDS) written into mscore.  Layer 1's position part is
+// [mbeg, mbeg+total) in LDS) written into mscore as integers.  Layer 1's position part is
 // accumulated once (lane = 4 hidden units); each chunk of 32 moves then runs
 // layer 2 as 16 MFMA steps whose A operand (move x 8 hidden units, BF16) is
 // built in registers from the position part plus the move's 3-4 feature rows.
-__device__ void mlp_score_moves(const SearchArgs &a, const Pos &p, int mbeg, int total, int lane, float *hpos,
-                                const u32 *mmove, int16_t *mscore) {
-  const zm::Weights &w = a.w;
+__device__ void mlp_score_moves(Args a, const Pos &p, int mbeg, int total, int lane, float *hpos,
+                                const u32 *mmove, u32 *mscore) {
+  const u16 *const w1f = a->w.w1f, *const w2t = a->w.w2t;
+  const float *const wb1 = a->w.b1;
   float h4[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) h4[j] = w.b1[lane * 4 + j];
+  for (int j = 0; j < 4; j++) h4[j] = wb1[lane * 4 + j];
   u64 occ = p.b1 | p.b2 | p.b3;
   while (occ) {
     const int sq = lsb(occ);
     occ &= occ - 1;
     const int f = zm::feat_ps(piece_at(p, sq), sq, p.stm);
-    const uint2 q = *(const uint2 *)(w.w1f + (size_t)f * zm::NH1 + lane * 4);
+    const uint2 q = *(const uint2 *)(w1f + (size_t)f * zm::NH1 + lane * 4);
     h4[0] += zm::bf2f((u16)(q.x & 0xFFFF));
     h4[1] += zm::bf2f((u16)(q.x >> 16));
     h4[2] += zm::bf2f((u16)(q.y & 0xFFFF));
@@ -422,7 +449,7 @@ __device__ void mlp_score_moves(const SearchArgs &a, const Pos &p, int mbeg, int
   for (int j = 0; j < 4; j++) hpos[lane * 4 + j] = h4[j];
   wsync();
   const int col = lane & 31, half = lane >> 5;
-  const float b2o = w.b2[col], w3o = w.w3[col], b3 = w.b3[0];
+  const float b2o = a->w.b2[col], w3o = a->w.w3[col], b3 = a->w.b3[0];
   for (int c0 = 0; c0 < total; c0 += 32) {
     const int mi = c0 + col;
     const u32 m = mi < total ? mmove[mbeg + mi] : 0u;
@@ -435,10 +462,10 @@ __device__ void mlp_score_moves(const SearchArgs &a, const Pos &p, int mbeg, int
 #pragma unroll
       for (int j = 0; j < 8; j++) x[j] = hpos[kb + j];
       if (m) {
-        add_row(x, w.w1f + (size_t)ff * zm::NH1 + kb);
-        add_row(x, w.w1f + (size_t)ft * zm::NH1 + kb);
-        add_row(x, w.w1f + (size_t)fp * zm::NH1 + kb);
-        if (fc >= 0) add_row(x, w.w1f + (size_t)fc * zm::NH1 + kb);
+        add_row(x, w1f + (size_t)ff * zm::NH1 + kb);
+        add_row(x, w1f + (size_t)ft * zm::NH1 + kb);
+        add_row(x, w1f + (size_t)fp * zm::NH1 + kb);
+        if (fc >= 0) add_row(x, w1f + (size_t)fc * zm::NH1 + kb);
       }
       bf16x8 av;
 #pragma unroll
@@ -446,7 +473,7 @@ __device__ void mlp_score_moves(const SearchArgs &a, const Pos &p, int mbeg, int
         const u16 hb = zm::f2bf(x[j] > 0.f ? x[j] : 0.f);
         av[j] = __builtin_bit_cast(__bf16, hb);
       }
-      const bf16x8 bv = *(const bf16x8 *)(w.w2t + (size_t)col * zm::NH1 + kb);
+      const bf16x8 bv = *(const bf16x8 *)(w2t + (size_t)col * zm::NH1 + kb);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
     }
     // layer 3: register i of lane l holds z2[move 8*(i/4)+4*half+i%4][unit col]
@@ -467,7 +494,7 @@ __device__ void mlp_score_moves(const SearchArgs &a, const Pos &p, int mbeg, int
         if (c0 + row < total) {
           float sc = (t[i] + b3) * 256.f;
           sc = sc > 31000.f ? 31000.f : (sc < -31000.f ? -31000.f : sc);
-          mscore[mbeg + c0 + row] = (int16_t)__float2int_rn(sc);
+          mscore[mbeg + c0 + row] = (u32)__float2int_rn(sc);
         }
       }
     }
@@ -477,8 +504,9 @@ __device__ void mlp_score_moves(const SearchArgs &a, const Pos &p, int mbeg, int
 
 // the plain ordering's score of a move (src/zeta.cl:2059-2082): MVV-LVA or
 // the piece-square delta, the killer's 1400 and the counter move's 1300
-__device__ __forceinline__ s32 plain_score(u32 stm, u32 m, u32 killer, u32 counter) {
-  s32 sc = order_score(stm, m);
+template <class T>
+__device__ __forceinline__ s32 plain_score(const T *tab, u32 stm, u32 m, u32 killer, u32 counter) {
+  s32 sc = order_score(tab, stm, m);
   sc = sc > 31999 ? 31999 : (sc < -31999 ? -31999 : sc);
   if (((mv_pcpt(m) >> 1) & 7) == PNONE) {
     if (m == killer) sc = KILLER_SCORE;
@@ -490,15 +518,14 @@ __device__ __forceinline__ s32 plain_score(u32 stm, u32 m, u32 killer, u32 count
 // Training pairs at a cut node of the full-width search whose cutoff move is
 // not the TT move (the TT move goes first whatever the network says): the
 // cutoff move against every other move of the node -- those searched before
-// it, which failed (scores marked USED), and those never searched, which the
+// it, which failed, and those never searched, which the
 // plain ordering ranked below it.  Each pair carries the plain ordering's
 // score difference (negative minus positive), which the ranking loss adds to
 // the network's, so that the network learns what to add to the plain
 // ordering.  Wave-compacted.
-__device__ void log_pairs(const SearchArgs &a, const Node &n, int lane, const u32 *mmove, const int16_t *mscore,
-                          u32 ttm, u32 killer, u32 counter, u32 &nrec) {
+__device__ void log_pairs(Args a, const Node &n, int lane, const u32 *mmove, const int16_t *tab, u32 ttm, u32 killer, u32 counter, u32 &nrec) {
   if (n.move == ttm) return;
-  const s32 ppos = plain_score(n.p.stm, n.move, killer, counter);
+  const s32 ppos = plain_score(tab, n.p.stm, n.move, killer, counter);
   for (int c0 = 0; c0 < n.mcnt; c0 += 64) {
     const int k = c0 + lane;
     bool neg = false;
@@ -511,14 +538,14 @@ __device__ void log_pairs(const SearchArgs &a, const Node &n, int lane, const u3
     if (!mask) continue;
     const u32 cnt = (u32)popc(mask);
     u64 base = 0;
-    if (lane == 0) base = atomicAdd((unsigned long long *)a.rec_count, (unsigned long long)cnt);
+    if (lane == 0) base = atomicAdd((unsigned long long *)a->rec_count, (unsigned long long)cnt);
     base = uf(base);
     if (neg) {
       const u64 slot = base + (u64)popc(mask & ((1ULL << lane) - 1));
-      if (slot < a.rec_cap) {
-        s32 dp = plain_score(n.p.stm, m, killer, counter) - ppos;
+      if (slot < a->rec_cap) {
+        s32 dp = plain_score(tab, n.p.stm, m, killer, counter) - ppos;
         dp = dp > zm::PAIR_OFFSET_MAX ? zm::PAIR_OFFSET_MAX : (dp < -zm::PAIR_OFFSET_MAX ? -zm::PAIR_OFFSET_MAX : dp);
-        u64 *rp = a.recs + slot * 6;
+        u64 *rp = a->recs + slot * 6;
         rp[0] = n.p.b0;
         rp[1] = n.p.b1;
         rp[2] = n.p.b2;
@@ -599,22 +626,22 @@ __device__ __forceinline__ u32 xcc_id() {
 // microseconds it mirrors the host words (ticket count, shutdown, cancel
 // generation) into device memory, so that the workers poll device memory
 // only, and it runs the watchdog on its own clock.
-__device__ void serve_scheduler(const SearchArgs &a, int lane) {
-  ServeDev *v = a.sv;
+__device__ void serve_scheduler(Args a, int lane) {
+  ServeDev *v = a->sv;
   u64 hb_seen = 0, hb_time = 0;
   u32 cg_seen = 0;
   for (;;) {
     u32 shut = 0, cg = 0;
     if (lane == 0) {
       const u64 now = wall_clock64();
-      const u64 sub = sys_load64(&a.sh->submitted);
-      const u64 hb = sys_load64(&a.sh->heartbeat);
-      shut = sys_load32(&a.sh->shutdown) ? 1u : 0u;
-      cg = sys_load32(&a.sh->cancel_gen);
+      const u64 sub = sys_load64(&a->sh->submitted);
+      const u64 hb = sys_load64(&a->sh->heartbeat);
+      shut = sys_load32(&a->sh->shutdown) ? 1u : 0u;
+      cg = sys_load32(&a->sh->cancel_gen);
       if (hb != hb_seen || hb_time == 0) {
         hb_seen = hb;
         hb_time = now;
-      } else if (a.watchdog_ticks && now - hb_time > a.watchdog_ticks) {
+      } else if (a->watchdog_ticks && now - hb_time > a->watchdog_ticks) {
         shut = 2;
         ag_store(&v->exit_now, now);
         ag_store(&v->exit_arg, hb_time);
@@ -624,7 +651,7 @@ __device__ void serve_scheduler(const SearchArgs &a, int lane) {
     }
     cg = uf(cg);
     if (cg != cg_seen) {
-      for (int s = lane; s < a.nslots; s += 64) ag_store(&a.dcancel[s], sys_load64(&a.scancel[s]));
+      for (int s = lane; s < a->nslots; s += 64) ag_store(&a->dcancel[s], sys_load64(&a->scancel[s]));
       cg_seen = cg;
     }
     shut = uf(shut);
@@ -638,39 +665,39 @@ __device__ void serve_scheduler(const SearchArgs &a, int lane) {
 
 // serving: claim the next published ticket, else join the running request
 // with the fewest workers; returns its slot and ticket+1, or -1 on shutdown
-__device__ int serve_pick(const SearchArgs &a, int lane, u64 &tk_out) {
+__device__ int serve_pick(Args a, int lane, u64 &tk_out) {
   int backoff = 1;
   for (;;) {
     int res = -2;
     u64 tk = 0;
     if (lane == 0) {
-      if (ag_load(&a.sv->shut)) {
+      if (ag_load(&a->sv->shut)) {
         res = -1;
       } else {
-        const u64 c = ag_load(&a.sv->claimed);
-        if (c < ag_load(&a.sv->sub) && ag_cas(&a.sv->claimed, c, c + 1)) {
-          const int qi = (int)(c % (u64)a.qcap);
-          const u64 s = sys_load64(&a.squeue[qi]);
-          if (s >= (u64)a.nslots) {
-            ag_store(&a.sv->exit_now, c);
-            ag_store(&a.sv->exit_arg, s);
-            ag_store(&a.sv->shut, 3u);  // the host broke the protocol: stop serving
+        const u64 c = ag_load(&a->sv->claimed);
+        if (c < ag_load(&a->sv->sub) && ag_cas(&a->sv->claimed, c, c + 1)) {
+          const int qi = (int)(c % (u64)a->qcap);
+          const u64 s = sys_load64(&a->squeue[qi]);
+          if (s >= (u64)a->nslots) {
+            ag_store(&a->sv->exit_now, c);
+            ag_store(&a->sv->exit_arg, s);
+            ag_store(&a->sv->shut, 3u);  // the host broke the protocol: stop serving
             res = -1;
           } else {
-            ServeReq &d = a.dreq[s];
-            const ServeReq &h = a.slots[s].req;
+            ServeReq &d = a->dreq[s];
+            const ServeReq &h = a->slots[s].req;
             for (int k = 0; k < 8; k++) ag_store(&d.pos[k], sys_load64(&h.pos[k]));
             const s32 hw = (s32)sys_load32((const u32 *)&h.workers);
             ag_store(&d.depth, (s32)sys_load32((const u32 *)&h.depth));
             ag_store(&d.flags, (s32)sys_load32((const u32 *)&h.flags));
             ag_store(&d.workers, hw);
-            sys_store(&a.sack[qi], c + 1);
-            ag_store(&a.nodes[s], slot_tag(c + 1) << 48);
-            ag_store(&a.depth_done[s], (s32)(u32)(slot_tag(c + 1) << 16));
+            sys_store(&a->sack[qi], c + 1);
+            ag_store(&a->nodes[s], slot_tag(c + 1) << 48);
+            ag_store(&a->depth_done[s], (s32)(u32)(slot_tag(c + 1) << 16));
             const u64 wmax = (u64)(hw < 1 ? 1 : (hw > 255 ? 255 : hw));
             // release: the request copy above is visible to every helper
             // that joins through this word (one write-back per request)
-            __hip_atomic_store(&a.sw[s], (u64)(((c + 1) << 24) | (wmax << 16) | (u64)4 | (u64)SV_RUN),
+            __hip_atomic_store(&a->sw[s], (u64)(((c + 1) << 24) | (wmax << 16) | (u64)4 | (u64)SV_RUN),
                                __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
             res = (int)s;
             tk = c + 1;
@@ -685,14 +712,14 @@ __device__ int serve_pick(const SearchArgs &a, int lane, u64 &tk_out) {
     }
     // no new request: the running request with the fewest workers below its maximum
     u32 bestkey = 0;
-    for (int base = 0; base < a.nslots; base += 64) {
+    for (int base = 0; base < a->nslots; base += 64) {
       const int s = base + lane;
-      if (s < a.nslots) {
-        const u64 v = ag_load(&a.sw[s]);
+      if (s < a->nslots) {
+        const u64 v = ag_load(&a->sw[s]);
         const int w = sw_w(v);
         // a cancelled request takes no new helpers: its workers drain and the
         // last one publishes the cancellation
-        if (sw_tk(v) && sw_st(v) == SV_RUN && w >= 1 && w < sw_max(v) && ag_load(&a.dcancel[s]) != sw_tk(v))
+        if (sw_tk(v) && sw_st(v) == SV_RUN && w >= 1 && w < sw_max(v) && ag_load(&a->dcancel[s]) != sw_tk(v))
           bestkey = max(bestkey, ((u32)(255 - w) << 16) | (u32)(0xFFFF - s));
       }
     }
@@ -701,11 +728,11 @@ __device__ int serve_pick(const SearchArgs &a, int lane, u64 &tk_out) {
       const int s = 0xFFFF - (int)(bestkey & 0xFFFF);
       int got = -1;
       if (lane == 0) {
-        const u64 v = ag_load(&a.sw[s]);
+        const u64 v = ag_load(&a->sw[s]);
         u64 e = v;
         if (sw_tk(v) && sw_st(v) == SV_RUN && sw_w(v) >= 1 && sw_w(v) < sw_max(v) &&
-            ag_load(&a.dcancel[s]) != sw_tk(v) &&
-            __hip_atomic_compare_exchange_strong(&a.sw[s], &e, v + 4, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
+            ag_load(&a->dcancel[s]) != sw_tk(v) &&
+            __hip_atomic_compare_exchange_strong(&a->sw[s], &e, v + 4, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT)) {  // acquire: once per join
           got = s;
           tk = sw_tk(v);
@@ -726,9 +753,9 @@ __device__ int serve_pick(const SearchArgs &a, int lane, u64 &tk_out) {
 }
 
 // serving: abort test at the periodic poll
-__device__ __forceinline__ bool serve_abort(const SearchArgs &a, int r, u64 tk) {
-  const u64 v = ag_load(&a.sw[r]);
-  return sw_tk(v) != tk || sw_st(v) != SV_RUN || ag_load(&a.dcancel[r]) == tk || ag_load(&a.sv->shut) != 0;
+__device__ __forceinline__ bool serve_abort(Args a, int r, u64 tk) {
+  const u64 v = ag_load(&a->sw[r]);
+  return sw_tk(v) != tk || sw_st(v) != SV_RUN || ag_load(&a->dcancel[r]) == tk || ag_load(&a->sv->shut) != 0;
 }
 
 // serving: leave the request.  The worker that completes it (or fails it)
@@ -737,10 +764,10 @@ __device__ __forceinline__ bool serve_abort(const SearchArgs &a, int r, u64 tk) 
 // publishes the result to the host slot -- DONE or FAILED as set, or
 // CANCELLED when every worker left a running request -- so the published
 // node count includes every worker's nodes.
-__device__ void serve_leave(const SearchArgs &a, int r, u64 tk, bool aborted, bool failed, s32 score, u32 move) {
-  if (!aborted && !failed) ag_store(&a.dres[r], (u64)(u32)score | ((u64)move << 32));
+__device__ void serve_leave(Args a, int r, u64 tk, bool aborted, bool failed, s32 score, u32 move) {
+  if (!aborted && !failed) ag_store(&a->dres[r], (u64)(u32)score | ((u64)move << 32));
   for (;;) {
-    const u64 v = ag_load(&a.sw[r]);
+    const u64 v = ag_load(&a->sw[r]);
     if (sw_tk(v) != tk) return;  // the slot has moved on
     int st = sw_st(v);
     if (st == SV_RUN) {
@@ -752,18 +779,18 @@ __device__ void serve_leave(const SearchArgs &a, int r, u64 tk, bool aborted, bo
     // release: the result recorded above before the status that announces
     // it; acquire: the last worker sees the result the completing one wrote
     u64 e = v;
-    if (!__hip_atomic_compare_exchange_strong(&a.sw[r], &e, nv, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
+    if (!__hip_atomic_compare_exchange_strong(&a->sw[r], &e, nv, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT))
       continue;
     if (last) {
       const int pub = st == SV_RUN ? SV_CANCELLED : st;
-      const u64 res = pub == SV_DONE ? ag_load(&a.dres[r]) : 0ULL;
-      ServeSlot &sl = a.slots[r];
+      const u64 res = pub == SV_DONE ? ag_load(&a->dres[r]) : 0ULL;
+      ServeSlot &sl = a->slots[r];
       sys_store(&sl.score, (s32)(u32)res);
       sys_store(&sl.bestmove, (u32)(res >> 32));
-      sys_store(&sl.nodes, (u64)(ag_load(&a.nodes[r]) & 0xFFFFFFFFFFFFULL));
+      sys_store(&sl.nodes, (u64)(ag_load(&a->nodes[r]) & 0xFFFFFFFFFFFFULL));
       sys_store(&sl.ticket, tk);
-      sys_store(&sl.depth_done, (s32)(ag_load(&a.depth_done[r]) & 0xFFFF));
+      sys_store(&sl.depth_done, (s32)(ag_load(&a->depth_done[r]) & 0xFFFF));
       sys_store(&sl.status, (s32)pub);
       // the one ordering point: the result fields before the done flag
       __hip_atomic_store(&sl.state, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -772,49 +799,417 @@ __device__ void serve_leave(const SearchArgs &a, int r, u64 tk, bool aborted, bo
   }
 }
 
-// The moves of a node whose children are quiescence nodes (depth <= 1) that
-// the child's stand pat refutes: the child is not in check, is not extended,
-// is no draw, and its static evaluation is at or above its beta (-alpha here),
-// so searching it returns that evaluation and changes nothing at this node but
-// the node count.  Lane = move: 64 children are made and evaluated together
-// (the piece-square sum by the move's change of it, the pawn terms and the
-// check test set by set), where each alone costs the wavefront a pass through
-// ENTER and RETURN.  alpha only rises while a node is searched, so a flag set
-// for one alpha holds for every later one; after a rise the rest is tested
-// again.  The flagged moves are counted off in move order by NEXT.
-__device__ void mark_refuted(const Node &n, int lane, u32 *mmove, const int16_t *mscore) {
+constexpr u64 OUTER_RANKS = 0xFF000000000000FFULL;
+
+struct Lds {  // one worker's memory (23 KB: seven workers a CU)
+  Ply ply[MAXPLY + 2];
+  u32 mmove[MSTACK + MPAD];
+  u32 mkey[MSTACK];
+  __align__(16) u16 ctab[NCOUNTER];  // counter moves by the previous move's squares (cleared 16 B at a time)
+  u32 killers[MAXPLY + 2];
+  union {
+    float hpos[zm::NH1];  // the learned scorer's hidden vector
+    u8 mstart[64];        // move-list start marks (lane + 1 at its offset)
+  };
+  int16_t tab[7 * 64];    // EVAL_SQ
+};
+
+// what move generation needs of the lane's square, in registers for good
+struct LaneSq {
+  SqLines q;
+  u64 knight, king, wpawn, bpawn;
+};
+__device__ __forceinline__ LaneSq lane_sq(int sq) {
+  const u64 b = bit(sq);
+  return LaneSq{sq_lines(sq), knight_att(b), king_att(b), pawn_att(b, 0), pawn_att(b, 1)};
+}
+// the lines of a wave-uniform square k, the diagonals from the lane that has them
+__device__ __forceinline__ u64 lane_u64(u64 x, int k) {
+  return ((u64)(u32)__builtin_amdgcn_readlane((int)(u32)(x >> 32), k) << 32) |
+         (u32)__builtin_amdgcn_readlane((int)(u32)x, k);
+}
+__device__ __forceinline__ SqLines uniform_lines(const LaneSq &me, int k) {
+  const u64 b = bit(k);
+  return SqLines{b, bit(63 - k), rank_line(k) ^ b, file_line(k) ^ b, lane_u64(me.q.diag, k), lane_u64(me.q.anti, k)};
+}
+
+__device__ __forceinline__ s32 static_eval(const Pos &p, int lane) {
+  const s32 e = wave_sum_i(eval_square(p, lane)) + eval_bishop_pair(p);
+  return p.stm ? -e : e;
+}
+
+// Periodic test (every POLL_EVERY nodes): true when the worker has to leave the
+// root; renews the root bound `ra` the other workers have published.
+__device__ __forceinline__ bool poll_root(Args a, int lane, bool serving, int r, u64 ticket, int id, u64 nodes,
+                                          s32 final_score, u32 final_move, s32 &ra) {
+  u32 d = 0;
+  if (lane == 0) {
+    if (serving) {
+      d = serve_abort(a, r, ticket);
+    } else {
+      // stop when the root is finished or given up, or the host aborts
+      d = (__atomic_load_n(&a->done[r], __ATOMIC_RELAXED) != 0u || sys_load32(a->habort) != 0u) ? 1u : 0u;
+      if (!d && a->max_nodes && nodes > a->max_nodes) {
+        // over the node budget: give the root up, so that no worker picks it
+        // again (a fresh budget on the same iteration could repeat forever);
+        // its result is this worker's deepest completed iteration
+        if (atomicCAS(&a->done[r], 0u, 3u) == 0u) {
+          a->score[r] = final_score;
+          a->bestmove[r] = final_move;
+        }
+        d = 1;
+      }
+    }
+  }
+  if (uf(d)) return true;
+  u64 rb = 0;
+  if (lane == 0) rb = ag_load(&a->rbound[r]);
+  rb = uf(rb);
+  if ((rb >> 32) == (ticket & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == id) ra = (s32)(rb & 0xFFFF) - 32768;
+  return false;
+}
+
+// What the key of a move says of the child c it makes, a quiescence node: in
+// check, nothing (a draw or a sum beyond 16 bits, which a visit finds), or its evaluation for the side
+// to move: `base` = the parent's sum of eval_piece, q / kb the king that is to
+// move in the child.
+__device__ __forceinline__ u32 child_key(const int16_t *tab, const Pos &c, u32 m, s32 base, const SqLines &q, u64 kb,
+                                         u32 stm) {
+  const u64 occ = c.b1 | c.b2 | c.b3;
+  const s32 e = base + eval_move_delta(tab, m) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ occ, c.b0) + eval_bishop_pair(c);
+  const u32 known = (u32)((stm ? e : -e) + 32768);
+  const bool fits = (u32)(e + 31000) <= 62000u;
+  return king_attacked(c, q, kb, stm) ? KEY_CHECK : (popc(occ) <= 2 || !fits ? KEY_OPEN : known);
+}
+// the node's sum of eval_piece: lane = square
+__device__ __forceinline__ s32 piece_sum(const int16_t *tab, u32 pc, int lane) {
+  return wave_sum_i(eval_piece(tab, pc, lane));
+}
+
+// The children of a depth-1 node, one a lane: those that are quiescence nodes
+// get their evaluation and their check flag into the move's key.  More than
+// half of all nodes are children whose evaluation is already at or above their
+// beta (stand pat); pick_move counts these without a visit, which would cost
+// the wavefront a pass through ENTER and RETURN each.
+__device__ __forceinline__ void key_children(Lds &L, const Node &n, int lane) {
   const u64 occ = n.p.b1 | n.p.b2 | n.p.b3;
-  const u64 kings = n.p.b1 & n.p.b2 & ~n.p.b3;
-  const u64 kb = kings & (n.p.stm ? (n.p.b0 ^ occ) : n.p.b0);  // the opponent's king, to move in every child
-  const int k2 = kb ? lsb(kb) : 0;
-  const u32 pc = piece_at(n.p, lane);
-  const s32 base = wave_sum_i(((pc >> 1) & 7) != PNONE ? eval_piece(pc, lane) : 0);
-  const s32 limit = -n.alpha;  // the children's beta
+  const u64 kb = n.p.b1 & n.p.b2 & ~n.p.b3 & (n.p.stm ? (n.p.b0 ^ occ) : n.p.b0);  // the opponent's king
+  const SqLines q = sq_lines(kb ? lsb(kb) : 0);
+  const s32 base = piece_sum(L.tab, piece_at(n.p, lane), lane);
   for (int k = lane; k < n.mcnt; k += 64) {
-    const u32 mf = mmove[n.mbeg + k];
-    if (mscore[n.mbeg + k] == (int16_t)USED || (mf & (DEFERRED | REFUTED))) continue;
-    const Pos c = apply(n.p, mf, false);
-    const u64 cocc = c.b1 | c.b2 | c.b3;
-    const s32 e = base + eval_move_delta(mf) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ cocc, c.b0) + eval_bishop_pair(c);
-    const s32 ev = n.p.stm ? e : -e;  // for the side to move in the child
-    const bool ext = !n.qs && is_promo(mf);
-    if (ev >= limit && !ext && child_hmc(n.hmc, mf) < 100 && popc(cocc) > 2 && !king_attacked(c, k2, kb))
-      mmove[n.mbeg + k] = mf | REFUTED;
+    const u32 m = L.mmove[n.mbeg + k] & MOVE_BITS;
+    u32 key = child_key(L.tab, apply(n.p, m, false), m, base, q, kb, n.p.stm);
+    // a check or a promotion extends the child, a full half-move clock draws it
+    if (key == KEY_CHECK || is_promo(m) || child_hmc(n.hmc, m) >= 100) key = KEY_OPEN;
+    u32 *const kp = &L.mkey[n.mbeg + k];
+    *kp = (*kp & 0xFFFF0000u) | key;
   }
 }
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_search(SearchArgs a) {
-  __shared__ Ply ply[MAXPLY + 2];
-  __shared__ u32 mmove[MSTACK];
-  __shared__ int16_t mscore[MSTACK];
-  __shared__ __align__(16) u16 ctab[NCOUNTER];  // counter moves by the previous move's squares (cleared 16 B at a time)
-  __shared__ u32 killers[MAXPLY + 2];
-  __shared__ float hpos[zm::NH1];
-  __shared__ u8 mstart[64];  // move-list start marks (lane + 1 at its offset)
-  const int lane = threadIdx.x;
-  const int hstart = (int)((blockIdx.x * 7919u) % (unsigned)(a.nroots > 0 ? a.nroots : 1));
+// The next move of the list [mbeg, mbeg + mcnt): the highest score, the lowest
+// slot among equals (wave arg-max); marks it searched and gives its key before
+// that.  Moves whose child is known to stand pat at or above `limit` (the
+// child's beta; 2 * INF: no such test) return at once in a visit and change
+// nothing at the node but the node count, for a limit that only falls while
+// the node is searched: those ahead of the next move are counted here, up to
+// the periodic poll, whose turn comes in the visit of the child it falls on.
+// defer: the list holds deferred moves, which pass 2 takes and pass 1 skips.
+__device__ __forceinline__ int pick_move(Lds &L, int lane, int mbeg, int mcnt, s32 limit, bool defer, bool pass2,
+                                         int &poll, u64 &nodes, int &searched, u32 &mk) {
+  const u32 lim = (u32)(limit + 32768);
+  for (;;) {
+    u32 best = 0, top = 0;
+    for (int k = lane; k < mcnt; k += 64) {
+      const u32 key = L.mkey[mbeg + k];
+      u32 sk = key >> 16 ? (key & 0xFFFF0000u) | (0xFFFFu - (u32)k) : 0u;
+      if (defer && ((L.mmove[mbeg + k] & DEFERRED) != 0u) != pass2) sk = 0;
+      top = sk > top ? sk : top;
+      if ((key & 0xFFFFu) > KEY_OPEN && (key & 0xFFFFu) >= lim) sk = 0;
+      best = sk > best ? sk : best;
+    }
+    best = wave_max_u32(best);
+    int c = 0;
+    if (__ballot(top > best)) {
+      for (int k0 = 0; k0 < mcnt; k0 += 64) {
+        const int k = k0 + lane;
+        const u32 key = k < mcnt ? L.mkey[mbeg + k] : 0u;
+        const u32 sk = key >> 16 ? (key & 0xFFFF0000u) | (0xFFFFu - (u32)k) : 0u;
+        c += popc(__ballot(sk > best && (key & 0xFFFFu) > KEY_OPEN && (key & 0xFFFFu) >= lim));
+      }
+      u32 upto = best;
+      if (poll + c >= POLL_EVERY) {
+        // a poll falls among them: one at a time up to it
+        top = wave_max_u32(top);
+        c = poll + 1 >= POLL_EVERY ? 0 : 1;
+        upto = top - 1;
+        if (!c) best = top;
+      }
+      if (c) {
+        for (int k = lane; k < mcnt; k += 64) {
+          const u32 key = L.mkey[mbeg + k];
+          const u32 sk = key >> 16 ? (key & 0xFFFF0000u) | (0xFFFFu - (u32)k) : 0u;
+          if (sk > upto && (key & 0xFFFFu) > KEY_OPEN && (key & 0xFFFFu) >= lim) L.mkey[mbeg + k] = key & 0xFFFFu;
+        }
+        poll += c;
+        nodes += (u64)c;
+        if (!pass2) searched += c;
+        wsync();
+        if (upto != best) continue;
+      }
+    }
+    if (best == 0) return -1;
+    const int k = (int)(0xFFFFu - (best & 0xFFFFu));
+    mk = uf(L.mkey[mbeg + k]);
+    wsync();
+    if (lane == 0) L.mkey[mbeg + k] = mk & 0xFFFFu;
+    return k;
+  }
+}
 
-  const bool serving = a.slots != nullptr;
+// The captures of a quiescence node (e.p. included), in the order of origin,
+// then target, with their keys; returns how many, or -1 when they do not fit
+// the move stack.  Lane = square gives the targets; then lane = capture makes
+// the child, tests its legality (the own king not attacked, only when a check,
+// a slider lined up with the king or several kings' squares make it a
+// question) and finds what the key says of it.  ep = the bit of the pawn that
+// may be taken en passant, or 0.
+__device__ __forceinline__ int gen_captures(Lds &L, const LaneSq &me, int lane, const Pos &p, u64 ep, bool kic,
+                                            int mbeg) {
+  const u64 occ = p.b1 | p.b2 | p.b3;
+  const u64 white = p.b0 ^ occ;
+  const u64 own = p.stm ? p.b0 : white, opp = p.stm ? white : p.b0;
+  const u64 rq = p.b3 & (p.b1 ^ p.b2), bq = p.b3 & ~p.b1;
+  const u64 kings = p.b1 & p.b2 & ~p.b3, kbb = own & kings, okb = opp & kings;
+  const u32 pc = piece_at(p, lane);
+  const u32 type = pc >> 1;
+  const bool mine = type != PNONE && (pc & 1u) == p.stm;
+  u64 t = sel(type == ROOK || type == QUEEN, rook_sq(me.q, occ)) | sel(type == BISHOP || type == QUEEN, bishop_sq(me.q, occ));
+  t = type == KNIGHT ? me.knight : t;
+  t = type == KING ? me.king : t;
+  t = type == PAWN ? (p.stm ? me.bpawn : me.wpawn) : t;
+  t = mine ? t & opp : 0;
+  if (__ballot(type == KING && t != 0)) {
+    // squares the king may not step to: attacked with the king off the board
+    const u64 o2 = occ ^ kbb;
+    u64 at = (rook_sq(me.q, o2) & rq) | (bishop_sq(me.q, o2) & bq);
+    at |= me.knight & ~p.b1 & p.b2 & ~p.b3;
+    at |= me.king & kings;
+    at |= (p.stm ? me.bpawn : me.wpawn) & p.b1 & ~p.b2 & ~p.b3;
+    const u64 A = __ballot((at & opp) != 0);
+    if (type == KING) t &= ~A;
+  }
+  const int ksq = kbb ? lsb(kbb) : 0;
+  if (ep) {
+    const int sqep = lsb(ep);
+    const bool cand = mine && type == PAWN && (((p.stm ? RANK4 : RANK5) & (bit(sqep + 1) | bit(sqep - 1))) >> lane) & 1;
+    if (__ballot(cand)) {
+      Node0 B;
+      B.own = own;
+      B.opp = opp;
+      B.occ = occ;
+      B.kbb = kbb;
+      B.pawns = p.b1 & ~p.b2 & ~p.b3;
+      B.knights = ~p.b1 & p.b2 & ~p.b3;
+      B.kings = kings;
+      B.rq = rq;
+      B.bq = bq;
+      B.ksq = ksq;
+      B.stm = p.stm;
+      const int to = (p.stm ? sqep - 8 : sqep + 8) & 63;
+      if (cand && ep_legal0(B, lane, to, sqep)) t |= bit(to);
+    }
+  }
+  int total;
+  const int off = wave_exscan_i(popc(t), lane, total);
+  if (total == 0) return 0;
+  if (mbeg + total > MSTACK + MPAD) return -1;
+  u32 *out = L.mmove + mbeg + off;
+  while (t) {
+    *out++ = (u32)lane | ((u32)lsb(t) << 6);
+    t &= t - 1;
+  }
+  wsync();
+  const SqLines kq = uniform_lines(me, ksq);
+  const bool test = kbb && (kic || ((kq.rank | kq.file) & opp & rq) || ((kq.diag | kq.anti) & opp & bq));
+  const SqLines oq = uniform_lines(me, okb ? lsb(okb) : 0);
+  const s32 base = piece_sum(L.tab, pc, lane);
+  const bool odd_pawns = (p.b1 & ~p.b2 & ~p.b3 & OUTER_RANKS) != 0;  // the pawn sums want none there
+  int kept = 0;
+  for (int c0 = 0; c0 < total; c0 += 64) {
+    const bool act = c0 + lane < total;
+    const u32 raw = act ? L.mmove[mbeg + c0 + lane] : 0u;
+    const int from = (int)(raw & 63u), to = (int)(raw >> 6);
+    const u32 pf = (u32)__shfl((int)pc, from, 64);
+    u32 cap = (u32)__shfl((int)pc, to, 64);
+    const bool pawn = (pf >> 1) == PAWN, isep = pawn && cap == 0;
+    int x = to;
+    if (ep) {  // wave-uniform
+      x = isep ? (p.stm ? to + 8 : to - 8) & 63 : to;
+      cap = (u32)__shfl((int)pc, x, 64);
+    }
+    const u32 pt = pawn && (p.stm ? to < 8 : to >= 56) ? ((QUEEN << 1) | p.stm) : pf;
+    const u32 m = mv_make((u32)from, (u32)to, (u32)x, pf, pt, cap);
+    const Pos c = apply_capture(p, m);
+    bool legal = act;
+    if (test) legal = act && ((pf >> 1) == KING || isep || !king_attacked(c, kq, kbb, p.stm ^ 1u));
+    u32 key = child_key(L.tab, c, m, base, oq, okb, p.stm);
+    if (odd_pawns && key > KEY_OPEN) key = KEY_OPEN;
+    const u64 lm = __ballot(legal);
+    const int slot = mbeg + kept + popc(lm & ((1ULL << lane) - 1));
+    kept += popc(lm);
+    if (mbeg + kept > MSTACK) return -1;
+    wsync();
+    if (legal) {
+      L.mmove[slot] = m;
+      L.mkey[slot] = move_key(piece_value(cap >> 1) * 16 - piece_value(pt >> 1), key);
+    }
+  }
+  wsync();
+  return kept;
+}
+
+// v_writelane_b32: x with lane k (a constant) set to v
+extern "C" __device__ int write_lane(int v, int k, int x) __asm("llvm.amdgcn.writelane.i32");
+
+enum { QS_DONE = 0, QS_ABORTED, QS_FAILED };
+
+// A quiescence node and everything below it, which is quiescence too: captures
+// only, stand pat when not in check, no table, no hash, no extension, no
+// deferral.  Apart from the full-width loop it keeps a few scalars a ply: the
+// four planes, the window and the list, one word a lane in the ply's record,
+// stored and loaded with one LDS access.  ev / known: the evaluation, if the
+// parent has it; kic: in check; polled: the visit has been counted to the poll.
+__device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p, s32 alpha, s32 beta, u32 hmc,
+                                       const int sd0, int mbeg, s32 ev, bool known, bool kic, bool polled, bool serving,
+                                       int r, u64 ticket, int id, s32 final_score, u32 final_move, u64 &nodes, int &poll,
+                                       s32 &ra, u32 &cvec, s32 &vout) {
+  int sd = sd0, mcnt = 0, unused = 0;
+  u64 ep = ~p.cr & RANKS45;  // captures leave none behind
+  s32 v = 0;
+  bool enter = true;
+  for (;;) {
+    if (enter) {
+      if (!polled && ++poll >= POLL_EVERY) {
+        poll = 0;
+        if (poll_root(args(), lane, serving, r, ticket, id, nodes, final_score, final_move, ra)) return QS_ABORTED;
+      }
+      polled = false;
+      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) alpha = ra - 1;
+      const bool draw = hmc >= 100 || popc(p.b1 | p.b2 | p.b3) <= 2;
+      // stand pat before any move generation: the reference returns the static
+      // evaluation both on a stand-pat cutoff and when no capture exists
+      // (src/zeta.cl:1597-1605)
+      bool leaf = false;
+      if (!kic) {
+        if (draw) {
+          v = 0;
+          leaf = true;
+        } else {
+          if (!known) ev = static_eval(p, lane);
+          if (ev >= beta || sd >= MAXPLY) {
+            if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
+            v = ev;
+            leaf = true;
+          }
+        }
+      }
+      if (!leaf) {
+        mcnt = gen_captures(L, me, lane, p, ep, kic, mbeg);
+        if (mcnt < 0) {
+          if (lane == 0) atomicOr(args()->err, 1u);
+          return QS_FAILED;
+        }
+        if (draw) {
+          v = 0;
+          leaf = true;
+        } else if (mcnt == 0 || sd >= MAXPLY) {
+          if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
+          v = kic ? static_eval(p, lane) : ev;
+          leaf = true;
+        } else if (!kic && ev > alpha) {
+          alpha = ev;
+        }
+      }
+      ep = 0;
+      hmc = 0;
+      enter = !leaf;
+    } else {
+      enter = true;
+    }
+    // enter: go on with this node's moves; else return v to the parent
+    int k = -1;
+    u32 mk = 0;
+    if (enter) {
+      k = pick_move(L, lane, mbeg, mcnt, sd + 1 < MAXPLY ? -alpha : 2 * INF, false, false, poll, nodes, unused, mk);
+      if (k < 0) v = alpha;
+    }
+    if (k >= 0) {
+      const u32 m = uf(L.mmove[mbeg + k]);
+      int w = 0;
+      w = write_lane((int)(u32)p.b0, 0, w);
+      w = write_lane((int)(u32)(p.b0 >> 32), 1, w);
+      w = write_lane((int)(u32)p.b1, 2, w);
+      w = write_lane((int)(u32)(p.b1 >> 32), 3, w);
+      w = write_lane((int)(u32)p.b2, 4, w);
+      w = write_lane((int)(u32)(p.b2 >> 32), 5, w);
+      w = write_lane((int)(u32)p.b3, 6, w);
+      w = write_lane((int)(u32)(p.b3 >> 32), 7, w);
+      w = write_lane((int)(((u32)alpha & 0xFFFFu) | ((u32)beta << 16)), 8, w);
+      w = write_lane((int)((u32)mbeg | ((u32)mcnt << 16)), 9, w);
+      if (lane < 10) ((int *)&L.ply[sd])[lane] = w;
+      nodes++;
+      p = apply_capture(p, m);
+      const s32 t = alpha;
+      alpha = -beta;
+      beta = -t;
+      mbeg += mcnt;
+      kic = (mk & 0xFFFFu) == KEY_CHECK;
+      known = (mk & 0xFFFFu) > KEY_OPEN;
+      ev = (s32)(mk & 0xFFFFu) - 32768;
+      sd++;
+      enter = true;
+      continue;
+    }
+    for (;;) {
+      if (sd == sd0) {
+        vout = v;
+        return QS_DONE;
+      }
+      sd--;
+      wsync();
+      const int w = ((const int *)&L.ply[sd])[lane & 15];
+      auto word = [&](int i) { return (u32)__builtin_amdgcn_readlane(w, i); };
+      p.b0 = ((u64)word(1) << 32) | word(0);
+      p.b1 = ((u64)word(3) << 32) | word(2);
+      p.b2 = ((u64)word(5) << 32) | word(4);
+      p.b3 = ((u64)word(7) << 32) | word(6);
+      p.stm ^= 1u;
+      alpha = (s32)(int16_t)(u16)word(8);
+      beta = (s32)word(8) >> 16;
+      mbeg = (int)(word(9) & 0xFFFFu);
+      mcnt = (int)(word(9) >> 16);
+      const s32 sc = -v;
+      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) alpha = ra - 1;
+      if (sc > alpha) alpha = sc;
+      if (alpha < beta) break;
+      v = alpha;
+    }
+    enter = false;
+  }
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_search(SearchArgs) {
+  __shared__ Lds L;
+  Ply *const ply = L.ply;
+  u32 *const mmove = L.mmove, *const mkey = L.mkey, *const killers = L.killers;
+  u16 *const ctab = L.ctab;
+  const int lane = threadIdx.x;
+  const LaneSq me = lane_sq(lane);
+  for (int k = lane; k < 7 * 64; k += 64) L.tab[k] = (int16_t)EVAL_SQ.v[k];
+  const Args a = args();
+  const int hstart = (int)((blockIdx.x * 7919u) % (unsigned)(a->nroots > 0 ? a->nroots : 1));
+
+  const bool serving = a->slots != nullptr;
   if (serving && blockIdx.x == gridDim.x - 1) {
     serve_scheduler(a, lane);
     return;
@@ -826,15 +1221,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       r = serve_pick(a, lane, ticket);
     } else {
       u32 ab = 0;
-      if (lane == 0) ab = sys_load32(a.habort);
+      if (lane == 0) ab = sys_load32(a->habort);
       r = uf(ab) ? -1 : pick_root(a, hstart, lane);
     }
     if (r < 0) return;
-    int depth_r = a.depth;
-    bool mlp_r = a.use_mlp != 0;
+    int depth_r = a->depth;
+    bool mlp_r = a->use_mlp != 0;
     if (serving) {
-      depth_r = uf(ag_load(&a.dreq[r].depth));
-      mlp_r = mlp_r && (uf(ag_load(&a.dreq[r].flags)) & 1);
+      depth_r = uf(ag_load(&a->dreq[r].depth));
+      mlp_r = mlp_r && (uf(ag_load(&a->dreq[r].flags)) & 1);
       if (depth_r < 1) depth_r = 1;
       if (depth_r > MAXPLY - 1) depth_r = MAXPLY - 1;
     }
@@ -842,10 +1237,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     // ---------------------------------------------------------------- root set-up
     // (the root position is re-read at every iteration rather than held in
     // scalar registers through the search)
-    const u64 *const rootq = serving ? (const u64 *)a.dreq[r].pos : a.roots + (size_t)r * 8;
+    const u64 *const rootq = serving ? (const u64 *)a->dreq[r].pos : a->roots + (size_t)r * 8;
     int hl = 0;
-    if (a.hist) {
-      hl = uf(a.hlen[r]);
+    if (a->hist) {
+      hl = uf(a->hlen[r]);
       hl = hl < 0 ? 0 : (hl > ZETA_HISTORY ? ZETA_HISTORY : hl);
     }
     // killers and counter moves start empty for every root (they persist
@@ -868,7 +1263,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     // iteration in progress: the earlier ones would only repeat work whose
     // moves are in the shared TT (the final iteration alone sets the score)
     int id0 = 1;
-    if (lane == 0) id0 = (__atomic_load_n(&a.depth_done[r], __ATOMIC_RELAXED) & (serving ? 0xFFFF : ~0)) + 1;
+    if (lane == 0) id0 = (__atomic_load_n(&a->depth_done[r], __ATOMIC_RELAXED) & (serving ? 0xFFFF : ~0)) + 1;
     id0 = uf(id0);
     id0 = id0 < 1 ? 1 : (id0 > depth_r ? depth_r : id0);
     for (int id = id0; id <= depth_r && !aborted && !failed; id++) {
@@ -879,7 +1274,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         // a worker joining the iteration starts from the bound the root's
         // other workers have published
         u64 rb = 0;
-        if (lane == 0) rb = ag_load(&a.rbound[r]);
+        if (lane == 0) rb = ag_load(&a->rbound[r]);
         rb = uf(rb);
         if ((rb >> 32) == (ticket & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == id)
           ra = (s32)(rb & 0xFFFF) - 32768;
@@ -916,61 +1311,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       n.iter = 1;
       n.ndefer = 0;
       n.searched = 0;
-      n.ralpha = -INF;
+      n.keyed = false;
       int sd = 1;
-      bool parent_qs = false;
+      s32 qev = 0;  // S_QS: the node's evaluation, whether it is known, and whether this visit has polled
+      bool qknown = false, polled = false;
       s32 rootscore = 0;  // DRAWSCORE until a root move raises alpha (src/zeta.cl:986)
       u32 rootmove = 0;
       s32 v = 0;
       int state = S_ENTER;
 
       for (;;) {
+        const Args a = args();  // loads of arguments stay in this pass
         if (state == S_ENTER) {
           // ---------------- ENTER: analyse, extend, generate, terminal tests
           if (++poll >= POLL_EVERY) {
             poll = 0;
-            u32 d = 0;
-            if (lane == 0) {
-              if (serving) {
-                d = serve_abort(a, r, ticket);
-              } else {
-                // stop when the root is finished or given up, or the host aborts
-                d = (__atomic_load_n(&a.done[r], __ATOMIC_RELAXED) != 0u || sys_load32(a.habort) != 0u) ? 1u : 0u;
-                if (!d && a.max_nodes && nodes > a.max_nodes) {
-                  // over the node budget: give the root up, so that no worker
-                  // picks it again (a fresh budget on the same iteration could
-                  // repeat forever); its result is this worker's deepest
-                  // completed iteration
-                  if (atomicCAS(&a.done[r], 0u, 3u) == 0u) {
-                    a.score[r] = final_score;
-                    a.bestmove[r] = final_move;
-                  }
-                  d = 1;
-                }
-              }
-            }
-            if (uf(d)) {
+            if (poll_root(a, lane, serving, r, ticket, id, nodes, final_score, final_move, ra)) {
               aborted = true;
               break;
             }
-            u64 rb = 0;
-            if (lane == 0) rb = ag_load(&a.rbound[r]);
-            rb = uf(rb);
-            if ((rb >> 32) == (ticket & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == id)
-              ra = (s32)(rb & 0xFFFF) - 32768;
           }
           const int plyn = sd - 1;
           // issue the TT load early: its latency overlaps the analysis below
-          const bool early = a.ttmask && sd > 1 && n.depth >= 1;
+          const bool early = a->ttmask && sd > 1 && n.depth >= 1;
           const u64 key = tt_key(n.hash, n.p.cr);
           u32x4 tte = {0u, 0u, 0u, 0u};
-          if (early) tte = *(const u32x4 *)(a.tt + 2 * (key & a.ttmask));
+          if (early) tte = *glob((const u32x4 *)(a->tt + 2 * (key & a->ttmask)));
           // node analysis, uniform part (king-square attackers by single-square
           // sliders): gives the in-check flag before the quiescence stand pat
           Node0 B;
           node_basics(n.p, B);
           n.kic = B.checkers != 0;
-          if (n.depth >= 0 && !parent_qs && (n.kic || is_promo(n.lastmove))) n.depth++;
+          if (n.depth >= 0 && (n.kic || is_promo(n.lastmove))) n.depth++;
           n.qs = n.depth <= 0;
           // Another worker's root move reached ra: at the root's side (odd
           // plies from 3 on) a value at or below ra - 1 cannot make this root
@@ -982,32 +1354,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.iter = 1;
           n.ndefer = 0;
           n.searched = 0;
-          n.ralpha = -INF;
+          n.keyed = false;
           n.mcnt = 0;
-          s32 ev0 = 0;
-          bool have_ev = false;
-          if (n.qs && !n.kic) {
-            // quiescence stand pat before any move generation: the reference
-            // returns the static eval both on a stand-pat cutoff and when no
-            // capture exists (src/zeta.cl:1597-1605), so eval >= beta ends the
-            // node with the same value either way
-            const bool qdraw = sd > 1 && (n.hmc >= 100 || popc(n.p.b1 | n.p.b2 | n.p.b3) <= 2);
-            if (qdraw) {
-              v = 0;
-              state = S_RETURN;
-              wsync();
-              continue;
-            }
-            const s32 e = wave_sum_i(eval_square(n.p, lane)) + eval_bishop_pair(n.p);
-            ev0 = n.p.stm ? -e : e;
-            have_ev = true;
-            if (ev0 >= n.beta || sd >= MAXPLY) {
-              if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
-              v = ev0;
-              state = S_RETURN;
-              wsync();
-              continue;
-            }
+          if (n.qs) {
+            // a quiescence node whose parent did not know it for one
+            qev = 0;
+            qknown = false;
+            polled = true;
+            state = S_QS;
+            continue;
           }
           // move generation, lane = square: the lanes answer "is my square
           // attacked" (a ballot gives the attack map) and "which targets has
@@ -1015,39 +1370,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // the attack map is read only for king moves and castling: skip it
           // (a uniform branch) when the king has no target square to test
           u64 A = 0;
-          const u64 kt = king_att(B.kbb) & (n.qs ? B.opp : ~B.own);
-          if (kt || (!n.qs && (n.p.cr & SMCRALL))) A = __ballot(attacked_nk(B, lane));
+          const u64 kt = king_att(B.kbb) & ~B.own;
+          if (kt || (n.p.cr & SMCRALL)) A = __ballot(attacked_nk(B, lane));
           u64 t = 0;
-          if ((B.own >> lane) & 1) t = lane_targets(n.p, B, A, lane, n.qs);
+          if ((B.own >> lane) & 1) t = lane_targets(n.p, B, A, lane, false);
           int total;
           const int off = wave_exscan_i(popc(t), lane, total);
           n.mcnt = total;
           if (n.mbeg + total > MSTACK) {
-            if (lane == 0) atomicOr(a.err, 1u);
+            if (lane == 0) atomicOr(a->err, 1u);
             failed = true;
             break;
           }
-          // killer and counter move (quiescence nodes have no quiet moves)
-          const u32 kil = killers[sd], cm = n.qs ? 0u : (u32)ctab[counter_index(n.lastmove)];
+          const u32 kil = killers[sd], cm = (u32)ctab[counter_index(n.lastmove)];
           {
             auto put = [&](int k, int from, int to) {
               const u32 m = make_code(n.p, from, to);
-              s32 sc = order_score(n.p.stm, m);
-              sc = sc > 31999 ? 31999 : (sc < -31999 ? -31999 : sc);
-              if (((mv_pcpt(m) >> 1) & 7) == PNONE) {
-                if (m == kil) sc = KILLER_SCORE;
-                else if (counter_code(m) == cm) sc = COUNTER_SCORE;
-              }
               mmove[k] = m;
-              mscore[k] = (int16_t)sc;
+              mkey[k] = move_key(plain_score(L.tab, n.p.stm, m, kil, cm), KEY_OPEN);
             };
-            if (!n.qs && total <= 64) {
+            if (total <= 64) {
               // lane j writes move j of the list (the same order as the loop
               // below: origin lanes ascending, then targets ascending): its
               // origin is the last lane with targets whose offset is <= j (a
               // prefix max over start marks), its target the (j - offset)-th
               // bit of that lane's set -- one pass instead of as many loop
               // trips as the busiest lane has targets
+              u8 *const mstart = L.mstart;
               mstart[lane] = 0;
               wsync();
               if (t) mstart[off] = (u8)(lane + 1);
@@ -1067,66 +1416,54 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               }
             }
           }
-          if (mlp_r && !n.qs && n.depth >= a.mlp_min_depth && total > 1) {
+          if (mlp_r && n.depth >= a->mlp_min_depth && total > 1) {
             wsync();
-            mlp_score_moves(a, n.p, n.mbeg, total, lane, hpos, mmove, mscore);
+            mlp_score_moves(a, n.p, n.mbeg, total, lane, L.hpos, mmove, mkey);
             // every move's key is its plain score plus the network's, in
             // plain-score units (zm::PLAIN_PER_LOGIT per unit of the
             // network's output, the scale the ranking loss is trained at);
             // the TT move still goes first
             for (int k = lane; k < total; k += 64) {
               const u32 m = mmove[n.mbeg + k];
-              s32 sc = plain_score(n.p.stm, m, kil, cm) +
-                       (s32)mscore[n.mbeg + k] * zm::PLAIN_PER_LOGIT / 256;
+              s32 sc = plain_score(L.tab, n.p.stm, m, kil, cm) +
+                       (s32)mkey[n.mbeg + k] * zm::PLAIN_PER_LOGIT / 256;
               sc = sc > 31999 ? 31999 : (sc < -31999 ? -31999 : sc);
-              mscore[n.mbeg + k] = (int16_t)sc;
+              mkey[n.mbeg + k] = move_key(sc, KEY_OPEN);
             }
             wsync();
             lcount(cvec, C_MLP_NODES, 1);
           }
           // terminal / draw tests in the reference's order (src/zeta.cl:1554-1609)
           bool draw = false;
-          if (total > 0 && !n.qs && sd > 1) {
+          if (total > 0 && sd > 1) {
             // repetition against plies plyn-2, plyn-4, .. >= plyn-hmc: the
             // searched path, then the game history before the root
             bool hit = false;
             const int nn = plyn - 2 - 2 * lane;
             if (nn >= plyn - (int)n.hmc) {
               if (nn >= 0) hit = ply[nn + 1].hash == n.hash;
-              else if (-nn - 1 < hl) hit = a.hist[(size_t)r * ZETA_HISTORY + (-nn - 1)] == n.hash;
+              else if (-nn - 1 < hl) hit = a->hist[(size_t)r * ZETA_HISTORY + (-nn - 1)] == n.hash;
             }
             draw = __ballot(hit) != 0;
           }
           if (sd > 1 && n.hmc >= 100) draw = true;
           if (sd > 1 && popc(B.occ) <= 2) draw = true;
-          const bool need_eval = !draw && ((n.qs && !n.kic) || (n.qs && total == 0) || (sd >= MAXPLY && total > 0));
-          s32 ev = 0;
-          if (need_eval && have_ev) {
-            ev = ev0;
-          } else if (need_eval) {
-            const s32 e = wave_sum_i(eval_square(n.p, lane)) + eval_bishop_pair(n.p);
-            ev = n.p.stm ? -e : e;
-          }
           state = S_NEXT;
           if (draw) {
             v = 0;
             state = S_RETURN;
-          } else if (!n.qs && total == 0) {
+          } else if (total == 0) {
             v = n.kic ? -INF + plyn : 0;
             state = S_RETURN;
-          } else if (sd >= MAXPLY || total == 0) {
-            if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
-            v = ev;
-            state = S_RETURN;
-          } else if (n.qs && !n.kic && ev >= n.beta) {
-            v = ev;  // stand pat, fail soft
+          } else if (sd >= MAXPLY) {
+            lcount(cvec, C_MAXPLY, 1);
+            v = static_eval(n.p, lane);
             state = S_RETURN;
           } else {
-            if (n.qs && !n.kic && ev > n.alpha) n.alpha = ev;
             // TT probe: move for ordering; score under the exact-depth rule
             u32 ttmove = 0;
-            if (a.ttmask && !n.qs && sd > 1) {
-              if (!early) tte = *(const u32x4 *)(a.tt + 2 * (key & a.ttmask));
+            if (a->ttmask && sd > 1) {
+              if (!early) tte = *glob((const u32x4 *)(a->tt + 2 * (key & a->ttmask)));
               const u64 w0 = uf(((u64)tte.y << 32) | tte.x), w1 = uf(((u64)tte.w << 32) | tte.z);
               lcount(cvec, C_TT_PROBE, 1);
               if ((w0 ^ w1) == key && ((w1 >> 57) & 1)) {
@@ -1157,17 +1494,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             }
             if (state == S_NEXT && ttmove) {
               for (int k = lane; k < total; k += 64)
-                if (mmove[n.mbeg + k] == ttmove) mscore[n.mbeg + k] = (int16_t)TTMOVE_SCORE;
+                if (mmove[n.mbeg + k] == ttmove) mkey[n.mbeg + k] = move_key(TTMOVE_SCORE, KEY_OPEN);
             }
-            if (a.recs && lane == 0) ply[sd].ttm = ttmove;
-            if (state == S_NEXT && a.hint && !n.qs) {
+            if (a->recs && lane == 0) ply[sd].ttm = ttmove;
+            if (state == S_NEXT && a->hint) {
               // the hint table (a completed search's table): its move first
-              const u32x4 he = *(const u32x4 *)(a.hint + 2 * (key & a.ttmask));
+              const u32x4 he = *glob((const u32x4 *)(a->hint + 2 * (key & a->ttmask)));
               const u64 h0 = uf(((u64)he.y << 32) | he.x), h1 = uf(((u64)he.w << 32) | he.z);
               if ((h0 ^ h1) == key && ((h1 >> 57) & 1)) {
                 const u32 hm = (u32)h1;
                 for (int k = lane; k < total; k += 64)
-                  if (mmove[n.mbeg + k] == hm) mscore[n.mbeg + k] = (int16_t)HINT_SCORE;
+                  if (mmove[n.mbeg + k] == hm) mkey[n.mbeg + k] = move_key(HINT_SCORE, KEY_OPEN);
               }
             }
           }
@@ -1176,71 +1513,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         }
 
         if (state == S_NEXT) {
-          // ---------------- NEXT: pick the best remaining move (wave arg-max)
-          // a node whose children are quiescence nodes: first flag the moves
-          // that a child's stand pat refutes (the pawn sums want no pawn on
-          // the outer ranks; a child at MAXPLY is counted, so made)
-          const bool leafward = n.depth <= 1 && sd + 1 < MAXPLY;
-          if (leafward && n.alpha > n.ralpha && !(n.p.b1 & ~n.p.b2 & ~n.p.b3 & 0xFF000000000000FFULL)) {
-            mark_refuted(n, lane, mmove, mscore);
-            n.ralpha = n.alpha;
+          // ---------------- NEXT: pick the best remaining move
+          // a node whose children are quiescence nodes: first find out what a
+          // lane each can tell of them (the pawn sums want no pawn on the
+          // outer ranks; a child at MAXPLY is counted, so made)
+          const bool leafward = n.depth <= 1 && sd + 1 < MAXPLY && n.alpha > -INF;
+          if (leafward && !n.keyed) {
+            n.keyed = true;
+            if (!(n.p.b1 & ~n.p.b2 & ~n.p.b3 & OUTER_RANKS)) key_children(L, n, lane);
           }
-          u32 bestkey = 0, topkey = 0;  // the best move to search, the best of all (flagged ones included)
-          for (int k = lane; k < n.mcnt; k += 64) {
-            const s32 sc = mscore[n.mbeg + k];
-            const u32 mf = mmove[n.mbeg + k];
-            const bool fl = (mf & DEFERRED) != 0u;
-            const bool ok = sc != USED && (n.iter == 1 ? !fl : fl);
-            if (ok) {
-              const u32 key = ((u32)(sc + 32768) << 16) | (0xFFFFu - (u32)k);
-              topkey = key > topkey ? key : topkey;
-              if (!(mf & REFUTED)) bestkey = key > bestkey ? key : bestkey;
-            }
-          }
-          bestkey = wave_max_u32(bestkey);
-          if (leafward) {
-            // flagged moves ahead of the best: visited here, as their order
-            // has it, by counting them
-            int c = 0;
-            for (int k0 = 0; k0 < n.mcnt; k0 += 64) {
-              const int k = k0 + lane;
-              bool ahead = false;
-              if (k < n.mcnt) {
-                const s32 sc = mscore[n.mbeg + k];
-                ahead = sc != USED && (mmove[n.mbeg + k] & REFUTED) &&
-                        (((u32)(sc + 32768) << 16) | (0xFFFFu - (u32)k)) > bestkey;
-              }
-              c += popc(__ballot(ahead));
-            }
-            if (c) {
-              u32 upto = bestkey;
-              if (poll + c >= POLL_EVERY) {
-                // a poll falls among them: one at a time up to it, and the
-                // child whose turn it is is entered as any other
-                topkey = wave_max_u32(topkey);
-                if (poll + 1 >= POLL_EVERY) {
-                  bestkey = topkey;
-                  c = 0;
-                } else {
-                  upto = topkey - 1;
-                  c = 1;
-                }
-              }
-              if (c) {
-                for (int k = lane; k < n.mcnt; k += 64) {
-                  const s32 sc = mscore[n.mbeg + k];
-                  if (sc != USED && (mmove[n.mbeg + k] & REFUTED) &&
-                      (((u32)(sc + 32768) << 16) | (0xFFFFu - (u32)k)) > upto)
-                    mscore[n.mbeg + k] = (int16_t)USED;
-                }
-                poll += c;
-                nodes += (u64)c;
-                n.searched += c;
-                if (upto != bestkey) continue;
-              }
-            }
-          }
-          if (bestkey == 0) {
+          u32 mk = 0;
+          const int pk = pick_move(L, lane, n.mbeg, n.mcnt, leafward ? -n.alpha : 2 * INF, n.ndefer > 0, n.iter == 2,
+                                   poll, nodes, n.searched, mk);
+          if (pk < 0) {
             if (n.iter == 1 && n.ndefer > 0) {
               n.iter = 2;
               continue;
@@ -1250,20 +1535,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             state = S_RETURN;
             continue;
           }
-          const int k = n.mbeg + (int)(0xFFFFu - (bestkey & 0xFFFFu));
+          const int k = n.mbeg + pk;
           const u32 m = uf(mmove[k]) & MOVE_BITS;
-          const s32 sk = (s32)(bestkey >> 16) - 32768;
           wsync();
-          if (lane == 0) mscore[k] = (int16_t)USED;
           const Pos c = apply(n.p, m, false);
           u64 ch, cph;
           child_hash(n, m, c, ch, cph);
           // ABDADA: defer a sibling that another worker is already searching
           bool cbusy = false;
-          if (a.workers > 1 && n.depth - 1 >= a.split_depth) {
-            const u32 bidx = (u32)(tt_key(ch, c.cr) >> 40) & a.busymask;
+          if (a->workers > 1 && n.depth - 1 >= a->split_depth) {
+            const u32 bidx = (u32)(tt_key(ch, c.cr) >> 40) & a->busymask;
             u32 b = 0;
-            if (lane == 0) b = __atomic_load_n(&a.busy[bidx], __ATOMIC_RELAXED);
+            if (lane == 0) b = __atomic_load_n(&a->busy[bidx], __ATOMIC_RELAXED);
             b = uf(b);
             // batch searches defer a busy first child too, from ply 3 down:
             // a worker that finds it busy moves on to the siblings and comes
@@ -1279,7 +1562,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             // the first-child deferral at every ply)
             if (n.iter == 1 && b && (n.searched > 0 || (!serving && sd >= 3))) {
               if (lane == 0) {
-                mscore[k] = (int16_t)sk;
+                mkey[k] = mk;
                 mmove[k] = m | DEFERRED;
               }
               n.ndefer++;
@@ -1287,7 +1570,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               wsync();
               continue;
             }
-            if (lane == 0) atomicAdd(&a.busy[bidx], 1u);
+            if (lane == 0) atomicAdd(&a->busy[bidx], 1u);
             cbusy = true;
           }
           if (n.iter == 1) n.searched++;
@@ -1295,7 +1578,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.move = m;
           if (lane == 0) save(ply[sd], n);
           // descend
-          parent_qs = n.qs;
           Node cn;
           cn.p = c;
           cn.hash = ch;
@@ -1315,11 +1597,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           cn.iter = 1;
           cn.ndefer = 0;
           cn.searched = 0;
-          cn.ralpha = -INF;
+          cn.keyed = false;
           n = cn;
           sd++;
           wsync();
           state = S_ENTER;
+          if ((mk & 0xFFFFu) > KEY_OPEN) {
+            // a quiescence node, not in check, its evaluation known
+            qev = (s32)(mk & 0xFFFFu) - 32768;
+            qknown = true;
+            polled = false;
+            n.qs = true;
+            state = S_QS;
+          }
+          continue;
+        }
+
+        if (state == S_QS) {
+          // ---------------- a quiescence node and all below it
+          const int st = qsearch(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, polled, serving,
+                                 r, ticket, id, final_score, final_move, nodes, poll, ra, cvec, v);
+          if (st != QS_DONE) {
+            aborted = st == QS_ABORTED;
+            failed = !aborted;
+            break;
+          }
+          state = S_RETURN;
           continue;
         }
 
@@ -1346,20 +1649,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             rootscore = sc;
             rootmove = n.move;
             if (lane == 0)
-              atomicMax((unsigned long long *)&a.rbound[r],
+              atomicMax((unsigned long long *)&a->rbound[r],
                         (unsigned long long)(((ticket & 0xFFFFFFFFULL) << 32) | ((u64)id << 16) | (u64)(u16)(sc + 32768)));
           }
         }
         if (n.alpha >= n.beta) {
-          if (a.recs && !n.qs && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
-              ((u32)(n.hash >> 40) & a.rec_mask) == 0) {
+          if (a->recs && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
+              ((u32)(n.hash >> 40) & a->rec_mask) == 0) {
             u32 nrec = 0;
-            log_pairs(a, n, lane, mmove, mscore, ply[sd].ttm, killers[sd], (u32)ctab[counter_index(n.lastmove)], nrec);
+            log_pairs(a, n, lane, mmove, L.tab, ply[sd].ttm, killers[sd], (u32)ctab[counter_index(n.lastmove)], nrec);
             lcount(cvec, C_RECORDS, nrec);
           }
           // a quiet move that fails high becomes the ply's killer and the
           // counter move of the move before it (src/zeta.cl:1916-1933)
-          if (!n.qs && ((mv_pcpt(n.move) >> 1) & 7) == PNONE && lane == 0) {
+          if (((mv_pcpt(n.move) >> 1) & 7) == PNONE && lane == 0) {
             killers[sd] = n.move;
             ctab[counter_index(n.lastmove)] = counter_code(n.move);
           }
@@ -1383,8 +1686,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       final_score = (rootscore == INF || rootscore == -INF) ? 0 : rootscore;  // src/search.c:137
       final_move = rootmove;
       if (lane == 0) {
-        if (serving) slot_max_depth(&a.depth_done[r], ticket, id);
-        else atomicMax(&a.depth_done[r], id);
+        if (serving) slot_max_depth(&a->depth_done[r], ticket, id);
+        else atomicMax(&a->depth_done[r], id);
       }
       // a mate within this iteration's depth is the score of every deeper
       // iteration too: iterative deepening stops there (src/search.c:177-186)
@@ -1392,22 +1695,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     }
 
     // ---------------------------------------------------------------- publish
-    if (lane < C_NODES && cvec) atomicAdd((unsigned long long *)&a.ctr[lane], (unsigned long long)cvec);
+    if (lane < C_NODES && cvec) atomicAdd((unsigned long long *)&a->ctr[lane], (unsigned long long)cvec);
     if (lane == 0) {
       // before leaving: the last worker to leave publishes the request's
       // count, which then holds every worker's nodes
-      if (serving) slot_add_nodes(&a.nodes[r], ticket, nodes);
-      else atomicAdd((unsigned long long *)&a.nodes[r], (unsigned long long)nodes);
-      atomicAdd((unsigned long long *)&a.ctr[C_NODES], (unsigned long long)nodes);
+      if (serving) slot_add_nodes(&a->nodes[r], ticket, nodes);
+      else atomicAdd((unsigned long long *)&a->nodes[r], (unsigned long long)nodes);
+      atomicAdd((unsigned long long *)&a->ctr[C_NODES], (unsigned long long)nodes);
       if (serving) {
         serve_leave(a, r, ticket, aborted, failed, final_score, final_move);
       } else {
-        if (!aborted && !failed && atomicCAS(&a.done[r], 0u, 1u) == 0u) {
-          a.score[r] = final_score;
-          a.bestmove[r] = final_move;
+        if (!aborted && !failed && atomicCAS(&a->done[r], 0u, 1u) == 0u) {
+          a->score[r] = final_score;
+          a->bestmove[r] = final_move;
         }
-        if (failed) atomicCAS(&a.done[r], 0u, 2u);
-        atomicSub(&a.nworkers[r], 1);
+        if (failed) atomicCAS(&a->done[r], 0u, 2u);
+        atomicSub(&a->nworkers[r], 1);
       }
     }
     wsync();
@@ -1416,11 +1719,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 
 // the search's learned-ordering routine applied to given moves (for tests and
 // external callers): one wave per position, up to MSTACK moves each
-__global__ __launch_bounds__(64) void k_mlp_score(SearchArgs a, const u64 *pos, const u32 *moves, const int *off,
+__global__ __launch_bounds__(64) void k_mlp_score(SearchArgs, const u64 *pos, const u32 *moves, const int *off,
                                                  float *out) {
   __shared__ u32 mmove[MSTACK];
-  __shared__ int16_t mscore[MSTACK];
+  __shared__ u32 mscore[MSTACK];
   __shared__ float hpos[zm::NH1];
+  const Args a = args();
   const int lane = threadIdx.x, i = blockIdx.x;
   const u64 *q = pos + (size_t)i * 8;
   Pos p;
@@ -1434,7 +1738,7 @@ __global__ __launch_bounds__(64) void k_mlp_score(SearchArgs a, const u64 *pos, 
   for (int k = lane; k < n; k += 64) mmove[k] = moves[b + k];
   wsync();
   mlp_score_moves(a, p, 0, n, lane, hpos, mmove, mscore);
-  for (int k = lane; k < n; k += 64) out[b + k] = (float)mscore[k] / 256.f;
+  for (int k = lane; k < n; k += 64) out[b + k] = (float)(s32)mscore[k] / 256.f;
 }
 
 // Principal variation after a search: the best root move, then the moves the
