@@ -19,7 +19,12 @@ extern "C" void hs_child(const uint64_t *b, int stm, uint32_t m, int32_t *out) {
   }
   const Pos c = apply(p, m, false);
   const u64 occ = c.b1 | c.b2 | c.b3;
-  out[0] = base + eval_move_delta(EVAL_SQ.v, m) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ occ, c.b0) + eval_bishop_pair(c);
+  out[0] = base + eval_move_delta<true>(EVAL_SQ.v, p.stm, m) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ occ, c.b0) + eval_bishop_pair(c);
+  if (((m >> 27) & 7) != PNONE) {  // captures: the two short forms
+    const Pos q = apply_capture(p, m);
+    if (q.b0 != c.b0 || q.b1 != c.b1 || q.b2 != c.b2 || q.b3 != c.b3 || q.stm != c.stm) out[0] = 1 << 30;
+    if (eval_move_delta<false>(EVAL_SQ.v, p.stm, m) != eval_move_delta<true>(EVAL_SQ.v, p.stm, m)) out[0] = 1 << 30;
+  }
   out[1] = eval_bishop_pair(c);
   for (int sq = 0; sq < 64; sq++) out[1] += eval_square(c, sq);
   const u64 kb = c.b1 & c.b2 & ~c.b3 & (c.stm ? c.b0 : (c.b0 ^ occ));

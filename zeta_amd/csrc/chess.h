@@ -589,6 +589,19 @@ ZD bool ep_legal0(const Node0 &B, int from, int to, int sqep) {
   return att == 0;
 }
 
+// castling targets of the king on k, its own rooks and the attack map A given
+// (castle_targets with each square's condition written out: one king a wave)
+ZD u64 castle_squares(const Pos &p, u64 ownrooks, u64 occ, u64 A, int k) {
+  const bool okq = p.stm ? ((~p.cr & SMCRBLACKQ) == SMCRBLACKQ) : ((~p.cr & SMCRWHITEQ) == SMCRWHITEQ);
+  const bool okk = p.stm ? ((~p.cr & SMCRBLACKK) == SMCRBLACKK) : ((~p.cr & SMCRWHITEK) == SMCRWHITEK);
+  const u64 q = sel(okq && (ownrooks & bit(k - 4)) && !(occ & (bit(k - 1) | bit(k - 2) | bit(k - 3))) &&
+                        !(A & (bit(k) | bit(k - 1) | bit(k - 2))),
+                    bit(k - 2));
+  return q | sel(okk && (ownrooks & bit(k + 3)) && !(occ & (bit(k + 1) | bit(k + 2))) &&
+                     !(A & (bit(k) | bit(k + 1) | bit(k + 2))),
+                 bit(k + 2));
+}
+
 // legal targets of the own piece on sq; A = squares attacked with the own
 // king transparent (only read for the king)
 ZD u64 lane_targets(const Pos &p, const Node0 &B, u64 A, int sq, bool qs) {
@@ -597,18 +610,7 @@ ZD u64 lane_targets(const Pos &p, const Node0 &B, u64 A, int sq, bool qs) {
   const u64 own = B.own, occ = B.occ;
   if (type == KING) {
     u64 t = king_att(b) & (qs ? B.opp : ~own) & ~A;
-    if (!qs && (p.cr & SMCRALL)) {
-      const int k = sq;
-      const bool okq = p.stm ? ((~p.cr & SMCRBLACKQ) == SMCRBLACKQ) : ((~p.cr & SMCRWHITEQ) == SMCRWHITEQ);
-      const bool okk = p.stm ? ((~p.cr & SMCRBLACKK) == SMCRBLACKK) : ((~p.cr & SMCRWHITEK) == SMCRWHITEK);
-      const u64 ownrooks = own & B.rq & ~p.b2;
-      t |= sel(okq && (ownrooks & bit(k - 4)) && !(occ & (bit(k - 1) | bit(k - 2) | bit(k - 3))) &&
-                   !(A & (bit(k) | bit(k - 1) | bit(k - 2))),
-               bit(k - 2));
-      t |= sel(okk && (ownrooks & bit(k + 3)) && !(occ & (bit(k + 1) | bit(k + 2))) &&
-                   !(A & (bit(k) | bit(k + 1) | bit(k + 2))),
-               bit(k + 2));
-    }
+    if (!qs && (p.cr & SMCRALL)) t |= castle_squares(p, own & B.rq & ~p.b2, occ, A, sq);
     return t;
   }
   const u64 pm = pin_line(B, sq);

@@ -129,20 +129,20 @@ ZD int32_t eval_piece(const T *tab, u32 pc, int sq) {
   return (pc & 1) ? -v : v;
 }
 
-// How a move changes the sum of eval_piece over the board (the castle rook
-// included).
-template <class T>
-ZD int32_t eval_move_delta(const T *tab, u32 m) {
-  const int f = (int)mv_from(m), t = (int)mv_to(m);
-  const u32 pf = mv_pfrom(m), pc = mv_pcpt(m);
-  int32_t d = eval_piece(tab, mv_pto(m), t) - eval_piece(tab, pf, f);
-  d -= eval_piece(tab, pc, (int)mv_cpt(m));  // no piece: the table's first 64 entries are 0
-  if (((pf >> 1) & 7) == KING && (f - t == 2 || t - f == 2)) {
-    const u32 rook = (ROOK << 1) | (pf & 1);
-    d += f - t == 2 ? eval_piece(tab, rook, (t + 1) & 63) - eval_piece(tab, rook, (f - 4) & 63)
-                    : eval_piece(tab, rook, (t - 1) & 63) - eval_piece(tab, rook, (f + 3) & 63);
+// How a move of `stm` changes the sum of eval_piece over the board (white
+// positive); CASTLING: the move may be one, the rook's step is included.
+template <bool CASTLING, class T>
+ZD int32_t eval_move_delta(const T *tab, u32 stm, u32 m) {
+  const u32 flip = stm ? 0 : 56;
+  const u32 f = mv_from(m), t = mv_to(m), pf = (mv_pfrom(m) >> 1) & 7;
+  // (no captured piece: the table's first 64 entries are 0)
+  int32_t d = (int32_t)tab[((mv_pto(m) >> 1) & 7) * 64 + (t ^ flip)] - (int32_t)tab[pf * 64 + (f ^ flip)] +
+              (int32_t)tab[((mv_pcpt(m) >> 1) & 7) * 64 + (mv_cpt(m) ^ flip ^ 56)];
+  if (CASTLING && pf == KING && (f - t == 2 || t - f == 2)) {
+    const u32 to = f - t == 2 ? t + 1 : t - 1, from = f - t == 2 ? f - 4 : f + 3;
+    d += (int32_t)tab[ROOK * 64 + ((to & 63) ^ flip)] - (int32_t)tab[ROOK * 64 + ((from & 63) ^ flip)];
   }
-  return d;
+  return stm ? -d : d;
 }
 
 // EVAL_VALUE / 100 of the seven piece types as nibbles of a constant: no load

@@ -60,7 +60,9 @@ constexpr s32 HINT_SCORE = 32100;    // the hint table's move, above the TT move
 // move's squares), quiet moves only: src/zeta.cl:2073-2082
 constexpr s32 KILLER_SCORE = 1400;
 constexpr s32 COUNTER_SCORE = 1300;
-constexpr int NCOUNTER = 64 * 64;  // counter-move table entries per worker (LDS)
+// counter-move table entries per worker: in device memory (its 8 KB would take
+// two of eight workers' room in LDS), read once a node, ahead of its use
+constexpr int NCOUNTER = 64 * 64;
 constexpr u32 DEFERRED = 0x80000000u;  // move-stack flag: deferred by ABDADA (move codes use bits 0-29)
 constexpr u32 MOVE_BITS = 0x3FFFFFFFu;
 constexpr int ABDADA_MIN_DEPTH = 2;  // default split depth (zeta_search_opts.split_depth)
@@ -120,6 +122,7 @@ struct SearchArgs {
   u64 *rbound;       // per root (slot): best root score so far, ticket << 32 | iteration << 16 | score + 32768
   u32 *busy;
   u32 busymask;
+  u16 *ctab;          // counter moves, NCOUNTER per worker (block)
   int *queue;
   u32 *done;
   int *nworkers;
@@ -183,19 +186,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 enum { C_TT_PROBE = 0, C_TT_HIT, C_TT_CUT, C_TT_STORE, C_DEFER, C_MAXPLY, C_MLP_NODES, C_RECORDS, C_NODES, C_NCTR = 16 };
 
-// One ply of a worker's stack in LDS (64 B).  The board itself is not kept:
-// a parent board is recovered with undo() when a child returns.
-struct Ply {
-  u64 cr, hash, phash;
-  s32 alpha, beta;
-  int16_t depth;
-  u16 keyed;
-  u32 move, best, lastmove;
-  u16 mbeg, mcnt;
-  u8 stm, hmc, qs, kic, iter, ndefer, busy, searched;
-  u32 ttm;  // the node's TT move (written at its analysis, read by the pair log)
-};
-
 __device__ __forceinline__ void wsync() { __syncthreads(); }  // one wave per block
 
 // Wave-uniform values: readfirstlane puts them in SGPRs, so the node logic
@@ -235,63 +225,18 @@ __device__ __forceinline__ bool is_promo(u32 m) {
   return m && ((mv_pfrom(m) >> 1) & 7) == PAWN && ((mv_pto(m) >> 1) & 7) == QUEEN;
 }
 
-struct Node {  // the current node (wave-uniform)
+struct Node {  // the current full-width node (wave-uniform)
   Pos p;
   u64 hash, phash;
   s32 alpha, beta, depth;
-  u32 move, best, lastmove;
+  u32 move, best, ttm;
   int mbeg, mcnt;
+  u64 left;         // moves not searched yet (lists of up to 64)
   u32 hmc;
-  bool qs, kic;
-  int iter, ndefer, searched;
+  bool kic, pass2;  // in check; second pass (deferred moves)
+  int ndefer, searched;
   bool busy;
-  bool keyed;  // the move keys hold what is known of the children (key_children)
 };
-
-__device__ __forceinline__ void save(Ply &y, const Node &n) {
-  y.cr = n.p.cr;
-  y.hash = n.hash;
-  y.phash = n.phash;
-  y.alpha = n.alpha;
-  y.beta = n.beta;
-  y.depth = (int16_t)n.depth;
-  y.keyed = n.keyed;
-  y.move = n.move;
-  y.best = n.best;
-  y.lastmove = n.lastmove;
-  y.mbeg = (u16)n.mbeg;
-  y.mcnt = (u16)n.mcnt;
-  y.stm = (u8)n.p.stm;
-  y.hmc = (u8)n.hmc;
-  y.qs = n.qs;
-  y.kic = n.kic;
-  y.iter = (u8)n.iter;
-  y.ndefer = (u8)n.ndefer;
-  y.busy = n.busy;
-  y.searched = (u8)n.searched;
-}
-// parent node from its LDS record and the returning child's board
-__device__ __forceinline__ void restore(const Ply &y, const Pos &child, Node &n) {
-  n.hash = uf(y.hash);
-  n.phash = uf(y.phash);
-  n.alpha = uf(y.alpha);
-  n.beta = uf(y.beta);
-  n.depth = uf((s32)y.depth);
-  n.keyed = uf((u32)y.keyed) != 0;
-  n.move = uf(y.move);
-  n.best = uf(y.best);
-  n.lastmove = uf(y.lastmove);
-  n.mbeg = (int)uf((u32)y.mbeg);
-  n.mcnt = (int)uf((u32)y.mcnt);
-  n.hmc = uf((u32)y.hmc);
-  n.qs = uf((u32)y.qs) != 0;
-  n.kic = uf((u32)y.kic) != 0;
-  n.iter = (int)uf((u32)y.iter);
-  n.ndefer = (int)uf((u32)y.ndefer);
-  n.busy = uf((u32)y.busy) != 0;
-  n.searched = (int)uf((u32)y.searched);
-  n.p = undo(child, n.move, uf(y.cr));
-}
 
 // child hash of the alpha-beta move-up (src/zeta.cl:2297-2359), incremental
 __device__ __forceinline__ void child_hash(const Node &n, u32 m, const Pos &c, u64 &hash, u64 &phash) {
@@ -323,7 +268,7 @@ __device__ __forceinline__ u32 child_hmc(u32 hmc, u32 m) {
   return (hmc + 1) & 0xFF;
 }
 
-enum { S_ENTER = 0, S_NEXT = 1, S_RETURN = 2, S_QS = 3 };
+enum { S_ENTER = 0, S_NEXT, S_RETURN, S_QS };
 
 // TT store when a full-width node returns: with a move that raised alpha, a
 // lower bound of the node's value and that move; with none (every move
@@ -332,8 +277,8 @@ enum { S_ENTER = 0, S_NEXT = 1, S_RETURN = 2, S_QS = 3 };
 // depth-limited subtree, which a node with a zero half-move clock cannot see
 // depend on the path above it: entries are used at the same depth and clock
 // only, so no root value depends on them.
-__device__ __forceinline__ u32 tt_store(Args a, const Node &n, int sd, int lane) {
-  if (!a->ttmask || n.qs || n.depth < 1) return 0;
+__device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Node &n, int sd, int lane) {
+  if (!ttmask) return 0;
   s32 s = n.alpha;
   const int plyn = sd - 1;
   if (is_mate(s) && s > 0) s += plyn;
@@ -348,7 +293,7 @@ __device__ __forceinline__ u32 tt_store(Args a, const Node &n, int sd, int lane)
     e.y = (u32)(w0 >> 32);
     e.z = (u32)w1;
     e.w = (u32)(w1 >> 32);
-    *glob((u32x4 *)(a->tt + 2 * (key & a->ttmask))) = e;  // one 16-byte vector store
+    *glob((u32x4 *)(a->tt + 2 * (key & ttmask))) = e;  // one 16-byte vector store
   }
   return 1;
 }
@@ -423,12 +368,13 @@ __device__ __forceinline__ void add_row(float x[8], const u16 *row) {
 }
 
 // Learned ordering: network score of every move of the node (moves
-// [mbeg, mbeg+total) in LDS) written into mscore as integers.  Layer 1's position part is
+// [mbeg, mbeg+total) in LDS) given to out(slot, score), once each.  Layer 1's position part is
 // accumulated once (lane = 4 hidden units); each chunk of 32 moves then runs
 // layer 2 as 16 MFMA steps whose A operand (move x 8 hidden units, BF16) is
 // built in registers from the position part plus the move's 3-4 feature rows.
+template <class Out>
 __device__ void mlp_score_moves(Args a, const Pos &p, int mbeg, int total, int lane, float *hpos,
-                                const u32 *mmove, u32 *mscore) {
+                                const u32 *mmove, Out &&out) {
   const u16 *const w1f = a->w.w1f, *const w2t = a->w.w2t;
   const float *const wb1 = a->w.b1;
   float h4[4];
@@ -494,7 +440,7 @@ __device__ void mlp_score_moves(Args a, const Pos &p, int mbeg, int total, int l
         if (c0 + row < total) {
           float sc = (t[i] + b3) * 256.f;
           sc = sc > 31000.f ? 31000.f : (sc < -31000.f ? -31000.f : sc);
-          mscore[mbeg + c0 + row] = (u32)__float2int_rn(sc);
+          out(mbeg + c0 + row, __float2int_rn(sc));
         }
       }
     }
@@ -801,18 +747,95 @@ __device__ void serve_leave(Args a, int r, u64 tk, bool aborted, bool failed, s3
 
 constexpr u64 OUTER_RANKS = 0xFF000000000000FFULL;
 
-struct Lds {  // one worker's memory (23 KB: seven workers a CU)
+// One ply of a worker's stack: a node as 32-bit words, stored and loaded with
+// one word a lane in one LDS access (field by field, and with the parent's
+// board taken back from the child's by undoing the move, a visit spent 1100
+// instructions on it).
+constexpr int NWORDS = 23;
+enum { W_PLANES = 0, W_CR = 8, W_HASH = 10, W_PHASH = 12, W_LEFT = 14, W_WINDOW = 16, W_MOVE, W_BEST, W_LIST, W_COUNTS, W_FLAGS, W_TTM };
+struct Ply {
+  u32 w[24];
+};
+
+struct Lds {  // one worker's memory: eight workers a CU
+  __align__(16) u64 lines[64][4];  // rank, file, diagonal, anti-diagonal through a square, without it
   Ply ply[MAXPLY + 2];
   u32 mmove[MSTACK + MPAD];
   u32 mkey[MSTACK];
-  __align__(16) u16 ctab[NCOUNTER];  // counter moves by the previous move's squares (cleared 16 B at a time)
   u32 killers[MAXPLY + 2];
   union {
     float hpos[zm::NH1];  // the learned scorer's hidden vector
     u8 mstart[64];        // move-list start marks (lane + 1 at its offset)
   };
   int16_t tab[7 * 64];    // EVAL_SQ
+  // the root in progress: its ticket (serving), index and depth, the iteration,
+  // its best move so far, and the result of the last completed one
+  u64 ticket;
+  int root, depth, iteration;
+  s32 best_score, final_score;
+  u32 best_move, final_move;
 };
+
+// v_writelane_b32: x with lane k (a constant) set to v
+extern "C" __device__ int write_lane(int v, int k, int x) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ int put32(int w, int k, u32 v) { return write_lane((int)v, k, w); }
+__device__ __forceinline__ int put64(int w, int k, u64 v) { return put32(put32(w, k, (u32)v), k + 1, (u32)(v >> 32)); }
+__device__ __forceinline__ u32 get32(int w, int k) { return (u32)__builtin_amdgcn_readlane(w, k); }
+__device__ __forceinline__ u64 get64(int w, int k) { return ((u64)get32(w, k + 1) << 32) | get32(w, k); }
+__device__ __forceinline__ int put_planes(int w, const Pos &p) {
+  return put64(put64(put64(put64(w, W_PLANES, p.b0), W_PLANES + 2, p.b1), W_PLANES + 4, p.b2), W_PLANES + 6, p.b3);
+}
+__device__ __forceinline__ void get_planes(int w, Pos &p) {
+  p.b0 = get64(w, W_PLANES);
+  p.b1 = get64(w, W_PLANES + 2);
+  p.b2 = get64(w, W_PLANES + 4);
+  p.b3 = get64(w, W_PLANES + 6);
+}
+__device__ __forceinline__ u32 window(s32 alpha, s32 beta) { return ((u32)alpha & 0xFFFFu) | ((u32)beta << 16); }
+
+enum { F_STM = 1, F_CHECK = 2, F_PASS2 = 4, F_BUSY = 8 };
+
+__device__ __forceinline__ void save(Ply &y, const Node &n, int lane) {
+  int w = put_planes(0, n.p);
+  w = put64(w, W_CR, n.p.cr);
+  w = put64(w, W_HASH, n.hash);
+  w = put64(w, W_PHASH, n.phash);
+  w = put64(w, W_LEFT, n.left);
+  w = put32(w, W_WINDOW, window(n.alpha, n.beta));
+  w = put32(w, W_MOVE, n.move);
+  w = put32(w, W_BEST, n.best);
+  w = put32(w, W_LIST, (u32)n.mbeg | ((u32)n.mcnt << 16));
+  w = put32(w, W_COUNTS, (u32)n.depth | (n.hmc << 8) | ((u32)n.searched << 16) | ((u32)n.ndefer << 24));
+  w = put32(w, W_FLAGS, (n.p.stm ? F_STM : 0) | (n.kic ? F_CHECK : 0) | (n.pass2 ? F_PASS2 : 0) | (n.busy ? F_BUSY : 0));
+  w = put32(w, W_TTM, n.ttm);
+  if (lane < NWORDS) y.w[lane] = (u32)w;
+}
+__device__ __forceinline__ void restore(const Ply &y, Node &n, int lane) {
+  const int w = (int)y.w[lane < NWORDS ? lane : 0];
+  get_planes(w, n.p);
+  n.p.cr = get64(w, W_CR);
+  n.hash = get64(w, W_HASH);
+  n.phash = get64(w, W_PHASH);
+  n.left = get64(w, W_LEFT);
+  const u32 win = get32(w, W_WINDOW), list = get32(w, W_LIST), cnt = get32(w, W_COUNTS), fl = get32(w, W_FLAGS);
+  n.alpha = (s32)(int16_t)(u16)win;
+  n.beta = (s32)win >> 16;
+  n.move = get32(w, W_MOVE);
+  n.best = get32(w, W_BEST);
+  n.mbeg = (int)(list & 0xFFFFu);
+  n.mcnt = (int)(list >> 16);
+  n.depth = (s32)(cnt & 0xFFu);
+  n.hmc = (cnt >> 8) & 0xFFu;
+  n.searched = (int)((cnt >> 16) & 0xFFu);
+  n.ndefer = (int)(cnt >> 24);
+  n.p.stm = fl & F_STM ? 1u : 0u;
+  n.kic = (fl & F_CHECK) != 0;
+  n.pass2 = (fl & F_PASS2) != 0;
+  n.busy = (fl & F_BUSY) != 0;
+  n.ttm = get32(w, W_TTM);
+}
+// the move that led to the node at ply sd, 0 at the root
+__device__ __forceinline__ u32 last_move(const Lds &L, int sd) { return sd > 1 ? uf(L.ply[sd - 1].w[W_MOVE]) : 0u; }
 
 // what move generation needs of the lane's square, in registers for good
 struct LaneSq {
@@ -823,158 +846,194 @@ __device__ __forceinline__ LaneSq lane_sq(int sq) {
   const u64 b = bit(sq);
   return LaneSq{sq_lines(sq), knight_att(b), king_att(b), pawn_att(b, 0), pawn_att(b, 1)};
 }
-// the lines of a wave-uniform square k, the diagonals from the lane that has them
-__device__ __forceinline__ u64 lane_u64(u64 x, int k) {
-  return ((u64)(u32)__builtin_amdgcn_readlane((int)(u32)(x >> 32), k) << 32) |
-         (u32)__builtin_amdgcn_readlane((int)(u32)x, k);
-}
-__device__ __forceinline__ SqLines uniform_lines(const LaneSq &me, int k) {
+// the lines of a wave-uniform square, in vector registers (24 scalar ones for
+// the two kings are more than the search has to spare)
+__device__ __forceinline__ SqLines lds_lines(const Lds &L, int k) {
   const u64 b = bit(k);
-  return SqLines{b, bit(63 - k), rank_line(k) ^ b, file_line(k) ^ b, lane_u64(me.q.diag, k), lane_u64(me.q.anti, k)};
+  const u64 *q = L.lines[k];
+  return SqLines{b, bit(63 - k), q[0], q[1], q[2], q[3]};
 }
 
+// the static evaluation for the side to move: lane = square
 __device__ __forceinline__ s32 static_eval(const Pos &p, int lane) {
+  // the square is hidden from the compiler, which would keep a 64-bit mask of
+  // lanes for every condition on it through the whole search
+  asm volatile("" : "+v"(lane));
   const s32 e = wave_sum_i(eval_square(p, lane)) + eval_bishop_pair(p);
   return p.stm ? -e : e;
 }
 
-// Periodic test (every POLL_EVERY nodes): true when the worker has to leave the
-// root; renews the root bound `ra` the other workers have published.
-__device__ __forceinline__ bool poll_root(Args a, int lane, bool serving, int r, u64 ticket, int id, u64 nodes,
-                                          s32 final_score, u32 final_move, s32 &ra) {
-  u32 d = 0;
+// The periodic test (every POLL_EVERY nodes) looks at words that were loaded at
+// the test before it: the abort word lies in host memory, a read of 2 us.
+struct Poll {
+  int count;      // nodes since the last test
+  u64 nodes;      // nodes made at this root
+  u64 state;      // done (batch) or the slot word (serving)
+  u64 cancel;     // abort word, or the slot's cancelled ticket
+  u32 shut;       // serving: the grid shuts down
+  u64 rbound;     // the root bound published by the root's workers
+};
+__device__ __forceinline__ void poll_load(Args a, int r, int lane, Poll &q) {
   if (lane == 0) {
-    if (serving) {
-      d = serve_abort(a, r, ticket);
+    if (a->slots) {
+      q.state = ag_load(glob(&a->sw[r]));
+      q.cancel = ag_load(glob(&a->dcancel[r]));
+      q.shut = ag_load(&glob(a->sv)->shut);
     } else {
-      // stop when the root is finished or given up, or the host aborts
-      d = (__atomic_load_n(&a->done[r], __ATOMIC_RELAXED) != 0u || sys_load32(a->habort) != 0u) ? 1u : 0u;
-      if (!d && a->max_nodes && nodes > a->max_nodes) {
-        // over the node budget: give the root up, so that no worker picks it
-        // again (a fresh budget on the same iteration could repeat forever);
-        // its result is this worker's deepest completed iteration
-        if (atomicCAS(&a->done[r], 0u, 3u) == 0u) {
-          a->score[r] = final_score;
-          a->bestmove[r] = final_move;
-        }
-        d = 1;
+      q.state = ag_load(glob(&a->done[r]));
+      q.cancel = sys_load32(glob(a->habort));
+    }
+    q.rbound = ag_load(glob(&a->rbound[r]));
+  }
+}
+// true when the worker has to leave the root; renews the root bound `ra`
+__device__ __forceinline__ bool poll_root(Args a, const Lds &L, int lane, Poll &q, s32 &ra) {
+  q.count = 0;
+  const int r = uf(L.root);
+  bool d;
+  if (a->slots) {
+    d = sw_tk(q.state) != L.ticket || sw_st(q.state) != SV_RUN || q.cancel == L.ticket || q.shut != 0;
+  } else {
+    // stop when the root is finished or given up, or the host aborts
+    d = q.state != 0 || q.cancel != 0;
+    if (!d && a->max_nodes && q.nodes > a->max_nodes) {
+      // over the node budget: give the root up, so that no worker picks it
+      // again (a fresh budget on the same iteration could repeat forever);
+      // its result is this worker's deepest completed iteration
+      if (lane == 0 && atomicCAS(&a->done[r], 0u, 3u) == 0u) {
+        a->score[r] = L.final_score;
+        a->bestmove[r] = L.final_move;
       }
+      d = true;
     }
   }
-  if (uf(d)) return true;
-  u64 rb = 0;
-  if (lane == 0) rb = ag_load(&a->rbound[r]);
-  rb = uf(rb);
-  if ((rb >> 32) == (ticket & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == id) ra = (s32)(rb & 0xFFFF) - 32768;
+  if (uf((u32)d)) return true;
+  const u64 rb = uf(q.rbound);
+  if ((rb >> 32) == (uf(L.ticket) & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == uf(L.iteration))
+    ra = (s32)(rb & 0xFFFF) - 32768;
+  poll_load(a, r, lane, q);
   return false;
 }
 
-// What the key of a move says of the child c it makes, a quiescence node: in
-// check, nothing (a draw or a sum beyond 16 bits, which a visit finds), or its evaluation for the side
-// to move: `base` = the parent's sum of eval_piece, q / kb the king that is to
-// move in the child.
-__device__ __forceinline__ u32 child_key(const int16_t *tab, const Pos &c, u32 m, s32 base, const SqLines &q, u64 kb,
-                                         u32 stm) {
-  const u64 occ = c.b1 | c.b2 | c.b3;
-  const s32 e = base + eval_move_delta(tab, m) + pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ occ, c.b0) + eval_bishop_pair(c);
-  const u32 known = (u32)((stm ? e : -e) + 32768);
-  const bool fits = (u32)(e + 31000) <= 62000u;
-  return king_attacked(c, q, kb, stm) ? KEY_CHECK : (popc(occ) <= 2 || !fits ? KEY_OPEN : known);
-}
-// the node's sum of eval_piece: lane = square
-__device__ __forceinline__ s32 piece_sum(const int16_t *tab, u32 pc, int lane) {
-  return wave_sum_i(eval_piece(tab, pc, lane));
+// A node's move list while it is the current one: lane j holds move j and its
+// key (of lists of up to 64 moves; longer ones are read from the move stack,
+// where every list is kept).
+struct List {
+  u32 move, key;
+};
+__device__ __forceinline__ List load_list(const Lds &L, int lane, int mbeg) {
+  // lanes past the list's end read other slots of the worker's memory
+  const int k = mbeg + lane < MSTACK ? mbeg + lane : 0;
+  return List{L.mmove[k], L.mkey[k]};
 }
 
-// The children of a depth-1 node, one a lane: those that are quiescence nodes
-// get their evaluation and their check flag into the move's key.  More than
-// half of all nodes are children whose evaluation is already at or above their
-// beta (stand pat); pick_move counts these without a visit, which would cost
-// the wavefront a pass through ENTER and RETURN each.
-__device__ __forceinline__ void key_children(Lds &L, const Node &n, int lane) {
-  const u64 occ = n.p.b1 | n.p.b2 | n.p.b3;
-  const u64 kb = n.p.b1 & n.p.b2 & ~n.p.b3 & (n.p.stm ? (n.p.b0 ^ occ) : n.p.b0);  // the opponent's king
-  const SqLines q = sq_lines(kb ? lsb(kb) : 0);
-  const s32 base = piece_sum(L.tab, piece_at(n.p, lane), lane);
-  for (int k = lane; k < n.mcnt; k += 64) {
-    const u32 m = L.mmove[n.mbeg + k] & MOVE_BITS;
-    u32 key = child_key(L.tab, apply(n.p, m, false), m, base, q, kb, n.p.stm);
-    // a check or a promotion extends the child, a full half-move clock draws it
-    if (key == KEY_CHECK || is_promo(m) || child_hmc(n.hmc, m) >= 100) key = KEY_OPEN;
-    u32 *const kp = &L.mkey[n.mbeg + k];
-    *kp = (*kp & 0xFFFF0000u) | key;
-  }
-}
-
-// The next move of the list [mbeg, mbeg + mcnt): the highest score, the lowest
-// slot among equals (wave arg-max); marks it searched and gives its key before
-// that.  Moves whose child is known to stand pat at or above `limit` (the
+// The next move of a node's list: the highest score, the lowest slot among
+// equals (wave arg-max); takes it out of the list and gives its slot, code and
+// key, or -1.  Moves whose child is known to stand pat at or above `limit` (the
 // child's beta; 2 * INF: no such test) return at once in a visit and change
 // nothing at the node but the node count, for a limit that only falls while
-// the node is searched: those ahead of the next move are counted here, up to
-// the periodic poll, whose turn comes in the visit of the child it falls on.
+// the node is searched: those ahead of the next move are counted here (more
+// than half of all nodes), up to the periodic poll, whose turn comes in the
+// visit of the child it falls on.
 // defer: the list holds deferred moves, which pass 2 takes and pass 1 skips.
-__device__ __forceinline__ int pick_move(Lds &L, int lane, int mbeg, int mcnt, s32 limit, bool defer, bool pass2,
-                                         int &poll, u64 &nodes, int &searched, u32 &mk) {
-  const u32 lim = (u32)(limit + 32768);
+__device__ __forceinline__ int pick_move(Lds &L, int lane, int mbeg, int mcnt, const List &li, u64 &left, s32 limit,
+                                         bool defer, bool pass2, Poll &q, int &searched, u32 &m, u32 &mk) {
+  u32 lim = (u32)(limit + 32768);
+  lim = lim > KEY_OPEN ? lim : KEY_OPEN + 1;
+  if (mcnt <= 64) {
+    const u32 sk = (li.key | 0xFFFFu) - (u32)lane;
+    const u64 refuted = __ballot((li.key & 0xFFFFu) >= lim);
+    u64 avail = left;
+    if (defer) {
+      const u64 d = __ballot((L.mmove[mbeg + lane < MSTACK ? mbeg + lane : 0] & DEFERRED) != 0u);
+      avail &= pass2 ? d : ~d;
+    }
+    for (;;) {
+      u32 best = wave_max_u32(__builtin_amdgcn_inverse_ballot_w64(avail & ~refuted) ? sk : 0u);
+      u64 ahead = avail & refuted & __ballot(sk > best);
+      if (ahead) {
+        int c = popc(ahead);
+        bool one = false;
+        if (q.count + c >= POLL_EVERY) {
+          // a poll falls among them: one at a time up to it
+          const u32 top = wave_max_u32(__builtin_amdgcn_inverse_ballot_w64(ahead) ? sk : 0u);
+          one = q.count + 1 < POLL_EVERY;
+          if (one) ahead = 1ULL << (0xFFFFu - (top & 0xFFFFu));
+          else best = top;
+          c = one ? 1 : 0;
+        }
+        if (c) {
+          left &= ~ahead;
+          avail &= ~ahead;
+          q.count += c;
+          q.nodes += (u64)c;
+          if (!pass2) searched += c;
+          if (one) continue;
+        }
+      }
+      if (best == 0) return -1;
+      const int k = (int)(0xFFFFu - (best & 0xFFFFu));
+      left &= ~(1ULL << k);
+      m = get32((int)li.move, k) & MOVE_BITS;
+      mk = get32((int)li.key, k);
+      return k;
+    }
+  }
+  // a longer list: its searched moves lose the score in their keys
+  auto sort_key = [&](int k) {
+    if (k >= mcnt) return 0u;
+    const u32 key = L.mkey[mbeg + k];
+    u32 sk = key >> 16 ? (key | 0xFFFFu) - (u32)k : 0u;
+    if (defer && ((L.mmove[mbeg + k] & DEFERRED) != 0u) != pass2) sk = 0;
+    return sk;
+  };
+  auto refuted = [&](int k) { return k < mcnt && (L.mkey[mbeg + k] & 0xFFFFu) >= lim; };
   for (;;) {
     u32 best = 0, top = 0;
     for (int k = lane; k < mcnt; k += 64) {
-      const u32 key = L.mkey[mbeg + k];
-      u32 sk = key >> 16 ? (key & 0xFFFF0000u) | (0xFFFFu - (u32)k) : 0u;
-      if (defer && ((L.mmove[mbeg + k] & DEFERRED) != 0u) != pass2) sk = 0;
-      top = sk > top ? sk : top;
-      if ((key & 0xFFFFu) > KEY_OPEN && (key & 0xFFFFu) >= lim) sk = 0;
-      best = sk > best ? sk : best;
+      const u32 sk = sort_key(k);
+      if (refuted(k)) top = sk > top ? sk : top;
+      else best = sk > best ? sk : best;
     }
     best = wave_max_u32(best);
-    int c = 0;
-    if (__ballot(top > best)) {
-      for (int k0 = 0; k0 < mcnt; k0 += 64) {
-        const int k = k0 + lane;
-        const u32 key = k < mcnt ? L.mkey[mbeg + k] : 0u;
-        const u32 sk = key >> 16 ? (key & 0xFFFF0000u) | (0xFFFFu - (u32)k) : 0u;
-        c += popc(__ballot(sk > best && (key & 0xFFFFu) > KEY_OPEN && (key & 0xFFFFu) >= lim));
-      }
-      u32 upto = best;
-      if (poll + c >= POLL_EVERY) {
-        // a poll falls among them: one at a time up to it
-        top = wave_max_u32(top);
-        c = poll + 1 >= POLL_EVERY ? 0 : 1;
-        upto = top - 1;
-        if (!c) best = top;
-      }
-      if (c) {
-        for (int k = lane; k < mcnt; k += 64) {
-          const u32 key = L.mkey[mbeg + k];
-          const u32 sk = key >> 16 ? (key & 0xFFFF0000u) | (0xFFFFu - (u32)k) : 0u;
-          if (sk > upto && (key & 0xFFFFu) > KEY_OPEN && (key & 0xFFFFu) >= lim) L.mkey[mbeg + k] = key & 0xFFFFu;
-        }
-        poll += c;
-        nodes += (u64)c;
-        if (!pass2) searched += c;
+    top = wave_max_u32(top);
+    if (top > best) {
+      // one refuted move at a time, and a visit where the poll falls
+      best = top;
+      if (q.count + 1 < POLL_EVERY) {
+        const int k = (int)(0xFFFFu - (best & 0xFFFFu));
+        if (lane == 0) L.mkey[mbeg + k] &= 0xFFFFu;
+        q.count++;
+        q.nodes++;
+        if (!pass2) searched++;
         wsync();
-        if (upto != best) continue;
+        continue;
       }
     }
     if (best == 0) return -1;
     const int k = (int)(0xFFFFu - (best & 0xFFFFu));
+    m = uf(L.mmove[mbeg + k]) & MOVE_BITS;
     mk = uf(L.mkey[mbeg + k]);
     wsync();
     if (lane == 0) L.mkey[mbeg + k] = mk & 0xFFFFu;
+    wsync();
     return k;
   }
 }
 
-// The captures of a quiescence node (e.p. included), in the order of origin,
-// then target, with their keys; returns how many, or -1 when they do not fit
-// the move stack.  Lane = square gives the targets; then lane = capture makes
-// the child, tests its legality (the own king not attacked, only when a check,
-// a slider lined up with the king or several kings' squares make it a
-// question) and finds what the key says of it.  ep = the bit of the pawn that
-// may be taken en passant, or 0.
-__device__ __forceinline__ int gen_captures(Lds &L, const LaneSq &me, int lane, const Pos &p, u64 ep, bool kic,
-                                            int mbeg) {
+// The legal moves of a node -- QS: its captures, e.p. included -- in the order
+// of origin, then target, with their keys; returns how many, or -1 when they
+// do not fit the move stack.  Lane = square gives the targets of its piece;
+// then lane = move makes the child, tests its legality (own king not attacked;
+// only when the king is in check or a slider is lined up with it, king moves
+// by the attack map instead, e.p. on its own) and finds what the key says of
+// the child: in check, and, where the children are quiescence nodes
+// (leafward), the evaluation: the parent's piece-square sum by the move's
+// change of it, the pawn terms set by set.
+// ep = the bit of the pawn that may be taken en passant, or 0.
+template <bool QS>
+__device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, const Pos &p, u64 ep, bool kic, u32 hmc,
+                                         int mbeg, bool leafward, u32 killer, u32 counter, List &li) {
   const u64 occ = p.b1 | p.b2 | p.b3;
   const u64 white = p.b0 ^ occ;
   const u64 own = p.stm ? p.b0 : white, opp = p.stm ? white : p.b0;
@@ -983,20 +1042,30 @@ __device__ __forceinline__ int gen_captures(Lds &L, const LaneSq &me, int lane, 
   const u32 pc = piece_at(p, lane);
   const u32 type = pc >> 1;
   const bool mine = type != PNONE && (pc & 1u) == p.stm;
+  const u64 patt = p.stm ? me.bpawn : me.wpawn;
   u64 t = sel(type == ROOK || type == QUEEN, rook_sq(me.q, occ)) | sel(type == BISHOP || type == QUEEN, bishop_sq(me.q, occ));
   t = type == KNIGHT ? me.knight : t;
   t = type == KING ? me.king : t;
-  t = type == PAWN ? (p.stm ? me.bpawn : me.wpawn) : t;
-  t = mine ? t & opp : 0;
-  if (__ballot(type == KING && t != 0)) {
+  t &= QS ? opp : ~own;
+  if (QS) {
+    t = type == PAWN ? patt & opp : t;
+  } else {
+    const u64 s1 = (p.stm ? me.q.b >> 8 : me.q.b << 8) & ~occ;
+    const u64 s2 = (p.stm ? (s1 & RANK6) >> 8 : (s1 & RANK3) << 8) & ~occ;
+    t = type == PAWN ? (patt & opp) | s1 | s2 : t;
+  }
+  t = mine ? t : 0;
+  const bool rights = !QS && (p.cr & SMCRALL);
+  if (rights || __ballot(type == KING && t != 0)) {
     // squares the king may not step to: attacked with the king off the board
     const u64 o2 = occ ^ kbb;
     u64 at = (rook_sq(me.q, o2) & rq) | (bishop_sq(me.q, o2) & bq);
     at |= me.knight & ~p.b1 & p.b2 & ~p.b3;
     at |= me.king & kings;
-    at |= (p.stm ? me.bpawn : me.wpawn) & p.b1 & ~p.b2 & ~p.b3;
+    at |= patt & p.b1 & ~p.b2 & ~p.b3;
     const u64 A = __ballot((at & opp) != 0);
     if (type == KING) t &= ~A;
+    if (rights && type == KING && mine) t |= castle_squares(p, own & rq & ~p.b2, occ, A, lane);
   }
   const int ksq = kbb ? lsb(kbb) : 0;
   if (ep) {
@@ -1022,99 +1091,128 @@ __device__ __forceinline__ int gen_captures(Lds &L, const LaneSq &me, int lane, 
   int total;
   const int off = wave_exscan_i(popc(t), lane, total);
   if (total == 0) return 0;
-  if (mbeg + total > MSTACK + MPAD) return -1;
-  u32 *out = L.mmove + mbeg + off;
-  while (t) {
-    *out++ = (u32)lane | ((u32)lsb(t) << 6);
-    t &= t - 1;
+  int from = 0, to = 0;  // of the lane's move
+  const bool small = !QS && total <= 64;
+  if (small) {
+    // lane j takes move j of the list: its origin is the last lane with
+    // targets whose offset is <= j (a prefix max over start marks), its target
+    // the (j - offset)-th bit of that lane's set -- one pass instead of as
+    // many loop trips as the busiest lane has targets
+    L.mstart[lane] = 0;
+    wsync();
+    if (t) L.mstart[off] = (u8)(lane + 1);
+    wsync();
+    const int own1 = (int)zw::wave_scan_max(lane < total ? (u32)L.mstart[lane] : 0u);
+    from = (own1 > 0 ? own1 : 1) - 1;
+    const int k = lane - __shfl(off, from, 64);
+    const u64 ts = ((u64)(u32)__shfl((int)(u32)(t >> 32), from, 64) << 32) | (u32)__shfl((int)(u32)t, from, 64);
+    to = lane < total ? nth_bit(ts, k) : 0;
+  } else {
+    if (mbeg + total > MSTACK + MPAD) return -1;
+    u32 *out = L.mmove + mbeg + off;
+    while (t) {
+      *out++ = (u32)lane | ((u32)lsb(t) << 6);
+      t &= t - 1;
+    }
+    wsync();
   }
-  wsync();
-  const SqLines kq = uniform_lines(me, ksq);
-  const bool test = kbb && (kic || ((kq.rank | kq.file) & opp & rq) || ((kq.diag | kq.anti) & opp & bq));
-  const SqLines oq = uniform_lines(me, okb ? lsb(okb) : 0);
-  const s32 base = piece_sum(L.tab, pc, lane);
-  const bool odd_pawns = (p.b1 & ~p.b2 & ~p.b3 & OUTER_RANKS) != 0;  // the pawn sums want none there
+  const SqLines kq = lds_lines(L, ksq);
+  const bool test = kbb && (kic || __ballot(((((kq.rank | kq.file) & rq) | ((kq.diag | kq.anti) & bq)) & opp) != 0));
+  const SqLines oq = lds_lines(L, okb ? lsb(okb) : 0);
+  // the pawn sums want no pawn on the outer ranks
+  const bool keyed = leafward && !(p.b1 & ~p.b2 & ~p.b3 & OUTER_RANKS);
+  const s32 base = keyed ? wave_sum_i(eval_piece(L.tab, pc, lane)) : 0;
   int kept = 0;
   for (int c0 = 0; c0 < total; c0 += 64) {
     const bool act = c0 + lane < total;
-    const u32 raw = act ? L.mmove[mbeg + c0 + lane] : 0u;
-    const int from = (int)(raw & 63u), to = (int)(raw >> 6);
+    if (!small) {
+      const u32 raw = act ? L.mmove[mbeg + c0 + lane] : 0u;
+      from = (int)(raw & 63u);
+      to = (int)(raw >> 6);
+    }
     const u32 pf = (u32)__shfl((int)pc, from, 64);
     u32 cap = (u32)__shfl((int)pc, to, 64);
-    const bool pawn = (pf >> 1) == PAWN, isep = pawn && cap == 0;
+    const bool pawn = (pf >> 1) == PAWN;
+    bool isep = false;
     int x = to;
     if (ep) {  // wave-uniform
+      isep = pawn && cap == 0 && ((from ^ to) & 7);
       x = isep ? (p.stm ? to + 8 : to - 8) & 63 : to;
       cap = (u32)__shfl((int)pc, x, 64);
     }
     const u32 pt = pawn && (p.stm ? to < 8 : to >= 56) ? ((QUEEN << 1) | p.stm) : pf;
     const u32 m = mv_make((u32)from, (u32)to, (u32)x, pf, pt, cap);
-    const Pos c = apply_capture(p, m);
+    const Pos c = QS ? apply_capture(p, m) : apply(p, m, false);
     bool legal = act;
     if (test) legal = act && ((pf >> 1) == KING || isep || !king_attacked(c, kq, kbb, p.stm ^ 1u));
-    u32 key = child_key(L.tab, c, m, base, oq, okb, p.stm);
-    if (odd_pawns && key > KEY_OPEN) key = KEY_OPEN;
+    u32 key = KEY_OPEN;
+    if (keyed) {
+      const u64 cocc = c.b1 | c.b2 | c.b3;
+      const s32 e = base + (QS ? eval_move_delta<false>(L.tab, p.stm, m) : eval_move_delta<true>(L.tab, p.stm, m)) +
+                    pawn_terms(c.b1 & ~c.b2 & ~c.b3, c.b0 ^ cocc, c.b0) + eval_bishop_pair(c);
+      // a draw or a sum beyond 16 bits is left to the visit, so are
+      // promotions (extended) and full half-move clocks
+      bool known = popc(cocc) > 2 && (u32)(e + 31000) <= 62000u;
+      if (!QS) known = known && !is_promo(m) && child_hmc(hmc, m) < 100;
+      if (known) key = (u32)((p.stm ? e : -e) + 32768);
+    }
+    if (king_attacked(c, oq, okb, p.stm)) key = KEY_CHECK;
+    const s32 sc = QS ? piece_value(cap >> 1) * 16 - piece_value(pt >> 1) : plain_score(L.tab, p.stm, m, killer, counter);
     const u64 lm = __ballot(legal);
     const int slot = mbeg + kept + popc(lm & ((1ULL << lane) - 1));
     kept += popc(lm);
     if (mbeg + kept > MSTACK) return -1;
     wsync();
+    li = List{m, move_key(sc, key)};
     if (legal) {
       L.mmove[slot] = m;
-      L.mkey[slot] = move_key(piece_value(cap >> 1) * 16 - piece_value(pt >> 1), key);
+      L.mkey[slot] = li.key;
     }
   }
   wsync();
+  // illegal moves left out: the list's lanes close up
+  if (kept != total) li = load_list(L, lane, mbeg);
   return kept;
 }
-
-// v_writelane_b32: x with lane k (a constant) set to v
-extern "C" __device__ int write_lane(int v, int k, int x) __asm("llvm.amdgcn.writelane.i32");
+// the slots of a list of n moves
+__device__ __forceinline__ u64 all_moves(int n) { return n < 64 ? (1ULL << n) - 1 : ~0ULL; }
 
 enum { QS_DONE = 0, QS_ABORTED, QS_FAILED };
 
 // A quiescence node and everything below it, which is quiescence too: captures
 // only, stand pat when not in check, no table, no hash, no extension, no
 // deferral.  Apart from the full-width loop it keeps a few scalars a ply: the
-// four planes, the window and the list, one word a lane in the ply's record,
-// stored and loaded with one LDS access.  ev / known: the evaluation, if the
+// four planes, the window and the list.  ev / known: the evaluation, if the
 // parent has it; kic: in check; polled: the visit has been counted to the poll.
 __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p, s32 alpha, s32 beta, u32 hmc,
-                                       const int sd0, int mbeg, s32 ev, bool known, bool kic, bool polled, bool serving,
-                                       int r, u64 ticket, int id, s32 final_score, u32 final_move, u64 &nodes, int &poll,
-                                       s32 &ra, u32 &cvec, s32 &vout) {
+                                       const int sd0, int mbeg, s32 ev, bool known, bool kic, bool polled, Poll &q, s32 &ra,
+                                       u32 &cvec, s32 &vout) {
   int sd = sd0, mcnt = 0, unused = 0;
   u64 ep = ~p.cr & RANKS45;  // captures leave none behind
+  u64 left = 0;
+  List li = {};
   s32 v = 0;
-  bool enter = true;
+  bool arrive = true;  // at a new node; else back at a parent, with moves to go on with
   for (;;) {
-    if (enter) {
-      if (!polled && ++poll >= POLL_EVERY) {
-        poll = 0;
-        if (poll_root(args(), lane, serving, r, ticket, id, nodes, final_score, final_move, ra)) return QS_ABORTED;
-      }
+    bool leaf = false;  // the node's value is v
+    if (arrive) {
+      if (!polled && ++q.count >= POLL_EVERY && poll_root(args(), L, lane, q, ra)) return QS_ABORTED;
       polled = false;
       if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) alpha = ra - 1;
       const bool draw = hmc >= 100 || popc(p.b1 | p.b2 | p.b3) <= 2;
       // stand pat before any move generation: the reference returns the static
       // evaluation both on a stand-pat cutoff and when no capture exists
       // (src/zeta.cl:1597-1605)
-      bool leaf = false;
       if (!kic) {
-        if (draw) {
-          v = 0;
-          leaf = true;
-        } else {
-          if (!known) ev = static_eval(p, lane);
-          if (ev >= beta || sd >= MAXPLY) {
-            if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
-            v = ev;
-            leaf = true;
-          }
-        }
+        if (!known && !draw) ev = static_eval(p, lane);
+        if (draw) ev = 0;
+        leaf = draw || ev >= beta || sd >= MAXPLY;
+        if (!draw && sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
+        v = ev;
       }
       if (!leaf) {
-        mcnt = gen_captures(L, me, lane, p, ep, kic, mbeg);
+        mcnt = gen_moves<true>(L, me, lane, p, ep, kic, 0, mbeg, true, 0, 0, li);
+        left = all_moves(mcnt);
         if (mcnt < 0) {
           if (lane == 0) atomicOr(args()->err, 1u);
           return QS_FAILED;
@@ -1124,7 +1222,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
           leaf = true;
         } else if (mcnt == 0 || sd >= MAXPLY) {
           if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
-          v = kic ? static_eval(p, lane) : ev;
+          if (kic) v = static_eval(p, lane);
           leaf = true;
         } else if (!kic && ev > alpha) {
           alpha = ev;
@@ -1132,132 +1230,138 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
       }
       ep = 0;
       hmc = 0;
-      enter = !leaf;
-    } else {
-      enter = true;
     }
-    // enter: go on with this node's moves; else return v to the parent
-    int k = -1;
-    u32 mk = 0;
-    if (enter) {
-      k = pick_move(L, lane, mbeg, mcnt, sd + 1 < MAXPLY ? -alpha : 2 * INF, false, false, poll, nodes, unused, mk);
-      if (k < 0) v = alpha;
+    if (!leaf) {
+      u32 m, mk;
+      if (pick_move(L, lane, mbeg, mcnt, li, left, sd + 1 < MAXPLY ? -alpha : 2 * INF, false, false, q, unused, m, mk) >= 0) {
+        int w = put_planes(0, p);
+        w = put32(w, 8, window(alpha, beta));
+        w = put32(w, 9, (u32)mbeg | ((u32)mcnt << 16));
+        w = put64(w, 10, left);
+        if (lane < 12) L.ply[sd].w[lane] = (u32)w;
+        q.nodes++;
+        p = apply_capture(p, m);
+        const s32 t = alpha;
+        alpha = -beta;
+        beta = -t;
+        mbeg += mcnt;
+        kic = (mk & 0xFFFFu) == KEY_CHECK;
+        known = (mk & 0xFFFFu) > KEY_OPEN;
+        ev = (s32)(mk & 0xFFFFu) - 32768;
+        sd++;
+        arrive = true;
+        continue;
+      }
+      v = alpha;
     }
-    if (k >= 0) {
-      const u32 m = uf(L.mmove[mbeg + k]);
-      int w = 0;
-      w = write_lane((int)(u32)p.b0, 0, w);
-      w = write_lane((int)(u32)(p.b0 >> 32), 1, w);
-      w = write_lane((int)(u32)p.b1, 2, w);
-      w = write_lane((int)(u32)(p.b1 >> 32), 3, w);
-      w = write_lane((int)(u32)p.b2, 4, w);
-      w = write_lane((int)(u32)(p.b2 >> 32), 5, w);
-      w = write_lane((int)(u32)p.b3, 6, w);
-      w = write_lane((int)(u32)(p.b3 >> 32), 7, w);
-      w = write_lane((int)(((u32)alpha & 0xFFFFu) | ((u32)beta << 16)), 8, w);
-      w = write_lane((int)((u32)mbeg | ((u32)mcnt << 16)), 9, w);
-      if (lane < 10) ((int *)&L.ply[sd])[lane] = w;
-      nodes++;
-      p = apply_capture(p, m);
-      const s32 t = alpha;
-      alpha = -beta;
-      beta = -t;
-      mbeg += mcnt;
-      kic = (mk & 0xFFFFu) == KEY_CHECK;
-      known = (mk & 0xFFFFu) > KEY_OPEN;
-      ev = (s32)(mk & 0xFFFFu) - 32768;
-      sd++;
-      enter = true;
-      continue;
-    }
-    for (;;) {
+    // return v to the parent, and on while the parents fail high
+    do {
       if (sd == sd0) {
         vout = v;
         return QS_DONE;
       }
       sd--;
       wsync();
-      const int w = ((const int *)&L.ply[sd])[lane & 15];
-      auto word = [&](int i) { return (u32)__builtin_amdgcn_readlane(w, i); };
-      p.b0 = ((u64)word(1) << 32) | word(0);
-      p.b1 = ((u64)word(3) << 32) | word(2);
-      p.b2 = ((u64)word(5) << 32) | word(4);
-      p.b3 = ((u64)word(7) << 32) | word(6);
+      const int w = (int)L.ply[sd].w[lane < 12 ? lane : 0];
+      get_planes(w, p);
       p.stm ^= 1u;
-      alpha = (s32)(int16_t)(u16)word(8);
-      beta = (s32)word(8) >> 16;
-      mbeg = (int)(word(9) & 0xFFFFu);
-      mcnt = (int)(word(9) >> 16);
-      const s32 sc = -v;
+      const u32 win = get32(w, 8), list = get32(w, 9);
+      left = get64(w, 10);
+      alpha = (s32)(int16_t)(u16)win;
+      beta = (s32)win >> 16;
+      mbeg = (int)(list & 0xFFFFu);
+      mcnt = (int)(list >> 16);
+      v = -v;
       if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) alpha = ra - 1;
-      if (sc > alpha) alpha = sc;
-      if (alpha < beta) break;
+      if (v > alpha) alpha = v;
       v = alpha;
-    }
-    enter = false;
+    } while (alpha >= beta);
+    li = load_list(L, lane, mbeg);
+    arrive = false;
   }
 }
 
+// The TT (or hint) move of a list goes first: its key takes the score, in the
+// move stack and in the lanes.
+__device__ __forceinline__ void first_move(Lds &L, int lane, const Node &n, List &li, u32 m, s32 score) {
+  for (int k = lane; k < n.mcnt; k += 64)
+    if (L.mmove[n.mbeg + k] == m) L.mkey[n.mbeg + k] = move_key(score, L.mkey[n.mbeg + k] & 0xFFFFu);
+  wsync();
+  li = load_list(L, lane, n.mbeg);
+}
+
+// What the search asks of its arguments at every node, in one scalar register:
+// flags, the split depth (bits 8-15), the network's least depth (16-23) and
+// the logarithm of the table's size (24-31, 0 = no table).
+enum { CF_MLP = 1, CF_HINT = 2, CF_RECORDS = 4, CF_ABDADA = 8, CF_SERVING = 16 };
+__device__ __forceinline__ u32 search_config(Args a) {
+  const s32 least = a->mlp_min_depth;
+  return (a->use_mlp ? CF_MLP : 0) | (a->hint ? CF_HINT : 0) | (a->recs ? CF_RECORDS : 0) | (a->workers > 1 ? CF_ABDADA : 0) |
+         (a->slots ? CF_SERVING : 0) | ((u32)a->split_depth << 8) | ((u32)(least < 0 ? 0 : (least > 255 ? 255 : least)) << 16) |
+         ((u32)popc(a->ttmask) << 24);
+}
+__device__ __forceinline__ u64 tt_mask(u32 cfg) { return (1ULL << (cfg >> 24)) - 1; }
+
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_search(SearchArgs) {
   __shared__ Lds L;
-  Ply *const ply = L.ply;
   u32 *const mmove = L.mmove, *const mkey = L.mkey, *const killers = L.killers;
-  u16 *const ctab = L.ctab;
   const int lane = threadIdx.x;
   const LaneSq me = lane_sq(lane);
+  L.lines[lane][0] = me.q.rank;
+  L.lines[lane][1] = me.q.file;
+  L.lines[lane][2] = me.q.diag;
+  L.lines[lane][3] = me.q.anti;
   for (int k = lane; k < 7 * 64; k += 64) L.tab[k] = (int16_t)EVAL_SQ.v[k];
-  const Args a = args();
-  const int hstart = (int)((blockIdx.x * 7919u) % (unsigned)(a->nroots > 0 ? a->nroots : 1));
-
-  const bool serving = a->slots != nullptr;
-  if (serving && blockIdx.x == gridDim.x - 1) {
-    serve_scheduler(a, lane);
-    return;
-  }
   for (;;) {
+    const Args a = args();
+    const bool serving = a->slots != nullptr;
+    if (serving && blockIdx.x == gridDim.x - 1) {
+      serve_scheduler(a, lane);
+      return;
+    }
     int r;
     u64 ticket = 0;
     if (serving) {
       r = serve_pick(a, lane, ticket);
     } else {
+      const int hstart = (int)((blockIdx.x * 7919u) % (unsigned)(a->nroots > 0 ? a->nroots : 1));
       u32 ab = 0;
       if (lane == 0) ab = sys_load32(a->habort);
       r = uf(ab) ? -1 : pick_root(a, hstart, lane);
     }
     if (r < 0) return;
     int depth_r = a->depth;
-    bool mlp_r = a->use_mlp != 0;
+    u32 cfg = search_config(a);
+
     if (serving) {
       depth_r = uf(ag_load(&a->dreq[r].depth));
-      mlp_r = mlp_r && (uf(ag_load(&a->dreq[r].flags)) & 1);
+      if (!(uf(ag_load(&a->dreq[r].flags)) & 1)) cfg &= ~CF_MLP;
       if (depth_r < 1) depth_r = 1;
       if (depth_r > MAXPLY - 1) depth_r = MAXPLY - 1;
     }
 
     // ---------------------------------------------------------------- root set-up
-    // (the root position is re-read at every iteration rather than held in
-    // scalar registers through the search)
-    const u64 *const rootq = serving ? (const u64 *)a->dreq[r].pos : a->roots + (size_t)r * 8;
-    int hl = 0;
-    if (a->hist) {
-      hl = uf(a->hlen[r]);
-      hl = hl < 0 ? 0 : (hl > ZETA_HISTORY ? ZETA_HISTORY : hl);
-    }
     // killers and counter moves start empty for every root (they persist
     // across its iterations), so a root's search does not depend on which
     // worker searched what before
+    u16 *ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
     for (int k = lane; k < MAXPLY + 2; k += 64) killers[k] = 0;
     for (int k = lane; k < NCOUNTER / 8; k += 64) ((uint4 *)ctab)[k] = make_uint4(0u, 0u, 0u, 0u);
+    if (lane == 0) {
+      L.root = r;
+      L.depth = depth_r;
+      L.ticket = ticket;
+      L.final_score = 0;
+      L.final_move = 0;
+    }
     wsync();
 
     // per-root statistics in one vector register (counter k in lane k) rather
     // than in scalar registers, which the node state needs
     u32 cvec = 0;
-    u64 nodes = 0;
-    int poll = 0;
+    Poll poll = {};
+    poll_load(a, r, lane, poll);
     bool aborted = false, failed = false;
-    s32 final_score = 0;
-    u32 final_move = 0;
 
     // a worker joining a root that others are already searching starts at the
     // iteration in progress: the earlier ones would only repeat work whose
@@ -1266,7 +1370,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     if (lane == 0) id0 = (__atomic_load_n(&a->depth_done[r], __ATOMIC_RELAXED) & (serving ? 0xFFFF : ~0)) + 1;
     id0 = uf(id0);
     id0 = id0 < 1 ? 1 : (id0 > depth_r ? depth_r : id0);
-    for (int id = id0; id <= depth_r && !aborted && !failed; id++) {
+    for (int id = id0; !aborted && !failed && id <= uf(L.depth); id++) {
+      const Args a = args();
       // the best score any worker has found for a root move in this
       // iteration (refreshed at the poll); -INF until one has
       s32 ra = -INF;
@@ -1274,18 +1379,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         // a worker joining the iteration starts from the bound the root's
         // other workers have published
         u64 rb = 0;
-        if (lane == 0) rb = ag_load(&a->rbound[r]);
+        if (lane == 0) {
+          L.iteration = id;
+          L.best_score = 0;  // DRAWSCORE until a root move raises alpha (src/zeta.cl:986)
+          L.best_move = 0;
+          rb = ag_load(&a->rbound[r]);
+        }
         rb = uf(rb);
-        if ((rb >> 32) == (ticket & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == id)
+        if ((rb >> 32) == (uf(L.ticket) & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == id)
           ra = (s32)(rb & 0xFFFF) - 32768;
       }
+      const int r = uf(L.root);
       Node n;
       {
+        // (the root position is re-read at every iteration rather than held in
+        // scalar registers through the search)
         u64 q[8];
         if (serving) {
+          const u64 *const rootq = (const u64 *)a->dreq[r].pos;
           for (int k = 0; k < 8; k++) q[k] = uf(ag_load(&rootq[k]));
         } else {
-          for (int k = 0; k < 8; k++) q[k] = rootq[k];
+          const u64 *const rootq = glob(a->roots) + (size_t)r * 8;
+          for (int k = 0; k < 8; k++) q[k] = uf(rootq[k]);
         }
         n.p.b0 = q[0];
         n.p.b1 = q[1];
@@ -1300,50 +1415,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       n.alpha = -INF;
       n.beta = INF;
       n.depth = id;
-      n.lastmove = 0;
       n.mbeg = 0;
-      n.mcnt = 0;
       n.busy = false;
       n.move = 0;
-      n.best = 0;
-      n.qs = false;
-      n.kic = false;
-      n.iter = 1;
-      n.ndefer = 0;
-      n.searched = 0;
-      n.keyed = false;
+      {
+        const u64 occ = n.p.b1 | n.p.b2 | n.p.b3;
+        const u64 kbb = n.p.b1 & n.p.b2 & ~n.p.b3 & (n.p.stm ? n.p.b0 : n.p.b0 ^ occ);
+        n.kic = king_attacked(n.p, lds_lines(L, kbb ? lsb(kbb) : 0), kbb, n.p.stm ^ 1u);
+      }
       int sd = 1;
-      s32 qev = 0;  // S_QS: the node's evaluation, whether it is known, and whether this visit has polled
-      bool qknown = false, polled = false;
-      s32 rootscore = 0;  // DRAWSCORE until a root move raises alpha (src/zeta.cl:986)
-      u32 rootmove = 0;
+      u32 lastmove = 0;    // the move that led to the node being entered
       s32 v = 0;
+      List li = {};
+      s32 qev = 0;  // S_QS: the node's evaluation, if its parent knows it
+      bool qknown = false;
       int state = S_ENTER;
 
       for (;;) {
         const Args a = args();  // loads of arguments stay in this pass
         if (state == S_ENTER) {
-          // ---------------- ENTER: analyse, extend, generate, terminal tests
-          if (++poll >= POLL_EVERY) {
-            poll = 0;
-            if (poll_root(a, lane, serving, r, ticket, id, nodes, final_score, final_move, ra)) {
-              aborted = true;
-              break;
-            }
+          // ---------------- ENTER: extend, generate, terminal tests
+          if (++poll.count >= POLL_EVERY && poll_root(a, L, lane, poll, ra)) {
+            aborted = true;
+            break;
           }
           const int plyn = sd - 1;
-          // issue the TT load early: its latency overlaps the analysis below
-          const bool early = a->ttmask && sd > 1 && n.depth >= 1;
-          const u64 key = tt_key(n.hash, n.p.cr);
-          u32x4 tte = {0u, 0u, 0u, 0u};
-          if (early) tte = *glob((const u32x4 *)(a->tt + 2 * (key & a->ttmask)));
-          // node analysis, uniform part (king-square attackers by single-square
-          // sliders): gives the in-check flag before the quiescence stand pat
-          Node0 B;
-          node_basics(n.p, B);
-          n.kic = B.checkers != 0;
-          if (n.depth >= 0 && (n.kic || is_promo(n.lastmove))) n.depth++;
-          n.qs = n.depth <= 0;
+          if (n.kic || is_promo(lastmove)) n.depth++;
+          const bool qs = n.depth <= 0;
           // Another worker's root move reached ra: at the root's side (odd
           // plies from 3 on) a value at or below ra - 1 cannot make this root
           // move the best, so the window starts there.  A root move then
@@ -1351,103 +1449,69 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // score, which stays exact, as does its move.
           if ((sd & 1) && sd >= 3 && ra - 1 > n.alpha && ra - 1 < n.beta) n.alpha = ra - 1;
           n.best = 0;
-          n.iter = 1;
+          n.pass2 = false;
           n.ndefer = 0;
           n.searched = 0;
-          n.keyed = false;
           n.mcnt = 0;
-          if (n.qs) {
-            // a quiescence node whose parent did not know it for one
-            qev = 0;
+          n.ttm = 0;
+          if (qs) {
+            // a quiescence node whose evaluation its parent did not know
             qknown = false;
-            polled = true;
             state = S_QS;
             continue;
           }
-          // move generation, lane = square: the lanes answer "is my square
-          // attacked" (a ballot gives the attack map) and "which targets has
-          // my piece"; a wave prefix sum compacts the lists
-          // the attack map is read only for king moves and castling: skip it
-          // (a uniform branch) when the king has no target square to test
-          u64 A = 0;
-          const u64 kt = king_att(B.kbb) & ~B.own;
-          if (kt || (n.p.cr & SMCRALL)) A = __ballot(attacked_nk(B, lane));
-          u64 t = 0;
-          if ((B.own >> lane) & 1) t = lane_targets(n.p, B, A, lane, false);
-          int total;
-          const int off = wave_exscan_i(popc(t), lane, total);
-          n.mcnt = total;
-          if (n.mbeg + total > MSTACK) {
+          // issue the TT load early: its latency overlaps the generation below
+          const u64 ttmask = tt_mask(cfg);
+          const u64 key = tt_key(n.hash, n.p.cr);
+          u32x4 tte = {0u, 0u, 0u, 0u};
+          if (ttmask && sd > 1) tte = *glob((const u32x4 *)(a->tt + 2 * (key & ttmask)));
+          u16 *const ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
+          const u32 kil = killers[sd], cm = (u32)ctab[counter_index(lastmove)];
+          const int total = gen_moves<false>(L, me, lane, n.p, ~n.p.cr & RANKS45, n.kic, n.hmc, n.mbeg,
+                                             n.depth == 1 && sd + 1 < MAXPLY, kil, cm, li);
+          if (total < 0) {
             if (lane == 0) atomicOr(a->err, 1u);
             failed = true;
             break;
           }
-          const u32 kil = killers[sd], cm = (u32)ctab[counter_index(n.lastmove)];
-          {
-            auto put = [&](int k, int from, int to) {
-              const u32 m = make_code(n.p, from, to);
-              mmove[k] = m;
-              mkey[k] = move_key(plain_score(L.tab, n.p.stm, m, kil, cm), KEY_OPEN);
-            };
-            if (total <= 64) {
-              // lane j writes move j of the list (the same order as the loop
-              // below: origin lanes ascending, then targets ascending): its
-              // origin is the last lane with targets whose offset is <= j (a
-              // prefix max over start marks), its target the (j - offset)-th
-              // bit of that lane's set -- one pass instead of as many loop
-              // trips as the busiest lane has targets
-              u8 *const mstart = L.mstart;
-              mstart[lane] = 0;
-              wsync();
-              if (t) mstart[off] = (u8)(lane + 1);
-              wsync();
-              const int own1 = (int)zw::wave_scan_max(lane < total ? (u32)mstart[lane] : 0u);
-              const int from = (own1 > 0 ? own1 : 1) - 1;
-              const int k = lane - __shfl(off, from, 64);
-              const u64 ts = ((u64)(u32)__shfl((int)(u32)(t >> 32), from, 64) << 32) | (u32)__shfl((int)(u32)t, from, 64);
-              if (lane < total) put(n.mbeg + lane, from, nth_bit(ts, k));
-            } else {
-              int k = n.mbeg + off;
-              while (t) {
-                const int to = lsb(t);
-                t &= t - 1;
-                put(k, lane, to);
-                k++;
-              }
-            }
-          }
-          if (mlp_r && n.depth >= a->mlp_min_depth && total > 1) {
-            wsync();
-            mlp_score_moves(a, n.p, n.mbeg, total, lane, L.hpos, mmove, mkey);
-            // every move's key is its plain score plus the network's, in
-            // plain-score units (zm::PLAIN_PER_LOGIT per unit of the
-            // network's output, the scale the ranking loss is trained at);
-            // the TT move still goes first
-            for (int k = lane; k < total; k += 64) {
-              const u32 m = mmove[n.mbeg + k];
-              s32 sc = plain_score(L.tab, n.p.stm, m, kil, cm) +
-                       (s32)mkey[n.mbeg + k] * zm::PLAIN_PER_LOGIT / 256;
+          n.mcnt = total;
+          n.left = all_moves(total);
+          if ((cfg & CF_MLP) && n.depth >= (s32)((cfg >> 16) & 0xFFu) && total > 1) {
+            // every move's score is its plain score plus the network's, in
+            // plain-score units (zm::PLAIN_PER_LOGIT per unit of the network's
+            // output, the scale the ranking loss is trained at); the TT move
+            // still goes first
+            mlp_score_moves(a, n.p, n.mbeg, total, lane, L.hpos, mmove, [&](int k, s32 out) {
+              const u32 old = mkey[k];
+              s32 sc = (s32)(old >> 16) - 32768 + out * zm::PLAIN_PER_LOGIT / 256;
               sc = sc > 31999 ? 31999 : (sc < -31999 ? -31999 : sc);
-              mkey[n.mbeg + k] = move_key(sc, KEY_OPEN);
-            }
+              mkey[k] = move_key(sc, old & 0xFFFFu);
+            });
             wsync();
             lcount(cvec, C_MLP_NODES, 1);
+            li = load_list(L, lane, n.mbeg);
           }
           // terminal / draw tests in the reference's order (src/zeta.cl:1554-1609)
           bool draw = false;
-          if (total > 0 && sd > 1) {
+          if (total > 0 && sd > 1 && n.hmc >= 2) {
             // repetition against plies plyn-2, plyn-4, .. >= plyn-hmc: the
             // searched path, then the game history before the root
             bool hit = false;
             const int nn = plyn - 2 - 2 * lane;
             if (nn >= plyn - (int)n.hmc) {
-              if (nn >= 0) hit = ply[nn + 1].hash == n.hash;
-              else if (-nn - 1 < hl) hit = a->hist[(size_t)r * ZETA_HISTORY + (-nn - 1)] == n.hash;
+              if (nn >= 0) {
+                const u32 *const w = L.ply[nn + 1].w;
+                hit = (((u64)w[W_HASH + 1] << 32) | w[W_HASH]) == n.hash;
+              } else if (a->hist) {
+                int hl = a->hlen[L.root];
+                hl = hl > ZETA_HISTORY ? ZETA_HISTORY : hl;
+                if (-nn - 1 < hl) hit = a->hist[(size_t)L.root * ZETA_HISTORY + (-nn - 1)] == n.hash;
+              }
             }
             draw = __ballot(hit) != 0;
           }
           if (sd > 1 && n.hmc >= 100) draw = true;
-          if (sd > 1 && popc(B.occ) <= 2) draw = true;
+          if (sd > 1 && popc(n.p.b1 | n.p.b2 | n.p.b3) <= 2) draw = true;
           state = S_NEXT;
           if (draw) {
             v = 0;
@@ -1462,8 +1526,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           } else {
             // TT probe: move for ordering; score under the exact-depth rule
             u32 ttmove = 0;
-            if (a->ttmask && sd > 1) {
-              if (!early) tte = *glob((const u32x4 *)(a->tt + 2 * (key & a->ttmask)));
+            if (ttmask && sd > 1) {
               const u64 w0 = uf(((u64)tte.y << 32) | tte.x), w1 = uf(((u64)tte.w << 32) | tte.z);
               lcount(cvec, C_TT_PROBE, 1);
               if ((w0 ^ w1) == key && ((w1 >> 57) & 1)) {
@@ -1493,18 +1556,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               }
             }
             if (state == S_NEXT && ttmove) {
-              for (int k = lane; k < total; k += 64)
-                if (mmove[n.mbeg + k] == ttmove) mkey[n.mbeg + k] = move_key(TTMOVE_SCORE, KEY_OPEN);
+              n.ttm = ttmove;
+              first_move(L, lane, n, li, ttmove, TTMOVE_SCORE);
             }
-            if (a->recs && lane == 0) ply[sd].ttm = ttmove;
-            if (state == S_NEXT && a->hint) {
+            if (state == S_NEXT && (cfg & CF_HINT)) {
               // the hint table (a completed search's table): its move first
-              const u32x4 he = *glob((const u32x4 *)(a->hint + 2 * (key & a->ttmask)));
+              const u32x4 he = *glob((const u32x4 *)(a->hint + 2 * (key & ttmask)));
               const u64 h0 = uf(((u64)he.y << 32) | he.x), h1 = uf(((u64)he.w << 32) | he.z);
               if ((h0 ^ h1) == key && ((h1 >> 57) & 1)) {
-                const u32 hm = (u32)h1;
-                for (int k = lane; k < total; k += 64)
-                  if (mmove[n.mbeg + k] == hm) mkey[n.mbeg + k] = move_key(HINT_SCORE, KEY_OPEN);
+                first_move(L, lane, n, li, (u32)h1, HINT_SCORE);
               }
             }
           }
@@ -1514,39 +1574,49 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 
         if (state == S_NEXT) {
           // ---------------- NEXT: pick the best remaining move
-          // a node whose children are quiescence nodes: first find out what a
-          // lane each can tell of them (the pawn sums want no pawn on the
-          // outer ranks; a child at MAXPLY is counted, so made)
-          const bool leafward = n.depth <= 1 && sd + 1 < MAXPLY && n.alpha > -INF;
-          if (leafward && !n.keyed) {
-            n.keyed = true;
-            if (!(n.p.b1 & ~n.p.b2 & ~n.p.b3 & OUTER_RANKS)) key_children(L, n, lane);
-          }
-          u32 mk = 0;
-          const int pk = pick_move(L, lane, n.mbeg, n.mcnt, leafward ? -n.alpha : 2 * INF, n.ndefer > 0, n.iter == 2,
-                                   poll, nodes, n.searched, mk);
-          if (pk < 0) {
-            if (n.iter == 1 && n.ndefer > 0) {
-              n.iter = 2;
+          u32 m, mk;
+          const int k = pick_move(L, lane, n.mbeg, n.mcnt, li, n.left, n.depth == 1 && sd + 1 < MAXPLY ? -n.alpha : 2 * INF,
+                                  n.ndefer > 0, n.pass2, poll, n.searched, m, mk);
+          if (k < 0) {
+            if (!n.pass2 && n.ndefer > 0) {
+              n.pass2 = true;
               continue;
             }
             v = n.alpha;
-            lcount(cvec, C_TT_STORE, tt_store(a, n, sd, lane));
+            lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), n, sd, lane));
             state = S_RETURN;
             continue;
           }
-          const int k = n.mbeg + pk;
-          const u32 m = uf(mmove[k]) & MOVE_BITS;
-          wsync();
           const Pos c = apply(n.p, m, false);
+          if ((mk & 0xFFFFu) > KEY_OPEN) {
+            // a quiescence node, not in check, its evaluation known
+            if (!n.pass2) n.searched++;
+            poll.nodes++;
+            n.move = m;
+            save(L.ply[sd], n, lane);
+            const s32 t = n.alpha;
+            n.alpha = -n.beta;
+            n.beta = -t;
+            n.hmc = child_hmc(n.hmc, m);
+            n.mbeg += n.mcnt;
+            n.p = c;
+            n.busy = false;
+            n.kic = false;
+            qev = (s32)(mk & 0xFFFFu) - 32768;
+            qknown = true;
+            sd++;
+            wsync();
+            state = S_QS;
+            continue;
+          }
           u64 ch, cph;
           child_hash(n, m, c, ch, cph);
           // ABDADA: defer a sibling that another worker is already searching
           bool cbusy = false;
-          if (a->workers > 1 && n.depth - 1 >= a->split_depth) {
-            const u32 bidx = (u32)(tt_key(ch, c.cr) >> 40) & a->busymask;
+          if ((cfg & CF_ABDADA) && n.depth - 1 >= (s32)((cfg >> 8) & 0xFFu)) {
+            u32 *const bp = glob(a->busy) + ((u32)(tt_key(ch, c.cr) >> 40) & a->busymask);
             u32 b = 0;
-            if (lane == 0) b = __atomic_load_n(&a->busy[bidx], __ATOMIC_RELAXED);
+            if (lane == 0) b = __atomic_load_n(bp, __ATOMIC_RELAXED);
             b = uf(b);
             // batch searches defer a busy first child too, from ply 3 down:
             // a worker that finds it busy moves on to the siblings and comes
@@ -1560,70 +1630,52 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             // requests defer only later siblings (a depth 4-9 stream
             // completed 43 instead of 47 of 48 requests within 120 s with
             // the first-child deferral at every ply)
-            if (n.iter == 1 && b && (n.searched > 0 || (!serving && sd >= 3))) {
+            if (!n.pass2 && b && (n.searched > 0 || (!(cfg & CF_SERVING) && sd >= 3))) {
+              n.left |= 1ULL << (k & 63);
               if (lane == 0) {
-                mkey[k] = mk;
-                mmove[k] = m | DEFERRED;
+                mkey[n.mbeg + k] = mk;
+                mmove[n.mbeg + k] = m | DEFERRED;
               }
               n.ndefer++;
               lcount(cvec, C_DEFER, 1);
               wsync();
               continue;
             }
-            if (lane == 0) atomicAdd(&a->busy[bidx], 1u);
+            if (lane == 0) atomicAdd(bp, 1u);
             cbusy = true;
           }
-          if (n.iter == 1) n.searched++;
-          nodes++;
+          if (!n.pass2) n.searched++;
+          poll.nodes++;
           n.move = m;
-          if (lane == 0) save(ply[sd], n);
-          // descend
-          Node cn;
-          cn.p = c;
-          cn.hash = ch;
-          cn.phash = cph;
-          cn.alpha = -n.beta;
-          cn.beta = -n.alpha;
-          cn.depth = n.depth - 1;
-          cn.lastmove = m;
-          cn.hmc = child_hmc(n.hmc, m);
-          cn.mbeg = n.mbeg + n.mcnt;
-          cn.mcnt = 0;
-          cn.busy = cbusy;
-          cn.move = 0;
-          cn.best = 0;
-          cn.qs = false;
-          cn.kic = false;
-          cn.iter = 1;
-          cn.ndefer = 0;
-          cn.searched = 0;
-          cn.keyed = false;
-          n = cn;
+          save(L.ply[sd], n, lane);
+          // descend (ENTER sets the rest)
+          n.hmc = child_hmc(n.hmc, m);
+          n.p = c;
+          n.hash = ch;
+          n.phash = cph;
+          const s32 t = n.alpha;
+          n.alpha = -n.beta;
+          n.beta = -t;
+          n.depth--;
+          n.mbeg += n.mcnt;
+          n.busy = cbusy;
+          n.kic = (mk & 0xFFFFu) == KEY_CHECK;
+          lastmove = m;
           sd++;
           wsync();
           state = S_ENTER;
-          if ((mk & 0xFFFFu) > KEY_OPEN) {
-            // a quiescence node, not in check, its evaluation known
-            qev = (s32)(mk & 0xFFFFu) - 32768;
-            qknown = true;
-            polled = false;
-            n.qs = true;
-            state = S_QS;
-          }
           continue;
         }
 
         if (state == S_QS) {
           // ---------------- a quiescence node and all below it
-          const int st = qsearch(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, polled, serving,
-                                 r, ticket, id, final_score, final_move, nodes, poll, ra, cvec, v);
+          const int st = qsearch(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, !qknown, poll, ra,
+                                 cvec, v);
           if (st != QS_DONE) {
             aborted = st == QS_ABORTED;
             failed = !aborted;
             break;
           }
-          state = S_RETURN;
-          continue;
         }
 
         // ---------------- RETURN v from node sd
@@ -1631,10 +1683,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         if (sd == 1) break;
         sd--;
         wsync();
-        {
-          const Pos child = n.p;
-          restore(ply[sd], child, n);
-        }
+        restore(L.ply[sd], n, lane);
         const s32 sc = -v;
         if ((sd & 1) && sd >= 3 && ra - 1 > n.alpha && ra - 1 < n.beta) {
           // the root bound rose while this node's children were searched:
@@ -1645,31 +1694,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         if (sc > n.alpha) {
           n.alpha = sc;
           n.best = n.move;
-          if (sd == 1) {
-            rootscore = sc;
-            rootmove = n.move;
-            if (lane == 0)
-              atomicMax((unsigned long long *)&a->rbound[r],
-                        (unsigned long long)(((ticket & 0xFFFFFFFFULL) << 32) | ((u64)id << 16) | (u64)(u16)(sc + 32768)));
+          if (sd == 1 && lane == 0) {
+            L.best_score = sc;
+            L.best_move = n.move;
+            atomicMax((unsigned long long *)&a->rbound[L.root],
+                      (unsigned long long)(((L.ticket & 0xFFFFFFFFULL) << 32) | ((u64)(u32)L.iteration << 16) |
+                                           (u64)(u16)(sc + 32768)));
           }
         }
         if (n.alpha >= n.beta) {
-          if (a->recs && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
+          const u32 last = last_move(L, sd);
+          u16 *const ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
+          if ((cfg & CF_RECORDS) && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
               ((u32)(n.hash >> 40) & a->rec_mask) == 0) {
             u32 nrec = 0;
-            log_pairs(a, n, lane, mmove, L.tab, ply[sd].ttm, killers[sd], (u32)ctab[counter_index(n.lastmove)], nrec);
+            log_pairs(a, n, lane, mmove, L.tab, n.ttm, killers[sd], (u32)ctab[counter_index(last)], nrec);
             lcount(cvec, C_RECORDS, nrec);
           }
           // a quiet move that fails high becomes the ply's killer and the
           // counter move of the move before it (src/zeta.cl:1916-1933)
           if (((mv_pcpt(n.move) >> 1) & 7) == PNONE && lane == 0) {
             killers[sd] = n.move;
-            ctab[counter_index(n.lastmove)] = counter_code(n.move);
+            ctab[counter_index(last)] = counter_code(n.move);
           }
           v = n.alpha;
-          lcount(cvec, C_TT_STORE, tt_store(a, n, sd, lane));
+          lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), n, sd, lane));
           state = S_RETURN;
         } else {
+          li = load_list(L, lane, n.mbeg);
           state = S_NEXT;
         }
         wsync();
@@ -1677,24 +1729,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 
       if (aborted || failed) {
         // release the ABDADA marks still held along the path
+        const Args a = args();
         if (n.busy) busy_release(a, n.hash, n.p.cr, lane);
         wsync();
-        for (int k = 2; k < sd; k++)
-          if (ply[k].busy) busy_release(a, uf(ply[k].hash), uf(ply[k].cr), lane);
+        for (int k = 2; k < sd; k++) {
+          Node y;
+          restore(L.ply[k], y, lane);
+          if (y.busy) busy_release(a, y.hash, y.p.cr, lane);
+        }
         break;
       }
-      final_score = (rootscore == INF || rootscore == -INF) ? 0 : rootscore;  // src/search.c:137
-      final_move = rootmove;
+      const Args b = args();
+      wsync();
+      s32 fs = uf(L.best_score);
+      if (fs == INF || fs == -INF) fs = 0;  // src/search.c:137
       if (lane == 0) {
-        if (serving) slot_max_depth(&a->depth_done[r], ticket, id);
-        else atomicMax(&a->depth_done[r], id);
+        L.final_score = fs;
+        L.final_move = L.best_move;
+        if (cfg & CF_SERVING) slot_max_depth(&b->depth_done[L.root], L.ticket, id);
+        else atomicMax(&b->depth_done[L.root], id);
       }
       // a mate within this iteration's depth is the score of every deeper
       // iteration too: iterative deepening stops there (src/search.c:177-186)
-      if (is_mate(final_score) && id >= (final_score > 0 ? INF - final_score : INF + final_score)) break;
+      if (is_mate(fs) && id >= (fs > 0 ? INF - fs : INF + fs)) break;
     }
 
     // ---------------------------------------------------------------- publish
+    wsync();
+    const s32 final_score = L.final_score;
+    const u32 final_move = L.final_move;
+    const u64 nodes = poll.nodes;
+    ticket = L.ticket;
+    r = L.root;
     if (lane < C_NODES && cvec) atomicAdd((unsigned long long *)&a->ctr[lane], (unsigned long long)cvec);
     if (lane == 0) {
       // before leaving: the last worker to leave publishes the request's
@@ -1722,7 +1788,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 __global__ __launch_bounds__(64) void k_mlp_score(SearchArgs, const u64 *pos, const u32 *moves, const int *off,
                                                  float *out) {
   __shared__ u32 mmove[MSTACK];
-  __shared__ u32 mscore[MSTACK];
   __shared__ float hpos[zm::NH1];
   const Args a = args();
   const int lane = threadIdx.x, i = blockIdx.x;
@@ -1737,8 +1802,7 @@ __global__ __launch_bounds__(64) void k_mlp_score(SearchArgs, const u64 *pos, co
   const int b = off[i], n = off[i + 1] - off[i];
   for (int k = lane; k < n; k += 64) mmove[k] = moves[b + k];
   wsync();
-  mlp_score_moves(a, p, 0, n, lane, hpos, mmove, mscore);
-  for (int k = lane; k < n; k += 64) out[b + k] = (float)(s32)mscore[k] / 256.f;
+  mlp_score_moves(a, p, 0, n, lane, hpos, mmove, [&](int k, s32 sc) { out[b + k] = (float)sc / 256.f; });
 }
 
 // Principal variation after a search: the best root move, then the moves the
@@ -1790,7 +1854,7 @@ __global__ void k_clear_u64(u64 *p, size_t n) {
 
 struct SearchState {
   zr::DevBuf tt, busy, roots, queue, done, nworkers, score, bestmove, nodes, depth_done, err, ctr, hist, hlen, pv, hint,
-      rbound;
+      rbound, ctab;
   u64 tt_entries = 0;
   u64 last_ctr[C_NCTR] = {0};
 };
@@ -1808,7 +1872,7 @@ void search_release() {
   zr::release(g_ss.done); zr::release(g_ss.nworkers); zr::release(g_ss.score); zr::release(g_ss.bestmove);
   zr::release(g_ss.nodes); zr::release(g_ss.depth_done); zr::release(g_ss.err);
   zr::release(g_ss.ctr); zr::release(g_ss.hist); zr::release(g_ss.hlen); zr::release(g_ss.pv);
-  zr::release(g_ss.hint); zr::release(g_ss.rbound);
+  zr::release(g_ss.hint); zr::release(g_ss.rbound); zr::release(g_ss.ctab);
   g_ss.tt_entries = 0;
 }
 
@@ -1869,6 +1933,7 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   const u64 cap = (u64)per_cu * (u64)zr::ctx().cu_count;
   u64 want = (u64)n * (u64)workers;
   const unsigned grid = (unsigned)(want < cap ? want : cap);
+  if ((r = zr::ensure(g_ss.ctab, (size_t)grid * NCOUNTER * 2))) return r;
 
   SearchArgs sa;
   sa.roots = (const u64 *)g_ss.roots.p;
@@ -1882,6 +1947,7 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   sa.rbound = (u64 *)g_ss.rbound.p;
   sa.busy = (u32 *)g_ss.busy.p;
   sa.busymask = busy_entries - 1;
+  sa.ctab = (u16 *)g_ss.ctab.p;
   sa.queue = (int *)g_ss.queue.p;
   sa.done = (u32 *)g_ss.done.p;
   sa.nworkers = (int *)g_ss.nworkers.p;
@@ -2047,7 +2113,7 @@ struct ServeState {
   ServeHost *sh = nullptr;
   u64 *queue = nullptr, *ack = nullptr, *cancel = nullptr;
   ServeSlot *slots = nullptr;
-  zr::DevBuf sv, sw, dreq, dcancel, nodes, depth_done, busy, ctr, err, rbound, dres;
+  zr::DevBuf sv, sw, dreq, dcancel, nodes, depth_done, busy, ctr, err, rbound, dres, ctab;
   std::vector<u64> slot_ticket;  // ticket + 1 held by the slot, 0 = free
   std::vector<u64> slot_cost;
   std::vector<int> free_slots;
@@ -2105,6 +2171,7 @@ void sv_free_all() {
   zr::release(g_sv.sv); zr::release(g_sv.sw); zr::release(g_sv.dreq); zr::release(g_sv.dcancel);
   zr::release(g_sv.nodes); zr::release(g_sv.depth_done); zr::release(g_sv.busy); zr::release(g_sv.ctr);
   zr::release(g_sv.err); zr::release(g_sv.rbound); zr::release(g_sv.dres);
+  zr::release(g_sv.ctab);
   if (g_sv.pinned) (void)hipHostFree(g_sv.pinned);
   g_sv.pinned = nullptr;
   g_sv.sh = nullptr;
@@ -2214,6 +2281,10 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   const int cap = per_cu * zr::ctx().cu_count;
   int grid = o->grid > 0 && o->grid < cap ? o->grid : cap;
   if (grid < 2) grid = 2;  // one scheduler wavefront + at least one worker
+  if ((r = zr::ensure(S.ctab, (size_t)grid * NCOUNTER * 2))) {
+    sv_free_all();
+    return r;
+  }
 
   SearchArgs sa;
   memset(&sa, 0, sizeof(sa));
@@ -2223,6 +2294,7 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   sa.ttmask = tt_entries ? tt_entries - 1 : 0;
   sa.busy = (u32 *)S.busy.p;
   sa.busymask = busy_entries - 1;
+  sa.ctab = (u16 *)S.ctab.p;
   sa.nodes = (u64 *)S.nodes.p;
   sa.depth_done = (s32 *)S.depth_done.p;
   sa.err = (u32 *)S.err.p;
