@@ -43,7 +43,6 @@ ZD int pair_offset(u32 w) { return (int)w >> 8; }
 // device weight set used by the search and by training
 struct Weights {
   const u16 *w1f;   // BF16 [928][256]: W1, unit-contiguous (row gathers in the search)
-  const u16 *w1t;   // BF16 [256][928]: W1 transposed, input-contiguous
   const u16 *w2t;   // BF16 [32][256]
   const float *b1;  // [256]
   const float *b2;  // [32]

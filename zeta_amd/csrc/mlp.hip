@@ -10,15 +10,15 @@
 //   L = mean_p softplus(s(neg_p) - s(pos_p) + o_p / PLAIN_PER_LOGIT),
 // o_p the plain ordering's score difference of the pair: the search ranks
 // by plain score + PLAIN_PER_LOGIT x s, so s learns a correction of it.
-// One step is a feature pass and five products of one NT GEMM kernel,
-// C[M][N] = sum_k A[m][k] Bt[n][k], both operands BF16 with k contiguous,
-// one 32x32 C tile per wavefront built from v_mfma_f32_32x32x16_bf16, each
-// with its consumer fused in as the epilogue:
+// One step is two launches.  k_rows takes 32 rows a block from the records to
+// the gradient at the first layer's output, k_weights forms the weight
+// gradients and applies Adam to them in place.  The products, on
+// v_mfma_f32_32x32x16_bf16 tiles (BF16 operands, FP32 accumulation):
 //   z1   [B][256]   = X     [B][928]  . W1t  [256][928]  -> h1 = relu(z1 + b1)
 //   z2   [B][32]    = H1    [B][256]  . W2t  [32][256]   -> scores, loss, dz2
-//   gW2t [32][256]  = dZ2t  [32][B]   . H1t  [256][B]    split over K
 //   dH1  [B][256]   = dZ2   [B][32]   . W2   [256][32]   -> dz1, b1 gradient
-//   gW1t [256][928] = dZ1t  [256][B]  . Xt   [928][B]    split over K
+//   gW2t [32][256]  = dZ2t  [32][B]   . H1t  [256][B]
+//   gW1t [256][928] = dZ1t  [256][B]  . Xt   [928][B]
 #include <math.h>
 #include <string.h>
 
@@ -29,6 +29,7 @@
 
 using namespace zm;
 using zc::u32;
+using zc::u8;
 using zc::u64;
 
 namespace {
@@ -56,10 +57,6 @@ constexpr u16 BF_ONE = 0x3F80;
 // (the other move), so every 32-row tile of a product holds 16 whole pairs
 // and the loss is an epilogue of the layer-2 product.
 
-// One-hot features of 32 rows (16 pairs) per block, written densely in both
-// layouts (X [B][928] and Xt [928][B]) so that no clearing pass is needed:
-// the block (256 threads) collects a 32-bit row mask per feature in LDS,
-// then stores 16-B chunks of X rows and 64-B row segments of Xt.
 // record index of pair i of a training step: splitmix64 of (seed, i) mod nrec
 __device__ __forceinline__ u32 sample_index(u64 seed, int i, u64 nrec) {
   u64 z = seed + (u64)(i + 1) * 0x9E3779B97F4A7C15ULL;
@@ -69,326 +66,497 @@ __device__ __forceinline__ u32 sample_index(u64 seed, int i, u64 nrec) {
   return (u32)(z % nrec);
 }
 
-// nrec > 0: the step's pairs are drawn here (sample_index) and their indices
-// written to idx for the later kernels; nrec = 0: idx holds them already
-__global__ __launch_bounds__(256) void k_features(const PairRec *__restrict__ recs, u32 *__restrict__ idx,
-                                                  int B, u16 *X, u16 *Xt, u64 nrec, u64 seed) {
-  __shared__ u32 mask[NINP];
-  const int e0 = blockIdx.x * 32;
-  for (int f = threadIdx.x; f < NINP; f += blockDim.x) mask[f] = 0;
-  __syncthreads();
-  {
-    // eight threads per row, one rank of the board each (the first one also
-    // the move's features)
-    const int r = threadIdx.x >> 3, rank = threadIdx.x & 7, e = e0 + r;
-    u32 ri;
-    if (nrec) {
-      ri = sample_index(seed, e >> 1, nrec);
-      if (rank == 0 && !(e & 1)) idx[e >> 1] = ri;
-    } else {
-      ri = idx[e >> 1];
-    }
-    const PairRec rc = recs[ri];
-    zc::Pos p;
-    p.b0 = rc.b0; p.b1 = rc.b1; p.b2 = rc.b2; p.b3 = rc.b3; p.cr = 0; p.stm = rc.stm & 1u;
-    const u32 bit = 1u << r;
-    u64 occ = (p.b1 | p.b2 | p.b3) & (0xFFull << (8 * rank));
-    while (occ) {
-      const int sq = zc::lsb(occ);
-      occ &= occ - 1;
-      atomicOr(&mask[feat_ps(zc::piece_at(p, sq), sq, p.stm)], bit);
-    }
-    if (rank == 0) {
-      const u32 m = (e & 1) ? rc.mneg : rc.mpos;
-      atomicOr(&mask[feat_from(m, p.stm)], bit);
-      atomicOr(&mask[feat_to(m, p.stm)], bit);
-      atomicOr(&mask[feat_piece(m)], bit);
-      const int fc = feat_capt(m);
-      if (fc >= 0) atomicOr(&mask[fc], bit);
-    }
-  }
-  __syncthreads();
-  constexpr int CH = NINP / 8;  // 16-B chunks per X row
-  for (int c = threadIdx.x; c < 32 * CH; c += blockDim.x) {
-    const int r = c / CH, f0 = (c % CH) * 8;
-    u32 w[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      w[j] = (((mask[f0 + 2 * j] >> r) & 1u) ? BF_ONE : 0u) | (((mask[f0 + 2 * j + 1] >> r) & 1u) ? (u32)BF_ONE << 16 : 0u);
-    *(uint4 *)(X + (size_t)(e0 + r) * NINP + f0) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-  for (int c = threadIdx.x; c < NINP * 4; c += blockDim.x) {
-    const int f = c >> 2, r0 = (c & 3) * 8;
-    const u32 mk = mask[f] >> r0;
-    u32 w[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      w[j] = (((mk >> (2 * j)) & 1u) ? BF_ONE : 0u) | (((mk >> (2 * j + 1)) & 1u) ? (u32)BF_ONE << 16 : 0u);
-    *(uint4 *)(Xt + (size_t)f * B + e0 + r0) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
-
-// ---- NT GEMM on MFMA, C[M][N] = sum_k A[m][k] Bt[n][k], one wavefront per
-// 32x32 tile of C (and K slice), with the consumer of each product fused in
-// as its epilogue.  Accumulator layout of v_mfma_f32_32x32x16_bf16: register
-// i of lane l holds C[8*(i/4) + 4*(l/32) + i%4][l%32].
-enum { E_SPLITK, E_L1ACT, E_HEAD, E_L1BACK };
-struct Epi {
-  float *C;                   // E_SPLITK output, ldc = N
-  const float *prm;           // master weights (biases, head)
-  float *Zf;                  // E_L1ACT: h1 (FP32) out;  E_L1BACK: h1 in
-  u16 *H, *Ht;                // E_L1ACT: h1 BF16 [M][N] and [N][M];  E_L1BACK: Ht = dz1 [N][M];  E_HEAD: dz2, dz2t
-  float *grad, *loss;
-  const PairRec *recs;
-  const u32 *idx;
-  int P;
-};
-
 __device__ __forceinline__ uint2 pack4(const u16 *v) {
   return make_uint2((u32)v[0] | ((u32)v[1] << 16), (u32)v[2] | ((u32)v[3] << 16));
 }
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// C row of register i in lane half h
+__device__ __forceinline__ int c_row(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 
-// E_SPLITK: the four wavefronts of a block take four K slices of one tile and
-// add their partial tiles in LDS; the block then adds the sum into C (zeroed
-// before) with FP32 atomics, ksplit/4 blocks per tile.  E_HEAD: one block per
-// tile, its four wavefronts take four K slices and, after the LDS sum, one
-// row group (accumulator registers 4w..4w+3) each for the epilogue.
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm_nt(const u16 *__restrict__ A, int lda, const u16 *__restrict__ Bt,
-                                                 int ldb, int M, int N, int K, int ksplit, Epi ep) {
-  const int lane = threadIdx.x & 63;
-  const int tn_count = N / 32;
-  int tile, ks;
-  if (EPI == E_SPLITK || EPI == E_HEAD) {
-    const int bpt = ksplit / 4;
-    tile = blockIdx.x / bpt;
-    ks = (blockIdx.x % bpt) * 4 + (threadIdx.x >> 6);
-  } else if (EPI == E_L1BACK) {
-    // the four wavefronts of a block share a column tile (their b1 column
-    // sums meet in LDS)
-    tile = ((int)(blockIdx.x / tn_count) * 4 + (int)(threadIdx.x >> 6)) * tn_count + (int)(blockIdx.x % tn_count);
-    ks = 0;
-  } else {
-    tile = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    ks = 0;
+// A one-hot operand is eight feature bits of a row, or eight row bits of a
+// feature: a byte, turned into eight BF16 by a 4-KB table in LDS.
+struct OneHot {
+  bf16x8 v[256];
+};
+__device__ __forceinline__ void one_hot_table(OneHot &t, int tid) {
+  if (tid < 256) {
+    u32 w[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      w[j] = (((tid >> (2 * j)) & 1) ? (u32)BF_ONE : 0u) | (((tid >> (2 * j + 1)) & 1) ? (u32)BF_ONE << 16 : 0u);
+    *(uint4 *)&t.v[tid] = make_uint4(w[0], w[1], w[2], w[3]);
   }
-  const int tm = tile / tn_count, tn = tile % tn_count;
-  if (EPI != E_SPLITK && EPI != E_HEAD && EPI != E_L1BACK && tm * 32 >= M) return;
-  // K slices of whole 16-steps; the last ones may be short or empty
-  const bool live = tm * 32 < M;  // E_L1BACK: false for the waves past M
-  const int kc = ((K / 16 + ksplit - 1) / ksplit) * 16, k0 = ks * kc;
-  const int kn = !live ? 0 : (K - k0 < kc ? K - k0 : kc);
-  const int r = tm * 32 + (lane & 31), c = tn * 32 + (lane & 31);
-  const int kofs = (lane >> 5) * 8;
-  const u16 *pa = A + (size_t)r * lda + kofs + k0;
-  const u16 *pb = Bt + (size_t)c * ldb + kofs + k0;
-  // E_HEAD: the plain score differences of this lane's two pairs, loaded
-  // (index, then record) while the products run
-  u32 hdw[2] = {0u, 0u};
-  if (EPI == E_HEAD) {
-    const int rb = tm * 32 + 8 * (threadIdx.x >> 6) + 4 * (lane >> 5);
-    hdw[0] = ep.recs[ep.idx[rb >> 1]].depth;
-    hdw[1] = ep.recs[ep.idx[(rb + 2) >> 1]].depth;
+}
+
+// The 16-bit operands of the products lie in memory as the matrix unit takes
+// them: the 32x16 block (tile t, step s) is 1 KB, 16 bytes a lane -- index
+// c = t * 32 + (lane & 31), k = s * 16 + 8 * (lane >> 5) + 0..7 -- so that a
+// wavefront's operand is one contiguous load.  (Row by row, a load touched 64
+// lines a power of two apart: the weight gradients of 16384 pairs took 130 us.)
+__device__ __forceinline__ size_t frag(int t, int s, int steps) { return ((size_t)t * steps + s) * 512; }
+// element (c, k) of it
+__device__ __forceinline__ size_t frag_at(int c, int k, int steps) {
+  return frag(c >> 5, k >> 4, steps) + (((k >> 3) & 1) * 32 + (c & 31)) * 8 + (k & 7);
+}
+
+// A barrier for data in LDS: loads from and stores to device memory stay in
+// flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+constexpr int TPB = 512;       // eight wavefronts
+constexpr int NW = TPB / 64;
+constexpr int HS = NH1 + 8;    // LDS row strides that spread the banks
+constexpr int DS = NH2 + 8;
+
+// Gradients of the biases and the head, and the loss: each block of k_rows
+// leaves its part of every sum, [sum][block]; k_weights adds them up in 64
+// bits, always in the same order.
+constexpr int S_B1 = 0, S_B2 = NH1, S_W3 = S_B2 + NH2, S_B3 = S_W3 + NH2, S_LOSS = S_B3 + 1, NSUM = S_LOSS + 1;
+
+// Forward and backward of 32 rows (16 pairs) a block, from the records to
+// dz1, all of it on chip: the rows' features as bits, h1 = relu(z1 + b1) with a
+// 32-column tile a wavefront, kept in registers for relu' and as BF16 in LDS
+// for layer 2, then z2, the scores, the loss and dz2, then dz1.  What the
+// weight gradients need goes out as BF16 operands (h1, dz1, dz2) and as the
+// one-hot rows' bits, 1/16 of their BF16 size.  nrec > 0: the step's pairs are
+// drawn here (sample_index); nrec = 0: pair p is record p.
+// Bound: the W1 operand, 464 KB a block at the 64 bytes a cycle a CU loads
+// (3 us), and the record's latency; a third of it is asked for before the
+// records are looked at, a third while the features are taken apart.
+// At 2048 pairs 14.6 us, where features, layer 1, head and layer-1 backward as
+// launches of their own took 39 us; 51 us at 16384 pairs.
+__global__ __launch_bounds__(TPB) void k_rows(const PairRec *__restrict__ recs, int B, u64 nrec, u64 seed,
+                                              const float *__restrict__ prm, const u16 *__restrict__ w1x,
+                                              const u16 *__restrict__ w2t, const u16 *__restrict__ w2,
+                                              u32 *__restrict__ bits, u16 *__restrict__ h1x, u16 *__restrict__ dz2x,
+                                              u16 *__restrict__ dz1x, float *__restrict__ sums) {
+  __shared__ OneHot hot;
+  __shared__ u32 mask[NINP];       // feature -> rows
+  __shared__ u32 rowbits[32][NINP / 32];  // row -> features
+  __shared__ u32 depth[16];
+  __shared__ __align__(16) u16 h1s[32 * HS];
+  __shared__ __align__(16) u16 d2s[32 * DS];
+  __shared__ float red[4][16][64];
+  __shared__ float hs[4][2 * NH2 + 2];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, half = lane >> 5;
+  const int e0 = blockIdx.x * 32;
+  // operands that depend on nothing: layer 2 and its backward
+  const int c1 = 32 * w + r;  // this lane's hidden unit
+  constexpr int KS = NINP / 16, AHEAD = 20;  // layer-1 steps of 16 features; a third of them, loaded together
+  bf16x8 bw2[4], bw2t[2], bw1[AHEAD];
+  // sixteen threads per row, half a rank of the board each (the first one also
+  // the move's features)
+  const int row = tid >> 4, part = tid & 15, e = e0 + row;
+  const PairRec rc = recs[nrec ? sample_index(seed, e >> 1, nrec) : (u32)(e >> 1)];
+  const u16 *pb = w1x + frag(w, 0, KS) + lane * 8;
+  const int units = B / 16;
+#pragma unroll
+  for (int j = 0; j < AHEAD; j++) bw1[j] = *(const bf16x8 *)(pb + 512 * j);
+#pragma unroll
+  for (int j = 0; j < 4; j++) bw2[j] = *(const bf16x8 *)(w2t + (size_t)r * NH1 + (4 * (w & 3) + j) * 16 + 8 * half);
+#pragma unroll
+  for (int j = 0; j < 2; j++) bw2t[j] = *(const bf16x8 *)(w2 + (size_t)c1 * NH2 + 16 * j + 8 * half);
+  const float b1c = prm[I_B1 + c1], b2o = prm[I_B2 + r], w3o = prm[I_W3 + r], b3 = prm[I_B3];
+  one_hot_table(hot, tid);
+  for (int f = tid; f < NINP; f += TPB) {
+    mask[f] = 0;
+    ((u32 *)rowbits)[f] = 0;
   }
+  lds_barrier();
+  bf16x8 next[AHEAD];
+#pragma unroll
+  for (int j = 0; j < AHEAD; j++) next[j] = *(const bf16x8 *)(pb + 512 * (AHEAD + j));
+  {
+    zc::Pos p;
+    p.b0 = rc.b0; p.b1 = rc.b1; p.b2 = rc.b2; p.b3 = rc.b3; p.cr = 0; p.stm = rc.stm & 1u;
+    const u32 bit = 1u << row;
+    auto add = [&](int f) {
+      atomicOr(&mask[f], bit);
+      atomicOr(&rowbits[row][f >> 5], 1u << (f & 31));
+    };
+    u64 occ = (p.b1 | p.b2 | p.b3) & (0xFull << (4 * part));
+    while (occ) {
+      const int sq = zc::lsb(occ);
+      occ &= occ - 1;
+      add(feat_ps(zc::piece_at(p, sq), sq, p.stm));
+    }
+    if (part == 0) {
+      const u32 m = (e & 1) ? rc.mneg : rc.mpos;
+      add(feat_from(m, p.stm));
+      add(feat_to(m, p.stm));
+      add(feat_piece(m));
+      const int fc = feat_capt(m);
+      if (fc >= 0) add(fc);
+      if (!(row & 1)) depth[row >> 1] = rc.depth;
+    }
+  }
+  lds_barrier();
+  for (int f = tid; f < NINP; f += TPB) bits[(size_t)blockIdx.x * NINP + f] = mask[f];
+
+  // z1 = X . W1t^T
   f32x16 acc = {};
-  // four 16-steps per trip, the next trip's operands loaded before this
-  // trip's MFMAs: the loads of one trip overlap the products of the last
-  // instead of each product waiting for its own load
-  int k = 0;
-  if (kn >= 64) {
-    bf16x8 a[4], b[4];
+  {
+    auto row_operand = [&](int k) { return hot.v[(rowbits[r][k >> 1] >> (16 * (k & 1) + 8 * half)) & 0xFFu]; };
+    bf16x8 a[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      a[j] = *(const bf16x8 *)(pa + 16 * j);
-      b[j] = *(const bf16x8 *)(pb + 16 * j);
+    for (int j = 0; j < 4; j++) a[j] = row_operand(j);
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+      const int g = k / AHEAD, i = k % AHEAD;
+      acc = mfma(a[k & 3], g == 1 ? next[i] : bw1[i], acc);
+      if (k + 4 < KS) a[k & 3] = row_operand(k + 4);
+      if (g == 0 && 2 * AHEAD + i < KS) bw1[i] = *(const bf16x8 *)(pb + 512 * (2 * AHEAD + i));
     }
-    for (; k + 128 <= kn; k += 64) {
-      bf16x8 na[4], nb[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        na[j] = *(const bf16x8 *)(pa + k + 64 + 16 * j);
-        nb[j] = *(const bf16x8 *)(pb + k + 64 + 16 * j);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[j], b[j], acc, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        a[j] = na[j];
-        b[j] = nb[j];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[j], b[j], acc, 0, 0, 0);
-    k += 64;
   }
-  for (; k < kn; k += 16) {
-    const bf16x8 a = *(const bf16x8 *)(pa + k);
-    const bf16x8 b = *(const bf16x8 *)(pb + k);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-  }
-  const int half = lane >> 5, col = tn * 32 + (lane & 31);
-  if (EPI == E_SPLITK) {
-    __shared__ float red[3][16][64];
-    const int w = threadIdx.x >> 6;
-    if (w) {
-#pragma unroll
-      for (int i = 0; i < 16; i++) red[w - 1][i][lane] = acc[i];
-    }
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-      for (int i = 0; i < 16; i++)
-        atomicAdd(ep.C + (size_t)(tm * 32 + 8 * (i >> 2) + 4 * half + (i & 3)) * N + col,
-                  acc[i] + red[0][i][lane] + red[1][i][lane] + red[2][i][lane]);
-    }
-  } else if (EPI == E_L1ACT) {
-    // h1 = relu(z1 + b1): FP32 (kept for relu' in the backward pass), BF16 in both layouts
-    const float bb = ep.prm[I_B1 + col];
+  float h[16];
+  {
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-      const int rb = tm * 32 + 8 * g + 4 * half;
       u16 hb[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        float h = acc[4 * g + j] + bb;
-        h = h > 0.f ? h : 0.f;
-        ep.Zf[(size_t)(rb + j) * N + col] = h;
-        hb[j] = f2bf(h);
-        ep.H[(size_t)(rb + j) * N + col] = hb[j];
+        const float x = acc[4 * g + j] + b1c;
+        h[4 * g + j] = x > 0.f ? x : 0.f;
+        hb[j] = f2bf(h[4 * g + j]);
+        h1s[c_row(4 * g + j, half) * HS + c1] = hb[j];
       }
-      *(uint2 *)(ep.Ht + (size_t)col * M + rb) = pack4(hb);
+      *(uint2 *)(h1x + frag_at(c1, e0 + c_row(4 * g, half), units)) = pack4(hb);
     }
-  } else if (EPI == E_L1BACK) {
-    // dz1 = dh1 * relu'(h1): BF16 transposed for the W1 gradient; b1 gradient
-    float cs = 0.f;
-    if (live) {
+  }
+  lds_barrier();
+
+  // z2 = H1 . W2t^T on the first four wavefronts, a quarter of the hidden
+  // units each; the partial tiles are summed in LDS and wavefront w takes the
+  // rows of registers 4w .. 4w+3: h2 = relu(z2 + b2), s = w3.h2 + b3 (sum over
+  // the 32 lanes of a half), and for its 2 pairs per half the loss
+  // softplus(s_neg - s_pos + o/PLAIN_PER_LOGIT), dz2 and the b2, W3, b3
+  // gradients and the loss
+  if (w < 4) {
+    f32x16 z = {};
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int rb = tm * 32 + 8 * g + 4 * half;
-        u16 db[4];
+    for (int j = 0; j < 4; j++) z = mfma(*(const bf16x8 *)(h1s + r * HS + (4 * w + j) * 16 + 8 * half), bw2[j], z);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const float dz = ep.Zf[(size_t)(rb + j) * N + col] > 0.f ? acc[4 * g + j] : 0.f;
-          cs += dz;
-          db[j] = f2bf(dz);
-        }
-        *(uint2 *)(ep.Ht + (size_t)col * M + rb) = pack4(db);
-      }
-    }
-    cs += __shfl_xor(cs, 32, 64);
-    __shared__ float cls[4][32];
-    if (lane < 32) cls[threadIdx.x >> 6][lane] = cs;
-    __syncthreads();
-    if (threadIdx.x < 32)
-      atomicAdd(ep.grad + I_B1 + col, cls[0][lane] + cls[1][lane] + cls[2][lane] + cls[3][lane]);
-  } else if (EPI == E_HEAD) {
-    // N = 32: the tile holds all of layer 2.  The K slices' partial tiles
-    // are summed in LDS; wavefront w then takes rows 8w + 4*half + j (j < 4,
-    // registers 4w + j): h2 = relu(z2 + b2), s = w3.h2 + b3 (sum over the 32
-    // lanes of a half), and for its 2 pairs per half the loss
-    // softplus(s_neg - s_pos + o/PLAIN_PER_LOGIT), dz2 and the b2, W3, b3
-    // gradients and the loss summed per wavefront
-    __shared__ float red[4][16][64];
-    const int w = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < 16; i++) red[w][i][lane] = acc[i];
-    __syncthreads();
-    const int o = lane & 31;
-    const float b2o = ep.prm[I_B2 + o], w3o = ep.prm[I_W3 + o], b3 = ep.prm[I_B3];
-    float h[4], sc[4];
+    for (int i = 0; i < 16; i++) red[w][i][lane] = z[i];
+  }
+  lds_barrier();
+  if (w < 4) {
+    float h2[4], sc[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const int i = 4 * w + j;
       const float z = red[0][i][lane] + red[1][i][lane] + red[2][i][lane] + red[3][i][lane] + b2o;
-      h[j] = z > 0.f ? z : 0.f;
-      float t = w3o * h[j];
+      h2[j] = z > 0.f ? z : 0.f;
+      float t = w3o * h2[j];
 #pragma unroll
       for (int x = 16; x > 0; x >>= 1) t += __shfl_xor(t, x, 64);
       sc[j] = t + b3;
     }
-    const float invP = 1.f / (float)ep.P;
+    const float invP = 1.f / (float)(B / 2);
     float gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, gl = 0.f;
+    u16 dzb[4];
 #pragma unroll
     for (int q = 0; q < 2; q++) {
       const int j = 2 * q;  // rows j, j+1 of this lane's group: an even row (cutoff move) and its pair
-      const int row = tm * 32 + 8 * w + 4 * half + j;
-      const float d = sc[j + 1] - sc[j] + (float)pair_offset(hdw[q]) / (float)PLAIN_PER_LOGIT;
+      const u32 dw = depth[(c_row(4 * w, half) + j) >> 1];
+      const float d = sc[j + 1] - sc[j] + (float)pair_offset(dw) / (float)PLAIN_PER_LOGIT;
       const float sig = 1.f / (1.f + expf(-d));
       const float l = d > 0.f ? d + log1pf(expf(-d)) : log1pf(expf(d));
       const float ds0 = -sig * invP, ds1 = sig * invP;
-      const float dz0 = h[j] > 0.f ? ds0 * w3o : 0.f, dz1 = h[j + 1] > 0.f ? ds1 * w3o : 0.f;
-      const u16 d0 = f2bf(dz0), d1 = f2bf(dz1);
-      ep.H[(size_t)row * NH2 + o] = d0;
-      ep.H[(size_t)(row + 1) * NH2 + o] = d1;
-      *(u32 *)(ep.Ht + (size_t)o * M + row) = (u32)d0 | ((u32)d1 << 16);
+      const float dz0 = h2[j] > 0.f ? ds0 * w3o : 0.f, dz1 = h2[j + 1] > 0.f ? ds1 * w3o : 0.f;
+      dzb[j] = f2bf(dz0);
+      dzb[j + 1] = f2bf(dz1);
       gb2 += dz0 + dz1;
-      gw3 += ds0 * h[j] + ds1 * h[j + 1];
-      if (o == 0) {
+      gw3 += ds0 * h2[j] + ds1 * h2[j + 1];
+      if (r == 0) {
         gb3 += ds0 + ds1;
         gl += l * invP;
       }
     }
+    const int row0 = c_row(4 * w, half);
+#pragma unroll
+    for (int j = 0; j < 4; j++) d2s[(row0 + j) * DS + r] = dzb[j];
+    *(uint2 *)(dz2x + frag_at(r, e0 + row0, units)) = pack4(dzb);
     gb2 += __shfl_xor(gb2, 32, 64);
     gw3 += __shfl_xor(gw3, 32, 64);
     gb3 += __shfl_xor(gb3, 32, 64);
     gl += __shfl_xor(gl, 32, 64);
-    // the four wavefronts' sums meet in LDS: one atomic per value and block
-    // (every block adds into the same 66 words)
-    __shared__ float hs[4][2 * NH2 + 2];
     if (lane < 32) {
-      hs[w][o] = gb2;
-      hs[w][NH2 + o] = gw3;
+      hs[w][r] = gb2;
+      hs[w][NH2 + r] = gw3;
     }
     if (lane == 0) {
       hs[w][2 * NH2] = gb3;
       hs[w][2 * NH2 + 1] = gl;
     }
-    __syncthreads();
-    const int t = threadIdx.x;
-    if (t < 2 * NH2 + 2) {
-      const float v = hs[0][t] + hs[1][t] + hs[2][t] + hs[3][t];
-      float *dst = t < NH2 ? ep.grad + I_B2 + t
-                           : (t < 2 * NH2 ? ep.grad + I_W3 + (t - NH2) : (t == 2 * NH2 ? ep.grad + I_B3 : ep.loss));
-      atomicAdd(dst, v);
+  }
+  lds_barrier();
+  if (tid < 2 * NH2 + 2)
+    sums[(size_t)(S_B2 + tid) * gridDim.x + blockIdx.x] = hs[0][tid] + hs[1][tid] + hs[2][tid] + hs[3][tid];
+
+  // dh1 = dZ2 . W2^T -> dz1 = dh1 * relu'(h1); b1 gradient
+  f32x16 dh = {};
+#pragma unroll
+  for (int j = 0; j < 2; j++) dh = mfma(*(const bf16x8 *)(d2s + r * DS + 16 * j + 8 * half), bw2t[j], dh);
+  float cs = 0.f;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    u16 db[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float dz = h[4 * g + j] > 0.f ? dh[4 * g + j] : 0.f;
+      cs += dz;
+      db[j] = f2bf(dz);
     }
+    *(uint2 *)(dz1x + frag_at(c1, e0 + c_row(4 * g, half), units)) = pack4(db);
+  }
+  cs += __shfl_xor(cs, 32, 64);
+  if (lane < 32) sums[(size_t)(S_B1 + c1) * gridDim.x + blockIdx.x] = cs;
+}
+
+// ---- weight gradients, and the use made of them in the same pass
+struct Adam {
+  float lr, b1, b2, eps, c1, c2;
+  float *prm, *m, *v;
+  u16 *w1x, *w1f, *w2t, *w2;  // BF16 working copies of the weights
+};
+struct AdamState {
+  float p, m, v;
+};
+__device__ __forceinline__ AdamState adam_load(const Adam &a, int i) { return AdamState{a.prm[i], a.m[i], a.v[i]}; }
+__device__ __forceinline__ float adam_step(const Adam &a, int i, const AdamState &s, float g) {
+  const float mi = a.b1 * s.m + (1.f - a.b1) * g;
+  const float vi = a.b2 * s.v + (1.f - a.b2) * g * g;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float p = s.p - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+  a.prm[i] = p;
+  return p;
+}
+
+__device__ __forceinline__ int w2_slices(int B) {
+  int n = 4;
+  while (n < 128 && B / (2 * n) >= 128) n *= 2;
+  return n;
+}
+
+constexpr int W1_TILES = (NH1 / 32) * (NINP / 32), W2_TILES = NH1 / 32;
+constexpr int SUM_BLOCKS = (NSUM + 31) / 32;  // 32 sums a block
+
+// gW1t [256][928] = dZ1t . X and gW2t [32][256] = dZ2t . H1: one 32x32 tile a
+// block, the batch split over its eight wavefronts and summed in LDS, so that
+// the block holds the whole gradient of its weights.  UPDATE: Adam on them
+// and their BF16 copies here (no gradient goes to memory and no pass of its
+// own updates the weights); else the gradient in the ABI's layout.  The last
+// blocks do the same for the biases and the head, whose sums k_rows left.
+// X comes from its bits (a byte is one operand).
+// At 2048 pairs 9.2 us, where the two products (22 us) and the update (6.6 us)
+// were passes of their own; at 16384 pairs 49 us, near the 64 bytes a cycle a
+// CU loads.
+template <bool UPDATE>
+__global__ __launch_bounds__(TPB) void k_weights(int B, const u32 *__restrict__ bits, const u16 *__restrict__ h1x,
+                                                 const u16 *__restrict__ dz2x, const u16 *__restrict__ dz1x, const float *__restrict__ sums,
+                                                 Adam ad, float *__restrict__ gout, float *__restrict__ loss) {
+  __shared__ OneHot hot;
+  __shared__ float red[NW][16][64];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, half = lane >> 5;
+  if (blockIdx.x >= W1_TILES + W2_TILES) {
+    const int nblk = B / 32;
+    for (int q = w; q < 32; q += NW) {
+      const int t = (blockIdx.x - (W1_TILES + W2_TILES)) * 32 + q;
+      if (t >= NSUM) break;
+      double d = 0.;
+      for (int k = lane; k < nblk; k += 64) d += (double)sums[(size_t)t * nblk + k];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+      if (lane == 0) {
+        const float g = (float)d;
+        const int i = t < S_B2 ? I_B1 + t : (t < S_W3 ? I_B2 + t - S_B2 : I_W3 + t - S_W3);
+        if (t == S_LOSS) *loss = g;
+        else if (UPDATE) (void)adam_step(ad, i, adam_load(ad, i), g);
+        else gout[t < S_B2 ? P_B1 + t : P_B2 + t - S_B2] = g;
+      }
+    }
+    return;
+  }
+  const bool second = blockIdx.x >= W1_TILES;
+  const int tile = second ? blockIdx.x - W1_TILES : blockIdx.x;
+  const int tm = second ? 0 : tile % (NH1 / 32), tn = second ? tile : tile / (NH1 / 32);
+  // The batch is cut into slices of whole 16-row products, each with an
+  // accumulator of its own, and the slices are added four at a time: eight
+  // slices (four below 1024 rows) for W1, one a wavefront; up to 128 of at
+  // least 128 rows for W2, groups of four a wavefront.  (FP32 sums taken in
+  // another order move the trained weights by 3e-4 within 100 steps.)
+  const int units = B / 16;
+  const int nslice = second ? w2_slices(B) : (B >= 1024 ? 8 : 4);
+  const int per = (units + nslice - 1) / nslice;
+  // the weights' own state, asked for before the products
+  AdamState own[2];
+  if (UPDATE) {
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      const int e = tid + q * TPB, row = e >> 5, col = e & 31;
+      own[q] = adam_load(ad, second ? I_W2T + row * NH1 + 32 * tn + col : I_W1T + (32 * tm + row) * NINP + 32 * tn + col);
+    }
+  }
+  auto slice_end = [&](int u0) { return u0 + per < units ? u0 + per : units; };
+  f32x16 acc = {};
+  // two sets of eight products' operands take turns: one is loaded while the
+  // other is used (16 KB a wavefront in flight; the scheduler would sink the
+  // loads to their uses)
+  constexpr int SET = 8;
+  auto pipeline = [&](int u0, int u1, auto &&load, auto &&use) {
+    if (u0 >= u1) return;
+    load(0, u0);
+    for (int u = u0; u < u1; u += 2 * SET) {
+      load(1, u + SET);
+      __builtin_amdgcn_sched_barrier(0);
+      use(0, u);
+      load(0, u + 2 * SET);
+      __builtin_amdgcn_sched_barrier(0);
+      use(1, u + SET);
+    }
+  };
+  if (second) {
+    const u16 *pa = dz2x + lane * 8, *pb = h1x + frag(tn, 0, units) + lane * 8;
+    for (int g = w; g < nslice / 4; g += NW) {
+      f32x16 group = {};
+      for (int q = 0; q < 4; q++) {
+        const int u0 = (4 * g + q) * per, u1 = slice_end(u0);
+        f32x16 part = {};
+        for (int u = u0; u < u1; u += SET) {
+          bf16x8 a[SET], b[SET];
+#pragma unroll
+          for (int j = 0; j < SET; j++) {
+            const int t = u + j < u1 ? u + j : u1 - 1;
+            a[j] = *(const bf16x8 *)(pa + (size_t)512 * t);
+            b[j] = *(const bf16x8 *)(pb + (size_t)512 * t);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < SET; j++) part = mfma(u + j < u1 ? a[j] : bf16x8{}, b[j], part);
+        }
+        group += part;
+      }
+      acc += group;
+    }
+  } else {
+    one_hot_table(hot, tid);
+    lds_barrier();
+    const u16 *pa = dz1x + frag(tm, 0, units) + lane * 8;
+    const u32 *px = bits + 32 * tn + r;
+    const int u0 = w * per, u1 = w < nslice ? slice_end(u0) : u0;
+    bf16x8 a[2][SET];
+    u32 x[2][SET];
+    pipeline(
+        u0, u1,
+        [&](int k, int u) {
+#pragma unroll
+          for (int j = 0; j < SET; j++) {
+            const int t = u + j < u1 ? u + j : u1 - 1;
+            a[k][j] = *(const bf16x8 *)(pa + (size_t)512 * t);
+            x[k][j] = px[(size_t)(t >> 1) * NINP];
+          }
+        },
+        [&](int k, int u) {
+#pragma unroll
+          for (int j = 0; j < SET; j++)
+            acc = mfma(a[k][j], hot.v[u + j < u1 ? (x[k][j] >> (16 * ((u + j) & 1) + 8 * half)) & 0xFFu : 0u], acc);
+        });
+  }
+#pragma unroll
+  for (int i = 0; i < 16; i++) red[w][i][lane] = acc[i];
+  lds_barrier();
+  // two elements a thread; the row (internal layout) or the column (ABI) runs
+  // over the threads' low bits, as their arrays lie in memory
+  __shared__ u16 copy[32][34];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const int e = tid + q * TPB;
+    const int row = UPDATE ? e >> 5 : e & 31, col = UPDATE ? e & 31 : e >> 5;
+    const int i = 4 * (row >> 3) + (row & 3), l = 32 * ((row >> 2) & 1) + col;
+    // (the W2 sum, whose order is free, in 64 bits)
+    float g = second ? (float)((double)red[0][i][l] + red[1][i][l] + red[2][i][l] + red[3][i][l] + red[4][i][l] +
+                               red[5][i][l] + red[6][i][l] + red[7][i][l])
+                     : (red[0][i][l] + red[1][i][l] + red[2][i][l] + red[3][i][l]) +
+                           (red[4][i][l] + red[5][i][l] + red[6][i][l] + red[7][i][l]);
+    if (second) {
+      const int o = row, u = 32 * tn + col;
+      if (UPDATE) {
+        const u16 b = f2bf(adam_step(ad, I_W2T + o * NH1 + u, own[q], g));
+        ad.w2t[o * NH1 + u] = b;
+        ad.w2[u * NH2 + o] = b;
+      } else {
+        gout[P_W2 + u * NH2 + o] = g;
+      }
+    } else {
+      const int u = 32 * tm + row, f = 32 * tn + col;
+      if (UPDATE) {
+        u16 b = 0;  // padded inputs keep zero weights
+        if (f < NIN) b = f2bf(adam_step(ad, I_W1T + u * NINP + f, own[q], g));
+        ad.w1x[frag_at(u, f, NINP / 16)] = b;
+        copy[col][row] = b;
+      } else if (f < NIN) {
+        gout[P_W1 + f * NH1 + u] = g;
+      }
+    }
+  }
+  if (UPDATE && !second) {
+    lds_barrier();
+    const int col = tid >> 4, row = 2 * (tid & 15);
+    *(u32 *)(ad.w1f + (size_t)(32 * tn + col) * NH1 + 32 * tm + row) = *(const u32 *)&copy[col][row];
   }
 }
 
-// Adam on the internal layout (padded W1 columns stay zero), and in the
-// same pass the BF16 working copies of the updated W1 and W2
-__global__ void k_adam(float *prm, const float *__restrict__ grad, float *m, float *v, int n, float lr, float b1,
-                       float b2, float eps, float c1, float c2, u16 *w1t, u16 *w1f, u16 *w2t, u16 *w2) {
+// ABI layout -> master weights and their BF16 copies; master weights -> ABI
+__global__ void k_set(const float *__restrict__ in, float *prm, u16 *w1x, u16 *w1f, u16 *w2t, u16 *w2) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float p = prm[i];
-  if (!(i < I_B1 && (i % NINP) >= NIN)) {
-    const float g = grad[i];
-    const float mi = b1 * m[i] + (1.f - b1) * g;
-    const float vi = b2 * v[i] + (1.f - b2) * g * g;
-    m[i] = mi;
-    v[i] = vi;
-    p -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    prm[i] = p;
-  }
+  if (i >= NINT) return;
+  float p;
   if (i < I_B1) {
+    const int u = i / NINP, f = i % NINP;
+    p = f < NIN ? in[P_W1 + f * NH1 + u] : 0.f;
     const u16 b = f2bf(p);
-    w1t[i] = b;
-    w1f[(i % NINP) * NH1 + i / NINP] = b;
-  } else if (i >= I_W2T && i < I_B2) {
-    const int j = i - I_W2T;
+    w1x[frag_at(u, f, NINP / 16)] = b;
+    w1f[f * NH1 + u] = b;
+  } else if (i < I_W2T) {
+    p = in[P_B1 + i - I_B1];
+  } else if (i < I_B2) {
+    const int j = i - I_W2T, o = j / NH1, u = j % NH1;
+    p = in[P_W2 + u * NH2 + o];
     const u16 b = f2bf(p);
     w2t[j] = b;
-    w2[(j % NH1) * NH2 + j / NH1] = b;
+    w2[u * NH2 + o] = b;
+  } else {
+    p = in[P_B2 + i - I_B2];
   }
+  prm[i] = p;
+}
+__global__ void k_get(const float *__restrict__ prm, float *__restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= NPARAMS) return;
+  float p;
+  if (i < P_B1) p = prm[I_W1T + (i % NH1) * NINP + i / NH1];
+  else if (i < P_W2) p = prm[I_B1 + i - P_B1];
+  else if (i < P_B2) p = prm[I_W2T + ((i - P_W2) % NH2) * NH1 + (i - P_W2) / NH2];
+  else p = prm[I_B2 + i - P_B2];
+  out[i] = p;
 }
 
 // BF16 working copies of the master weights
-__global__ void k_refresh(const float *__restrict__ prm, u16 *w1t, u16 *w1f, u16 *w2t, u16 *w2) {
+__global__ void k_refresh(const float *__restrict__ prm, u16 *w1x, u16 *w1f, u16 *w2t, u16 *w2) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < NH1 * NINP) {
     const u16 b = f2bf(prm[I_W1T + i]);
-    w1t[i] = b;
     const int u = i / NINP, f = i % NINP;
+    w1x[frag_at(u, f, NINP / 16)] = b;
     w1f[f * NH1 + u] = b;
   }
   if (i < NH2 * NH1) {
@@ -418,8 +586,8 @@ __global__ void k_init(float *prm, u64 seed) {
 }
 
 struct MlpState {
-  zr::DevBuf prm, grad, m, v, w1t, w1f, w2t, w2;     // weights
-  zr::DevBuf X, Xt, Z1, H1, H1t, dZ2, dZ2t, dZ1t, idx, loss, recs_scratch;
+  zr::DevBuf prm, grad, m, v, w1x, w1f, w2t, w2;     // weights
+  zr::DevBuf bits, h1x, dz2x, dz1x, sums, loss, recs_scratch;  // a batch
   int cap_pairs = 0;
   bool ready = false;
   int step = 0;
@@ -430,7 +598,7 @@ int ensure_weights() {
   int r;
   if ((r = zr::ensure(g_ms.prm, NINT * 4)) || (r = zr::ensure(g_ms.grad, NINT * 4)) ||
       (r = zr::ensure(g_ms.m, NINT * 4)) || (r = zr::ensure(g_ms.v, NINT * 4)) ||
-      (r = zr::ensure(g_ms.w1t, NH1 * NINP * 2)) || (r = zr::ensure(g_ms.w1f, NH1 * NINP * 2)) ||
+      (r = zr::ensure(g_ms.w1x, NH1 * NINP * 2)) || (r = zr::ensure(g_ms.w1f, NH1 * NINP * 2)) ||
       (r = zr::ensure(g_ms.w2t, NH2 * NH1 * 2)) ||
       (r = zr::ensure(g_ms.w2, NH2 * NH1 * 2)))
     return r;
@@ -441,11 +609,9 @@ int ensure_batch(int P) {
   if (g_ms.cap_pairs >= P) return ZETA_OK;
   const size_t B = 2 * (size_t)P;
   int r;
-  if ((r = zr::ensure(g_ms.X, B * NINP * 2)) || (r = zr::ensure(g_ms.Xt, B * NINP * 2)) ||
-      (r = zr::ensure(g_ms.Z1, B * NH1 * 4)) || (r = zr::ensure(g_ms.H1, B * NH1 * 2)) ||
-      (r = zr::ensure(g_ms.H1t, B * NH1 * 2)) || (r = zr::ensure(g_ms.dZ2, B * NH2 * 2)) ||
-      (r = zr::ensure(g_ms.dZ2t, B * NH2 * 2)) || (r = zr::ensure(g_ms.dZ1t, B * NH1 * 2)) ||
-      (r = zr::ensure(g_ms.idx, (size_t)P * 4)) || (r = zr::ensure(g_ms.loss, 64)))
+  if ((r = zr::ensure(g_ms.bits, B / 32 * NINP * 4)) || (r = zr::ensure(g_ms.h1x, B * NH1 * 2)) ||
+      (r = zr::ensure(g_ms.dz2x, B * NH2 * 2)) || (r = zr::ensure(g_ms.dz1x, B * NH1 * 2)) ||
+      (r = zr::ensure(g_ms.sums, B / 32 * NSUM * 4)) || (r = zr::ensure(g_ms.loss, 64)))
     return r;
   g_ms.cap_pairs = P;
   return ZETA_OK;
@@ -453,101 +619,29 @@ int ensure_batch(int P) {
 
 inline unsigned nb(size_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
-// C = A . Bt^T with epilogue EPI.  E_SPLITK: C was zeroed and K slices add
-// into it, so a product with few output tiles splits its K to fill the device
-template <int EPI>
-int gemm(const u16 *A, int lda, const u16 *Bt, int ldb, int M, int N, int K, int kid, const Epi &ep) {
-  const size_t tiles = (size_t)(M / 32) * (N / 32);
-  int ksplit = 1;
-  if (EPI == E_SPLITK) {
-    ksplit = 4;
-    while (tiles * ksplit < 1024 && K / (2 * ksplit) >= 128) ksplit *= 2;
-  } else if (EPI == E_HEAD) {
-    if (N != 32) return zr::fail(ZETA_EINVAL, "mlp gemm: the head product needs N = 32");
-    ksplit = 4;
-  }
-  if (M % 32 || N % 32 || K % 16) return zr::fail(ZETA_EINVAL, "mlp gemm: shape %d x %d x %d", M, N, K);
-  // E_L1BACK: blocks of four row tiles in one column tile (the last block's
-  // extra waves, past M, only join its barrier)
-  const size_t blocks = EPI == E_L1BACK ? (size_t)((M / 32 + 3) / 4) * (N / 32) : nb(tiles * ksplit * 64, 256);
-  ZLAUNCH(kid, (u64)M * N * K * 2, k_gemm_nt<EPI>, blocks, 256, 0, A, lda, Bt, ldb, M, N, K, ksplit, ep);
-  return ZETA_OK;
-}
-
-// forward + backward of one batch of P pairs; gradients into g_ms.grad, mean
-// loss into g_ms.loss.  nrec = 0: the record indices are in g_ms.idx already;
-// nrec > 0: the feature kernel draws them from nrec records with seed
-int fwd_bwd(const PairRec *recs, int P, u64 nrec, u64 seed) {
-  hipStream_t st = zr::ctx().stream;
+// forward and backward of one batch of P pairs (nrec = 0: the first P records;
+// nrec > 0: drawn from nrec records with seed); `ad` given: Adam with the
+// gradients, else the gradients into gout in the ABI's layout.  The mean loss
+// goes to *loss.
+int step(const PairRec *recs, int P, u64 nrec, u64 seed, const Adam *ad, float *gout, float *loss) {
   const int B = 2 * P;
-  int r;
-  ZCHECK(hipMemsetAsync(g_ms.grad.p, 0, NINT * 4, st));
-  ZCHECK(hipMemsetAsync(g_ms.loss.p, 0, 4, st));
-  u32 *idx = (u32 *)g_ms.idx.p;
-  ZLAUNCH(zr::K_MLP_FWD, B, k_features, B / 32, 256, 0, recs, idx, B, (u16 *)g_ms.X.p, (u16 *)g_ms.Xt.p, nrec,
-          seed);
-  Epi ep = {};
-  ep.prm = (const float *)g_ms.prm.p;
-  ep.grad = (float *)g_ms.grad.p;
-  ep.loss = (float *)g_ms.loss.p;
-  ep.recs = recs;
-  ep.idx = idx;
-  ep.P = P;
-  // z1 = X . W1t^T -> h1
-  ep.Zf = (float *)g_ms.Z1.p;
-  ep.H = (u16 *)g_ms.H1.p;
-  ep.Ht = (u16 *)g_ms.H1t.p;
-  if ((r = gemm<E_L1ACT>((const u16 *)g_ms.X.p, NINP, (const u16 *)g_ms.w1t.p, NINP, B, NH1, NINP, zr::K_MLP_FWD,
-                         ep)))
-    return r;
-  // z2 = H1 . W2t^T -> scores, loss, dz2 and the head's gradients
-  ep.H = (u16 *)g_ms.dZ2.p;
-  ep.Ht = (u16 *)g_ms.dZ2t.p;
-  if ((r = gemm<E_HEAD>((const u16 *)g_ms.H1.p, NH1, (const u16 *)g_ms.w2t.p, NH1, B, NH2, NH1, zr::K_MLP_BWD, ep)))
-    return r;
-  // gW2t = dZ2t . H1t^T
-  ep.C = (float *)g_ms.grad.p + I_W2T;
-  if ((r = gemm<E_SPLITK>((const u16 *)g_ms.dZ2t.p, B, (const u16 *)g_ms.H1t.p, B, NH2, NH1, B, zr::K_MLP_BWD, ep)))
-    return r;
-  // dh1 = dZ2 . W2^T -> dz1 (transposed), b1 gradient
-  ep.Ht = (u16 *)g_ms.dZ1t.p;
-  if ((r = gemm<E_L1BACK>((const u16 *)g_ms.dZ2.p, NH2, (const u16 *)g_ms.w2.p, NH2, B, NH1, NH2, zr::K_MLP_BWD,
-                          ep)))
-    return r;
-  // gW1t = dZ1t . Xt^T
-  ep.C = (float *)g_ms.grad.p + I_W1T;
-  if ((r = gemm<E_SPLITK>((const u16 *)g_ms.dZ1t.p, B, (const u16 *)g_ms.Xt.p, B, NH1, NINP, B, zr::K_MLP_BWD, ep)))
-    return r;
+  const unsigned tiles = W1_TILES + W2_TILES + SUM_BLOCKS;
+  ZLAUNCH(zr::K_MLP_FWD, B, k_rows, B / 32, TPB, 0, recs, B, nrec, seed, (const float *)g_ms.prm.p,
+          (const u16 *)g_ms.w1x.p, (const u16 *)g_ms.w2t.p, (const u16 *)g_ms.w2.p, (u32 *)g_ms.bits.p,
+          (u16 *)g_ms.h1x.p, (u16 *)g_ms.dz2x.p, (u16 *)g_ms.dz1x.p, (float *)g_ms.sums.p);
+  if (ad)
+    ZLAUNCH(zr::K_MLP_BWD, B, k_weights<true>, tiles, TPB, 0, B, (const u32 *)g_ms.bits.p, (const u16 *)g_ms.h1x.p,
+            (const u16 *)g_ms.dz2x.p, (const u16 *)g_ms.dz1x.p, (const float *)g_ms.sums.p, *ad, (float *)nullptr, loss);
+  else
+    ZLAUNCH(zr::K_MLP_BWD, B, k_weights<false>, tiles, TPB, 0, B, (const u32 *)g_ms.bits.p, (const u16 *)g_ms.h1x.p,
+            (const u16 *)g_ms.dz2x.p, (const u16 *)g_ms.dz1x.p, (const float *)g_ms.sums.p, Adam{}, gout, loss);
   return ZETA_OK;
 }
 
 int refresh() {
   ZLAUNCH(zr::K_MLP_ADAM, NH1 * NINP, k_refresh, nb((size_t)NH1 * NINP, 256), 256, 0, (const float *)g_ms.prm.p,
-          (u16 *)g_ms.w1t.p, (u16 *)g_ms.w1f.p, (u16 *)g_ms.w2t.p, (u16 *)g_ms.w2.p);
+          (u16 *)g_ms.w1x.p, (u16 *)g_ms.w1f.p, (u16 *)g_ms.w2t.p, (u16 *)g_ms.w2.p);
   return ZETA_OK;
-}
-
-// ABI layout <-> internal layout
-void to_internal(const float *in, std::vector<float> &out) {
-  out.assign(NINT, 0.f);
-  for (int f = 0; f < NIN; f++)
-    for (int u = 0; u < NH1; u++) out[I_W1T + u * NINP + f] = in[P_W1 + f * NH1 + u];
-  for (int u = 0; u < NH1; u++) out[I_B1 + u] = in[P_B1 + u];
-  for (int u = 0; u < NH1; u++)
-    for (int o = 0; o < NH2; o++) out[I_W2T + o * NH1 + u] = in[P_W2 + u * NH2 + o];
-  for (int o = 0; o < NH2; o++) out[I_B2 + o] = in[P_B2 + o];
-  for (int o = 0; o < NH2; o++) out[I_W3 + o] = in[P_W3 + o];
-  out[I_B3] = in[P_B3];
-}
-void to_abi(const std::vector<float> &in, float *out) {
-  for (int f = 0; f < NIN; f++)
-    for (int u = 0; u < NH1; u++) out[P_W1 + f * NH1 + u] = in[I_W1T + u * NINP + f];
-  for (int u = 0; u < NH1; u++) out[P_B1 + u] = in[I_B1 + u];
-  for (int u = 0; u < NH1; u++)
-    for (int o = 0; o < NH2; o++) out[P_W2 + u * NH2 + o] = in[I_W2T + o * NH1 + u];
-  for (int o = 0; o < NH2; o++) out[P_B2 + o] = in[I_B2 + o];
-  for (int o = 0; o < NH2; o++) out[P_W3 + o] = in[I_W3 + o];
-  out[P_B3] = in[I_B3];
 }
 
 }  // namespace
@@ -596,7 +690,6 @@ const zm::Weights *mlp_weights() {
   static zm::Weights w;
   if (!g_ms.ready) return nullptr;
   const float *prm = (const float *)g_ms.prm.p;
-  w.w1t = (const u16 *)g_ms.w1t.p;
   w.w1f = (const u16 *)g_ms.w1f.p;
   w.w2t = (const u16 *)g_ms.w2t.p;
   w.b1 = prm + I_B1;
@@ -607,9 +700,8 @@ const zm::Weights *mlp_weights() {
 }
 
 void mlp_release() {
-  zr::DevBuf *bufs[] = {&g_ms.prm, &g_ms.grad, &g_ms.m,   &g_ms.v,    &g_ms.w1t,  &g_ms.w1f, &g_ms.w2t, &g_ms.w2,
-                        &g_ms.X,   &g_ms.Xt,   &g_ms.Z1,  &g_ms.H1,   &g_ms.H1t,  &g_ms.dZ2,
-                        &g_ms.dZ2t, &g_ms.dZ1t, &g_ms.idx, &g_ms.loss, &g_ms.recs_scratch};
+  zr::DevBuf *bufs[] = {&g_ms.prm,  &g_ms.grad, &g_ms.m,    &g_ms.v,    &g_ms.w1x,  &g_ms.w1f,  &g_ms.w2t,         &g_ms.w2,
+                        &g_ms.bits, &g_ms.h1x,  &g_ms.dz2x, &g_ms.dz1x, &g_ms.sums, &g_ms.loss, &g_ms.recs_scratch};
   for (auto *b : bufs) zr::release(*b);
   g_ms.cap_pairs = 0;
   g_ms.ready = false;
@@ -639,13 +731,12 @@ extern "C" int zeta_mlp_set(const float *params, size_t n) {
   if (r) return r;
   if (!params || n != (size_t)NPARAMS) return zr::fail(ZETA_EINVAL, "zeta_mlp_set: expected %d floats", NPARAMS);
   if ((r = ensure_weights())) return r;
-  std::vector<float> in;
-  to_internal(params, in);
   hipStream_t st = zr::ctx().stream;
-  ZCHECK(hipMemcpyAsync(g_ms.prm.p, in.data(), NINT * 4, hipMemcpyHostToDevice, st));
+  ZCHECK(hipMemcpyAsync(g_ms.grad.p, params, (size_t)NPARAMS * 4, hipMemcpyHostToDevice, st));
+  ZLAUNCH(zr::K_MLP_ADAM, NINT, k_set, nb(NINT, 256), 256, 0, (const float *)g_ms.grad.p, (float *)g_ms.prm.p,
+          (u16 *)g_ms.w1x.p, (u16 *)g_ms.w1f.p, (u16 *)g_ms.w2t.p, (u16 *)g_ms.w2.p);
   ZCHECK(hipMemsetAsync(g_ms.m.p, 0, NINT * 4, st));
   ZCHECK(hipMemsetAsync(g_ms.v.p, 0, NINT * 4, st));
-  if ((r = refresh())) return r;
   ZCHECK(hipStreamSynchronize(st));
   zr::time_collect();
   g_ms.step = 0;
@@ -658,10 +749,10 @@ extern "C" int zeta_mlp_get(float *params, size_t n) {
   if (r) return r;
   if (!g_ms.ready) return zr::fail(ZETA_ESTATE, "zeta_mlp_get: no network (zeta_mlp_init / zeta_mlp_set first)");
   if (!params || n != (size_t)NPARAMS) return zr::fail(ZETA_EINVAL, "zeta_mlp_get: expected %d floats", NPARAMS);
-  std::vector<float> in(NINT);
-  ZCHECK(hipMemcpyAsync(in.data(), g_ms.prm.p, NINT * 4, hipMemcpyDeviceToHost, zr::ctx().stream));
+  ZLAUNCH(zr::K_MLP_ADAM, NPARAMS, k_get, nb(NPARAMS, 256), 256, 0, (const float *)g_ms.prm.p, (float *)g_ms.grad.p);
+  ZCHECK(hipMemcpyAsync(params, g_ms.grad.p, (size_t)NPARAMS * 4, hipMemcpyDeviceToHost, zr::ctx().stream));
   ZCHECK(hipStreamSynchronize(zr::ctx().stream));
-  to_abi(in, params);
+  zr::time_collect();
   return ZETA_OK;
 }
 
@@ -675,18 +766,14 @@ extern "C" int zeta_mlp_grad(const void *pairs, int npairs, float *loss, float *
   if ((r = ensure_batch(npairs)) || (r = zr::ensure(g_ms.recs_scratch, (size_t)npairs * sizeof(PairRec))))
     return r;
   hipStream_t st = zr::ctx().stream;
-  std::vector<u32> idx(npairs);
-  for (int i = 0; i < npairs; i++) idx[i] = (u32)i;
   ZCHECK(hipMemcpyAsync(g_ms.recs_scratch.p, pairs, (size_t)npairs * sizeof(PairRec), hipMemcpyHostToDevice, st));
-  ZCHECK(hipMemcpyAsync(g_ms.idx.p, idx.data(), (size_t)npairs * 4, hipMemcpyHostToDevice, st));
-  if ((r = fwd_bwd((const PairRec *)g_ms.recs_scratch.p, npairs, 0, 0))) return r;
-  std::vector<float> g(NINT);
+  if ((r = step((const PairRec *)g_ms.recs_scratch.p, npairs, 0, 0, nullptr, (float *)g_ms.grad.p, (float *)g_ms.loss.p)))
+    return r;
   float l = 0.f;
-  ZCHECK(hipMemcpyAsync(g.data(), g_ms.grad.p, NINT * 4, hipMemcpyDeviceToHost, st));
+  ZCHECK(hipMemcpyAsync(grads, g_ms.grad.p, (size_t)NPARAMS * 4, hipMemcpyDeviceToHost, st));
   ZCHECK(hipMemcpyAsync(&l, g_ms.loss.p, 4, hipMemcpyDeviceToHost, st));
   ZCHECK(hipStreamSynchronize(st));
   zr::time_collect();
-  to_abi(g, grads);
   if (loss) *loss = l;
   return ZETA_OK;
 }
@@ -705,25 +792,31 @@ extern "C" int zeta_mlp_train(int steps, int pairs_per_step, float lr, uint64_t 
   }
   if (nrec > zrec::g_cap) nrec = zrec::g_cap;
   if (nrec == 0) return zr::fail(ZETA_ESTATE, "zeta_mlp_train: no logged training pairs");
-  if ((r = ensure_batch(pairs_per_step))) return r;
+  if ((r = ensure_batch(pairs_per_step)) || (r = zr::ensure(g_ms.loss, (size_t)steps * 4))) return r;
   hipStream_t st = zr::ctx().stream;
-  std::vector<float> lv(steps > 0 ? steps : 1);
-  const float b1 = 0.9f, b2 = 0.999f;
+  Adam ad;
+  ad.lr = lr;
+  ad.b1 = 0.9f;
+  ad.b2 = 0.999f;
+  ad.eps = 1e-8f;
+  ad.prm = (float *)g_ms.prm.p;
+  ad.m = (float *)g_ms.m.p;
+  ad.v = (float *)g_ms.v.p;
+  ad.w1x = (u16 *)g_ms.w1x.p;
+  ad.w1f = (u16 *)g_ms.w1f.p;
+  ad.w2t = (u16 *)g_ms.w2t.p;
+  ad.w2 = (u16 *)g_ms.w2.p;
   for (int s = 0; s < steps; s++) {
-    if ((r = fwd_bwd((const PairRec *)zrec::g_recs.p, pairs_per_step, nrec,
-                     (u64)seed + (u64)s * 0xD1B54A32D192ED03ULL)))
-      return r;
     g_ms.step++;
-    const float c1 = 1.f - powf(b1, (float)g_ms.step), c2 = 1.f - powf(b2, (float)g_ms.step);
-    ZLAUNCH(zr::K_MLP_ADAM, NINT, k_adam, nb(NINT, 256), 256, 0, (float *)g_ms.prm.p, (const float *)g_ms.grad.p,
-            (float *)g_ms.m.p, (float *)g_ms.v.p, NINT, lr, b1, b2, 1e-8f, c1, c2, (u16 *)g_ms.w1t.p,
-            (u16 *)g_ms.w1f.p, (u16 *)g_ms.w2t.p, (u16 *)g_ms.w2.p);
-    if (losses) ZCHECK(hipMemcpyAsync(&lv[s], g_ms.loss.p, 4, hipMemcpyDeviceToHost, st));
+    ad.c1 = 1.f - powf(ad.b1, (float)g_ms.step);
+    ad.c2 = 1.f - powf(ad.b2, (float)g_ms.step);
+    if ((r = step((const PairRec *)zrec::g_recs.p, pairs_per_step, nrec, (u64)seed + (u64)s * 0xD1B54A32D192ED03ULL, &ad,
+                  nullptr, (float *)g_ms.loss.p + s)))
+      return r;
   }
+  if (losses && steps) ZCHECK(hipMemcpyAsync(losses, g_ms.loss.p, (size_t)steps * 4, hipMemcpyDeviceToHost, st));
   ZCHECK(hipStreamSynchronize(st));
   zr::time_collect();
-  if (losses)
-    for (int s = 0; s < steps; s++) losses[s] = lv[s];
   return ZETA_OK;
 }
 
