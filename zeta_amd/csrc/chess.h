@@ -88,6 +88,23 @@ ZD u64 and_or(u64 a, u64 b, u64 c) {
 #endif
 }
 
+// Any function of three boards in one v_bitop3_b32 a half: F is its truth
+// table, written as the same expression of TA, TB and TC.
+constexpr u32 TA = 0xF0, TB = 0xCC, TC = 0xAA;
+template <u32 F>
+ZD u64 bop3(u64 a, u64 b, u64 c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const u32 lo = __builtin_amdgcn_bitop3_b32((u32)a, (u32)b, (u32)c, F & 0xFF);
+  const u32 hi = __builtin_amdgcn_bitop3_b32((u32)(a >> 32), (u32)(b >> 32), (u32)(c >> 32), F & 0xFF);
+  return whole(((u64)hi << 32) | lo);
+#else
+  u64 r = 0;
+  for (u32 k = 0; k < 8; k++)
+    if (F >> k & 1) r |= (k & 4 ? a : ~a) & (k & 2 ? b : ~b) & (k & 1 ? c : ~c);
+  return r;
+#endif
+}
+
 // ---- move code: the reference's 32-bit packing (src/types.h:67-74,126-141)
 ZD u32 mv_from(u32 m) { return m & 63; }
 ZD u32 mv_to(u32 m) { return (m >> 6) & 63; }
@@ -173,6 +190,10 @@ template <int D>
 ZD u64 slide_raw(u64 g, u64 empty) {
   return shift_raw<D>(ks_fill<D>(g, empty));
 }
+template <int D>
+struct Dir {
+  static constexpr int value = D;
+};
 ZD u64 rook_att(u64 g, u64 empty) {
   return slide<0>(g, empty) | slide<1>(g, empty) | slide<2>(g, empty) | slide<3>(g, empty);
 }
@@ -189,6 +210,17 @@ ZD u64 king_att(u64 k) {
   u64 a = k | ((k << 1) & NOTA) | ((k >> 1) & NOTH);
   a |= (a << 8) | (a >> 8);
   return a ^ k;
+}
+// the same for boards that differ by lane (a uniform one keeps to the scalar
+// unit above): fused logic and whole shifts
+ZD u64 knight_att_v(u64 n) {
+  const u64 h1 = and_or(whole(n >> 1), NOTH, whole(n << 1) & NOTA);
+  const u64 h2 = and_or(whole(n >> 2), 0x3F3F3F3F3F3F3F3FULL, whole(n << 2) & 0xFCFCFCFCFCFCFCFCULL);
+  return bop3<(TA | TB | TC)>(whole(h1 << 16), whole(h1 >> 16), whole(h2 << 8)) | whole(h2 >> 8);
+}
+ZD u64 king_att_v(u64 k) {
+  const u64 a = and_or(whole(k << 1), NOTA, and_or(whole(k >> 1), NOTH, k));
+  return bop3<(TA | TB | TC)>(a, whole(a << 8), whole(a >> 8)) ^ k;
 }
 ZD u64 pawn_att(u64 p, u32 color) {
   return color ? (((p >> 7) & NOTA) | ((p >> 9) & NOTH)) : (((p << 9) & NOTA) | ((p << 7) & NOTH));
@@ -249,58 +281,113 @@ struct Legal {
   u32 stm;
 };
 
-// Checkers, check ray, x-ray and pins along one line through the king, from
-// occluded fills in its two directions U and V: R = the rays of the opponent
-// sliders S that move along the line, K = the king's own rays (each up to and
-// including the first blocker).  The first piece on the king's U ray is a
-// checker if it is in S; an own piece there is pinned if an S ray in
-// direction V reaches it from the far side.  A checker's attack continues
-// through the king along the king's opposite ray (`xray`: squares the king
-// cannot step to).  Returns the pinned pieces; adds the rays to the attack
-// map A.
-template <int U, int V>
-ZD u64 king_line(u64 S, u64 kbb, u64 own, u64 e, u64 &A, u64 &checkers, u64 &chkray, u64 &xray) {
-  const u64 Ru = slide<U>(S, e), Rv = slide<V>(S, e);
-  const u64 Ku = slide<U>(kbb, e), Kv = slide<V>(kbb, e);
-  A |= Ru | Rv;
-  const u64 cu = Ku & S, cv = Kv & S;
-  checkers |= cu | cv;
-  const bool hu = cu != 0, hv = cv != 0;
-  chkray |= sel(hu, Ku) | sel(hv, Kv);
-  xray |= sel(hu, Kv) | sel(hv, Ku);
-  return ((Ku & Rv) | (Kv & Ru)) & own;
+// ---- rank rays by a carry: added to the empty squares, a piece shifted one
+// square on runs through them and sets the first that is not empty (a blocker
+// or the edge file, which `e` leaves out).  Pieces are not empty, so a ray ends
+// at the next one and all rays of a set come from one addition.  West runs on
+// the reversed board.  s: occupied squares; e: empty & NOTH.
+ZD u64 ray_east(u64 s, u64 e) { return whole(((s & NOTH) << 1) + e) ^ e; }
+
+// Legality context of a board with several own kings (no game reaches it):
+// the check rays are all the kings' rays in a checked direction, and so are
+// the squares behind them.
+ZD void many_kings(Legal &L, u64 e, u64 &A, u64 &chkray) {
+  const u64 orq = L.opp & L.rq, obq = L.opp & L.bq;
+  auto line = [&](u64 S, u64 Ku, u64 Kv) {
+    const bool hu = (Ku & S) != 0, hv = (Kv & S) != 0;
+    chkray |= sel(hu, Ku) | sel(hv, Kv);
+    A |= sel(hu, Kv) | sel(hv, Ku);
+  };
+  chkray = 0;
+  line(orq, slide<0>(L.kbb, e), slide<1>(L.kbb, e));
+  line(orq, slide<2>(L.kbb, e), slide<3>(L.kbb, e));
+  line(obq, slide<4>(L.kbb, e), slide<7>(L.kbb, e));
+  line(obq, slide<5>(L.kbb, e), slide<6>(L.kbb, e));
 }
 
+// Per line through the king, from occluded fills in its two directions U and
+// V: R = the rays of the opponent's sliders that move along the line, K = the
+// king's own rays (each up to and including the first blocker).  Where a ray
+// of the king meets the opposite ray of a slider, an own piece is pinned and
+// an empty square lies between the king and a checker.  Both lie strictly
+// inside the line, never on an edge file of a rank or diagonal: the diagonals'
+// rays go unmasked (their last step may wrap onto an edge file) and the wraps
+// fall to the mask of what meets them, or to one mask a union.
+// A holds, of the squares behind the king on a checked line, the next one: the
+// king steps no further, and a king in check does not castle.
+// Bound: VALU issue where a lane takes a position (perft).  The three fills of
+// a direction share the doubled empty sets; three-operand logic and the rank
+// carries, here, in apply_v and in count_legal, took a perft leaf from 990 to
+// 880 lane-instructions (130.8 M leaves: 3.42 to 3.25 ms).
 ZD void analyse(const Pos &p, Legal &L) {
-  const u64 occ = p.b1 | p.b2 | p.b3;
-  const u64 white = p.b0 ^ occ;
+  const u64 occ = bop3<(TA | TB | TC)>(p.b1, p.b2, p.b3);
+  const u64 black = 0 - (u64)(p.stm & 1u);
   L.stm = p.stm;
   L.occ = occ;
-  L.own = p.stm ? p.b0 : white;
-  L.opp = p.stm ? white : p.b0;
-  L.pawns = p.b1 & ~p.b2 & ~p.b3;
-  L.knights = ~p.b1 & p.b2 & ~p.b3;
-  L.kings = p.b1 & p.b2 & ~p.b3;
-  L.rq = p.b3 & (p.b1 ^ p.b2);  // rook 101, queen 110
-  L.bq = p.b3 & ~p.b1;          // bishop 100, queen 110
-  L.kbb = L.own & L.kings;
-  L.ksq = L.kbb ? lsb(L.kbb) : 0;
+  L.own = bop3<(TA ^ (TB & ~TC))>(p.b0, occ, black);
+  L.opp = bop3<(TA ^ (TB & TC))>(p.b0, occ, black);
+  L.pawns = bop3<(TA & ~TB & ~TC)>(p.b1, p.b2, p.b3);
+  L.knights = bop3<(~TA & TB & ~TC)>(p.b1, p.b2, p.b3);
+  L.kings = bop3<(TA & TB & ~TC)>(p.b1, p.b2, p.b3);
+  L.rq = bop3<((TA ^ TB) & TC)>(p.b1, p.b2, p.b3);  // rook 101, queen 110
+  L.bq = p.b3 & ~p.b1;                              // bishop 100, queen 110
+  const u64 kbb = L.own & L.kings;
+  L.kbb = kbb;
+  L.ksq = kbb ? lsb(kbb) : 0;
   const u64 orq = L.opp & L.rq, obq = L.opp & L.bq;
-  // the opponent's attacks with the own king as a blocker (every fill shares
-  // the empty set, and with it the doubling masks, with the move counts),
-  // completed by the squares the checking sliders attack through the king
+  const u64 opawns = L.opp & L.pawns, oknights = L.opp & L.knights;
   const u64 e = ~occ;
-  u64 A = pawn_att(L.opp & L.pawns, p.stm ^ 1u) | knight_att(L.opp & L.knights) | king_att(L.opp & L.kings);
-  u64 checkers = (pawn_att(L.kbb, p.stm) & L.opp & L.pawns) | (knight_att(L.kbb) & L.opp & L.knights);
-  u64 chkray = 0, xray = 0;
-  L.pinF = king_line<0, 1>(orq, L.kbb, L.own, e, A, checkers, chkray, xray);
-  L.pinR = king_line<2, 3>(orq, L.kbb, L.own, e, A, checkers, chkray, xray);
-  L.pinD = king_line<4, 7>(obq, L.kbb, L.own, e, A, checkers, chkray, xray);
-  L.pinA = king_line<5, 6>(obq, L.kbb, L.own, e, A, checkers, chkray, xray);
-  L.A = A | xray;
-  L.checkers = checkers;
-  const int n = popc(checkers);
-  L.cmask = n == 0 ? FULL : (n == 1 ? (checkers | chkray) : 0ULL);
+  constexpr u64 INNER = NOTA & NOTH;
+  // a slider's ray that reaches the (one) king goes one square on
+  const bool many = (kbb & (kbb - 1)) != 0;
+  const u64 kx = sel(!many, kbb), kxA = kx & NOTA, kxH = kx & NOTH;
+  auto ray = [&](auto D, u64 k, u64 g) {
+    constexpr int d = decltype(D)::value;
+    return shift_raw<d>(and_or(shift_raw<d>(g), k, g));
+  };
+  // files
+  const u64 rn = ray(Dir<0>(), kx, ks_fill<0>(orq, e)), rs = ray(Dir<1>(), kx, ks_fill<1>(orq, e));
+  const u64 kn = slide_raw<0>(kbb, e), ks = slide_raw<1>(kbb, e);
+  const u64 xf = and_or(kn, rs, ks & rn);
+  // ranks
+  const u64 ee = e & NOTH, er = rev64(e) & NOTH;
+  u64 re = ray_east(orq, ee), rw = ray_east(rev64(orq), er);
+  const u64 ke = ray_east(kbb, ee), kw = rev64(ray_east(rev64(kbb), er));
+  rw = rev64(rw);
+  re |= whole((re & kxH) << 1);
+  rw |= whole((rw & kxA) >> 1);
+  const u64 xr = and_or(ke, rw, kw & re);
+  // diagonals
+  const u64 rne = ray(Dir<4>(), kxA, ks_fill<4>(obq, e)), rsw = ray(Dir<7>(), kxH, ks_fill<7>(obq, e));
+  const u64 kne = slide_raw<4>(kbb, e), ksw = slide_raw<7>(kbb, e);
+  const u64 xd = and_or(kne, rsw, ksw & rne);
+  const u64 rnw = ray(Dir<5>(), kxH, ks_fill<5>(obq, e)), rse = ray(Dir<6>(), kxA, ks_fill<6>(obq, e));
+  const u64 knw = slide_raw<5>(kbb, e), kse = slide_raw<6>(kbb, e);
+  const u64 xa = and_or(knw, rse, kse & rnw);
+  L.pinF = xf & L.own;
+  L.pinR = xr & L.own;
+  const u64 owni = L.own & INNER;
+  L.pinD = xd & owni;
+  L.pinA = xa & owni;
+  u64 chkray = bop3<((TA | TB) & TC)>(xf, xr, e) | bop3<((TA | TB) & TC)>(xd, xa, e & INNER);
+  // the opponent's pawns one rank on, and the king's
+  const int up = p.stm & 1u ? 0 : 8, down = 8 - up;
+  const u64 pf = (opawns << down) >> up, kf = (kbb << up) >> down;
+  const u64 kpawn = and_or(whole(kf << 1), NOTA, whole(kf >> 1) & NOTH);
+  u64 A = bop3<(TA | TB | TC)>(rn, rs, re) | rw;
+  A = bop3<(TA | TB | TC)>(A, knight_att_v(oknights), king_att_v(L.opp & L.kings));
+  A = and_or(bop3<(TA | TB | TC)>(rne, rse, whole(pf << 1)), NOTA, A);
+  A = and_or(bop3<(TA | TB | TC)>(rnw, rsw, whole(pf >> 1)), NOTH, A);
+  u64 ch = bop3<((TA | TB) & TC)>(bop3<(TA | TB | TC)>(kn, ks, ke), kw, orq);
+  ch |= bop3<((TA | TB) & TC)>(kne, kse, obq & NOTA);
+  ch |= bop3<((TA | TB) & TC)>(knw, ksw, obq & NOTH);
+  ch = and_or(kpawn, opawns, ch);
+  ch = and_or(knight_att_v(kbb), oknights, ch);
+  if (many) many_kings(L, e, A, chkray);
+  L.A = A;
+  L.checkers = ch;
+  const int n = popc(ch);
+  L.cmask = n == 0 ? FULL : (n == 1 ? (ch | chkray) : 0ULL);
 }
 
 // is the side to move's king attacked after the e.p. capture from->to taking
@@ -310,6 +397,15 @@ ZD void analyse(const Pos &p, Legal &L) {
 // not eight occluded fills); a king never checks
 ZD bool ep_legal(const Legal &L, int from, int to, int sqep) {
   if (!L.kbb) return true;
+  // nearly always nothing can open: no check, the capturing pawn not pinned,
+  // and the captured one neither on the king's rank nor on its diagonals (its
+  // file stays closed by the capturing pawn).  Boards that no game reaches may
+  // break the last: their e.p. flag can name an empty square or any piece, so
+  // an opponent's pawn has to stand there, and the capture's target be empty.
+  const int dr = (sqep >> 3) - (L.ksq >> 3), df = (sqep & 7) - (L.ksq & 7);
+  const u64 pinned = L.pinR | L.pinF | L.pinD | L.pinA;
+  const bool plain = ((L.opp & L.pawns) >> sqep & 1) && !((L.occ >> to) & 1) && L.cmask == FULL;
+  if (plain && !((pinned >> from) & 1) && dr != 0 && dr != df && dr != -df) return true;
   const u64 occ2 = (L.occ ^ bit(from) ^ bit(sqep)) | bit(to);
   const u64 opp2 = L.opp & ~bit(sqep);
   const u64 att = (rook_sq(L.ksq, occ2) & opp2 & L.rq) | (bishop_sq(L.ksq, occ2) & opp2 & L.bq) |
@@ -355,42 +451,40 @@ ZD int count_legal(const Pos &p, const Legal &L, bool qs) {
   // the target set with each edge-file mask applied once (a shifted set
   // masked and then intersected with T is the shifted set intersected with
   // the masked T)
-  const u64 TA = T & NOTA, TH = T & NOTH;
-  const u64 pinned = L.pinR | L.pinF | L.pinD | L.pinA;
-  int cnt = popc(king_att(L.kbb) & (qs ? L.opp : ~own) & ~L.A);
-  const u64 kn = own & L.knights & ~pinned;
+  const u64 TnA = T & NOTA, TnH = T & NOTH;
+  const u64 pinned = bop3<(TA | TB | TC)>(L.pinR, L.pinF, L.pinD) | L.pinA;
+  int cnt = popc(bop3<(TA & TB & ~TC)>(king_att_v(L.kbb), qs ? L.opp : ~own, L.A));
+  const u64 kn = bop3<(TA & TB & ~TC)>(own, L.knights, pinned);
   const u64 TAB = T & 0xFCFCFCFCFCFCFCFCULL, TGH = T & 0x3F3F3F3F3F3F3F3FULL;
-  cnt += popc((kn << 17) & TA) + popc((kn << 15) & TH) + popc((kn << 10) & TAB) + popc((kn << 6) & TGH);
-  cnt += popc((kn >> 6) & TAB) + popc((kn >> 10) & TGH) + popc((kn >> 15) & TA) + popc((kn >> 17) & TH);
+  cnt += popc(whole(kn << 17) & TnA) + popc(whole(kn << 15) & TnH) + popc(whole(kn << 10) & TAB) + popc(whole(kn << 6) & TGH);
+  cnt += popc(whole(kn >> 6) & TAB) + popc(whole(kn >> 10) & TGH) + popc(whole(kn >> 15) & TnA) + popc(whole(kn >> 17) & TnH);
   const u64 e = ~occ;
   const u64 orq = own & L.rq, obq = own & L.bq;
-  cnt += popc(slide_raw<0>(orq & (~pinned | L.pinF), e) & T);
-  cnt += popc(slide_raw<1>(orq & (~pinned | L.pinF), e) & T);
-  cnt += popc(slide_raw<2>(orq & (~pinned | L.pinR), e) & TA);
-  cnt += popc(slide_raw<3>(orq & (~pinned | L.pinR), e) & TH);
-  cnt += popc(slide_raw<4>(obq & (~pinned | L.pinD), e) & TA);
-  cnt += popc(slide_raw<7>(obq & (~pinned | L.pinD), e) & TH);
-  cnt += popc(slide_raw<5>(obq & (~pinned | L.pinA), e) & TH);
-  cnt += popc(slide_raw<6>(obq & (~pinned | L.pinA), e) & TA);
+  const u64 sf = bop3<(TA & (~TB | TC))>(orq, pinned, L.pinF), sr = bop3<(TA & (~TB | TC))>(orq, pinned, L.pinR);
+  const u64 sd = bop3<(TA & (~TB | TC))>(obq, pinned, L.pinD), sa = bop3<(TA & (~TB | TC))>(obq, pinned, L.pinA);
+  cnt += popc(slide_raw<0>(sf, e) & T);
+  cnt += popc(slide_raw<1>(sf, e) & T);
+  const u64 ee = e & NOTH, er = rev64(e) & NOTH;
+  cnt += popc(ray_east(sr, ee) & T);
+  cnt += popc(ray_east(rev64(sr), er) & rev64(T));
+  cnt += popc(slide_raw<4>(sd, e) & TnA);
+  cnt += popc(slide_raw<7>(sd, e) & TnH);
+  cnt += popc(slide_raw<5>(sa, e) & TnH);
+  cnt += popc(slide_raw<6>(sa, e) & TnA);
+  // pawns: one rank on, then one file east or west.  East captures run along
+  // the a1-h8 diagonals for white and the others for black.
   const u64 P = own & L.pawns;
-  const u64 capD = P & (~pinned | L.pinD), capA = P & (~pinned | L.pinA);
+  const int up = p.stm & 1u ? 0 : 8, down = 8 - up;
+  const u64 pinE = p.stm & 1u ? L.pinA : L.pinD, pinW = p.stm & 1u ? L.pinD : L.pinA;
+  const u64 capE = (bop3<(TA & (~TB | TC))>(P, pinned, pinE) << up) >> down;
+  const u64 capW = (bop3<(TA & (~TB | TC))>(P, pinned, pinW) << up) >> down;
   const u64 tgt = L.opp & L.cmask;
-  if (p.stm) {
-    cnt += popc(((capD >> 9) & NOTH) & tgt) + popc(((capA >> 7) & NOTA) & tgt);
-  } else {
-    cnt += popc(((capD << 9) & NOTA) & tgt) + popc(((capA << 7) & NOTH) & tgt);
-  }
+  cnt += popc(bop3<(TA & TB & TC)>(whole(capE << 1), tgt, NOTA)) + popc(bop3<(TA & TB & TC)>(whole(capW >> 1), tgt, NOTH));
   if (!qs) {
-    const u64 pp = P & (~pinned | L.pinF);
-    u64 s1, s2;
-    if (p.stm) {
-      s1 = (pp >> 8) & e;
-      s2 = ((s1 & RANK6) >> 8) & e;
-    } else {
-      s1 = (pp << 8) & e;
-      s2 = ((s1 & RANK3) << 8) & e;
-    }
-    cnt += popc(s1 & L.cmask) + popc(s2 & L.cmask);
+    const u64 pp = bop3<(TA & (~TB | TC))>(P, pinned, L.pinF);
+    const u64 s1 = whole((pp << up) >> down) & e;
+    const u64 s2 = whole(((s1 & (p.stm & 1u ? RANK6 : RANK3)) << up) >> down);
+    cnt += popc(s1 & L.cmask) + popc(bop3<(TA & TB & TC)>(s2, e, L.cmask));
     cnt += popc(castle_targets(p, L));
   }
   int sqep;
@@ -690,6 +784,39 @@ ZD Pos apply(const Pos &p, u32 m, bool rook_flag) {
   const bool dbl = ((pf >> 1) & 7) == PAWN && rt - rf == 2;
   cr |= RANKS45;
   if (dbl) cr &= ~bit(t);
+  c.cr = cr;
+  c.stm = p.stm ^ 1u;
+  return c;
+}
+
+// apply() where every lane has a position of its own (perft): fused logic, the
+// castling rook behind a branch that few wavefronts take
+ZD Pos apply_v(const Pos &p, u32 m) {
+  Pos c;
+  const int f = (int)mv_from(m), t = (int)mv_to(m);
+  const u64 tb = bit(t);
+  const u64 gone = bop3<(TA | TB | TC)>(bit(f), bit((int)mv_cpt(m)), tb);
+  const u32 pf = mv_pfrom(m), pt = mv_pto(m);
+  c.b0 = and_or(0 - (u64)(pt & 1), tb, p.b0 & ~gone);
+  c.b1 = and_or(0 - (u64)((pt >> 1) & 1), tb, p.b1 & ~gone);
+  c.b2 = and_or(0 - (u64)((pt >> 2) & 1), tb, p.b2 & ~gone);
+  c.b3 = and_or(0 - (u64)((pt >> 3) & 1), tb, p.b3 & ~gone);
+  u64 cr = bop3<(TA | TB | TC)>(p.cr, gone, RANKS45);
+  const u32 type = (pf >> 1) & 7;
+  if (type == KING && (f - t == 2 || t - f == 2)) {
+    // the rook goes to the king's other side
+    const int r = f - t == 2 ? f - 4 : f + 3, s = f - t == 2 ? t + 1 : t - 1;
+    const u64 keep = ~bit(r);
+    c.b0 &= keep;
+    c.b1 &= keep;
+    c.b2 &= keep;
+    c.b3 &= keep;
+    put_piece(c, s, (ROOK << 1) | (pf & 1));
+    cr |= bit(r);
+  }
+  const u32 col = pf & 1;
+  const int rf = col ? ((f >> 3) ^ 7) : (f >> 3), rt = col ? ((t >> 3) ^ 7) : (t >> 3);
+  if (type == PAWN && rt - rf == 2) cr &= ~tb;
   c.cr = cr;
   c.stm = p.stm ^ 1u;
   return c;

@@ -217,7 +217,7 @@ __global__ __launch_bounds__(TPB) void k_apply(Front f, const u64 *__restrict__ 
   const u64 e = pm[j];
   const u32 pi = (u32)(e >> 32);
   const Pos p = load_pos(f, pi);
-  const Pos c = apply(p, (u32)e, true);
+  const Pos c = apply_v(p, (u32)e);
   store_pos(g, j, c, f.meta[pi] >> 1);
   Legal L;
   analyse(c, L);
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(TPB) void k_leaf(Front f, const u64 *__restrict__ p
     const u64 e = pm[j];
     const u32 pi = (u32)(e >> 32);
     const Pos p = load_pos(f, pi);
-    const Pos c = apply(p, (u32)e, true);
+    const Pos c = apply_v(p, (u32)e);
     Legal L;
     analyse(c, L);
     if (nobulk) {
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(TPB) void k_playout(u64 seed, int n, int minply, in
       const int pick = (int)(rnd() % (u64)nl);
       const u32 m = nth_legal(p, L, pick);
       hmc = next_hmc(hmc, m);
-      p = apply(p, m, true);
+      p = apply_v(p, m);
     }
     if (ok) {
       Legal L;
