@@ -26,7 +26,7 @@ def H(tmp_path_factory):
     return L
 
 
-def _board(rng, pieces, stm):
+def _board(rng, pieces, stm, kings=False):
     b = np.zeros(7, dtype=np.uint64)
     squares = rng.permutation(64)[:pieces]
     while max(abs(int(squares[0]) % 8 - int(squares[1]) % 8), abs(int(squares[0]) // 8 - int(squares[1]) // 8)) < 2:
@@ -35,7 +35,7 @@ def _board(rng, pieces, stm):
         piece, black = int(rng.integers(1, 7)), int(rng.integers(0, 2))  # the king is piece 3
         if i < 2:
             piece, black = 3, i
-        elif piece == 3 or piece == 1 and not 8 <= sq < 56:
+        elif (piece == 3 and not kings) or piece == 1 and not 8 <= sq < 56:
             piece = int(rng.integers(4, 7))
         for bit in range(3):
             if piece >> bit & 1:
@@ -57,7 +57,7 @@ def _board(rng, pieces, stm):
 
 def test_counts_on_any_board(H):
     rng = np.random.default_rng(12)
-    out = np.zeros(2, dtype=np.int32)
+    out = np.zeros(3, dtype=np.int32)
     p = np.zeros(1, dtype=R.POS_DTYPE)
     checks = 0
     for k in range(4000):
@@ -69,6 +69,26 @@ def test_counts_on_any_board(H):
         assert out[1] == out[0], (k, [hex(int(v)) for v in b])  # as many are emitted, and made alike
         checks += out[0] < 8
     assert checks > 100
+
+
+def test_emitted_moves_of_several_kings(H):
+    # the places of a position's moves are laid out by count_emitted, on every
+    # board: a king step and a castling can be one move where kings are many
+    rng = np.random.default_rng(14)
+    out = np.zeros(3, dtype=np.int32)
+    kings = np.zeros(7, dtype=np.uint64)  # white kings e1 and g2 with a rook on h1, black's on a8
+    for sq, piece, black in [(4, 3, 0), (14, 3, 0), (7, 5, 0), (56, 3, 1)]:
+        for bit in range(3):
+            kings[1 + bit] |= np.uint64((piece >> bit & 1) << sq)
+        kings[0] |= np.uint64(black << sq)
+    kings[4] = np.uint64(0x6EFFFFFFFFFFFF6E)
+    differ = 0
+    for k in range(4000):
+        b = kings if k == 0 else _board(rng, int(rng.integers(2, 50)), k & 1, kings=True)
+        H.rh_count(b.ctypes.data, k & 1, out.ctypes.data)
+        assert out[1] == out[2], (k, [hex(int(v)) for v in b])
+        differ += out[0] != out[2]
+    assert differ  # the first one
 
 
 def test_rank_rays(H):

@@ -822,6 +822,22 @@ ZD Pos apply_v(const Pos &p, u32 m) {
   return c;
 }
 
+// apply_v() of a position that is only counted: the e.p. flag is dropped when
+// no pawn stands to use it (positions that differ only there have the same
+// legal moves and descendants).
+ZD Pos apply_count(const Pos &p, u32 m) {
+  Pos c = apply_v(p, m);
+  const u64 w = ~c.cr & RANKS45;
+  if (w) {
+    const u64 occ = c.b1 | c.b2 | c.b3;
+    const u64 mine = c.stm ? c.b0 : c.b0 ^ occ;
+    const int sq = lsb(w);
+    const u64 cand = mine & c.b1 & ~c.b2 & ~c.b3 & (c.stm ? RANK4 : RANK5) & (bit(sq + 1) | bit(sq - 1));
+    if (!cand) c.cr |= RANKS45;
+  }
+  return c;
+}
+
 // apply() of a capture (e.p. and promotions included, no castling): the
 // planes and the side to move; the moved flags are the parent's.
 ZD Pos apply_capture(const Pos &p, u32 m) {
@@ -1041,6 +1057,12 @@ ZD void for_each_legal(const Pos &p, const Legal &L, Emit &&emit) {
       if (ep_legal(L, f, to, sqep)) emit(make_code(p, f, to));
     }
   }
+}
+
+// How many moves for_each_legal emits: a board with several kings of one side
+// can have a king step and a castling with one target, which is one move there.
+ZD int count_emitted(const Pos &p, const Legal &L) {
+  return count_legal(p, L, false) - popc(king_att(L.kbb) & ~L.own & ~L.A & castle_targets(p, L));
 }
 
 // host domove half-move clock rule (src/bitboard.c:604-689): +1, reset by

@@ -3,18 +3,21 @@
 // Replaces perft_gpu (src/zetaperft.cl:801-1477), which walks ONE root with
 // one 64-lane work-group, and its host driver (src/search.c:225-271,
 // src/clrun.c:979-1147).  Design: a level-synchronous frontier over all roots
-// of the batch, one lane per position:
-//   level 0 = roots (SoA in HBM) with their legal-move counts;
-//   count -> exclusive scan -> expand writes (parent, move) pairs of level L+1
-//   -> apply materialises level L+1 (SoA) and counts its moves;
-//   the last level is never materialised: perft_leaf applies each move to its
-//   parent and adds the child's legal-move count (bulk counting at depth-1)
-//   to its root's u64 counter with one wavefront-aggregated atomic per root.
-// Every leaf-level lane does the same branch-free set-wise counting, so the
-// uneven subtree sizes of a batch cost no SIMD divergence.  Levels that would
-// exceed the frontier budget are split into chunks (depth-first over chunks).
+// of the batch (SoA in HBM); the last level is never materialised: its moves
+// are applied to their parents and the children's legal moves counted (bulk
+// counting at depth-1) into the roots' u64 counters.  Every leaf-level lane
+// does the same branch-free set-wise counting, so the uneven subtree sizes of a
+// batch cost no SIMD divergence.  Two drivers:
+//   the chain (fast_perft) queues all levels without waiting for their sizes,
+//   and counts positions that several move orders reach once;
+//   the chunked one (process) reads each level's size, splits levels that
+//   exceed the frontier budget into chunks (depth-first over chunks), and works
+//   in fixed buffers where the call may not allocate.  Its levels:
+//     count -> exclusive scan -> expand writes (parent, move) pairs of level
+//     L+1 -> apply materialises level L+1 and counts its moves.
 #include <string.h>
 
+#include <type_traits>
 #include <vector>
 
 #include "chess.h"
@@ -267,6 +270,433 @@ __global__ __launch_bounds__(TPB) void k_leaf(Front f, const u64 *__restrict__ p
     pending &= ~mask;
     active = active && !mine;
   }
+}
+
+// ========================================================== the chain
+// A call's levels in one chain of launches without a wait between them: the
+// host sizes the buffers by what earlier calls needed, every kernel reads its
+// level's count from device memory, and a level that did not fit reports its
+// size at the end (the chain then runs again with room for it, or, past the
+// frontier budget, the chunked driver takes the call).
+//   wide    one wavefront a parent, lane = square, then lane = move: few
+//           positions in few microseconds
+//   spread  one parent a lane, the moves of 128 parents meet in LDS and are
+//           made one a lane: many positions
+// Levels 3 and deeper merge transpositions: positions of a root reached by
+// several move orders become one node that carries their number (k_merge).
+// Measured against the chunked driver (host waits for every level, three scan
+// launches each): one position at depth 4 139 -> 47 us, at depth 6 (119 M and
+// 8 G leaves) 2.05 -> 0.39 and 5.8 -> 0.52 ms.  The first of these is launches
+// and the host's one wait; the others are bound by the leaves' VALU issue.
+struct Level {
+  u64 *b0, *b1, *b2, *b3, *cr;
+  u64 *wt;    // paths from the root that the node stands for
+  u32 *meta;  // root index << 1 | side to move
+  u32 *mv;    // the move that led to it
+  u32 *par;   // its parent's index in the level above
+  u64 *count; // nodes wanted so far (those past the capacity are not stored)
+  u64 cap;
+};
+
+__device__ __forceinline__ Pos level_pos(const Level &f, size_t i) {
+  Pos p;
+  p.b0 = f.b0[i];
+  p.b1 = f.b1[i];
+  p.b2 = f.b2[i];
+  p.b3 = f.b3[i];
+  p.cr = f.cr[i];
+  p.stm = f.meta[i] & 1u;
+  return p;
+}
+__device__ __forceinline__ void level_store(const Level &f, size_t i, const Pos &c, u32 root, u32 mv, u32 par, u64 wt) {
+  f.b0[i] = c.b0;
+  f.b1[i] = c.b1;
+  f.b2[i] = c.b2;
+  f.b3[i] = c.b3;
+  f.cr[i] = c.cr;
+  f.meta[i] = (root << 1) | c.stm;
+  f.mv[i] = mv;
+  f.par[i] = par;
+  f.wt[i] = wt;
+}
+// (a level that did not fit counts as empty: nothing below it is worked on)
+__device__ __forceinline__ u64 level_size(const Level &f) {
+  const u64 n = *f.count;
+  return n <= f.cap ? n : 0;
+}
+__device__ __forceinline__ Pos root_pos(const u64 *in, size_t i) {
+  const u64 *q = in + i * 8;  // zeta_pos = 7 x u64 + stm + pad
+  Pos p;
+  p.b0 = q[0];
+  p.b1 = q[1];
+  p.b2 = q[2];
+  p.b3 = q[3];
+  p.cr = q[4];
+  p.stm = (u32)(q[7] & 1u);
+  return p;
+}
+
+// ---- depth 1: the roots' own move counts
+__global__ __launch_bounds__(64) void k_count_roots(const u64 *__restrict__ in, int n, u64 *__restrict__ counts) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  if (i >= n) return;
+  const Pos p = root_pos(in, i);
+  Legal L;
+  analyse(p, L);
+  counts[i] = (u64)count_legal(p, L, false);
+}
+
+// ---- wide: the legal moves of one position, spread over a wavefront: lane
+// takes move number `lane` + 64 k of list[0 .. n).  A position without exactly
+// one king of its own is enumerated by one lane (the per-square form below
+// takes each king for itself).
+__device__ __forceinline__ int wide_moves(const Pos &p, int lane, u32 *list) {
+  Node0 B;
+  node_basics(p, B);
+  if (popc(B.kbb) != 1) {
+    int n = 0;
+    if (lane == 0) {
+      Legal L;
+      analyse(p, L);
+      for_each_legal(p, L, [&](u32 code) { list[n++] = code; });
+    }
+    return __shfl(n, 0, 64);
+  }
+  const u64 A = __ballot(attacked_nk(B, lane));
+  u64 t = (B.own >> lane) & 1 ? lane_targets(p, B, A, lane, false) : 0;
+  const int incl = zw::wave_scan_add(popc(t));
+  int k = incl - popc(t);
+  while (t) {
+    list[k++] = make_code(p, lane, lsb(t));
+    t &= t - 1;
+  }
+  return __builtin_amdgcn_readlane(incl, 63);
+}
+
+// most moves of a position with one king to move, on any board: a piece has at
+// most 27 (the king 10), a square can be reached from at most 8 lines, 8
+// knights, a king and 2 more pawns: with k pieces no more than
+// min(27 k + 10, 19 (64 - k)), below 740 for every k
+constexpr int MAXMOVES = 768;
+constexpr int WIDE_TPB = 512;
+
+// level 0 (in != null) or f -> g; also clears the counts of the roots
+__global__ __launch_bounds__(WIDE_TPB) void k_wide(const u64 *__restrict__ in, int nroots, Level f, Level g,
+                                                   u64 *__restrict__ counts) {
+  __shared__ u32 list[WIDE_TPB / 64][MAXMOVES];
+  __shared__ u32 num[WIDE_TPB / 64];
+  __shared__ u64 lbase;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const u64 n = in ? (u64)nroots : level_size(f);
+  for (u64 i0 = (u64)blockIdx.x * (WIDE_TPB / 64); i0 < n; i0 += (u64)gridDim.x * (WIDE_TPB / 64)) {
+    const u64 i = i0 + w;
+    Pos p = {};
+    u32 root = 0;
+    u64 wt = 1;
+    int m = 0;
+    if (i < n) {
+      p = in ? root_pos(in, i) : level_pos(f, i);
+      root = in ? (u32)i : f.meta[i] >> 1;
+      if (!in) wt = f.wt[i];
+      if (in && lane == 0) counts[i] = 0;
+      m = wide_moves(p, lane, list[w]);
+    }
+    if (lane == 0) num[w] = (u32)m;
+    __syncthreads();
+    // one atomic a block: they are a chain of 10 ns each
+    u32 before = 0, total = 0;
+#pragma unroll
+    for (int k = 0; k < WIDE_TPB / 64; k++) {
+      before += k < w ? num[k] : 0u;
+      total += num[k];
+    }
+    if (threadIdx.x == 0) lbase = total ? atomicAdd((unsigned long long *)g.count, (unsigned long long)total) : 0;
+    __syncthreads();
+    const u64 base = lbase + before;
+    for (int k = lane; k < m; k += 64)
+      if (base + k < g.cap) level_store(g, base + k, apply_count(p, list[w][k]), root, list[w][k], (u32)i, wt);
+    __syncthreads();
+  }
+}
+
+// the last level below few parents: each lane makes a child and counts its
+// moves (nobulk: generates them and counts the child itself)
+__global__ __launch_bounds__(WIDE_TPB) void k_wide_leaf(const u64 *__restrict__ in, int nroots, Level f,
+                                                        u64 *__restrict__ counts, int nobulk) {
+  __shared__ u32 list[WIDE_TPB / 64][MAXMOVES];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const u64 n = in ? (u64)nroots : level_size(f);
+  const u64 step = (u64)gridDim.x * (WIDE_TPB / 64);
+  for (u64 i = (u64)blockIdx.x * (WIDE_TPB / 64) + w; i < n; i += step) {
+    const Pos p = in ? root_pos(in, i) : level_pos(f, i);
+    const int m = wide_moves(p, lane, list[w]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    u32 v = 0;
+    for (int k = lane; k < m; k += 64) {
+      const Pos c = apply_v(p, list[w][k]);
+      Legal L;
+      analyse(c, L);
+      v += nobulk ? 1u + (u32)(count_legal(c, L, true) > 4096) : (u32)count_legal(c, L, false);
+    }
+    const u64 s = (u64)(u32)__builtin_amdgcn_readlane(zw::wave_scan_add((int)v), 63);
+    if (lane == 0) {
+      if (in) counts[i] = s;
+      else if (s) atomicAdd((unsigned long long *)&counts[f.meta[i] >> 1], (unsigned long long)(s * f.wt[i]));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+}
+
+// ---- spread: 128 parents a block, one a lane; their moves meet in LDS (those
+// beyond its list wait in the output itself) and are made one a lane, so that
+// the stores are coalesced.  PAIRS: the moves are not made but written as
+// (parent << 32 | move) for the leaf kernel.  Takes the parents [i0, i1).
+// Bound: VALU issue of the move loops, where a wavefront runs as many steps as
+// its busiest lane has of each kind (4.2 M parents, 130 M pairs: 0.54 ms; the
+// stores alone would take 0.22).
+template <bool PAIRS>
+__global__ __launch_bounds__(XTPB) void k_spread(Level f, u64 i0, u64 i1, Level g, u64 *__restrict__ pm) {
+  __shared__ u32 lcode[XCAP];
+  __shared__ u8 llane[XCAP];
+  __shared__ u64 lb0[XTPB], lb1[XTPB], lb2[XTPB], lb3[XTPB], lcr[XTPB], lwt[XTPB];
+  __shared__ u32 lmeta[XTPB];
+  __shared__ u32 wsum[XTPB / 64];
+  __shared__ u64 lbase;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const u64 size = level_size(f), n = size < i1 ? size : i1;
+  for (u64 c0 = i0 + (u64)blockIdx.x * XTPB; c0 < n; c0 += (u64)gridDim.x * XTPB) {
+    const u64 i = c0 + tid;
+    Pos p;
+    Legal L;
+    u32 cnt = 0;
+    if (i < n) {
+      p = level_pos(f, i);
+      if (!PAIRS) {
+        lb0[tid] = p.b0;
+        lb1[tid] = p.b1;
+        lb2[tid] = p.b2;
+        lb3[tid] = p.b3;
+        lcr[tid] = p.cr;
+        lwt[tid] = f.wt[i];
+        lmeta[tid] = f.meta[i];
+      }
+      analyse(p, L);
+      cnt = (u32)count_emitted(p, L);
+    }
+    const u32 incl = (u32)zw::wave_scan_add((int)cnt);
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    const u32 total = wsum[0] + wsum[1];
+    if (tid == 0) lbase = atomicAdd((unsigned long long *)g.count, (unsigned long long)total);
+    __syncthreads();
+    const u64 base = lbase;
+    if (i < n) {
+      u32 o = incl - cnt + (w ? wsum[0] : 0u);
+      for_each_legal(p, L, [&](u32 code) {
+        if (o < (u32)XCAP) {
+          lcode[o] = code;
+          llane[o] = (u8)tid;
+        } else if (base + o < g.cap) {
+          if (PAIRS) {
+            pm[base + o] = i << 32 | code;
+          } else {
+            g.mv[base + o] = code;
+            g.par[base + o] = (u32)i;
+          }
+        }
+        o++;
+      });
+    }
+    __syncthreads();
+    for (u32 k = tid; k < total && base + k < g.cap; k += XTPB) {
+      if (PAIRS) {
+        if (k >= (u32)XCAP) break;
+        pm[base + k] = (c0 + llane[k]) << 32 | lcode[k];
+      } else {
+        const u32 l = k < (u32)XCAP ? llane[k] : (u32)(g.par[base + k] - c0);
+        const u32 code = k < (u32)XCAP ? lcode[k] : g.mv[base + k];
+        Pos q;
+        q.b0 = lb0[l];
+        q.b1 = lb1[l];
+        q.b2 = lb2[l];
+        q.b3 = lb3[l];
+        q.cr = lcr[l];
+        q.stm = lmeta[l] & 1u;
+        level_store(g, base + k, apply_count(q, code), lmeta[l] >> 1, code, (u32)(c0 + l), lwt[l]);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ---- leaf: the children of `f` that the pairs name, counted into their roots.
+// Bound: VALU issue (0.99 of it); a child costs about 850 lane-instructions.
+// A wavefront takes runs of 512 pairs in turn, one atomic a root of the run; of
+// the grid about three blocks a CU are resident, and the rest of its 48 a CU
+// fills the places of those that end first (3.20 ms for 130 M pairs, 3.59 ms
+// with a grid of the resident ones).
+// WT: f is a merged level, whose nodes count as often as they have paths.
+constexpr int LEAF_BLOCKS = 48;
+constexpr u32 LEAF_RUN = 512;
+template <bool WT, bool NOBULK>
+__global__ __launch_bounds__(TPB) void k_leaves(Level f, const u64 *__restrict__ pm, const u64 *__restrict__ npm, u64 cap,
+                                                u64 *__restrict__ counts) {
+  using Sum = std::conditional_t<WT, u64, u32>;  // a run: 512 pairs of at most 740 moves
+  const int lane = threadIdx.x & 63;
+  const u64 m = *npm;
+  if (m > cap) return;
+  const u64 waves = (u64)gridDim.x * (TPB / 64), w = (u64)blockIdx.x * (TPB / 64) + (threadIdx.x >> 6);
+  for (u64 r0 = w * LEAF_RUN; r0 < m; r0 += waves * LEAF_RUN) {
+    const u32 n = m - r0 < LEAF_RUN ? (u32)(m - r0) : LEAF_RUN;
+    Sum acc = 0;  // this lane's part of the sum of root cur
+    u32 cur = 0;
+    auto flush = [&] {
+      u64 s;
+      if constexpr (WT) {
+        s = acc;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      } else {
+        s = (u64)(u32)__builtin_amdgcn_readlane(zw::wave_scan_add((int)acc), 63);
+      }
+      if (lane == 0 && s) atomicAdd((unsigned long long *)&counts[cur], (unsigned long long)s);
+      acc = 0;
+    };
+    for (u32 j0 = 0; j0 < n; j0 += 64) {
+      const bool on = j0 + lane < n;
+      Sum v = 0;
+      u32 root = 0;
+      if (on) {
+        const u64 e = pm[r0 + j0 + lane];
+        const u32 pi = (u32)(e >> 32);
+        const u32 meta = f.meta[pi];
+        Pos p;
+        p.b0 = f.b0[pi];
+        p.b1 = f.b1[pi];
+        p.b2 = f.b2[pi];
+        p.b3 = f.b3[pi];
+        p.cr = f.cr[pi];
+        p.stm = meta & 1u;
+        const Pos c = apply_v(p, (u32)e);
+        Legal L;
+        analyse(c, L);
+        // nobulk: the reference visits every leaf: it generates the leaf's
+        // (quiescence) moves and counts one node (src/zetaperft.cl:1316-1326)
+        v = NOBULK ? 1u + (u32)(count_legal(c, L, true) > 4096) : (u32)count_legal(c, L, false);
+        if constexpr (WT) v *= f.wt[pi];
+        root = meta >> 1;
+      }
+      u64 pending = __ballot(on);
+      while (pending) {
+        const u32 rl = (u32)__builtin_amdgcn_readlane((int)root, __builtin_ctzll(pending));
+        if (rl != cur) {
+          flush();
+          cur = rl;
+        }
+        const bool its = on && root == rl;
+        acc += its ? v : 0;
+        pending &= ~__ballot(its);
+      }
+    }
+    flush();
+  }
+}
+
+// ---- merging a stored level.  k_merge enters every node of `f` into a hash
+// table (64-bit words: half of the hash, index + 1); a node that meets an equal
+// one -- same root, planes and flags, compared in full -- gives it its paths
+// and leaves.  k_compact writes those that stay to `g`.  Bound: the random
+// accesses (16 us a level of 0.1 M nodes); a level keeps some 60 % of its nodes
+// and everything below shrinks with it.
+__device__ __forceinline__ u64 node_hash(const Pos &p, u32 meta) {
+  u64 h = p.b0 * 0x9E3779B97F4A7C15ULL ^ (p.b1 + 0x7F4A7C15ULL) * 0xBF58476D1CE4E5B9ULL;
+  h = (h ^ (h >> 32)) + p.b2 * 0x94D049BB133111EBULL;
+  h = (h ^ (h >> 29)) * 0xD1B54A32D192ED03ULL + p.b3 * 0x9E3779B97F4A7C15ULL;
+  h = (h ^ (h >> 32)) * 0xBF58476D1CE4E5B9ULL + (p.cr ^ ((u64)meta << 8)) * 0x94D049BB133111EBULL;
+  return h ^ (h >> 31);
+}
+__global__ __launch_bounds__(TPB) void k_table_clear(u64 *__restrict__ tab, Level f, u64 tabcap) {
+  // two slots a node, a power of two
+  const u64 n = level_size(f);
+  u64 slots = 1024;
+  while (slots < 2 * n && slots < tabcap) slots *= 2;
+  for (u64 i = (u64)blockIdx.x * TPB + threadIdx.x; i < slots; i += (u64)gridDim.x * TPB) tab[i] = 0;
+}
+__global__ __launch_bounds__(TPB) void k_merge(u64 *__restrict__ tab, Level f, u64 tabcap) {
+  const u64 n = level_size(f);
+  u64 slots = 1024;
+  while (slots < 2 * n && slots < tabcap) slots *= 2;
+  for (u64 i = (u64)blockIdx.x * TPB + threadIdx.x; i < n; i += (u64)gridDim.x * TPB) {
+    const Pos p = level_pos(f, i);
+    const u32 meta = f.meta[i];
+    const u64 h = node_hash(p, meta);
+    const u64 e = (h & 0xFFFFFFFF00000000ULL) | (i + 1);
+    u64 s = h & (slots - 1);
+    for (;;) {
+      const u64 old = atomicCAS((unsigned long long *)&tab[s], 0ULL, (unsigned long long)e);
+      if (old == 0) break;
+      if ((old ^ e) >> 32 == 0) {
+        const u64 j = (old & 0xFFFFFFFFULL) - 1;
+        const Pos q = level_pos(f, j);
+        if (q.b0 == p.b0 && q.b1 == p.b1 && q.b2 == p.b2 && q.b3 == p.b3 && q.cr == p.cr && f.meta[j] == meta) {
+          // the one in the table keeps its place; this one's paths are its own
+          // until here (only entered nodes receive any)
+          atomicAdd((unsigned long long *)&f.wt[j], (unsigned long long)f.wt[i]);
+          f.par[i] = ~0u;  // gone
+          break;
+        }
+      }
+      s = (s + 1) & (slots - 1);
+    }
+  }
+}
+__global__ __launch_bounds__(TPB) void k_compact(Level f, Level g) {
+  __shared__ u32 part[TPB / 64];
+  __shared__ u64 base;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const u64 n = level_size(f);
+  for (u64 i0 = (u64)blockIdx.x * TPB; i0 < n; i0 += (u64)gridDim.x * TPB) {
+    const u64 i = i0 + threadIdx.x;
+    const bool stay = i < n && f.par[i] != ~0u;
+    const u64 b = __ballot(stay);
+    __syncthreads();
+    if (lane == 0) part[w] = (u32)popc(b);
+    __syncthreads();
+    if (threadIdx.x == 0)
+      base = atomicAdd((unsigned long long *)g.count, (unsigned long long)(part[0] + part[1] + part[2] + part[3]));
+    __syncthreads();
+    u64 o = base + (u64)popc(b & ((1ULL << lane) - 1));
+    for (int k = 0; k < w; k++) o += part[k];
+    if (stay && o < g.cap) level_store(g, o, level_pos(f, i), f.meta[i] >> 1, f.mv[i], f.par[i], f.wt[i]);
+  }
+}
+// the roots as level 0 (many roots)
+__global__ __launch_bounds__(TPB) void k_load_roots(const u64 *__restrict__ in, int n, Level f, u64 *__restrict__ counts) {
+  const int i = blockIdx.x * TPB + threadIdx.x;
+  if (i >= n) return;
+  if (i == 0) *f.count = (u64)n;
+  level_store(f, i, root_pos(in, i), (u32)i, 0, (u32)i, 1);
+  counts[i] = 0;
+}
+// The end of a chain: the sizes of its levels to the host's words (and cleared
+// for the next call), the counts to host memory where the call wants them.
+// Words: level sizes [0, 14), the most pairs of a pass, the pairs of the
+// current one, sizes before merging [16, 30), all pairs.
+constexpr int CTL_WORDS = 32, CTL_MOST = 14, CTL_PAIRS = 15, CTL_ALL = 30;
+// after a pass over the last level's parents
+__global__ void k_pass(u64 *ctl) {
+  const u64 n = ctl[CTL_PAIRS];
+  if (n > ctl[CTL_MOST]) ctl[CTL_MOST] = n;
+  ctl[CTL_ALL] += n;
+  ctl[CTL_PAIRS] = 0;
+}
+__global__ __launch_bounds__(TPB) void k_end(u64 *ctl, u64 *host, const u64 *__restrict__ counts, u64 *hcounts, int n) {
+  const int i = blockIdx.x * TPB + threadIdx.x;
+  if (i < CTL_WORDS) {
+    host[i] = ctl[i];
+    ctl[i] = 0;
+  }
+  if (hcounts && i < n) hcounts[i] = counts[i];
 }
 
 __global__ void k_u32_to_u64(const u32 *a, u64 *b, int n) {
@@ -552,6 +982,249 @@ int perft_device(const void *d_pos, int n, int depth, u64 *d_counts, int flags) 
   return process(0, 0, (size_t)n, D, d_counts, nobulk);
 }
 
+// ---- host side of the fast path
+// Expected parents (32 moves a position) up to which a wavefront takes each.
+// Two plies from n positions, a wavefront each against a lane each: n = 1 18
+// and 29 us, 4096 33 and 73, 8192 51 and 71, 16384 85 and 72, 32768 145 and 86.
+constexpr u64 WIDE_PARENTS = 16384;
+constexpr int MERGE_LEVEL = 3;  // the first level with transpositions: x, y, z and z, y, x
+
+struct LevelMem {
+  zr::DevBuf b0, b1, b2, b3, cr, wt, meta, mv, par;
+  u64 cap = 0;
+};
+struct FastState {
+  LevelMem lev[MAXLEV], cand;  // cand: a level before it is merged
+  zr::DevBuf ctl, table, pairs;
+  u64 tabcap = 0;
+  bool ctl_clean = false;
+};
+FastState g_fs;
+
+void release_level(LevelMem &m) {
+  for (zr::DevBuf *b : {&m.b0, &m.b1, &m.b2, &m.b3, &m.cr, &m.wt, &m.meta, &m.mv, &m.par}) zr::release(*b);
+  m.cap = 0;
+}
+int ensure_fast(LevelMem &m, u64 n) {
+  if (m.cap >= n) return ZETA_OK;
+  m.cap = 0;
+  int r;
+  for (zr::DevBuf *b : {&m.b0, &m.b1, &m.b2, &m.b3, &m.cr, &m.wt})
+    if ((r = zr::ensure(*b, n * 8))) return r;
+  for (zr::DevBuf *b : {&m.meta, &m.mv, &m.par})
+    if ((r = zr::ensure(*b, n * 4))) return r;
+  m.cap = n;
+  return ZETA_OK;
+}
+Level level_of(LevelMem &m, int word, u64 cap) {
+  return Level{(u64 *)m.b0.p,   (u64 *)m.b1.p, (u64 *)m.b2.p,  (u64 *)m.b3.p, (u64 *)m.cr.p,
+               (u64 *)m.wt.p,   (u32 *)m.meta.p, (u32 *)m.mv.p, (u32 *)m.par.p, (u64 *)g_fs.ctl.p + word, cap};
+}
+
+// One call's shape, and its buffers' capacities (a level's, and before merging).
+struct Chain {
+  const u64 *pos;  // device-visible
+  int n, D;
+  bool nobulk;
+  u64 *counts, *hcounts;  // device; where the host reads them, or null
+  u64 caps[MAXLEV], ccaps[MAXLEV], paircap;
+  double expect(int L) const {  // parents at level L
+    double e = n;
+    for (int k = 0; k < L; k++) e *= 32;
+    return e;
+  }
+  bool wide(int L) const { return expect(L) <= (double)WIDE_PARENTS; }
+  bool merged(int L) const { return !nobulk && L >= MERGE_LEVEL; }
+};
+
+unsigned wide_blocks(double e) { return (unsigned)(e < 8 * 2048 ? (e + 7) / 8 : 2048); }
+unsigned grid_blocks(double e, int per, int most) {
+  const double b = e / per + 1, cap = (double)most * zr::ctx().cu_count;
+  return (unsigned)(b < cap ? b : cap);
+}
+Level chain_level(const Chain &q, int L) { return level_of(g_fs.lev[L], L, q.caps[L]); }
+
+// levels 1 .. D - 2
+int launch_levels(const Chain &q) {
+  for (int L = 0; L < q.D - 2; L++) {
+    const bool merge = q.merged(L + 1);
+    const Level out = merge ? level_of(g_fs.cand, 16 + L + 1, q.ccaps[L + 1]) : chain_level(q, L + 1);
+    const double e = q.expect(L);
+    if (q.wide(L)) {
+      ZLAUNCH(zr::K_PERFT_EXPAND, 0, k_wide, wide_blocks(e), WIDE_TPB, 0, L ? (const u64 *)nullptr : q.pos, q.n,
+              chain_level(q, L), out, q.counts);
+    } else {
+      if (L == 0)
+        ZLAUNCH(zr::K_PERFT_ROOTS, q.n, k_load_roots, blocks(q.n, TPB), TPB, 0, q.pos, q.n, chain_level(q, 0), q.counts);
+      ZLAUNCH(zr::K_PERFT_EXPAND, 0, k_spread<false>, grid_blocks(e, XTPB, 6), XTPB, 0, chain_level(q, L), (u64)0,
+              ~(u64)0, out, (u64 *)nullptr);
+    }
+    if (merge) {
+      const unsigned nb = grid_blocks(e * 32, TPB, 8);
+      ZLAUNCH(zr::K_PERFT_APPLY, 0, k_table_clear, nb, TPB, 0, (u64 *)g_fs.table.p, out, g_fs.tabcap);
+      ZLAUNCH(zr::K_PERFT_APPLY, 0, k_merge, nb, TPB, 0, (u64 *)g_fs.table.p, out, g_fs.tabcap);
+      ZLAUNCH(zr::K_PERFT_APPLY, 0, k_compact, nb, TPB, 0, out, chain_level(q, L + 1));
+    }
+  }
+  return ZETA_OK;
+}
+
+int launch_end(const Chain &q) {
+  ZLAUNCH(zr::K_PERFT_SCAN, 0, k_end, q.hcounts ? blocks(q.n, TPB) : 1, TPB, 0, (u64 *)g_fs.ctl.p,
+          (u64 *)zr::ctx().perft_ctl_dev, q.counts, q.hcounts, q.n);
+  return ZETA_OK;
+}
+
+// the last level, below the parents of level D - 2: a wavefront a parent, or
+// passes over [0, size) of `step` parents each
+int launch_leaves(const Chain &q, u64 size, u64 step) {
+  const int L = q.D - 2;
+  const double e = q.expect(L);
+  if (q.wide(L)) {
+    // (a root's children: nothing is summed over blocks)
+    ZLAUNCH(zr::K_PERFT_LEAF, 0, k_wide_leaf, wide_blocks(e), WIDE_TPB, 0, L ? (const u64 *)nullptr : q.pos, q.n,
+            chain_level(q, L), L == 0 && q.hcounts ? q.hcounts : q.counts, q.nobulk ? 1 : 0);
+    return ZETA_OK;
+  }
+  if (L == 0) ZLAUNCH(zr::K_PERFT_ROOTS, q.n, k_load_roots, blocks(q.n, TPB), TPB, 0, q.pos, q.n, chain_level(q, 0), q.counts);
+  const Level pairs = level_of(g_fs.cand, CTL_PAIRS, q.paircap);
+  const auto leaves = q.nobulk ? k_leaves<false, true> : L >= MERGE_LEVEL ? k_leaves<true, false> : k_leaves<false, false>;
+  for (u64 i = 0; i < size; i += step) {
+    const double here = e < (double)step ? e : (double)step;
+    ZLAUNCH(zr::K_PERFT_EXPAND, 0, k_spread<true>, grid_blocks(here, XTPB, 6), XTPB, 0, chain_level(q, L), i, i + step,
+            pairs, (u64 *)g_fs.pairs.p);
+    ZLAUNCH(zr::K_PERFT_LEAF, 0, leaves, grid_blocks(here * 32, TPB, LEAF_BLOCKS), TPB, 0, chain_level(q, L),
+            (const u64 *)g_fs.pairs.p, (const u64 *)pairs.count, q.paircap, q.counts);
+    ZLAUNCH(zr::K_PERFT_SCAN, 0, k_pass, 1, 1, 0, (u64 *)g_fs.ctl.p);
+  }
+  return ZETA_OK;
+}
+
+void fast_release() {
+  for (auto &l : g_fs.lev) release_level(l);
+  release_level(g_fs.cand);
+  zr::release(g_fs.ctl);
+  zr::release(g_fs.table);
+  zr::release(g_fs.pairs);
+  g_fs.tabcap = 0;
+  g_fs.ctl_clean = false;
+}
+// the device is full: the chunked path, which needs less, takes the call
+int no_room() {
+  (void)hipGetLastError();
+  fast_release();
+  return ZETA_OK;
+}
+
+// The whole call; *done = false: a level is beyond the frontier budget (or the
+// call is one the fast path does not take) and nothing has been counted.
+int fast_perft(const u64 *pos, int n, int depth, u64 *counts, u64 *hcounts, int flags, bool *done) {
+  zr::Ctx &c = zr::ctx();
+  *done = false;
+  const bool nobulk = (flags & ZETA_PERFT_NOBULK) != 0;
+  const int D = nobulk ? depth + 1 : depth;
+  const u64 budget = c.cfg.frontier_budget;
+  if (depth < 1 || D >= MAXLEV || budget < 512 || (u64)n > budget || !c.perft_ctl_dev) return ZETA_OK;
+  int r;
+  if ((r = zr::ensure(g_fs.ctl, CTL_WORDS * 8))) return r;
+  if (!g_fs.ctl_clean) {
+    ZCHECK(hipMemsetAsync(g_fs.ctl.p, 0, CTL_WORDS * 8, c.stream));
+    g_fs.ctl_clean = true;
+  }
+  if (D == 1) {
+    ZLAUNCH(zr::K_PERFT_ROOTS, n, k_count_roots, blocks(n, 64), 64, 0, pos, n, hcounts ? hcounts : counts);
+    ZCHECK(hipStreamSynchronize(c.stream));
+    *done = true;
+    return ZETA_OK;
+  }
+  Chain q = {pos, n, D, nobulk, counts, hcounts, {0}, {0}, 0};
+  const u64 *const want = c.perft_ctl_host;
+  // waits for the chain; the sizes it reports are in `want`
+  auto finish = [&](int rc) {
+    const hipError_t e = hipStreamSynchronize(c.stream);
+    if (rc || e != hipSuccess) g_fs.ctl_clean = false;
+    return rc ? rc : e != hipSuccess ? zr::hip_fail(e, "perft sync", __FILE__, __LINE__) : ZETA_OK;
+  };
+  auto clear_words = [&] { memset(c.perft_ctl_host, 0, CTL_WORDS * 8); };
+  const int last = D - 2;
+  // pairs a pass may hold and parents whose pairs they are: 64 moves a parent
+  // at first, in the end as many as a parent can have
+  u64 moves = 64;
+  for (int tries = 0; tries < 3 * MAXLEV; tries++) {
+    // room for every level: at first 40 moves a position up to 16 M nodes,
+    // later what the levels have asked for
+    double e = n;
+    u64 cand = 0;
+    for (int L = 0; L <= last; L++, e *= 40) {
+      const double first = e < 65536 ? 65536 : (e > (double)(1 << 24) ? (double)(1 << 24) : e);
+      u64 room = (u64)first > g_fs.lev[L].cap ? (u64)first : g_fs.lev[L].cap;
+      if (L == 0) room = (u64)n;
+      if (room > budget) room = budget;
+      if (ensure_fast(g_fs.lev[L], room)) return no_room();
+      q.caps[L] = g_fs.lev[L].cap < budget ? g_fs.lev[L].cap : budget;
+      if (q.merged(L) && room > cand) cand = room;
+    }
+    if (cand) {
+      if (ensure_fast(g_fs.cand, cand)) return no_room();
+      for (int L = 0; L <= last; L++) q.ccaps[L] = g_fs.cand.cap < budget ? g_fs.cand.cap : budget;
+      u64 t = 1024;
+      while (t < 2 * g_fs.cand.cap) t *= 2;
+      if (t > g_fs.tabcap) {
+        g_fs.tabcap = 0;
+        if (zr::ensure(g_fs.table, t * 8)) return no_room();
+        g_fs.tabcap = t;
+      }
+    }
+    const bool wide = q.wide(last);
+    u64 step = ~(u64)0 >> 1;
+    if (!wide) {
+      u64 pairs = q.caps[last] > (u64)(1 << 27) / moves ? (u64)(1 << 27) : q.caps[last] * moves;
+      if (pairs > budget) pairs = budget;
+      if (pairs < (u64)MAXMOVES) return ZETA_OK;
+      if (zr::ensure(g_fs.pairs, pairs * 8)) return no_room();
+      q.paircap = pairs;
+      step = pairs / moves;
+    }
+    // one chain where one pass holds every parent there can be, else the
+    // level's size is read first
+    const bool whole = wide || q.caps[last] <= step;
+    clear_words();
+    r = launch_levels(q);
+    if (!r && whole) r = launch_leaves(q, 1, step);
+    if (!r && !(wide && last == 0)) r = launch_end(q);
+    if ((r = finish(r))) return r;
+    bool again = false;
+    for (int L = 1; L <= last && !again; L++) {
+      if (q.merged(L) && want[16 + L] > q.ccaps[L]) {
+        if (want[16 + L] > budget) return ZETA_OK;
+        if (ensure_fast(g_fs.cand, want[16 + L] + want[16 + L] / 4)) return no_room();
+        again = true;
+      } else if (want[L] > q.caps[L]) {
+        if (want[L] > budget) return ZETA_OK;
+        if (ensure_fast(g_fs.lev[L], want[L] + want[L] / 4)) return no_room();
+        again = true;
+      }
+    }
+    if (again) continue;
+    if (!whole) {
+      // the level's count is a word the end has cleared: give it back
+      const u64 size = last ? want[last] : (u64)n;
+      ZLAUNCH(zr::K_PERFT_SCAN, 0, k_fill_u64, 1, 1, 0, (u64 *)g_fs.ctl.p + last, 1, size);
+      r = launch_leaves(q, size, step);
+      if (!r) r = launch_end(q);
+      if ((r = finish(r))) return r;
+    }
+    if (!wide && want[CTL_MOST] > q.paircap) {
+      moves = moves == 64 ? 256 : (u64)MAXMOVES;
+      continue;
+    }
+    if (c.timing) c.kstat[zr::K_PERFT_LEAF].items += want[CTL_ALL];
+    *done = true;
+    return ZETA_OK;
+  }
+  return zr::fail(ZETA_ENOMEM, "perft: the levels keep growing");
+}
+
 }  // namespace
 
 void perft_release() {
@@ -566,12 +1239,21 @@ void perft_release() {
   zr::release(g_ps.counts);
   zr::release(g_ps.fails);
   zr::release(g_ps.cuts);
+  fast_release();
 }
 
 extern "C" int zeta_perft_batch_device(const void *d_pos, int n, int depth, void *d_counts, int flags) {
   int r = zr::require_up();
   if (r) return r;
   if ((!d_pos || !d_counts) && n > 0) return zr::fail(ZETA_EINVAL, "perft: null pointer");
+  bool done = false;
+  if (n > 0 && depth > 0) {
+    r = fast_perft((const u64 *)d_pos, n, depth, (u64 *)d_counts, nullptr, flags, &done);
+    if (r || done) {
+      zr::time_collect();
+      return r;
+    }
+  }
   use_growable_bufs();
   r = perft_device(d_pos, n, depth, (u64 *)d_counts, flags);
   hipError_t e = hipStreamSynchronize(zr::ctx().stream);
@@ -692,7 +1374,32 @@ extern "C" int zeta_perft_batch(const zeta_pos *pos, int n, int depth, uint64_t 
   if (n == 0) return ZETA_OK;
   if ((r = zr::ensure(g_ps.roots, (size_t)n * sizeof(zeta_pos))) || (r = zr::ensure(g_ps.counts, (size_t)n * 8)))
     return r;
-  ZCHECK(hipMemcpyAsync(g_ps.roots.p, pos, (size_t)n * sizeof(zeta_pos), hipMemcpyHostToDevice, zr::ctx().stream));
+  zr::Ctx &c = zr::ctx();
+  // few positions go through pinned host memory, which the kernels read and
+  // write themselves: two copies less in the chain
+  const bool pinned = n <= zr::PERFT_STAGE;
+  if (pinned) memcpy(c.perft_stage_host, pos, (size_t)n * sizeof(zeta_pos));
+  else ZCHECK(hipMemcpyAsync(g_ps.roots.p, pos, (size_t)n * sizeof(zeta_pos), hipMemcpyHostToDevice, c.stream));
+  if (depth > 0) {
+    bool done = false;
+    r = fast_perft(pinned ? (const u64 *)c.perft_stage_dev : (const u64 *)g_ps.roots.p, n, depth, (u64 *)g_ps.counts.p,
+                   pinned ? (u64 *)c.perft_counts_dev : nullptr, 0, &done);
+    if (r) {
+      zr::time_collect();
+      return r;
+    }
+    if (done) {
+      if (pinned) {
+        memcpy(counts, c.perft_counts_host, (size_t)n * 8);
+      } else {
+        ZCHECK(hipMemcpyAsync(counts, g_ps.counts.p, (size_t)n * 8, hipMemcpyDeviceToHost, c.stream));
+        ZCHECK(hipStreamSynchronize(c.stream));
+      }
+      zr::time_collect();
+      return ZETA_OK;
+    }
+  }
+  if (pinned) ZCHECK(hipMemcpyAsync(g_ps.roots.p, pos, (size_t)n * sizeof(zeta_pos), hipMemcpyHostToDevice, c.stream));
   use_growable_bufs();
   r = perft_device(g_ps.roots.p, n, depth, (u64 *)g_ps.counts.p, 0);
   if (r) {

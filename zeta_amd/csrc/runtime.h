@@ -35,6 +35,9 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
+// perft calls of up to this many positions exchange them in pinned host memory
+constexpr int PERFT_STAGE = 256;
+
 struct Ctx {
   bool up = false;
   int device = 0;
@@ -44,10 +47,17 @@ struct Ctx {
   int cu_count = 0;
   bool timing = false;
   bool serving = false;  // a persistent serving grid owns the stream (zeta_serve_start .. stop)
-  // 64 bytes of coherent pinned host memory, allocated by zeta_init:
-  // bytes 0-3 the search abort word (zeta_search_abort) that the search
-  // workers poll at abort_dev, bytes 8-15 the perft level total the host
-  // waits for (perft_total_host, after ev_total)
+  // coherent pinned host memory, allocated by zeta_init (HOST_BYTES): bytes
+  // 0-3 the search abort word (zeta_search_abort) that the search workers poll
+  // at abort_dev, bytes 8-15 the perft level total the host waits for
+  // (perft_total_host, after ev_total), from 256 the sizes of a perft call's
+  // levels (perft_ctl_*), from 1024 its positions and from 1024 +
+  // 64 * PERFT_STAGE their counts
+  static constexpr size_t HOST_BYTES = 1024 + 72 * (size_t)PERFT_STAGE;
+  uint64_t *perft_ctl_host = nullptr;
+  const uint64_t *perft_counts_host = nullptr;
+  void *perft_ctl_dev = nullptr, *perft_stage_dev = nullptr, *perft_counts_dev = nullptr;
+  void *perft_stage_host = nullptr;
   uint32_t *abort_host = nullptr;
   const uint32_t *abort_dev = nullptr;
   uint64_t *perft_total_host = nullptr;

@@ -151,13 +151,13 @@ extern "C" int zeta_init(const zeta_config *cfg) {
   e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
   if (e != hipSuccess) return fail(ZETA_ENODEV, "hipStreamCreate: %s", hipGetErrorString(e));
   void *ab = nullptr;
-  e = hipHostMalloc(&ab, 64, hipHostMallocCoherent | hipHostMallocMapped);
+  e = hipHostMalloc(&ab, Ctx::HOST_BYTES, hipHostMallocCoherent | hipHostMallocMapped);
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c.stream);
     c.stream = nullptr;
     return fail(ZETA_ENOMEM, "hipHostMalloc of the abort word: %s", hipGetErrorString(e));
   }
-  memset(ab, 0, 64);
+  memset(ab, 0, Ctx::HOST_BYTES);
   void *abd = nullptr;
   e = hipHostGetDevicePointer(&abd, ab, 0);
   if (e != hipSuccess) {
@@ -169,6 +169,12 @@ extern "C" int zeta_init(const zeta_config *cfg) {
   c.abort_host = (uint32_t *)ab;
   c.abort_dev = (const uint32_t *)abd;
   c.perft_total_host = (uint64_t *)((char *)ab + 8);
+  c.perft_ctl_host = (uint64_t *)((char *)ab + 256);
+  c.perft_ctl_dev = (char *)abd + 256;
+  c.perft_stage_host = (char *)ab + 1024;
+  c.perft_stage_dev = (char *)abd + 1024;
+  c.perft_counts_host = (const uint64_t *)((char *)ab + 1024 + 64 * PERFT_STAGE);
+  c.perft_counts_dev = (char *)abd + 1024 + 64 * PERFT_STAGE;
   e = hipEventCreateWithFlags(&c.ev_total, hipEventDisableTiming);
   if (e == hipSuccess && (rc = perft_setup()) != ZETA_OK) e = hipErrorUnknown;
   if (e != hipSuccess) {
@@ -178,6 +184,8 @@ extern "C" int zeta_init(const zeta_config *cfg) {
     c.abort_host = nullptr;
     c.abort_dev = nullptr;
     c.perft_total_host = nullptr;
+    c.perft_ctl_host = nullptr;
+    c.perft_ctl_dev = nullptr;
     (void)hipStreamDestroy(c.stream);
     c.stream = nullptr;
     return rc ? rc : fail(ZETA_ENODEV, "hipEventCreate: %s", hipGetErrorString(e));
@@ -211,6 +219,8 @@ extern "C" int zeta_shutdown(void) {
   c.abort_host = nullptr;
   c.abort_dev = nullptr;
   c.perft_total_host = nullptr;
+  c.perft_ctl_host = nullptr;
+  c.perft_ctl_dev = nullptr;
   (void)hipStreamDestroy(c.stream);
   c.stream = nullptr;
   c.up = false;
