@@ -88,3 +88,16 @@ def test_levels_that_outgrow_their_buffers(zeta, oracle):
     finally:
         zeta.shutdown()
         zeta.init()
+
+
+@pytest.mark.parametrize("n,minply,maxply", [(1, 0, 0), (3, 1, 1), (5, 8, 40), (257, 0, 200), (4097, 20, 60)])
+def test_playouts_a_wavefront_each(zeta, oracle, n, minply, maxply):
+    g, o = zeta.playouts(7, n, minply, maxply), oracle.gen_playouts(7, n, minply, maxply)
+    assert (g["b"] == o["b"]).all() and (g["stm"] == o["stm"]).all()
+
+
+def test_playouts_either_way(zeta):
+    # position i depends on the seed and i only; the larger calls take a lane each
+    few = zeta.playouts(9, 3000, 0, 120)
+    for n in (40960, 40961, 100000):
+        assert (zeta.playouts(9, n, 0, 120)[:3000] == few).all()

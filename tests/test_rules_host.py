@@ -22,6 +22,9 @@ def H(tmp_path_factory):
     L = ctypes.CDLL(so)
     L.rh_count.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
     L.rh_count.restype = None
+    L.rh_lanes.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    L.rh_mod.argtypes = [ctypes.c_uint64, ctypes.c_uint32]
+    L.rh_mod.restype = ctypes.c_uint32
     L.rh_rays.argtypes = [ctypes.c_uint64, ctypes.c_uint64]
     return L
 
@@ -89,6 +92,27 @@ def test_emitted_moves_of_several_kings(H):
         assert out[1] == out[2], (k, [hex(int(v)) for v in b])
         differ += out[0] != out[2]
     assert differ  # the first one
+
+
+def test_moves_by_lane_out_of_check(H):
+    rng = np.random.default_rng(15)
+    p = np.zeros(1, dtype=R.POS_DTYPE)
+    free = 0
+    for k in range(4000):
+        p["b"][0] = _board(rng, int(rng.integers(2, 30)), k & 1)
+        p["stm"][0] = k & 1
+        b = np.ascontiguousarray(p["b"][0])
+        n = H.rh_lanes(b.ctypes.data, k & 1)
+        assert n == -2 or n == R.count_legal(p), (k, n, [hex(int(v)) for v in b])
+        free += n >= 0
+    assert free > 800
+
+
+def test_small_moduli(H):
+    rng = np.random.default_rng(16)
+    for n in range(1, 257):
+        for z in [0, n - 1, n, (1 << 64) - 1, (1 << 64) - n] + [int(v) for v in rng.integers(0, 1 << 64, 60, dtype=np.uint64)]:
+            assert H.rh_mod(z, n) == z % n
 
 
 def test_rank_rays(H):

@@ -631,6 +631,16 @@ ZD u64 line_att(const SqLines &q, u64 occ, u64 mask) {  // mask: one of q's line
 ZD u64 rook_sq(const SqLines &q, u64 occ) { return line_att(q, occ, q.rank) | line_att(q, occ, q.file); }
 ZD u64 bishop_sq(const SqLines &q, u64 occ) { return line_att(q, occ, q.diag) | line_att(q, occ, q.anti); }
 
+// what move generation needs of the lane's square, in registers for good
+struct LaneSq {
+  SqLines q;
+  u64 knight, king, wpawn, bpawn;
+};
+ZD LaneSq lane_sq(int sq) {
+  const u64 b = bit(sq);
+  return LaneSq{sq_lines(sq), knight_att(b), king_att(b), pawn_att(b, 0), pawn_att(b, 1)};
+}
+
 // Does the side `by` attack the king of the other side?  kb = the king's
 // bitboard (0 for no king: never), q = the lines of its square.
 // One position per lane, the same king square in every lane: the checkers of
@@ -731,6 +741,79 @@ ZD u64 lane_targets(const Pos &p, const Node0 &B, u64 A, int sq, bool qs) {
   const bool rk = type == ROOK || type == QUEEN, bs = type == BISHOP || type == QUEEN;
   t = sel(rk, rook_sq(sq, occ)) | sel(bs, bishop_sq(sq, occ)) | sel(type == KNIGHT, knight_att(b));
   return t & T;
+}
+
+// ---- lane = square of one position whose king is not in check: what a slider
+// on the lane's square would see
+struct LaneRays {
+  u64 rank, file, diag, anti;
+};
+ZD LaneRays lane_rays(const LaneSq &me, u64 occ) {
+  return LaneRays{line_att(me.q, occ, me.q.rank), line_att(me.q, occ, me.q.file), line_att(me.q, occ, me.q.diag),
+                  line_att(me.q, occ, me.q.anti)};
+}
+// is the lane's square attacked by the side that is not to move (the own king
+// a blocker)?
+ZD bool lane_attacked(const Pos &p, const LaneSq &me, const LaneRays &y) {
+  const u64 opp = p.stm ? p.b0 ^ (p.b1 | p.b2 | p.b3) : p.b0;
+  const u64 rq = p.b3 & (p.b1 ^ p.b2), bq = p.b3 & ~p.b1;
+  u64 a = ((y.rank | y.file) & rq) | ((y.diag | y.anti) & bq);
+  a |= (me.knight & ~p.b1 & p.b2 & ~p.b3) | (me.king & p.b1 & p.b2 & ~p.b3);
+  a |= (p.stm ? me.bpawn : me.wpawn) & p.b1 & ~p.b2 & ~p.b3;
+  return (a & opp) != 0;
+}
+// legal targets of the own piece on the lane's square; A: the squares that
+// lane_attacked is true for.  A piece that sees its king and, the other way on
+// the line, a slider of the line is pinned to it.
+ZD u64 lane_free_targets(const Pos &p, const LaneSq &me, const LaneRays &y, u64 A, int sq) {
+  const u64 b = me.q.b, occ = p.b1 | p.b2 | p.b3;
+  const u64 opp = p.stm ? p.b0 ^ occ : p.b0, own = occ ^ opp;
+  if (!(own & b)) return 0;
+  const u64 rq = p.b3 & (p.b1 ^ p.b2), bq = p.b3 & ~p.b1;
+  const u64 king = own & p.b1 & p.b2 & ~p.b3;
+  const u32 type = (u32)((p.b1 & b ? 1 : 0) | (p.b2 & b ? 2 : 0) | (p.b3 & b ? 4 : 0));
+  u64 pm = FULL;
+  if ((y.rank & king) && (y.rank & opp & rq)) pm = me.q.rank;
+  if ((y.file & king) && (y.file & opp & rq)) pm = me.q.file;
+  if ((y.diag & king) && (y.diag & opp & bq)) pm = me.q.diag;
+  if ((y.anti & king) && (y.anti & opp & bq)) pm = me.q.anti;
+  u64 t = sel(type == ROOK || type == QUEEN, y.rank | y.file) | sel(type == BISHOP || type == QUEEN, y.diag | y.anti) |
+          sel(type == KNIGHT, me.knight);
+  t &= ~own;
+  if (type == KING) {
+    t = me.king & ~own & ~A;
+    if (p.cr & SMCRALL) t |= castle_squares(p, own & rq & ~p.b2, occ, A, sq);
+  }
+  if (type == PAWN) {
+    const u64 s1 = (p.stm ? b >> 8 : b << 8) & ~occ;
+    const u64 s2 = (p.stm ? (s1 & RANK6) >> 8 : (s1 & RANK3) << 8) & ~occ;
+    t = ((p.stm ? me.bpawn : me.wpawn) & opp) | s1 | s2;
+  }
+  t &= pm;
+  const u64 w = ~p.cr & RANKS45;
+  if (type == PAWN && w) {
+    const int sqep = lsb(w);
+    if ((p.stm ? RANK4 : RANK5) & (bit(sqep + 1) | bit(sqep - 1)) & b) {
+      Node0 B;
+      node_basics(p, B);
+      const int to = (p.stm ? sqep - 8 : sqep + 8) & 63;
+      if (ep_legal0(B, sq, to, sqep)) t |= bit(to);
+    }
+  }
+  return t;
+}
+
+// z modulo n, n from 1 to 256, sixteen bits at a time: a remainder and the next
+// bits are below 2^24, where a float quotient is off by one at most
+ZD u32 mod_small(u64 z, u32 n) {
+  const float inv = 1.0f / (float)n;
+  u32 r = 0;
+  for (int s = 48; s >= 0; s -= 16) {
+    const u32 t = (r << 16) | (u32)((z >> s) & 0xFFFF);
+    const int d = (int)(t - (u32)((float)t * inv) * n);
+    r = (u32)(d < 0 ? d + (int)n : d >= (int)n ? d - (int)n : d);
+  }
+  return r;
 }
 
 // Pack from->to with the reference movepicker rules (src/zetaperft.cl:1363-1386):

@@ -709,31 +709,112 @@ __global__ void k_fill_u64(u64 *b, int n, u64 v) {
   if (i < n) b[i] = v;
 }
 
-// ---- playouts (workload generator), one lane per position
+// ---- playouts (workload generator)
+__device__ __forceinline__ Pos start_pos() {  // setboard of the standard FEN with KQkq
+  Pos p;
+  p.b0 = 0xFFFF000000000000ULL;
+  p.b1 = 0x91FF00000000FF91ULL;
+  p.b2 = 0x5A0000000000005AULL;
+  p.b3 = 0xAD000000000000ADULL;
+  p.cr = 0x6EFFFFFFFFFFFF6EULL;
+  p.stm = 0;
+  return p;
+}
+struct PlayRng {
+  u64 st;
+  __device__ __forceinline__ PlayRng(u64 seed, u32 i, u64 attempt)
+      : st(seed ^ ((u64)i * 0x9E3779B97F4A7C15ULL) ^ (attempt * 0xD1B54A32D192ED03ULL)) {}
+  __device__ __forceinline__ u64 next() {
+    u64 z = (st += 0x9E3779B97F4A7C15ULL);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
+    return z ^ (z >> 31);
+  }
+};
+__device__ __forceinline__ void store_playout(u64 *q, const Pos &p, u32 hmc) {
+  q[0] = p.b0;
+  q[1] = p.b1;
+  q[2] = p.b2;
+  q[3] = p.b3;
+  q[4] = p.cr;
+  q[5] = hash_full(p);
+  q[6] = hmc;
+  q[7] = p.stm;
+}
+
+// One wavefront a position, lane = square.  A playout is a chain of plies:
+// with a lane a position 4096 of them are 64 wavefronts on 1024 SIMDs, each as
+// slow as its longest playout and its busiest lane (1.84 ms at 20-60 plies,
+// 0.23 ms here).  Bound: instruction issue of one wavefront, about 650 a ply;
+// the rays of the lane's square serve the attack map, the pins and the targets,
+// and the x-rays through the king are left to the positions in check.
+__global__ __launch_bounds__(TPB) void k_playout_wide(u64 seed, int n, int minply, int maxply, u64 *out, u32 *fails) {
+  const int lane = threadIdx.x & 63;
+  const int i = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (TPB / 64) + (threadIdx.x >> 6)));
+  if (i >= n) return;
+  const LaneSq me = lane_sq(lane);
+  // the lane's legal targets; all of them, summed up to this lane: incl
+  auto targets = [&](const Pos &p, int &incl) {
+    const u64 occ = p.b1 | p.b2 | p.b3;
+    const LaneRays y = lane_rays(me, occ);
+    u64 A = __ballot(lane_attacked(p, me, y));
+    const u64 own = p.stm ? p.b0 : p.b0 ^ occ;
+    u64 t;
+    if (A & own & p.b1 & p.b2 & ~p.b3) {  // in check
+      Node0 B;
+      node_basics(p, B);
+      A = __ballot(attacked_nk(B, lane));
+      t = (own >> lane) & 1 ? lane_targets(p, B, A, lane, false) : 0;
+    } else {
+      t = lane_free_targets(p, me, y, A, lane);
+    }
+    incl = zw::wave_scan_add(popc(t));
+    return t;
+  };
+  for (u64 a = 0; a <= 1000; a++) {
+    PlayRng rng(seed, (u32)i, a);
+    const int plies = minply + (int)(rng.next() % (u64)(maxply - minply + 1));
+    Pos p = start_pos();
+    u32 hmc = 0;
+    bool ok = true;
+    for (int k = 0; k <= plies; k++) {
+      int incl;
+      const u64 t = targets(p, incl);
+      const int nl = __builtin_amdgcn_readlane(incl, 63);
+      if (nl == 0 || hmc >= 100) {
+        ok = false;
+        break;
+      }
+      if (k == plies) break;
+      const int pick = (int)mod_small(rng.next(), (u32)nl);
+      // the origin whose targets hold move `pick` (origins ascending, then targets)
+      const int f = __builtin_ctzll(__ballot(incl > pick));
+      const u64 tf = (u64)(u32)__builtin_amdgcn_readlane((int)(u32)t, f) |
+                     (u64)(u32)__builtin_amdgcn_readlane((int)(u32)(t >> 32), f) << 32;
+      const u32 m = make_code(p, f, nth_bit(tf, pick - __builtin_amdgcn_readlane(incl - popc(t), f)));
+      hmc = next_hmc(hmc, m);
+      p = apply(p, m, true);
+    }
+    if (ok) {
+      if (lane == 0) store_playout(out + (size_t)i * 8, p, hmc);
+      return;
+    }
+  }
+  if (lane == 0) atomicAdd(fails, 1u);
+}
+
+// one lane a position: more of them than the wavefronts the chip holds
 __global__ __launch_bounds__(TPB) void k_playout(u64 seed, int n, int minply, int maxply, u64 *out,
                                                  u32 *fails) {
   const int i = blockIdx.x * TPB + threadIdx.x;
   if (i >= n) return;
-  Pos s0;  // the initial position, setboard of the standard FEN with KQkq
-  s0.b0 = 0xFFFF000000000000ULL;
-  s0.b1 = 0x91FF00000000FF91ULL;
-  s0.b2 = 0x5A0000000000005AULL;
-  s0.b3 = 0xAD000000000000ADULL;
-  s0.cr = 0x6EFFFFFFFFFFFF6EULL;
-  s0.stm = 0;
   for (u64 a = 0; a <= 1000; a++) {
-    u64 st = seed ^ ((u64)i * 0x9E3779B97F4A7C15ULL) ^ (a * 0xD1B54A32D192ED03ULL);
-    auto rnd = [&st]() {
-      u64 z = (st += 0x9E3779B97F4A7C15ULL);
-      z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
-      z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
-      return z ^ (z >> 31);
-    };
-    const int plies = minply + (int)(rnd() % (u64)(maxply - minply + 1));
-    Pos p = s0;
+    PlayRng rng(seed, (u32)i, a);
+    const int plies = minply + (int)(rng.next() % (u64)(maxply - minply + 1));
+    Pos p = start_pos();
     u32 hmc = 0;
     bool ok = true;
-    for (int k = 0; k < plies; k++) {
+    for (int k = 0; k <= plies; k++) {
       Legal L;
       analyse(p, L);
       const int nl = count_legal(p, L, false);
@@ -741,26 +822,13 @@ __global__ __launch_bounds__(TPB) void k_playout(u64 seed, int n, int minply, in
         ok = false;
         break;
       }
-      const int pick = (int)(rnd() % (u64)nl);
-      const u32 m = nth_legal(p, L, pick);
+      if (k == plies) break;
+      const u32 m = nth_legal(p, L, (int)mod_small(rng.next(), (u32)nl));
       hmc = next_hmc(hmc, m);
       p = apply_v(p, m);
     }
     if (ok) {
-      Legal L;
-      analyse(p, L);
-      if (count_legal(p, L, false) == 0 || hmc >= 100) ok = false;
-    }
-    if (ok) {
-      u64 *q = out + (size_t)i * 8;
-      q[0] = p.b0;
-      q[1] = p.b1;
-      q[2] = p.b2;
-      q[3] = p.b3;
-      q[4] = p.cr;
-      q[5] = hash_full(p);
-      q[6] = hmc;
-      q[7] = p.stm;
+      store_playout(out + (size_t)i * 8, p, hmc);
       return;
     }
   }
@@ -987,6 +1055,11 @@ int perft_device(const void *d_pos, int n, int depth, u64 *d_counts, int flags) 
 // Two plies from n positions, a wavefront each against a lane each: n = 1 18
 // and 29 us, 4096 33 and 73, 8192 51 and 71, 16384 85 and 72, 32768 145 and 86.
 constexpr u64 WIDE_PARENTS = 16384;
+// Playouts up to which a wavefront takes each.  Kernel time at 20-60 plies, a
+// wavefront each against a lane each: n = 1 51 and 181 us, 4096 230 and 1802,
+// 32768 1139 and 1588, 65536 2129 and 1613; at 8-40 plies 32768 748 and 918,
+// 65536 1392 and 959.
+constexpr int WIDE_PLAYOUTS = 40960;
 constexpr int MERGE_LEVEL = 3;  // the first level with transpositions: x, y, z and z, y, x
 
 struct LevelMem {
@@ -1421,8 +1494,9 @@ extern "C" int zeta_playouts(uint64_t seed, int n, int minply, int maxply, zeta_
   if (n == 0) return ZETA_OK;
   if ((r = zr::ensure(g_ps.roots, (size_t)n * sizeof(zeta_pos))) || (r = zr::ensure(g_ps.fails, 4))) return r;
   ZCHECK(hipMemsetAsync(g_ps.fails.p, 0, 4, zr::ctx().stream));
-  ZLAUNCH(zr::K_PLAYOUT, n, k_playout, blocks(n, TPB), TPB, 0, seed, n, minply, maxply, (u64 *)g_ps.roots.p,
-          (u32 *)g_ps.fails.p);
+  const bool wide = n <= WIDE_PLAYOUTS;
+  ZLAUNCH(zr::K_PLAYOUT, n, wide ? k_playout_wide : k_playout, blocks(n, wide ? TPB / 64 : TPB), TPB, 0, seed, n, minply,
+          maxply, (u64 *)g_ps.roots.p, (u32 *)g_ps.fails.p);
   u32 fails = 0;
   ZCHECK(hipMemcpyAsync(out, g_ps.roots.p, (size_t)n * sizeof(zeta_pos), hipMemcpyDeviceToHost, zr::ctx().stream));
   ZCHECK(hipMemcpyAsync(&fails, g_ps.fails.p, 4, hipMemcpyDeviceToHost, zr::ctx().stream));

@@ -837,15 +837,6 @@ __device__ __forceinline__ void restore(const Ply &y, Node &n, int lane) {
 // the move that led to the node at ply sd, 0 at the root
 __device__ __forceinline__ u32 last_move(const Lds &L, int sd) { return sd > 1 ? uf(L.ply[sd - 1].w[W_MOVE]) : 0u; }
 
-// what move generation needs of the lane's square, in registers for good
-struct LaneSq {
-  SqLines q;
-  u64 knight, king, wpawn, bpawn;
-};
-__device__ __forceinline__ LaneSq lane_sq(int sq) {
-  const u64 b = bit(sq);
-  return LaneSq{sq_lines(sq), knight_att(b), king_att(b), pawn_att(b, 0), pawn_att(b, 1)};
-}
 // the lines of a wave-uniform square, in vector registers (24 scalar ones for
 // the two kings are more than the search has to spare)
 __device__ __forceinline__ SqLines lds_lines(const Lds &L, int k) {
