@@ -26,10 +26,9 @@
 //
 // Transposition table (2^k entries x 16 B in HBM, lockless: word0 =
 // key ^ word1): every entry supplies the move ordering's TT move; its score
-// is used to raise alpha only when it cannot change the root value: the
-// entry was stored at the same depth by a node whose half-move clock was 0
-// and the probing node's clock is 0 too (then neither subtree can see a
-// repetition above itself), and the key includes the exact castle squares.
+// is used only when it cannot change the root value: at the same depth, with
+// the exact castle squares in the key, and where neither the storing nor the
+// probing path can repeat a position above the node (path_free).
 #include <string.h>
 
 #include "chess.h"
@@ -236,6 +235,7 @@ struct Node {  // the current full-width node (wave-uniform)
   bool kic, pass2;  // in check; second pass (deferred moves)
   int ndefer, searched;
   bool busy;
+  u32 reach;        // see path_free
 };
 
 // child hash of the alpha-beta move-up (src/zeta.cl:2297-2359), incremental
@@ -269,34 +269,6 @@ __device__ __forceinline__ u32 child_hmc(u32 hmc, u32 m) {
 }
 
 enum { S_ENTER = 0, S_NEXT, S_RETURN, S_QS };
-
-// TT store when a full-width node returns: with a move that raised alpha, a
-// lower bound of the node's value and that move; with none (every move
-// failed low), an upper bound and no move (bit 58).  The score is kept as
-// distance-to-mate from this node.  Either bound is the value of the
-// depth-limited subtree, which a node with a zero half-move clock cannot see
-// depend on the path above it: entries are used at the same depth and clock
-// only, so no root value depends on them.
-__device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Node &n, int sd, int lane) {
-  if (!ttmask) return 0;
-  s32 s = n.alpha;
-  const int plyn = sd - 1;
-  if (is_mate(s) && s > 0) s += plyn;
-  if (is_mate(s) && s < 0) s -= plyn;
-  const u64 key = tt_key(n.hash, n.p.cr);
-  const u64 w1 = (u64)n.best | ((u64)(u16)(int16_t)s << 32) | ((u64)(n.depth & 0xFF) << 48) |
-                 ((u64)(n.hmc == 0 ? 1 : 0) << 56) | (1ULL << 57) | ((u64)(n.best ? 0 : 1) << 58);
-  if (lane == 0) {
-    const u64 w0 = key ^ w1;
-    u32x4 e;
-    e.x = (u32)w0;
-    e.y = (u32)(w0 >> 32);
-    e.z = (u32)w1;
-    e.w = (u32)(w1 >> 32);
-    *glob((u32x4 *)(a->tt + 2 * (key & ttmask))) = e;  // one 16-byte vector store
-  }
-  return 1;
-}
 
 // A counter move is a quiet move, which its from- and to-square and its
 // piece determine (sqcpt = to, no captured piece, pto = pfrom or the queen a
@@ -772,6 +744,7 @@ struct Lds {  // one worker's memory: eight workers a CU
   // its best move so far, and the result of the last completed one
   u64 ticket;
   int root, depth, iteration;
+  int hlen;  // positions of the game before the root
   s32 best_score, final_score;
   u32 best_move, final_move;
 };
@@ -793,7 +766,7 @@ __device__ __forceinline__ void get_planes(int w, Pos &p) {
 }
 __device__ __forceinline__ u32 window(s32 alpha, s32 beta) { return ((u32)alpha & 0xFFFFu) | ((u32)beta << 16); }
 
-enum { F_STM = 1, F_CHECK = 2, F_PASS2 = 4, F_BUSY = 8 };
+enum { F_STM = 1, F_CHECK = 2, F_PASS2 = 4, F_BUSY = 8, F_REACH = 16 };  // F_REACH: two bits
 
 __device__ __forceinline__ void save(Ply &y, const Node &n, int lane) {
   int w = put_planes(0, n.p);
@@ -806,7 +779,8 @@ __device__ __forceinline__ void save(Ply &y, const Node &n, int lane) {
   w = put32(w, W_BEST, n.best);
   w = put32(w, W_LIST, (u32)n.mbeg | ((u32)n.mcnt << 16));
   w = put32(w, W_COUNTS, (u32)n.depth | (n.hmc << 8) | ((u32)n.searched << 16) | ((u32)n.ndefer << 24));
-  w = put32(w, W_FLAGS, (n.p.stm ? F_STM : 0) | (n.kic ? F_CHECK : 0) | (n.pass2 ? F_PASS2 : 0) | (n.busy ? F_BUSY : 0));
+  w = put32(w, W_FLAGS, (n.p.stm ? F_STM : 0) | (n.kic ? F_CHECK : 0) | (n.pass2 ? F_PASS2 : 0) | (n.busy ? F_BUSY : 0) |
+                         n.reach * F_REACH);
   w = put32(w, W_TTM, n.ttm);
   if (lane < NWORDS) y.w[lane] = (u32)w;
 }
@@ -832,10 +806,63 @@ __device__ __forceinline__ void restore(const Ply &y, Node &n, int lane) {
   n.kic = (fl & F_CHECK) != 0;
   n.pass2 = (fl & F_PASS2) != 0;
   n.busy = (fl & F_BUSY) != 0;
+  n.reach = fl / F_REACH;
   n.ttm = get32(w, W_TTM);
 }
 // the move that led to the node at ply sd, 0 at the root
 __device__ __forceinline__ u32 last_move(const Lds &L, int sd) { return sd > 1 ? uf(L.ply[sd - 1].w[W_MOVE]) : 0u; }
+
+// Whether what a search below the node at ply sd found holds on any path to it.
+// Only positions searched in full width are tested for repetition.  `reach` is
+// how far below the node the search (or a table entry it used) tested one that
+// reversible moves lead to: 3 for 3 or more.  hr plies above the node are
+// reversibly connected to it.  A position k plies below repeats one above only
+// if they are 4, 6, .. plies apart: none while reach + hr <= 3.  One ply below,
+// 4 plies apart, the two moves of the side that moved last are both on the path
+// and have to take each other back.  The half-move clock has to stay clear of
+// 100 as well.  With a clock of 0 nothing above can be met again.
+// Most nodes have one ply left, no checking move and so reach 0: their bounds
+// serve every order of the moves that lead to them: 1.0 M of 4.1 M probes of a
+// 1024-position depth-4 batch end the node (before, with a clock of 0 on both
+// sides required, moves in another order were searched again), and the probe
+// comes ahead of the generation.
+__device__ __forceinline__ bool path_free(const Lds &L, const Node &n, u32 reach, int sd) {
+  if (n.hmc == 0) return true;
+  if (reach >= 3 || n.hmc >= 90) return false;
+  if (reach == 0) return true;
+  const int above = sd - 1 + uf(L.hlen), hr = (int)n.hmc < above ? (int)n.hmc : above;
+  if ((int)reach + hr <= 3) return true;
+  if (reach != 1 || hr > 4 || sd < 4) return false;
+  const u32 m = uf(L.ply[sd - 1].w[W_MOVE]), o = uf(L.ply[sd - 3].w[W_MOVE]);
+  return mv_from(m) != mv_to(o) || mv_to(m) != mv_from(o);
+}
+
+// TT store when a full-width node returns: with a move that raised alpha, a
+// lower bound of the node's value and that move; with none (every move
+// failed low), an upper bound and no move (bit 58).  The score is kept as
+// distance-to-mate from this node.  Bit 56: the bound does not depend on the
+// path above the node; bits 59-60: the node's reach (path_free).
+__device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Lds &L, const Node &n, int sd, int lane) {
+  if (!ttmask) return 0;
+  s32 s = n.alpha;
+  const int plyn = sd - 1;
+  if (is_mate(s) && s > 0) s += plyn;
+  if (is_mate(s) && s < 0) s -= plyn;
+  const u64 key = tt_key(n.hash, n.p.cr);
+  const u64 w1 = (u64)n.best | ((u64)(u16)(int16_t)s << 32) | ((u64)(n.depth & 0xFF) << 48) |
+                 ((u64)(path_free(L, n, n.reach, sd) ? 1 : 0) << 56) | (1ULL << 57) | ((u64)(n.best ? 0 : 1) << 58) |
+                 ((u64)n.reach << 59);
+  if (lane == 0) {
+    const u64 w0 = key ^ w1;
+    u32x4 e;
+    e.x = (u32)w0;
+    e.y = (u32)(w0 >> 32);
+    e.z = (u32)w1;
+    e.w = (u32)(w1 >> 32);
+    *glob((u32x4 *)(a->tt + 2 * (key & ttmask))) = e;  // one 16-byte vector store
+  }
+  return 1;
+}
 
 // the lines of a wave-uniform square, in vector registers (24 scalar ones for
 // the two kings are more than the search has to spare)
@@ -1344,6 +1371,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       L.ticket = ticket;
       L.final_score = 0;
       L.final_move = 0;
+      const s32 hl = a->hist ? a->hlen[r] : 0;
+      L.hlen = hl > ZETA_HISTORY ? ZETA_HISTORY : (hl < 0 ? 0 : hl);
     }
     wsync();
 
@@ -1445,17 +1474,71 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.searched = 0;
           n.mcnt = 0;
           n.ttm = 0;
+          n.reach = 0;
           if (qs) {
             // a quiescence node whose evaluation its parent did not know
             qknown = false;
             state = S_QS;
             continue;
           }
-          // issue the TT load early: its latency overlaps the generation below
           const u64 ttmask = tt_mask(cfg);
           const u64 key = tt_key(n.hash, n.p.cr);
           u32x4 tte = {0u, 0u, 0u, 0u};
           if (ttmask && sd > 1) tte = *glob((const u32x4 *)(a->tt + 2 * (key & ttmask)));
+          // draws that hold with and without moves
+          if (sd > 1 && (n.hmc >= 100 || popc(n.p.b1 | n.p.b2 | n.p.b3) <= 2)) {
+            v = 0;
+            state = S_RETURN;
+            continue;
+          }
+          bool repeated = false;
+          if (sd > 1 && n.hmc >= 2) {
+            // repetition against plies plyn-2, plyn-4, .. >= plyn-hmc: the
+            // searched path, then the game history before the root
+            bool hit = false;
+            const int nn = plyn - 2 - 2 * lane;
+            if (nn >= plyn - (int)n.hmc) {
+              if (nn >= 0) {
+                const u32 *const w = L.ply[nn + 1].w;
+                hit = (((u64)w[W_HASH + 1] << 32) | w[W_HASH]) == n.hash;
+              } else if (-nn - 1 < L.hlen) {
+                hit = a->hist[(size_t)L.root * ZETA_HISTORY + (-nn - 1)] == n.hash;
+              }
+            }
+            repeated = __ballot(hit) != 0;
+          }
+          // TT probe, before any move is generated (a stored node had moves):
+          // move for ordering; score where no path to the node changes it
+          u32 ttmove = 0;
+          if (ttmask && sd > 1) {
+            const u64 w0 = uf(((u64)tte.y << 32) | tte.x), w1 = uf(((u64)tte.w << 32) | tte.z);
+            lcount(cvec, C_TT_PROBE, 1);
+            if ((w0 ^ w1) == key && ((w1 >> 57) & 1)) {
+              lcount(cvec, C_TT_HIT, 1);
+              ttmove = (u32)w1;
+              s32 ts = (s32)(int16_t)(u16)(w1 >> 32);
+              const int d = (int)((w1 >> 48) & 0xFF);
+              const u32 reach = (u32)(w1 >> 59) & 3u;
+              if (is_mate(ts) && ts > 0) ts -= plyn;
+              if (is_mate(ts) && ts < 0) ts += plyn;
+              if (((w1 >> 56) & 1) && d == n.depth && ts > -INF && ts < INF && !repeated && sd < MAXPLY &&
+                  path_free(L, n, reach, sd)) {
+                // an upper bound at or below alpha: the node fails low; a
+                // lower bound raises alpha
+                const bool upper = (w1 >> 58) & 1;
+                if (upper ? ts <= n.alpha : ts > n.alpha) {
+                  lcount(cvec, C_TT_CUT, 1);
+                  n.reach = reach;
+                  if (!upper) n.alpha = ts;
+                  if (upper || n.alpha >= n.beta) {
+                    v = n.alpha;
+                    state = S_RETURN;
+                    continue;
+                  }
+                }
+              }
+            }
+          }
           u16 *const ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
           const u32 kil = killers[sd], cm = (u32)ctab[counter_index(lastmove)];
           const int total = gen_moves<false>(L, me, lane, n.p, ~n.p.cr & RANKS45, n.kic, n.hmc, n.mbeg,
@@ -1483,28 +1566,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             li = load_list(L, lane, n.mbeg);
           }
           // terminal / draw tests in the reference's order (src/zeta.cl:1554-1609)
-          bool draw = false;
-          if (total > 0 && sd > 1 && n.hmc >= 2) {
-            // repetition against plies plyn-2, plyn-4, .. >= plyn-hmc: the
-            // searched path, then the game history before the root
-            bool hit = false;
-            const int nn = plyn - 2 - 2 * lane;
-            if (nn >= plyn - (int)n.hmc) {
-              if (nn >= 0) {
-                const u32 *const w = L.ply[nn + 1].w;
-                hit = (((u64)w[W_HASH + 1] << 32) | w[W_HASH]) == n.hash;
-              } else if (a->hist) {
-                int hl = a->hlen[L.root];
-                hl = hl > ZETA_HISTORY ? ZETA_HISTORY : hl;
-                if (-nn - 1 < hl) hit = a->hist[(size_t)L.root * ZETA_HISTORY + (-nn - 1)] == n.hash;
-              }
-            }
-            draw = __ballot(hit) != 0;
-          }
-          if (sd > 1 && n.hmc >= 100) draw = true;
-          if (sd > 1 && popc(n.p.b1 | n.p.b2 | n.p.b3) <= 2) draw = true;
           state = S_NEXT;
-          if (draw) {
+          if (repeated && total > 0) {
             v = 0;
             state = S_RETURN;
           } else if (total == 0) {
@@ -1515,42 +1578,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             v = static_eval(n.p, lane);
             state = S_RETURN;
           } else {
-            // TT probe: move for ordering; score under the exact-depth rule
-            u32 ttmove = 0;
-            if (ttmask && sd > 1) {
-              const u64 w0 = uf(((u64)tte.y << 32) | tte.x), w1 = uf(((u64)tte.w << 32) | tte.z);
-              lcount(cvec, C_TT_PROBE, 1);
-              if ((w0 ^ w1) == key && ((w1 >> 57) & 1)) {
-                lcount(cvec, C_TT_HIT, 1);
-                ttmove = (u32)w1;
-                s32 ts = (s32)(int16_t)(u16)(w1 >> 32);
-                const int d = (int)((w1 >> 48) & 0xFF);
-                if (is_mate(ts) && ts > 0) ts -= plyn;
-                if (is_mate(ts) && ts < 0) ts += plyn;
-                if (((w1 >> 56) & 1) && n.hmc == 0 && d == n.depth && ts > -INF && ts < INF) {
-                  if ((w1 >> 58) & 1) {
-                    // upper bound at or below alpha: the node fails low
-                    if (ts <= n.alpha) {
-                      lcount(cvec, C_TT_CUT, 1);
-                      v = n.alpha;
-                      state = S_RETURN;
-                    }
-                  } else if (ts > n.alpha) {
-                    n.alpha = ts;
-                    lcount(cvec, C_TT_CUT, 1);
-                    if (n.alpha >= n.beta) {
-                      v = n.alpha;
-                      state = S_RETURN;
-                    }
-                  }
-                }
-              }
-            }
-            if (state == S_NEXT && ttmove) {
+            if (ttmove) {
               n.ttm = ttmove;
               first_move(L, lane, n, li, ttmove, TTMOVE_SCORE);
             }
-            if (state == S_NEXT && (cfg & CF_HINT)) {
+            if (cfg & CF_HINT) {
               // the hint table (a completed search's table): its move first
               const u32x4 he = *glob((const u32x4 *)(a->hint + 2 * (key & ttmask)));
               const u64 h0 = uf(((u64)he.y << 32) | he.x), h1 = uf(((u64)he.w << 32) | he.z);
@@ -1574,7 +1606,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               continue;
             }
             v = n.alpha;
-            lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), n, sd, lane));
+            lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
             state = S_RETURN;
             continue;
           }
@@ -1672,9 +1704,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         // ---------------- RETURN v from node sd
         if (n.busy) busy_release(a, n.hash, n.p.cr, lane);
         if (sd == 1) break;
+        // (quiescence nodes are not tested for repetition)
+        const u32 below = state == S_QS || n.hmc == 0 ? 0u : (n.reach < 3 ? n.reach + 1 : 3u);
         sd--;
         wsync();
         restore(L.ply[sd], n, lane);
+        n.reach = n.reach > below ? n.reach : below;
         const s32 sc = -v;
         if ((sd & 1) && sd >= 3 && ra - 1 > n.alpha && ra - 1 < n.beta) {
           // the root bound rose while this node's children were searched:
@@ -1709,7 +1744,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             ctab[counter_index(last)] = counter_code(n.move);
           }
           v = n.alpha;
-          lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), n, sd, lane));
+          lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
           state = S_RETURN;
         } else {
           li = load_list(L, lane, n.mbeg);
