@@ -53,3 +53,16 @@ def test_table_scores_hold_on_every_path(zeta, oracle, depth, with_history):
         got = zeta.search(pos, depth, workers=workers, tt_log2=tt, clear_tt=clear, history=hist)
         assert list(got["score"]) == want, (workers, tt, clear)
         assert (got["status"] == 0).all()
+
+
+@pytest.mark.parametrize("n,workers,depth", [(1, 1, 3), (40, 1, 2), (64, 2, 3), (200, 64, 2), (300, 8, 1)])
+def test_quiescence_table(zeta, oracle, n, workers, depth):
+    """From one worker (the smallest quiescence table) to a full grid (the
+    largest): captures in every order, e.p., checks, promotions, draws."""
+    pos = np.concatenate([oracle.setboard("8/2p5/3p4/KP5r/1R3p1k/8/4P1P1/8 w - - 98 60")] * (n > 1) +
+                         [oracle.gen_playouts(n + depth, n, 10, 80)])[:n]
+    want = [oracle.search(pos[i:i + 1], depth)[0] for i in range(n)]
+    for clear in (True, False):
+        got = zeta.search(pos, depth, workers=workers, tt_log2=18, clear_tt=clear)
+        assert list(got["score"]) == want
+        assert (got["status"] == 0).all()

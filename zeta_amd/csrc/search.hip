@@ -68,6 +68,22 @@ constexpr int ABDADA_MIN_DEPTH = 2;  // default split depth (zeta_search_opts.sp
 constexpr int POLL_EVERY = 64;
 
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));  // one 16-byte TT entry
+typedef u32 u32x2 __attribute__((ext_vector_type(2)));  // one 8-byte quiescence entry
+
+// The quiescence table.  A quiescence node's value is a function of its pieces
+// and side to move alone (captures only, no repetition, no castling), so the
+// captures of a position in another order, the other workers of a root and its
+// next iteration meet it again: three quarters of a search's time went into
+// quiescence trees, and trees of 10^5 nodes below one node kept a worker busy
+// after all others had ended.  An entry is 8 bytes, read and written whole: the
+// key's bits above QT_BITS (those below are in the index, of at least QT_BITS
+// bits, so that no two keys share an entry), the kind of bound, the value.
+// It starts empty in every call.  1024 positions, depth 4, 128 workers each:
+// 373 -> 151 ms (1057 -> 251 ms for a batch with one root of 89 M nodes); one
+// position, depth 5: 52 -> 45 ms.
+constexpr int QT_BITS = 18;
+enum { Q_LOWER = 1, Q_UPPER = 2, Q_EXACT = 3 };
+constexpr u64 QT_MIN = 1ULL << QT_BITS, QT_MAX = 1ULL << 22, QT_WORKER = 4096;  // entries: least, most, per worker
 
 // ---- serving (zeta_serve_*): the host publishes requests in coherent pinned
 // host memory; a persistent grid of workers claims them in ticket order,
@@ -117,6 +133,8 @@ struct SearchArgs {
   int split_depth;   // ABDADA deferral / busy marking at depth - 1 >= split_depth
   u64 *tt;           // 2 words per entry
   u64 ttmask;        // entries - 1 (0 = no TT)
+  u64 *qtt;          // quiescence table, see QEntry (used where there is a TT)
+  u64 qmask;         // its entries - 1
   const u64 *hint;   // read-only table in the TT's format whose moves go first (null = none)
   u64 *rbound;       // per root (slot): best root score so far, ticket << 32 | iteration << 16 | score + 32768
   u32 *busy;
@@ -843,7 +861,6 @@ __device__ __forceinline__ bool path_free(const Lds &L, const Node &n, u32 reach
 // distance-to-mate from this node.  Bit 56: the bound does not depend on the
 // path above the node; bits 59-60: the node's reach (path_free).
 __device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Lds &L, const Node &n, int sd, int lane) {
-  if (!ttmask) return 0;
   s32 s = n.alpha;
   const int plyn = sd - 1;
   if (is_mate(s) && s > 0) s += plyn;
@@ -1197,15 +1214,30 @@ __device__ __forceinline__ u64 all_moves(int n) { return n < 64 ? (1ULL << n) - 
 
 enum { QS_DONE = 0, QS_ABORTED, QS_FAILED };
 
+__device__ __forceinline__ void qt_store(const Pos &p, u64 phash, s32 v, u32 kind, int lane) {
+  if (lane != 0 || v != (s32)(int16_t)(u16)v) return;
+  const Args a = args();
+  const u64 key = phash ^ (u64)p.stm;
+  u32x2 e;
+  e.x = ((u32)(key >> QT_BITS) << QT_BITS) | (kind << 16) | ((u32)v & 0xFFFFu);
+  e.y = (u32)(key >> 32);
+  *glob((u32x2 *)(a->qtt + (key & a->qmask))) = e;
+}
+
 // A quiescence node and everything below it, which is quiescence too: captures
 // only, stand pat when not in check, no table, no hash, no extension, no
 // deferral.  Apart from the full-width loop it keeps a few scalars a ply: the
 // four planes, the window and the list.  ev / known: the evaluation, if the
 // parent has it; kic: in check; polled: the visit has been counted to the poll.
+template <bool TABLE>
 __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p, s32 alpha, s32 beta, u32 hmc,
-                                       const int sd0, int mbeg, s32 ev, bool known, bool kic, bool polled, Poll &q, s32 &ra,
-                                       u32 &cvec, s32 &vout) {
+                                       const int sd0, int mbeg, s32 ev, bool known, bool kic, bool polled, u64 phash,
+                                       Poll &q, s32 &ra, u32 &cvec, s32 &vout) {
   int sd = sd0, mcnt = 0, unused = 0;
+  // the node's value goes into the table; a move or the stand pat raised alpha;
+  // in this call a root bound has taken alpha's place (a value may then be a bound)
+  bool store = false, raised = false, clamped = false;
+  u32x2 qe = {0u, 0u};
   u64 ep = ~p.cr & RANKS45;  // captures leave none behind
   u64 left = 0;
   List li = {};
@@ -1216,7 +1248,11 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
     if (arrive) {
       if (!polled && ++q.count >= POLL_EVERY && poll_root(args(), L, lane, q, ra)) return QS_ABORTED;
       polled = false;
-      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) alpha = ra - 1;
+      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) {
+        alpha = ra - 1;
+        clamped = true;
+      }
+      store = raised = false;
       const bool draw = hmc >= 100 || popc(p.b1 | p.b2 | p.b3) <= 2;
       // stand pat before any move generation: the reference returns the static
       // evaluation both on a stand-pat cutoff and when no capture exists
@@ -1227,6 +1263,25 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
         leaf = draw || ev >= beta || sd >= MAXPLY;
         if (!draw && sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
         v = ev;
+      }
+      // (no deeper than 32 plies, the ply limit is out of reach below the node)
+      if (TABLE && !leaf && !ep && !draw && sd <= 32) {
+        const u64 key = phash ^ (u64)p.stm;
+        if (sd == sd0) qe = *glob((const u32x2 *)(args()->qtt + (key & args()->qmask)));
+        const u64 e = uf(((u64)qe.y << 32) | qe.x);
+        store = true;
+        if ((e >> QT_BITS) == (key >> QT_BITS)) {
+          const u32 kind = (u32)(e >> 16) & 3u;
+          const s32 ts = (s32)(int16_t)(u16)e;
+          leaf = kind == Q_EXACT || (kind == Q_LOWER && ts >= beta) || (kind == Q_UPPER && ts <= alpha);
+          if (leaf) {
+            v = ts;
+            store = false;
+          } else if (kind == Q_LOWER && ts > alpha) {
+            alpha = ts;
+            raised = true;
+          }
+        }
       }
       if (!leaf) {
         mcnt = gen_moves<true>(L, me, lane, p, ep, kic, 0, mbeg, true, 0, 0, li);
@@ -1242,8 +1297,10 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
           if (sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
           if (kic) v = static_eval(p, lane);
           leaf = true;
+          if (TABLE && store) qt_store(p, phash, v, Q_EXACT, lane);
         } else if (!kic && ev > alpha) {
           alpha = ev;
+          raised = true;
         }
       }
       ep = 0;
@@ -1256,8 +1313,18 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
         w = put32(w, 8, window(alpha, beta));
         w = put32(w, 9, (u32)mbeg | ((u32)mcnt << 16));
         w = put64(w, 10, left);
-        if (lane < 12) L.ply[sd].w[lane] = (u32)w;
+        if (TABLE) {
+          w = put64(w, 12, phash);
+          w = put32(w, 14, (store ? 1u : 0u) | (raised ? 2u : 0u));
+        }
+        if (lane < 15) L.ply[sd].w[lane] = (u32)w;
         q.nodes++;
+        if (TABLE) {
+          // the child's entry is on its way while the child is made
+          phash ^= piece_key(mv_pfrom(m), (int)mv_from(m)) ^ piece_key(mv_pto(m), (int)mv_to(m)) ^
+                   piece_key(mv_pcpt(m), (int)mv_cpt(m));
+          qe = *glob((const u32x2 *)(args()->qtt + ((phash ^ (u64)(p.stm ^ 1u)) & args()->qmask)));
+        }
         p = apply_capture(p, m);
         const s32 t = alpha;
         alpha = -beta;
@@ -1271,6 +1338,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
         continue;
       }
       v = alpha;
+      if (TABLE && store) qt_store(p, phash, v, raised ? (clamped ? Q_LOWER : Q_EXACT) : Q_UPPER, lane);
     }
     // return v to the parent, and on while the parents fail high
     do {
@@ -1280,8 +1348,13 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
       }
       sd--;
       wsync();
-      const int w = (int)L.ply[sd].w[lane < 12 ? lane : 0];
+      const int w = (int)L.ply[sd].w[lane < 15 ? lane : 0];
       get_planes(w, p);
+      if (TABLE) {
+        phash = get64(w, 12);
+        store = get32(w, 14) & 1u;
+        raised = get32(w, 14) & 2u;
+      }
       p.stm ^= 1u;
       const u32 win = get32(w, 8), list = get32(w, 9);
       left = get64(w, 10);
@@ -1290,9 +1363,17 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
       mbeg = (int)(list & 0xFFFFu);
       mcnt = (int)(list >> 16);
       v = -v;
-      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) alpha = ra - 1;
-      if (v > alpha) alpha = v;
+      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) {
+        alpha = ra - 1;
+        raised = false;
+        clamped = true;
+      }
+      if (v > alpha) {
+        alpha = v;
+        raised = true;
+      }
       v = alpha;
+      if (TABLE && store && alpha >= beta) qt_store(p, phash, v, Q_LOWER, lane);
     } while (alpha >= beta);
     li = load_list(L, lane, mbeg);
     arrive = false;
@@ -1320,6 +1401,10 @@ __device__ __forceinline__ u32 search_config(Args a) {
 }
 __device__ __forceinline__ u64 tt_mask(u32 cfg) { return (1ULL << (cfg >> 24)) - 1; }
 
+// TABLE: there is a transposition table, and with it a quiescence table.  The
+// search without them keeps no piece hash through quiescence and no reach: with
+// one kernel for both it took 4 % longer.
+template <bool TABLE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_search(SearchArgs) {
   __shared__ Lds L;
   u32 *const mmove = L.mmove, *const mkey = L.mkey, *const killers = L.killers;
@@ -1481,10 +1566,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             state = S_QS;
             continue;
           }
-          const u64 ttmask = tt_mask(cfg);
+          const u64 ttmask = TABLE ? tt_mask(cfg) : 0;
           const u64 key = tt_key(n.hash, n.p.cr);
           u32x4 tte = {0u, 0u, 0u, 0u};
-          if (ttmask && sd > 1) tte = *glob((const u32x4 *)(a->tt + 2 * (key & ttmask)));
+          if (TABLE && sd > 1) tte = *glob((const u32x4 *)(a->tt + 2 * (key & ttmask)));
           // draws that hold with and without moves
           if (sd > 1 && (n.hmc >= 100 || popc(n.p.b1 | n.p.b2 | n.p.b3) <= 2)) {
             v = 0;
@@ -1510,7 +1595,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // TT probe, before any move is generated (a stored node had moves):
           // move for ordering; score where no path to the node changes it
           u32 ttmove = 0;
-          if (ttmask && sd > 1) {
+          if (TABLE && sd > 1) {
             const u64 w0 = uf(((u64)tte.y << 32) | tte.x), w1 = uf(((u64)tte.w << 32) | tte.z);
             lcount(cvec, C_TT_PROBE, 1);
             if ((w0 ^ w1) == key && ((w1 >> 57) & 1)) {
@@ -1578,11 +1663,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             v = static_eval(n.p, lane);
             state = S_RETURN;
           } else {
-            if (ttmove) {
+            if (TABLE && ttmove) {
               n.ttm = ttmove;
               first_move(L, lane, n, li, ttmove, TTMOVE_SCORE);
             }
-            if (cfg & CF_HINT) {
+            if (TABLE && (cfg & CF_HINT)) {
               // the hint table (a completed search's table): its move first
               const u32x4 he = *glob((const u32x4 *)(a->hint + 2 * (key & ttmask)));
               const u64 h0 = uf(((u64)he.y << 32) | he.x), h1 = uf(((u64)he.w << 32) | he.z);
@@ -1606,12 +1691,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               continue;
             }
             v = n.alpha;
-            lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
+            if (TABLE) lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
             state = S_RETURN;
             continue;
           }
           const Pos c = apply(n.p, m, false);
-          if ((mk & 0xFFFFu) > KEY_OPEN) {
+          const bool quiet = (mk & 0xFFFFu) > KEY_OPEN;
+          u64 ch = 0, cph = 0;
+          if (TABLE || !quiet) child_hash(n, m, c, ch, cph);
+          if (quiet) {
             // a quiescence node, not in check, its evaluation known
             if (!n.pass2) n.searched++;
             poll.nodes++;
@@ -1627,13 +1715,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             n.kic = false;
             qev = (s32)(mk & 0xFFFFu) - 32768;
             qknown = true;
+            n.phash = cph;
             sd++;
             wsync();
             state = S_QS;
             continue;
           }
-          u64 ch, cph;
-          child_hash(n, m, c, ch, cph);
           // ABDADA: defer a sibling that another worker is already searching
           bool cbusy = false;
           if ((cfg & CF_ABDADA) && n.depth - 1 >= (s32)((cfg >> 8) & 0xFFu)) {
@@ -1692,7 +1779,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 
         if (state == S_QS) {
           // ---------------- a quiescence node and all below it
-          const int st = qsearch(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, !qknown, poll, ra,
+          const int st = qsearch<TABLE>(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, !qknown, n.phash,
+                                 poll, ra,
                                  cvec, v);
           if (st != QS_DONE) {
             aborted = st == QS_ABORTED;
@@ -1709,7 +1797,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         sd--;
         wsync();
         restore(L.ply[sd], n, lane);
-        n.reach = n.reach > below ? n.reach : below;
+        if (TABLE) n.reach = n.reach > below ? n.reach : below;
         const s32 sc = -v;
         if ((sd & 1) && sd >= 3 && ra - 1 > n.alpha && ra - 1 < n.beta) {
           // the root bound rose while this node's children were searched:
@@ -1744,7 +1832,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             ctab[counter_index(last)] = counter_code(n.move);
           }
           v = n.alpha;
-          lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
+          if (TABLE) lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
           state = S_RETURN;
         } else {
           li = load_list(L, lane, n.mbeg);
@@ -1880,11 +1968,25 @@ __global__ void k_clear_u64(u64 *p, size_t n) {
 
 struct SearchState {
   zr::DevBuf tt, busy, roots, queue, done, nworkers, score, bestmove, nodes, depth_done, err, ctr, hist, hlen, pv, hint,
-      rbound, ctab;
+      rbound, ctab, qtt;
   u64 tt_entries = 0;
   u64 last_ctr[C_NCTR] = {0};
 };
 SearchState g_ss;
+
+// the quiescence table of a call with `grid` workers, empty: 32 KB a worker,
+// between 2 MB (QT_BITS bits of index) and 32 MB
+int qt_clear(unsigned grid, hipStream_t st, SearchArgs &sa) {
+  u64 entries = QT_MIN;
+  while (entries < QT_MAX && entries < (u64)grid * QT_WORKER) entries *= 2;
+  const int r = zr::ensure(g_ss.qtt, entries * 8);
+  if (r) return r;
+  hipLaunchKernelGGL(k_clear_u64, dim3((unsigned)(entries / 1024)), dim3(256), 0, st, (u64 *)g_ss.qtt.p, (size_t)entries);
+  ZCHECK(hipGetLastError());
+  sa.qtt = (u64 *)g_ss.qtt.p;
+  sa.qmask = entries - 1;
+  return 0;
+}
 
 inline unsigned nblocks(size_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
@@ -1898,7 +2000,7 @@ void search_release() {
   zr::release(g_ss.done); zr::release(g_ss.nworkers); zr::release(g_ss.score); zr::release(g_ss.bestmove);
   zr::release(g_ss.nodes); zr::release(g_ss.depth_done); zr::release(g_ss.err);
   zr::release(g_ss.ctr); zr::release(g_ss.hist); zr::release(g_ss.hlen); zr::release(g_ss.pv);
-  zr::release(g_ss.hint); zr::release(g_ss.rbound); zr::release(g_ss.ctab);
+  zr::release(g_ss.hint); zr::release(g_ss.rbound); zr::release(g_ss.ctab); zr::release(g_ss.qtt);
   g_ss.tt_entries = 0;
 }
 
@@ -1953,7 +2055,7 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   ZCHECK(hipMemsetAsync(g_ss.busy.p, 0, (size_t)busy_entries * 4, st));
 
   int per_cu = 0;
-  ZCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_search, 64, 0));
+  ZCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, tt_entries ? k_search<true> : k_search<false>, 64, 0));
   if (opts->waves_per_simd > 0 && 4 * opts->waves_per_simd < per_cu) per_cu = 4 * opts->waves_per_simd;
   if (per_cu < 1) per_cu = 1;
   const u64 cap = (u64)per_cu * (u64)zr::ctx().cu_count;
@@ -1969,6 +2071,9 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   sa.split_depth = opts->split_depth > 0 ? opts->split_depth : ABDADA_MIN_DEPTH;
   sa.tt = (u64 *)g_ss.tt.p;
   sa.ttmask = tt_entries ? tt_entries - 1 : 0;
+  sa.qtt = nullptr;
+  sa.qmask = 0;
+  if (tt_entries && (r = qt_clear(grid, st, sa))) return r;
   sa.hint = opts->order_hint ? (const u64 *)g_ss.hint.p : nullptr;
   sa.rbound = (u64 *)g_ss.rbound.p;
   sa.busy = (u32 *)g_ss.busy.p;
@@ -2029,7 +2134,8 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
     sa.rec_count = cnt;
     sa.rec_cap = cap;
   }
-  ZLAUNCH(zr::K_SEARCH, (u64)n, k_search, grid, 64, 0, sa);
+  if (tt_entries) ZLAUNCH(zr::K_SEARCH, (u64)n, k_search<true>, grid, 64, 0, sa);
+  else ZLAUNCH(zr::K_SEARCH, (u64)n, k_search<false>, grid, 64, 0, sa);
 
   std::vector<s32> score(n), dd(n);
   std::vector<u32> bm(n), done(n);
@@ -2230,7 +2336,7 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   S.budget = o->mem_budget;
   S.use_mlp = w != nullptr;
   hipFuncAttributes fa;
-  ZCHECK(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(k_search)));
+  ZCHECK(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(k_search<true>)));
   S.worker_bytes = (u64)fa.sharedSizeBytes;
   const u64 tt_entries = tt_log2 > 0 ? (1ULL << tt_log2) : 0;
   S.tt_bytes = tt_entries * 16;
@@ -2302,7 +2408,8 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   const int wd_ms = o->watchdog_ms > 0 ? o->watchdog_ms : 10000;
 
   int per_cu = 0;
-  SV_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_search, 64, 0));
+  const auto kernel = tt_entries ? k_search<true> : k_search<false>;
+  SV_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0));
   if (per_cu < 1) per_cu = 1;
   const int cap = per_cu * zr::ctx().cu_count;
   int grid = o->grid > 0 && o->grid < cap ? o->grid : cap;
@@ -2321,6 +2428,10 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   sa.busy = (u32 *)S.busy.p;
   sa.busymask = busy_entries - 1;
   sa.ctab = (u16 *)S.ctab.p;
+  if (tt_entries && (r = qt_clear((unsigned)grid, st, sa))) {
+    sv_free_all();
+    return r;
+  }
   sa.nodes = (u64 *)S.nodes.p;
   sa.depth_done = (s32 *)S.depth_done.p;
   sa.err = (u32 *)S.err.p;
@@ -2349,7 +2460,7 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   S.slot_cost.assign(S.nslots, 0);
   S.on = true;
   zr::ctx().serving = true;
-  hipLaunchKernelGGL(k_search, dim3(grid), dim3(64), 0, st, sa);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, st, sa);
   SV_CHECK(hipGetLastError());
 #undef SV_CHECK
   return ZETA_OK;
