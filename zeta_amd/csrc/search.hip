@@ -64,7 +64,14 @@ constexpr s32 COUNTER_SCORE = 1300;
 constexpr int NCOUNTER = 64 * 64;
 constexpr u32 DEFERRED = 0x80000000u;  // move-stack flag: deferred by ABDADA (move codes use bits 0-29)
 constexpr u32 MOVE_BITS = 0x3FFFFFFFu;
-constexpr int ABDADA_MIN_DEPTH = 2;  // default split depth (zeta_search_opts.split_depth)
+// Default split depth (zeta_search_opts.split_depth), by workers per root: from
+// 16 on, workers meet at the nodes next to quiescence often enough that marking
+// those pays too (16 positions, depth 4: 229 ms with 1, 290 with 2 at 32
+// workers; one position, depth 5, 128 workers: 206, 229, and 278 with 3).  Up
+// to 8, single positions take 2-4 % longer with 1 (batches 10 % less), and a
+// root's nodes spread over its workers, so that per-worker node budgets end a
+// search later than they did.
+inline int default_split(int workers) { return workers >= 16 ? 1 : 2; }
 constexpr int POLL_EVERY = 64;
 
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));  // one 16-byte TT entry
@@ -254,6 +261,9 @@ struct Node {  // the current full-width node (wave-uniform)
   int ndefer, searched;
   bool busy;
   u32 reach;        // see path_free
+  bool scout;       // the move being searched has a window of one above `floor`
+  s32 floor;
+  u32 child;        // what its key says of the child
 };
 
 // child hash of the alpha-beta move-up (src/zeta.cl:2297-2359), incremental
@@ -287,6 +297,14 @@ __device__ __forceinline__ u32 child_hmc(u32 hmc, u32 m) {
 }
 
 enum { S_ENTER = 0, S_NEXT, S_RETURN, S_QS };
+
+// The value a move of the node has to exceed.  At the root that is the best of
+// all workers less one (ra - 1), not this worker's own: a worker that starts on
+// a root move with no score of its own would look at every reply to it (six
+// batches of 1024 positions, depth 4: 770 -> 698 ms).
+__device__ __forceinline__ s32 floor_of(const Node &n, int sd, s32 ra) {
+  return sd == 1 && ra - 1 > n.alpha ? ra - 1 : n.alpha;
+}
 
 // A counter move is a quiet move, which its from- and to-square and its
 // piece determine (sqcpt = to, no captured piece, pto = pfrom or the queen a
@@ -741,8 +759,8 @@ constexpr u64 OUTER_RANKS = 0xFF000000000000FFULL;
 // one word a lane in one LDS access (field by field, and with the parent's
 // board taken back from the child's by undoing the move, a visit spent 1100
 // instructions on it).
-constexpr int NWORDS = 23;
-enum { W_PLANES = 0, W_CR = 8, W_HASH = 10, W_PHASH = 12, W_LEFT = 14, W_WINDOW = 16, W_MOVE, W_BEST, W_LIST, W_COUNTS, W_FLAGS, W_TTM };
+constexpr int NWORDS = 24;
+enum { W_PLANES = 0, W_CR = 8, W_HASH = 10, W_PHASH = 12, W_LEFT = 14, W_WINDOW = 16, W_MOVE, W_BEST, W_LIST, W_COUNTS, W_FLAGS, W_TTM, W_FLOOR };
 struct Ply {
   u32 w[24];
 };
@@ -784,7 +802,7 @@ __device__ __forceinline__ void get_planes(int w, Pos &p) {
 }
 __device__ __forceinline__ u32 window(s32 alpha, s32 beta) { return ((u32)alpha & 0xFFFFu) | ((u32)beta << 16); }
 
-enum { F_STM = 1, F_CHECK = 2, F_PASS2 = 4, F_BUSY = 8, F_REACH = 16 };  // F_REACH: two bits
+enum { F_STM = 1, F_CHECK = 2, F_PASS2 = 4, F_BUSY = 8, F_REACH = 16, F_SCOUT = 64, F_CHILD = 1 << 16 };  // F_REACH: two bits, F_CHILD: 16
 
 __device__ __forceinline__ void save(Ply &y, const Node &n, int lane) {
   int w = put_planes(0, n.p);
@@ -798,8 +816,9 @@ __device__ __forceinline__ void save(Ply &y, const Node &n, int lane) {
   w = put32(w, W_LIST, (u32)n.mbeg | ((u32)n.mcnt << 16));
   w = put32(w, W_COUNTS, (u32)n.depth | (n.hmc << 8) | ((u32)n.searched << 16) | ((u32)n.ndefer << 24));
   w = put32(w, W_FLAGS, (n.p.stm ? F_STM : 0) | (n.kic ? F_CHECK : 0) | (n.pass2 ? F_PASS2 : 0) | (n.busy ? F_BUSY : 0) |
-                         n.reach * F_REACH);
+                         n.reach * F_REACH | (n.scout ? F_SCOUT : 0) | n.child * F_CHILD);
   w = put32(w, W_TTM, n.ttm);
+  w = put32(w, W_FLOOR, (u32)n.floor);
   if (lane < NWORDS) y.w[lane] = (u32)w;
 }
 __device__ __forceinline__ void restore(const Ply &y, Node &n, int lane) {
@@ -824,8 +843,11 @@ __device__ __forceinline__ void restore(const Ply &y, Node &n, int lane) {
   n.kic = (fl & F_CHECK) != 0;
   n.pass2 = (fl & F_PASS2) != 0;
   n.busy = (fl & F_BUSY) != 0;
-  n.reach = fl / F_REACH;
+  n.reach = (fl / F_REACH) & 3u;
+  n.scout = (fl & F_SCOUT) != 0;
+  n.child = fl / F_CHILD;
   n.ttm = get32(w, W_TTM);
+  n.floor = (s32)get32(w, W_FLOOR);
 }
 // the move that led to the node at ply sd, 0 at the root
 __device__ __forceinline__ u32 last_move(const Lds &L, int sd) { return sd > 1 ? uf(L.ply[sd - 1].w[W_MOVE]) : 0u; }
@@ -1535,6 +1557,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       s32 qev = 0;  // S_QS: the node's evaluation, if its parent knows it
       bool qknown = false;
       int state = S_ENTER;
+      bool again = false;  // S_NEXT: the move that a window of one was too small for
 
       for (;;) {
         const Args a = args();  // loads of arguments stay in this pass
@@ -1683,8 +1706,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         if (state == S_NEXT) {
           // ---------------- NEXT: pick the best remaining move
           u32 m, mk;
-          const int k = pick_move(L, lane, n.mbeg, n.mcnt, li, n.left, n.depth == 1 && sd + 1 < MAXPLY ? -n.alpha : 2 * INF,
-                                  n.ndefer > 0, n.pass2, poll, n.searched, m, mk);
+          int k = 0;
+          if (TABLE && again) {
+            m = n.move;
+            mk = n.child;
+          } else {
+            k = pick_move(L, lane, n.mbeg, n.mcnt, li, n.left, n.depth == 1 && sd + 1 < MAXPLY ? -n.alpha : 2 * INF,
+                          n.ndefer > 0, n.pass2, poll, n.searched, m, mk);
+          }
           if (k < 0) {
             if (!n.pass2 && n.ndefer > 0) {
               n.pass2 = true;
@@ -1697,17 +1726,27 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           }
           const Pos c = apply(n.p, m, false);
           const bool quiet = (mk & 0xFFFFu) > KEY_OPEN;
+          // Once a move has been searched, the others are expected to stay at
+          // or below the floor: a window of one shows it with fewer nodes, and
+          // a move that exceeds it is searched again with the node's window.
+          // Six batches of 1024 positions, depth 4: 1101 -> 698 ms.
+          const s32 lo = floor_of(n, sd, ra);
+          const bool repeat = TABLE && again;
+          again = false;
+          n.scout = TABLE && !repeat && n.searched > 0 && n.beta - lo > 1;
+          n.child = mk & 0xFFFFu;
+          n.floor = lo;
+          const s32 hi = n.scout ? lo + 1 : n.beta;
           u64 ch = 0, cph = 0;
           if (TABLE || !quiet) child_hash(n, m, c, ch, cph);
           if (quiet) {
             // a quiescence node, not in check, its evaluation known
-            if (!n.pass2) n.searched++;
+            if (!n.pass2 && !repeat) n.searched++;
             poll.nodes++;
             n.move = m;
             save(L.ply[sd], n, lane);
-            const s32 t = n.alpha;
-            n.alpha = -n.beta;
-            n.beta = -t;
+            n.alpha = -hi;
+            n.beta = -lo;
             n.hmc = child_hmc(n.hmc, m);
             n.mbeg += n.mcnt;
             n.p = c;
@@ -1740,7 +1779,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             // requests defer only later siblings (a depth 4-9 stream
             // completed 43 instead of 47 of 48 requests within 120 s with
             // the first-child deferral at every ply)
-            if (!n.pass2 && b && (n.searched > 0 || (!(cfg & CF_SERVING) && sd >= 3))) {
+            if (!n.pass2 && !repeat && b && (n.searched > 0 || (!(cfg & CF_SERVING) && sd >= 3))) {
               n.left |= 1ULL << (k & 63);
               if (lane == 0) {
                 mkey[n.mbeg + k] = mk;
@@ -1754,7 +1793,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             if (lane == 0) atomicAdd(bp, 1u);
             cbusy = true;
           }
-          if (!n.pass2) n.searched++;
+          if (!n.pass2 && !repeat) n.searched++;
           poll.nodes++;
           n.move = m;
           save(L.ply[sd], n, lane);
@@ -1763,9 +1802,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.p = c;
           n.hash = ch;
           n.phash = cph;
-          const s32 t = n.alpha;
-          n.alpha = -n.beta;
-          n.beta = -t;
+          n.alpha = -hi;
+          n.beta = -lo;
           n.depth--;
           n.mbeg += n.mcnt;
           n.busy = cbusy;
@@ -1805,6 +1843,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.alpha = ra - 1;
           n.best = 0;
         }
+        // (the floor it was searched with: the root's bound may have risen since)
+        if (TABLE && n.scout && sc > n.floor && sc < n.beta) {
+          again = true;
+          state = S_NEXT;
+          wsync();
+          continue;
+        }
         if (sc > n.alpha) {
           n.alpha = sc;
           n.best = n.move;
@@ -1816,7 +1861,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
                                            (u64)(u16)(sc + 32768)));
           }
         }
-        if (n.alpha >= n.beta) {
+        // (at the other side's plies: no better reply is needed to keep the root
+        // move at or below ra - 1)
+        if (n.alpha >= n.beta || (!(sd & 1) && ra > -INF && n.alpha >= 1 - ra)) {
           const u32 last = last_move(L, sd);
           u16 *const ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
           if ((cfg & CF_RECORDS) && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
@@ -2068,7 +2115,7 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   sa.nroots = n;
   sa.depth = opts->depth;
   sa.workers = workers;
-  sa.split_depth = opts->split_depth > 0 ? opts->split_depth : ABDADA_MIN_DEPTH;
+  sa.split_depth = opts->split_depth > 0 ? opts->split_depth : default_split(workers);
   sa.tt = (u64 *)g_ss.tt.p;
   sa.ttmask = tt_entries ? tt_entries - 1 : 0;
   sa.qtt = nullptr;
@@ -2422,7 +2469,7 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   SearchArgs sa;
   memset(&sa, 0, sizeof(sa));
   sa.workers = S.workers;
-  sa.split_depth = ABDADA_MIN_DEPTH;
+  sa.split_depth = default_split(S.workers);
   sa.tt = (u64 *)g_ss.tt.p;
   sa.ttmask = tt_entries ? tt_entries - 1 : 0;
   sa.busy = (u32 *)S.busy.p;
