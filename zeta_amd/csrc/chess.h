@@ -641,18 +641,22 @@ ZD LaneSq lane_sq(int sq) {
   return LaneSq{sq_lines(sq), knight_att(b), king_att(b), pawn_att(b, 0), pawn_att(b, 1)};
 }
 
-// Does the side `by` attack the king of the other side?  kb = the king's
-// bitboard (0 for no king: never), q = the lines of its square.
+// Does the side `by` attack the king of the other side?  q = the lines of its
+// square, knight and pawn = the squares from which those attack it (king false:
+// there is none).
 // One position per lane, the same king square in every lane: the checkers of
 // node_basics without the check mask.
-ZD bool king_attacked(const Pos &p, const SqLines &q, u64 kb, u32 by) {
+ZD bool king_attacked(const Pos &p, const SqLines &q, bool king, u64 knight, u64 pawn, u32 by) {
   const u64 occ = p.b1 | p.b2 | p.b3;
   const u64 them = by ? p.b0 : (p.b0 ^ occ);
   const u64 rq = p.b3 & (p.b1 ^ p.b2), bq = p.b3 & ~p.b1;
   u64 a = (rook_sq(q, occ) & rq) | (bishop_sq(q, occ) & bq);
-  a |= knight_att(kb) & ~p.b1 & p.b2 & ~p.b3;
-  a |= pawn_att(kb, by ^ 1u) & p.b1 & ~p.b2 & ~p.b3;
-  return kb && (a & them);
+  a |= knight & ~p.b1 & p.b2 & ~p.b3;
+  a |= pawn & p.b1 & ~p.b2 & ~p.b3;
+  return king && (a & them);
+}
+ZD bool king_attacked(const Pos &p, const SqLines &q, u64 kb, u32 by) {
+  return king_attacked(p, q, kb != 0, knight_att(kb), pawn_att(kb, by ^ 1u), by);
 }
 
 // is sq attacked by the opponent, the own king taken off the board?

@@ -849,6 +849,10 @@ __device__ __forceinline__ void restore(const Ply &y, Node &n, int lane) {
   n.ttm = get32(w, W_TTM);
   n.floor = (s32)get32(w, W_FLOOR);
 }
+// x of lane k (wave-uniform)
+__device__ __forceinline__ u64 lane64(u64 x, int k) {
+  return ((u64)(u32)__builtin_amdgcn_readlane((int)(x >> 32), k) << 32) | (u32)__builtin_amdgcn_readlane((int)x, k);
+}
 // the move that led to the node at ply sd, 0 at the root
 __device__ __forceinline__ u32 last_move(const Lds &L, int sd) { return sd > 1 ? uf(L.ply[sd - 1].w[W_MOVE]) : 0u; }
 
@@ -1102,6 +1106,9 @@ __device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, con
   const u32 type = pc >> 1;
   const bool mine = type != PNONE && (pc & 1u) == p.stm;
   const u64 patt = p.stm ? me.bpawn : me.wpawn;
+  // the pawn sums want no pawn on the outer ranks
+  const bool keyed = leafward && !(p.b1 & ~p.b2 & ~p.b3 & OUTER_RANKS);
+  const s32 psq = keyed ? eval_piece(L.tab, pc, lane) : 0;
   u64 t = sel(type == ROOK || type == QUEEN, rook_sq(me.q, occ)) | sel(type == BISHOP || type == QUEEN, bishop_sq(me.q, occ));
   t = type == KNIGHT ? me.knight : t;
   t = type == KING ? me.king : t;
@@ -1147,9 +1154,12 @@ __device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, con
       if (cand && ep_legal0(B, lane, to, sqep)) t |= bit(to);
     }
   }
-  int total;
-  const int off = wave_exscan_i(popc(t), lane, total);
+  // one scan for the slots (below 1024) and the piece-square sum
+  const s32 scan = zw::wave_scan_add(popc(t) + psq * 1024), last = (s32)__builtin_amdgcn_readlane(scan, 63);
+  const int total = last & 1023;
   if (total == 0) return 0;
+  const int off = (scan & 1023) - popc(t);
+  const s32 base = last >> 10;
   int from = 0, to = 0;  // of the lane's move
   const bool small = !QS && total <= 64;
   if (small) {
@@ -1177,10 +1187,13 @@ __device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, con
   }
   const SqLines kq = lds_lines(L, ksq);
   const bool test = kbb && (kic || __ballot(((((kq.rank | kq.file) & rq) | ((kq.diag | kq.anti) & bq)) & opp) != 0));
-  const SqLines oq = lds_lines(L, okb ? lsb(okb) : 0);
-  // the pawn sums want no pawn on the outer ranks
-  const bool keyed = leafward && !(p.b1 & ~p.b2 & ~p.b3 & OUTER_RANKS);
-  const s32 base = keyed ? wave_sum_i(eval_piece(L.tab, pc, lane)) : 0;
+  const int osq = okb ? lsb(okb) : 0;
+  const SqLines oq = lds_lines(L, osq);
+  // what attacks the kings' squares: the lanes of those squares hold it (made
+  // from the square it took 130 of a visit's 860 instructions, with the constants
+  // spilled; six batches of 1024 positions, depth 4: 635 -> 592 ms)
+  const u64 kknight = lane64(me.knight, ksq), kpawn = lane64(patt, ksq);
+  const u64 oknight = lane64(me.knight, osq), opawn = lane64(p.stm ? me.wpawn : me.bpawn, osq);
   int kept = 0;
   for (int c0 = 0; c0 < total; c0 += 64) {
     const bool act = c0 + lane < total;
@@ -1203,7 +1216,7 @@ __device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, con
     const u32 m = mv_make((u32)from, (u32)to, (u32)x, pf, pt, cap);
     const Pos c = QS ? apply_capture(p, m) : apply(p, m, false);
     bool legal = act;
-    if (test) legal = act && ((pf >> 1) == KING || isep || !king_attacked(c, kq, kbb, p.stm ^ 1u));
+    if (test) legal = act && ((pf >> 1) == KING || isep || !king_attacked(c, kq, true, kknight, kpawn, p.stm ^ 1u));
     u32 key = KEY_OPEN;
     if (keyed) {
       const u64 cocc = c.b1 | c.b2 | c.b3;
@@ -1215,7 +1228,7 @@ __device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, con
       if (!QS) known = known && !is_promo(m) && child_hmc(hmc, m) < 100;
       if (known) key = (u32)((p.stm ? e : -e) + 32768);
     }
-    if (king_attacked(c, oq, okb, p.stm)) key = KEY_CHECK;
+    if (king_attacked(c, oq, okb != 0, oknight, opawn, p.stm)) key = KEY_CHECK;
     const s32 sc = QS ? piece_value(cap >> 1) * 16 - piece_value(pt >> 1) : plain_score(L.tab, p.stm, m, killer, counter);
     const u64 lm = __ballot(legal);
     const int slot = mbeg + kept + popc(lm & ((1ULL << lane) - 1));
