@@ -75,6 +75,7 @@ inline int default_split(int workers) { return workers >= 16 ? 1 : 2; }
 constexpr int POLL_EVERY = 64;
 
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));  // one 16-byte TT entry
+typedef u32 u32x2 __attribute__((ext_vector_type(2)));  // one 8-byte quiescence entry
 
 // The quiescence table.  A quiescence node's value is a function of its pieces
 // and side to move alone (captures only, no repetition, no castling), so the
@@ -212,13 +213,22 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // chiplets shared next to nothing. (One position, depth 5: four workers made 3.7
 // times the nodes of one and were 5 % faster, now 1.6 times and 2.3 times as
 // fast; six positions with 128 workers 182 -> 113 ms.)
-__device__ __forceinline__ u32x4 tt_load(const u64 *p) {
-  const u64 a = __hip_atomic_load(glob(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const u64 b = __hip_atomic_load(glob(p) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return u32x4{(u32)a, (u32)(a >> 32), (u32)b, (u32)(b >> 32)};
+// A search with a node budget per worker shares less: plain accesses, no
+// quiescence table, no entries by path, full windows.  Its workers make about
+// the nodes they made before all that, so that the same budgets stop the same
+// searches (with it, a root of 30000 nodes over 8 workers ends within 2000 each).
+enum { T_NONE = 0, T_SHARED, T_BUDGET };  // a search's tables
+__device__ __forceinline__ u64 shared_load(const u64 *p) {
+  return __hip_atomic_load(glob(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void shared_store(u64 *p, u64 v) {
   __hip_atomic_store(glob(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int TABLE>
+__device__ __forceinline__ u32x4 tt_load(const u64 *p) {
+  if (TABLE == T_BUDGET) return *glob((const u32x4 *)p);
+  const u64 a = shared_load(p), b = shared_load(p + 1);
+  return u32x4{(u32)a, (u32)(a >> 32), (u32)b, (u32)(b >> 32)};
 }
 
 enum { C_TT_PROBE = 0, C_TT_HIT, C_TT_CUT, C_TT_STORE, C_DEFER, C_MAXPLY, C_MLP_NODES, C_RECORDS, C_NODES, C_NCTR = 16 };
@@ -308,6 +318,10 @@ __device__ __forceinline__ u32 child_hmc(u32 hmc, u32 m) {
   if (((pf >> 1) & 7) == KING && (f - t == 2 || t - f == 2)) return 0;
   return (hmc + 1) & 0xFF;
 }
+
+// least depth of nodes that are looked up under their path too (below, most
+// bounds hold on any path)
+constexpr int PATH_DEPTH = 2;
 
 enum { S_ENTER = 0, S_NEXT, S_RETURN, S_QS };
 
@@ -794,6 +808,7 @@ struct Lds {  // one worker's memory: eight workers a CU
   u64 ticket;
   int root, depth, iteration;
   int hlen;  // positions of the game before the root
+  u64 hsalt;  // of their hashes, see path_key
   s32 best_score, final_score;
   u32 best_move, final_move;
 };
@@ -894,28 +909,73 @@ __device__ __forceinline__ bool path_free(const Lds &L, const Node &n, u32 reach
   return mv_from(m) != mv_to(o) || mv_to(m) != mv_from(o);
 }
 
+// The positions above the node at ply sd that a search below it can repeat, as
+// one word: those of the path since the last irreversible move, the game's if
+// that lies before the root, and the half-move clock.  A bound that holds on
+// this path only is stored under the position's key and this one.  The workers
+// of a root share its nodes high in the tree through it, whose bounds depend on
+// the path (six positions, depth 5, 128 workers: 113 -> 107 ms).
+__device__ __forceinline__ u64 hash_mix(u64 x) {
+  x ^= x >> 32;
+  x *= 0x9E3779B97F4A7C15ULL;
+  return x ^ (x >> 29);
+}
+__device__ __forceinline__ u32 wave_xor(u32 x) {
+  x ^= (u32)zw::dpp0<0x111, 0xF>((int)x);
+  x ^= (u32)zw::dpp0<0x112, 0xF>((int)x);
+  x ^= (u32)zw::dpp0<0x114, 0xF>((int)x);
+  x ^= (u32)zw::dpp0<0x118, 0xF>((int)x);
+  x ^= (u32)zw::dpp0<0x142, 0xA>((int)x);
+  x ^= (u32)zw::dpp0<0x143, 0xC>((int)x);
+  return (u32)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ __forceinline__ u64 wave_xor(u64 x) { return ((u64)wave_xor((u32)(x >> 32)) << 32) | wave_xor((u32)x); }
+__device__ __forceinline__ u64 path_key(const Lds &L, const Node &n, int sd, int lane) {
+  u64 v = 0;
+  const int k = sd - 1 - lane;  // the node's ancestors are at plies 1 .. sd - 1
+  if (k >= 1 && lane < (int)n.hmc) {
+    const u32 *const w = L.ply[k].w;
+    v = hash_mix(((u64)w[W_HASH + 1] << 32) | w[W_HASH]);
+  }
+  u64 x = wave_xor(v) + (u64)(n.hmc + 1) * 0xD1B54A32D192ED03ULL;
+  if ((int)n.hmc >= sd) x += uf(L.hsalt);
+  return hash_mix(x);
+}
+template <int TABLE>
+__device__ __forceinline__ void tt_write(Args a, u64 ttmask, u64 key, u64 w1, int lane) {
+  if (lane == 0) {
+    const u64 w0 = key ^ w1;
+    u64 *const e = a->tt + 2 * (key & ttmask);
+    if (TABLE == T_BUDGET) {
+      *glob((u32x4 *)e) = u32x4{(u32)w0, (u32)(w0 >> 32), (u32)w1, (u32)(w1 >> 32)};
+    } else {
+      shared_store(e, w0);
+      shared_store(e + 1, w1);
+    }
+  }
+}
+
 // TT store when a full-width node returns: with a move that raised alpha, a
 // lower bound of the node's value and that move; with none (every move
 // failed low), an upper bound (bit 58) and the move that the table had before,
 // which the next iteration would otherwise lose (six batches of 1024 positions,
 // depth 4: 714 -> 645 ms).  The score is kept as
 // distance-to-mate from this node.  Bit 56: the bound does not depend on the
-// path above the node; bits 59-60: the node's reach (path_free).
+// path above the node, or the entry is under this path's key; bits 59-60: the
+// node's reach (path_free).
+template <int TABLE>
 __device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Lds &L, const Node &n, int sd, int lane) {
   s32 s = n.alpha;
   const int plyn = sd - 1;
   if (is_mate(s) && s > 0) s += plyn;
   if (is_mate(s) && s < 0) s -= plyn;
   const u64 key = tt_key(n.hash, n.p.cr);
+  const bool any = path_free(L, n, n.reach, sd);
   const u64 w1 = (u64)(n.best ? n.best : n.ttm) | ((u64)(u16)(int16_t)s << 32) | ((u64)(n.depth & 0xFF) << 48) |
-                 ((u64)(path_free(L, n, n.reach, sd) ? 1 : 0) << 56) | (1ULL << 57) | ((u64)(n.best ? 0 : 1) << 58) |
-                 ((u64)n.reach << 59);
-  if (lane == 0) {
-    const u64 w0 = key ^ w1;
-    u64 *const e = a->tt + 2 * (key & ttmask);
-    shared_store(e, w0);
-    shared_store(e + 1, w1);
-  }
+                 (1ULL << 57) | ((u64)(n.best ? 0 : 1) << 58) | ((u64)n.reach << 59);
+  tt_write<TABLE>(a, ttmask, key, w1 | ((u64)(any ? 1 : 0) << 56), lane);
+  if (TABLE == T_SHARED && !any && n.depth >= PATH_DEPTH)
+    tt_write<TABLE>(a, ttmask, key ^ path_key(L, n, sd, lane), w1 | (1ULL << 56), lane);
   return 1;
 }
 
@@ -1311,7 +1371,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
       // (no deeper than 32 plies, the ply limit is out of reach below the node)
       if (TABLE && !leaf && !ep && !draw && sd <= 32) {
         const u64 key = phash ^ (u64)p.stm;
-        if (sd == sd0) qe = __hip_atomic_load(glob(args()->qtt) + (key & args()->qmask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (sd == sd0) qe = shared_load(args()->qtt + (key & args()->qmask));
         const u64 e = uf(qe);
         store = true;
         if ((e >> QT_BITS) == (key >> QT_BITS)) {
@@ -1367,8 +1427,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
           // the child's entry is on its way while the child is made
           phash ^= piece_key(mv_pfrom(m), (int)mv_from(m)) ^ piece_key(mv_pto(m), (int)mv_to(m)) ^
                    piece_key(mv_pcpt(m), (int)mv_cpt(m));
-          qe = __hip_atomic_load(glob(args()->qtt) + ((phash ^ (u64)(p.stm ^ 1u)) & args()->qmask), __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
+          qe = shared_load(args()->qtt + ((phash ^ (u64)(p.stm ^ 1u)) & args()->qmask));
         }
         p = apply_capture(p, m);
         const s32 t = alpha;
@@ -1446,10 +1505,11 @@ __device__ __forceinline__ u32 search_config(Args a) {
 }
 __device__ __forceinline__ u64 tt_mask(u32 cfg) { return (1ULL << (cfg >> 24)) - 1; }
 
-// TABLE: there is a transposition table, and with it a quiescence table.  The
-// search without them keeps no piece hash through quiescence and no reach: with
-// one kernel for both it took 4 % longer.
-template <bool TABLE>
+// TABLE: none, shared (a transposition table, and with it a quiescence table and
+// windows of one) or that of a search with a node budget.  The search without
+// tables keeps no piece hash through quiescence and no reach: with one kernel
+// for all it took 4 % longer.
+template <int TABLE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_search(SearchArgs) {
   __shared__ Lds L;
   u32 *const mmove = L.mmove, *const mkey = L.mkey, *const killers = L.killers;
@@ -1503,6 +1563,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       L.final_move = 0;
       const s32 hl = a->hist ? a->hlen[r] : 0;
       L.hlen = hl > ZETA_HISTORY ? ZETA_HISTORY : (hl < 0 ? 0 : hl);
+    }
+    if (TABLE == T_SHARED) {
+      u64 h = 0;
+      wsync();
+      for (int k = lane; k < L.hlen; k += 64) h ^= hash_mix(a->hist[(size_t)r * ZETA_HISTORY + k]);
+      h = wave_xor(h);
+      if (lane == 0) L.hsalt = h;
     }
     wsync();
 
@@ -1615,7 +1682,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           const u64 ttmask = TABLE ? tt_mask(cfg) : 0;
           const u64 key = tt_key(n.hash, n.p.cr);
           u32x4 tte = {0u, 0u, 0u, 0u};
-          if (TABLE && sd > 1) tte = tt_load(a->tt + 2 * (key & ttmask));
+          if (TABLE && sd > 1) tte = tt_load<TABLE>(a->tt + 2 * (key & ttmask));
+          const bool by_path = TABLE == T_SHARED && sd > 1 && n.depth >= PATH_DEPTH && n.hmc != 0;
+          u64 key2 = 0;
+          u32x4 tte2 = {0u, 0u, 0u, 0u};
+          if (by_path) {
+            key2 = key ^ path_key(L, n, sd, lane);
+            tte2 = tt_load<TABLE>(a->tt + 2 * (key2 & ttmask));
+          }
           // draws that hold with and without moves
           if (sd > 1 && (n.hmc >= 100 || popc(n.p.b1 | n.p.b2 | n.p.b3) <= 2)) {
             v = 0;
@@ -1642,32 +1716,37 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // move for ordering; score where no path to the node changes it
           u32 ttmove = 0;
           if (TABLE && sd > 1) {
-            const u64 w0 = uf(((u64)tte.y << 32) | tte.x), w1 = uf(((u64)tte.w << 32) | tte.z);
             lcount(cvec, C_TT_PROBE, 1);
-            if ((w0 ^ w1) == key && ((w1 >> 57) & 1)) {
-              lcount(cvec, C_TT_HIT, 1);
-              ttmove = (u32)w1;
+            bool cut = false;
+            auto use = [&](const u32x4 &t, u64 k, bool path) {
+              const u64 w0 = uf(((u64)t.y << 32) | t.x), w1 = uf(((u64)t.w << 32) | t.z);
+              if ((w0 ^ w1) != k || !((w1 >> 57) & 1)) return;
+              if (!path) lcount(cvec, C_TT_HIT, 1);
+              if (!ttmove) ttmove = (u32)w1;
               s32 ts = (s32)(int16_t)(u16)(w1 >> 32);
               const int d = (int)((w1 >> 48) & 0xFF);
               const u32 reach = (u32)(w1 >> 59) & 3u;
               if (is_mate(ts) && ts > 0) ts -= plyn;
               if (is_mate(ts) && ts < 0) ts += plyn;
               if (((w1 >> 56) & 1) && d == n.depth && ts > -INF && ts < INF && !repeated && sd < MAXPLY &&
-                  path_free(L, n, reach, sd)) {
+                  (path || path_free(L, n, reach, sd))) {
                 // an upper bound at or below alpha: the node fails low; a
                 // lower bound raises alpha
                 const bool upper = (w1 >> 58) & 1;
                 if (upper ? ts <= n.alpha : ts > n.alpha) {
                   lcount(cvec, C_TT_CUT, 1);
-                  n.reach = reach;
+                  n.reach = n.reach > reach ? n.reach : reach;
                   if (!upper) n.alpha = ts;
-                  if (upper || n.alpha >= n.beta) {
-                    v = n.alpha;
-                    state = S_RETURN;
-                    continue;
-                  }
+                  cut = upper || n.alpha >= n.beta;
                 }
               }
+            };
+            use(tte, key, false);
+            if (by_path && !cut) use(tte2, key2, true);
+            if (cut) {
+              v = n.alpha;
+              state = S_RETURN;
+              continue;
             }
           }
           u16 *const ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
@@ -1730,7 +1809,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // ---------------- NEXT: pick the best remaining move
           u32 m, mk;
           int k = 0;
-          if (TABLE && again) {
+          if (TABLE == T_SHARED && again) {
             m = n.move;
             mk = n.child;
           } else {
@@ -1743,7 +1822,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               continue;
             }
             v = n.alpha;
-            if (TABLE) lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
+            if (TABLE) lcount(cvec, C_TT_STORE, tt_store<TABLE>(a, tt_mask(cfg), L, n, sd, lane));
             state = S_RETURN;
             continue;
           }
@@ -1754,14 +1833,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // a move that exceeds it is searched again with the node's window.
           // Six batches of 1024 positions, depth 4: 1101 -> 698 ms.
           const s32 lo = floor_of(n, sd, ra);
-          const bool repeat = TABLE && again;
+          const bool repeat = TABLE == T_SHARED && again;
           again = false;
-          n.scout = TABLE && !repeat && n.searched > 0 && n.beta - lo > 1;
+          n.scout = TABLE == T_SHARED && !repeat && n.searched > 0 && n.beta - lo > 1;
           n.child = mk & 0xFFFFu;
           n.floor = lo;
           const s32 hi = n.scout ? lo + 1 : n.beta;
           u64 ch = 0, cph = 0;
-          if (TABLE || !quiet) child_hash(n, m, c, ch, cph);
+          if (TABLE == T_SHARED || !quiet) child_hash(n, m, c, ch, cph);
           if (quiet) {
             // a quiescence node, not in check, its evaluation known
             if (!n.pass2 && !repeat) n.searched++;
@@ -1787,8 +1866,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           bool cbusy = false;
           if ((cfg & CF_ABDADA) && n.depth - 1 >= (s32)((cfg >> 8) & 0xFFu)) {
             u32 *const bp = glob(a->busy) + ((u32)(tt_key(ch, c.cr) >> 40) & a->busymask);
+            // test and mark in one: workers that start on a root together walk
+            // in step, and with a load ahead of the mark they all find the child
+            // free (16 workers on a position, depth 5: 184 -> 159 ms)
             u32 b = 0;
-            if (lane == 0) b = __atomic_load_n(bp, __ATOMIC_RELAXED);
+            if (lane == 0) b = atomicAdd(bp, 1u);
             b = uf(b);
             // batch searches defer a busy first child too, from ply 3 down:
             // a worker that finds it busy moves on to the siblings and comes
@@ -1805,6 +1887,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             if (!n.pass2 && !repeat && b && (n.searched > 0 || (!(cfg & CF_SERVING) && sd >= 3))) {
               n.left |= 1ULL << (k & 63);
               if (lane == 0) {
+                atomicSub(bp, 1u);
                 mkey[n.mbeg + k] = mk;
                 mmove[n.mbeg + k] = m | DEFERRED;
               }
@@ -1813,7 +1896,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               wsync();
               continue;
             }
-            if (lane == 0) atomicAdd(bp, 1u);
             cbusy = true;
           }
           if (!n.pass2 && !repeat) n.searched++;
@@ -1840,7 +1922,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 
         if (state == S_QS) {
           // ---------------- a quiescence node and all below it
-          const int st = qsearch<TABLE>(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, !qknown, n.phash,
+          const int st = qsearch<TABLE == T_SHARED>(L, me, lane, n.p, n.alpha, n.beta, n.hmc, sd, n.mbeg, qev, qknown, n.kic, !qknown, n.phash,
                                  poll, ra,
                                  cvec, v);
           if (st != QS_DONE) {
@@ -1867,7 +1949,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           n.best = 0;
         }
         // (the floor it was searched with: the root's bound may have risen since)
-        if (TABLE && n.scout && sc > n.floor && sc < n.beta) {
+        if (TABLE == T_SHARED && n.scout && sc > n.floor && sc < n.beta) {
           again = true;
           state = S_NEXT;
           wsync();
@@ -1902,7 +1984,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             ctab[counter_index(last)] = counter_code(n.move);
           }
           v = n.alpha;
-          if (TABLE) lcount(cvec, C_TT_STORE, tt_store(a, tt_mask(cfg), L, n, sd, lane));
+          if (TABLE) lcount(cvec, C_TT_STORE, tt_store<TABLE>(a, tt_mask(cfg), L, n, sd, lane));
           state = S_RETURN;
         } else {
           li = load_list(L, lane, n.mbeg);
@@ -2124,8 +2206,10 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   ZCHECK(hipMemsetAsync(g_ss.ctr.p, 0, C_NCTR * 8, st));
   ZCHECK(hipMemsetAsync(g_ss.busy.p, 0, (size_t)busy_entries * 4, st));
 
+  const int table = !tt_entries ? T_NONE : (opts->max_nodes ? T_BUDGET : T_SHARED);
+  const auto kernel = table == T_NONE ? k_search<T_NONE> : (table == T_BUDGET ? k_search<T_BUDGET> : k_search<T_SHARED>);
   int per_cu = 0;
-  ZCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, tt_entries ? k_search<true> : k_search<false>, 64, 0));
+  ZCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0));
   if (opts->waves_per_simd > 0 && 4 * opts->waves_per_simd < per_cu) per_cu = 4 * opts->waves_per_simd;
   if (per_cu < 1) per_cu = 1;
   const u64 cap = (u64)per_cu * (u64)zr::ctx().cu_count;
@@ -2143,7 +2227,7 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
   sa.ttmask = tt_entries ? tt_entries - 1 : 0;
   sa.qtt = nullptr;
   sa.qmask = 0;
-  if (tt_entries && (r = qt_clear(grid, st, sa))) return r;
+  if (table == T_SHARED && (r = qt_clear(grid, st, sa))) return r;
   sa.hint = opts->order_hint ? (const u64 *)g_ss.hint.p : nullptr;
   sa.rbound = (u64 *)g_ss.rbound.p;
   sa.busy = (u32 *)g_ss.busy.p;
@@ -2204,8 +2288,7 @@ extern "C" int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_o
     sa.rec_count = cnt;
     sa.rec_cap = cap;
   }
-  if (tt_entries) ZLAUNCH(zr::K_SEARCH, (u64)n, k_search<true>, grid, 64, 0, sa);
-  else ZLAUNCH(zr::K_SEARCH, (u64)n, k_search<false>, grid, 64, 0, sa);
+  ZLAUNCH(zr::K_SEARCH, (u64)n, kernel, grid, 64, 0, sa);
 
   std::vector<s32> score(n), dd(n);
   std::vector<u32> bm(n), done(n);
@@ -2406,7 +2489,7 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   S.budget = o->mem_budget;
   S.use_mlp = w != nullptr;
   hipFuncAttributes fa;
-  ZCHECK(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(k_search<true>)));
+  ZCHECK(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(k_search<T_SHARED>)));
   S.worker_bytes = (u64)fa.sharedSizeBytes;
   const u64 tt_entries = tt_log2 > 0 ? (1ULL << tt_log2) : 0;
   S.tt_bytes = tt_entries * 16;
@@ -2478,7 +2561,7 @@ extern "C" int zeta_serve_start(const zeta_serve_opts *o) {
   const int wd_ms = o->watchdog_ms > 0 ? o->watchdog_ms : 10000;
 
   int per_cu = 0;
-  const auto kernel = tt_entries ? k_search<true> : k_search<false>;
+  const auto kernel = tt_entries ? k_search<T_SHARED> : k_search<T_NONE>;
   SV_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0));
   if (per_cu < 1) per_cu = 1;
   const int cap = per_cu * zr::ctx().cu_count;
