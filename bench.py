@@ -24,25 +24,26 @@ VALU_PEAK = 256 * 4 * 16 * 2.4e9  # VALU lane-instructions/s: 256 CU x 4 SIMD x 
 HBM_PEAK = 8.0e12
 
 
-# Work of one k_leaf position (apply the parent's move, analyse, count the
+# Work of one leaf position (apply the parent's move, analyse, count the
 # legal moves), measured once with rocprofv3 --pmc on this workload and kept
 # as constants (profiles/perft_c2_pmc.md):
-#   SQ_INSTS_VALU = 1,993,137,114 wave instructions per launch of 128,916,248
-#   positions (one position per lane) -> 989.5 VALU lane-instructions per
-#   position; each wave64 instruction occupies a 16-lane SIMD for 4 cycles,
-#   so the issue peak is 256 CU x 4 SIMD x 16 lanes x 2.4 GHz = 39.3 T/s.
-#   FETCH_SIZE 777,423.5 KiB x 1.99991 + WRITE_SIZE 63,073.4 KiB x 0.99999
-#   per launch, the factors from the library's copy kernel over 1 GiB
-#   (FETCH_SIZE 524,311.3 KiB, WRITE_SIZE 1,048,586.0 KiB) -> 12.85 B of HBM
-#   traffic per position.
-VALU_LANE_INSTS_PER_POSITION = 989.5
-HBM_BYTES_PER_POSITION = 12.85
+#   SQ_INSTS_VALU = 1,742,005,837 wave instructions in the two k_leaves launches
+#   of a step, 128,916,248 positions (one position per lane) -> 864.8 VALU
+#   lane-instructions per position; each wave64 instruction occupies a 16-lane
+#   SIMD for 4 cycles, so the issue peak is 256 CU x 4 SIMD x 16 lanes x
+#   2.4 GHz = 39.3 T/s.
+#   FETCH_SIZE 612,571.4 KiB x 1.99991 + WRITE_SIZE 8,984.5 KiB x 0.99999 per
+#   step, the factors from the library's copy kernel over 1 GiB (FETCH_SIZE
+#   524,311.3 KiB, WRITE_SIZE 1,048,586.0 KiB) -> 9.80 B of HBM traffic per
+#   position.
+VALU_LANE_INSTS_PER_POSITION = 864.8
+HBM_BYTES_PER_POSITION = 9.80
 # k_search: one node per wavefront; SQ_INSTS_VALU and SQ_INSTS_SALU / nodes
 # over the depth-6 search leg (profiles/search_c3_pmc.md).  A CU's arbiter
 # issues at most one scalar instruction per cycle (each SIMD's waves get one
 # SALU slot every 4 cycles), so the SALU issue peak is 256 CU x 2.4 GHz.
-VALU_WAVE_INSTS_PER_NODE = 459.8
-SALU_INSTS_PER_NODE = 870.1
+VALU_WAVE_INSTS_PER_NODE = 312.8
+SALU_INSTS_PER_NODE = 280.6
 SALU_PEAK = 256 * 2.4e9
 # the ordering network: 908 -> 256 -> 32 -> 1, dense FLOP of one scored move
 # (2 x (908 x 256 + 256 x 32 + 32)); a training pair scores two moves and its
