@@ -1877,13 +1877,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
             // back to it in the second pass, which keeps helpers off the
             // path every worker starts on.  At the root and ply 2 the first
             // child is searched by every worker that reaches it: a sibling
-            // searched before the first child has set the root's bound runs
-            // with the full window (with 128 workers per root the depth-7
-            // 1024-root batch took 44-45 s this way against 64-67 s with
-            // the deferral at every ply, and 51 s from ply 4 down).  Served
-            // requests defer only later siblings (a depth 4-9 stream
-            // completed 43 instead of 47 of 48 requests within 120 s with
-            // the first-child deferral at every ply)
+            // searched before the first child has set the root's bound has
+            // no bound to fail against (six positions, depth 5, 128 workers:
+            // 107 ms this way, 130 with the deferral from ply 2, 103 from
+            // ply 4; six batches of 250 with the network 270, 304, 267).
+            // Served requests defer only later siblings
             if (!n.pass2 && !repeat && b && (n.searched > 0 || (!(cfg & CF_SERVING) && sd >= 3))) {
               n.left |= 1ULL << (k & 63);
               if (lane == 0) {
