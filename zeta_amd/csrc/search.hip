@@ -31,6 +31,7 @@
 // probing path can repeat a position above the node (path_free).
 #include <string.h>
 
+#include "bounds.h"
 #include "chess.h"
 #include "evaltab.h"
 #include "mlp.h"
@@ -962,9 +963,11 @@ __device__ __forceinline__ void tt_write(Args a, u64 ttmask, u64 key, u64 w1, in
 // depth 4: 714 -> 645 ms).  The score is kept as
 // distance-to-mate from this node.  Bit 56: the bound does not depend on the
 // path above the node, or the entry is under this path's key; bits 59-60: the
-// node's reach (path_free).
+// node's reach (path_free).  Nothing is stored where the root's bound may have
+// made the value (bound_holds).  Returns how many values were.
 template <int TABLE>
-__device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Lds &L, const Node &n, int sd, int lane) {
+__device__ __forceinline__ u32 tt_store(Args a, u64 ttmask, const Lds &L, const Node &n, int sd, s32 ra, int lane) {
+  if (!bound_holds(sd, ra, n.best != 0, n.alpha)) return 0;
   s32 s = n.alpha;
   const int plyn = sd - 1;
   if (is_mate(s) && s > 0) s += plyn;
@@ -1041,9 +1044,10 @@ __device__ __forceinline__ bool poll_root(Args a, const Lds &L, int lane, Poll &
     }
   }
   if (uf((u32)d)) return true;
+  // (the word may be older than the bound that the iteration started with)
   const u64 rb = uf(q.rbound);
-  if ((rb >> 32) == (uf(L.ticket) & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == uf(L.iteration))
-    ra = (s32)(rb & 0xFFFF) - 32768;
+  const s32 b = (s32)(rb & 0xFFFF) - 32768;
+  if ((rb >> 32) == (uf(L.ticket) & 0xFFFFFFFFULL) && (int)((rb >> 16) & 0xFFFF) == uf(L.iteration) && b > ra) ra = b;
   poll_load(a, r, lane, q);
   return false;
 }
@@ -1352,7 +1356,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
     if (arrive) {
       if (!polled && ++q.count >= POLL_EVERY && poll_root(args(), L, lane, q, ra)) return QS_ABORTED;
       polled = false;
-      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) {
+      if (floor_lifts(sd, ra, alpha, beta)) {
         alpha = ra - 1;
         clamped = true;
       }
@@ -1467,7 +1471,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
       mbeg = (int)(list & 0xFFFFu);
       mcnt = (int)(list >> 16);
       v = -v;
-      if ((sd & 1) && sd >= 3 && ra - 1 > alpha && ra - 1 < beta) {
+      if (floor_lifts(sd, ra, alpha, beta)) {
         alpha = ra - 1;
         raised = false;
         clamped = true;
@@ -1665,7 +1669,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           // move the best, so the window starts there.  A root move then
           // reports max(its value, a bound below ra) -- below the best root
           // score, which stays exact, as does its move.
-          if ((sd & 1) && sd >= 3 && ra - 1 > n.alpha && ra - 1 < n.beta) n.alpha = ra - 1;
+          if (floor_lifts(sd, ra, n.alpha, n.beta)) n.alpha = ra - 1;
           n.best = 0;
           n.pass2 = false;
           n.ndefer = 0;
@@ -1822,7 +1826,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
               continue;
             }
             v = n.alpha;
-            if (TABLE) lcount(cvec, C_TT_STORE, tt_store<TABLE>(a, tt_mask(cfg), L, n, sd, lane));
+            if (TABLE) lcount(cvec, C_TT_STORE, tt_store<TABLE>(a, tt_mask(cfg), L, n, sd, ra, lane));
             state = S_RETURN;
             continue;
           }
@@ -1940,7 +1944,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         restore(L.ply[sd], n, lane);
         if (TABLE) n.reach = n.reach > below ? n.reach : below;
         const s32 sc = -v;
-        if ((sd & 1) && sd >= 3 && ra - 1 > n.alpha && ra - 1 < n.beta) {
+        if (floor_lifts(sd, ra, n.alpha, n.beta)) {
           // the root bound rose while this node's children were searched:
           // its best move so far is below it, so no lower bound stands
           n.alpha = ra - 1;
@@ -1964,12 +1968,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
                                            (u64)(u16)(sc + 32768)));
           }
         }
-        // (at the other side's plies: no better reply is needed to keep the root
-        // move at or below ra - 1)
-        if (n.alpha >= n.beta || (!(sd & 1) && ra > -INF && n.alpha >= 1 - ra)) {
+        const bool cut = n.alpha >= n.beta;
+        if (cut || reply_suffices(sd, ra, n.alpha)) {
           const u32 last = last_move(L, sd);
           u16 *const ctab = glob(a->ctab) + (size_t)blockIdx.x * NCOUNTER;
-          if ((cfg & CF_RECORDS) && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
+          // the move refuted the one before it (not where only the root's bound
+          // ended the node, here or below)
+          const bool refutes = cut && bound_holds(sd, ra, true, n.alpha);
+          if (refutes && (cfg & CF_RECORDS) && n.depth >= 1 && n.searched >= 1 && n.mcnt >= 2 &&
               ((u32)(n.hash >> 40) & a->rec_mask) == 0) {
             u32 nrec = 0;
             log_pairs(a, n, lane, mmove, L.tab, n.ttm, killers[sd], (u32)ctab[counter_index(last)], nrec);
@@ -1977,12 +1983,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
           }
           // a quiet move that fails high becomes the ply's killer and the
           // counter move of the move before it (src/zeta.cl:1916-1933)
-          if (((mv_pcpt(n.move) >> 1) & 7) == PNONE && lane == 0) {
+          if (refutes && ((mv_pcpt(n.move) >> 1) & 7) == PNONE && lane == 0) {
             killers[sd] = n.move;
             ctab[counter_index(last)] = counter_code(n.move);
           }
           v = n.alpha;
-          if (TABLE) lcount(cvec, C_TT_STORE, tt_store<TABLE>(a, tt_mask(cfg), L, n, sd, lane));
+          if (TABLE) lcount(cvec, C_TT_STORE, tt_store<TABLE>(a, tt_mask(cfg), L, n, sd, ra, lane));
           state = S_RETURN;
         } else {
           li = load_list(L, lane, n.mbeg);
