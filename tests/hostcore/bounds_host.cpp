@@ -1,5 +1,5 @@
 // Host model of the search's windows (zeta_amd/csrc/bounds.h, the control flow
-// of search.hip's k_search) on random game graphs whose values are
+// of search.hip's k_search and qsearch) on random game graphs whose values are
 // known by plain minimax, with the bound of the root's other workers rising at
 // any visit.  Test-only.
 #include <stdint.h>
@@ -29,6 +29,8 @@ struct Model {
   std::vector<int> capture[STATES];
   int q[STATES], val[MAXDEPTH + 1][STATES];  // minimax, for the side to move
   Entry tt[MAXDEPTH + 1][STATES];
+  uint32_t qkind[STATES];
+  int qval[STATES];
   int ra = -INF, most = 0;  // most: the bound may rise to it
   long stores = 0, wrong = 0;
 
@@ -43,6 +45,7 @@ struct Model {
       }
       q[i] = eval[i];
       for (int c : capture[i]) q[i] = q[i] > -q[c] ? q[i] : -q[c];
+      qkind[i] = Q_NONE;
       val[0][i] = q[i];
     }
     for (int d = 1; d <= MAXDEPTH; d++)
@@ -62,18 +65,52 @@ struct Model {
     stores++;
     wrong += lower ? val[d][i] < v : val[d][i] > v;
   }
+  void qstore(int i, uint32_t kind, int v) {
+    if (kind == Q_NONE) return;
+    qkind[i] = kind;
+    qval[i] = v;
+    stores++;
+    wrong += ((kind & Q_LOWER) && q[i] < v) || ((kind & Q_UPPER) && q[i] > v);
+  }
+
   int quiesce(int i, int sd, int alpha, int beta) {
     visit();
     if (floor_lifts(sd, ra, alpha, beta)) alpha = ra - 1;
     if (eval[i] >= beta) return eval[i];
-    if (eval[i] > alpha) alpha = eval[i];
+    bool raised = false;
+    if (shared && qkind[i] != Q_NONE) {
+      if (qkind[i] == Q_EXACT || (qkind[i] == Q_LOWER && qval[i] >= beta) || (qkind[i] == Q_UPPER && qval[i] <= alpha))
+        return qval[i];
+      if (qkind[i] == Q_LOWER && qval[i] > alpha) {
+        alpha = qval[i];
+        raised = true;
+      }
+    }
+    if (capture[i].empty()) {
+      qstore(i, Q_EXACT, eval[i]);
+      return eval[i];
+    }
+    if (eval[i] > alpha) {
+      alpha = eval[i];
+      raised = true;
+    }
     for (int c : capture[i]) {
       const int v = -quiesce(c, sd + 1, -beta, -alpha);
-      if (floor_lifts(sd, ra, alpha, beta)) alpha = ra - 1;
-      if (v > alpha) alpha = v;
-      if (alpha >= beta) break;
+      if (floor_lifts(sd, ra, alpha, beta)) {
+        alpha = ra - 1;
+        raised = false;
+      }
+      if (v > alpha) {
+        alpha = v;
+        raised = true;
+      }
+      if (alpha >= beta) {
+        if (bound_holds(sd, ra, true, alpha)) qstore(i, Q_LOWER, alpha);
+        return alpha;
+      }
     }
-    return capture[i].empty() ? eval[i] : alpha;
+    qstore(i, bound_kind(sd, ra, raised, alpha), alpha);
+    return alpha;
   }
 
   int full(int i, int d, int sd, int alpha, int beta) {

@@ -32,6 +32,6 @@ def test_stored_bounds_hold(H, shared):
         H.hs_bounds(seed, shared, out.ctypes.data)
         total += out
     print("stored", total[0], "wrong", total[1], "searches", total[2], "off", total[3])
-    assert total[0] > 100000
+    assert total[0] > 1000000
     assert total[1] == 0
     assert total[3] == 0

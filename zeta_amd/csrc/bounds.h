@@ -29,4 +29,11 @@ ZD bool bound_holds(int sd, int32_t ra, bool lower, int32_t v) {
   return sd & 1 ? !lower || v >= ra : lower || v <= -ra;
 }
 
+// What a node that has seen all its moves with the result v, below beta, may
+// store: a move (or the stand pat) raised alpha to v, or none did.
+enum { Q_NONE = 0, Q_LOWER = 1, Q_UPPER = 2, Q_EXACT = 3 };
+ZD uint32_t bound_kind(int sd, int32_t ra, bool raised, int32_t v) {
+  return (raised && bound_holds(sd, ra, true, v) ? Q_LOWER : Q_NONE) | (bound_holds(sd, ra, false, v) ? Q_UPPER : Q_NONE);
+}
+
 }  // namespace zc

@@ -85,12 +85,12 @@ typedef u32 u32x2 __attribute__((ext_vector_type(2)));  // one 8-byte quiescence
 // quiescence trees, and trees of 10^5 nodes below one node kept a worker busy
 // after all others had ended.  An entry is 8 bytes, read and written whole: the
 // key's bits above QT_BITS (those below are in the index, of at least QT_BITS
-// bits, so that no two keys share an entry), the kind of bound, the value.
+// bits, so that no two keys share an entry), the kind of bound (Q_LOWER ..
+// Q_EXACT), the value.
 // It starts empty in every call.  1024 positions, depth 4, 128 workers each:
 // 373 -> 151 ms (1057 -> 251 ms for a batch with one root of 89 M nodes); one
 // position, depth 5: 52 -> 45 ms.
 constexpr int QT_BITS = 18;
-enum { Q_LOWER = 1, Q_UPPER = 2, Q_EXACT = 3 };
 constexpr u64 QT_MIN = 1ULL << QT_BITS, QT_MAX = 1ULL << 22, QT_WORKER = 4096;  // entries: least, most, per worker
 
 // ---- serving (zeta_serve_*): the host publishes requests in coherent pinned
@@ -1326,7 +1326,7 @@ __device__ __forceinline__ u64 all_moves(int n) { return n < 64 ? (1ULL << n) - 
 enum { QS_DONE = 0, QS_ABORTED, QS_FAILED };
 
 __device__ __forceinline__ void qt_store(const Pos &p, u64 phash, s32 v, u32 kind, int lane) {
-  if (lane != 0 || v != (s32)(int16_t)(u16)v) return;
+  if (lane != 0 || kind == Q_NONE || v != (s32)(int16_t)(u16)v) return;
   const Args a = args();
   const u64 key = phash ^ (u64)p.stm;
   shared_store(a->qtt + (key & a->qmask), (key >> QT_BITS << QT_BITS) | (kind << 16) | ((u32)v & 0xFFFFu));
@@ -1342,9 +1342,8 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
                                        const int sd0, int mbeg, s32 ev, bool known, bool kic, bool polled, u64 phash,
                                        Poll &q, s32 &ra, u32 &cvec, s32 &vout) {
   int sd = sd0, mcnt = 0, unused = 0;
-  // the node's value goes into the table; a move or the stand pat raised alpha;
-  // in this call a root bound has taken alpha's place (a value may then be a bound)
-  bool store = false, raised = false, clamped = false;
+  // the node's value goes into the table; a move or the stand pat raised alpha
+  bool store = false, raised = false;
   u64 qe = 0;
   u64 ep = ~p.cr & RANKS45;  // captures leave none behind
   u64 left = 0;
@@ -1356,10 +1355,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
     if (arrive) {
       if (!polled && ++q.count >= POLL_EVERY && poll_root(args(), L, lane, q, ra)) return QS_ABORTED;
       polled = false;
-      if (floor_lifts(sd, ra, alpha, beta)) {
-        alpha = ra - 1;
-        clamped = true;
-      }
+      if (floor_lifts(sd, ra, alpha, beta)) alpha = ra - 1;
       store = raised = false;
       const bool draw = hmc >= 100 || popc(p.b1 | p.b2 | p.b3) <= 2;
       // stand pat before any move generation: the reference returns the static
@@ -1446,7 +1442,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
         continue;
       }
       v = alpha;
-      if (TABLE && store) qt_store(p, phash, v, raised ? (clamped ? Q_LOWER : Q_EXACT) : Q_UPPER, lane);
+      if (TABLE && store) qt_store(p, phash, v, bound_kind(sd, ra, raised, v), lane);
     }
     // return v to the parent, and on while the parents fail high
     do {
@@ -1474,14 +1470,13 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
       if (floor_lifts(sd, ra, alpha, beta)) {
         alpha = ra - 1;
         raised = false;
-        clamped = true;
       }
       if (v > alpha) {
         alpha = v;
         raised = true;
       }
       v = alpha;
-      if (TABLE && store && alpha >= beta) qt_store(p, phash, v, Q_LOWER, lane);
+      if (TABLE && store && alpha >= beta && bound_holds(sd, ra, true, v)) qt_store(p, phash, v, Q_LOWER, lane);
     } while (alpha >= beta);
     li = load_list(L, lane, mbeg);
     arrive = false;
