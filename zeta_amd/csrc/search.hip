@@ -1564,9 +1564,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
       L.hlen = hl > ZETA_HISTORY ? ZETA_HISTORY : (hl < 0 ? 0 : hl);
     }
     if (TABLE == T_SHARED) {
+      // (each with its place: a position that occurred twice would cancel itself)
       u64 h = 0;
       wsync();
-      for (int k = lane; k < L.hlen; k += 64) h ^= hash_mix(a->hist[(size_t)r * ZETA_HISTORY + k]);
+      for (int k = lane; k < L.hlen; k += 64)
+        h ^= hash_mix(a->hist[(size_t)r * ZETA_HISTORY + k] + (u64)(k + 1) * 0xD1B54A32D192ED03ULL);
       h = wave_xor(h);
       if (lane == 0) L.hsalt = h;
     }
