@@ -1189,7 +1189,14 @@ int no_room() {
   return ZETA_OK;
 }
 
-// The whole call; *done = false: a level is beyond the frontier budget (or the
+// depth 1, queued only: the caller waits, behind the copy of the counts if it
+// takes one (two waits: 300 positions 45 us, one 33)
+int count_roots(const u64 *pos, int n, u64 *counts) {
+  ZLAUNCH(zr::K_PERFT_ROOTS, n, k_count_roots, blocks(n, 64), 64, 0, pos, n, counts);
+  return ZETA_OK;
+}
+
+// The whole call, depth 2 or more; *done = false: a level is beyond the frontier budget (or the
 // call is one the fast path does not take) and nothing has been counted.
 int fast_perft(const u64 *pos, int n, int depth, u64 *counts, u64 *hcounts, int flags, bool *done) {
   zr::Ctx &c = zr::ctx();
@@ -1197,18 +1204,12 @@ int fast_perft(const u64 *pos, int n, int depth, u64 *counts, u64 *hcounts, int 
   const bool nobulk = (flags & ZETA_PERFT_NOBULK) != 0;
   const int D = nobulk ? depth + 1 : depth;
   const u64 budget = c.cfg.frontier_budget;
-  if (depth < 1 || D >= MAXLEV || budget < 512 || (u64)n > budget || !c.perft_ctl_dev) return ZETA_OK;
+  if (D < 2 || D >= MAXLEV || budget < 512 || (u64)n > budget || !c.perft_ctl_dev) return ZETA_OK;
   int r;
   if ((r = zr::ensure(g_fs.ctl, CTL_WORDS * 8))) return r;
   if (!g_fs.ctl_clean) {
     ZCHECK(hipMemsetAsync(g_fs.ctl.p, 0, CTL_WORDS * 8, c.stream));
     g_fs.ctl_clean = true;
-  }
-  if (D == 1) {
-    ZLAUNCH(zr::K_PERFT_ROOTS, n, k_count_roots, blocks(n, 64), 64, 0, pos, n, hcounts ? hcounts : counts);
-    ZCHECK(hipStreamSynchronize(c.stream));
-    *done = true;
-    return ZETA_OK;
   }
   Chain q = {pos, n, D, nobulk, counts, hcounts, {0}, {0}, 0};
   const u64 *const want = c.perft_ctl_host;
@@ -1320,6 +1321,11 @@ extern "C" int zeta_perft_batch_device(const void *d_pos, int n, int depth, void
   if (r) return r;
   if ((!d_pos || !d_counts) && n > 0) return zr::fail(ZETA_EINVAL, "perft: null pointer");
   bool done = false;
+  if (n > 0 && depth == 1 && !(flags & ZETA_PERFT_NOBULK)) {
+    if (!(r = count_roots((const u64 *)d_pos, n, (u64 *)d_counts))) ZCHECK(hipStreamSynchronize(zr::ctx().stream));
+    zr::time_collect();
+    return r;
+  }
   if (n > 0 && depth > 0) {
     r = fast_perft((const u64 *)d_pos, n, depth, (u64 *)d_counts, nullptr, flags, &done);
     if (r || done) {
@@ -1454,20 +1460,18 @@ extern "C" int zeta_perft_batch(const zeta_pos *pos, int n, int depth, uint64_t 
   if (pinned) memcpy(c.perft_stage_host, pos, (size_t)n * sizeof(zeta_pos));
   else ZCHECK(hipMemcpyAsync(g_ps.roots.p, pos, (size_t)n * sizeof(zeta_pos), hipMemcpyHostToDevice, c.stream));
   if (depth > 0) {
-    bool done = false;
-    r = fast_perft(pinned ? (const u64 *)c.perft_stage_dev : (const u64 *)g_ps.roots.p, n, depth, (u64 *)g_ps.counts.p,
-                   pinned ? (u64 *)c.perft_counts_dev : nullptr, 0, &done);
+    bool done = depth == 1;
+    const u64 *const in = pinned ? (const u64 *)c.perft_stage_dev : (const u64 *)g_ps.roots.p;
+    u64 *const out = (u64 *)g_ps.counts.p, *const hout = pinned ? (u64 *)c.perft_counts_dev : nullptr;
+    r = depth == 1 ? count_roots(in, n, pinned ? hout : out) : fast_perft(in, n, depth, out, hout, 0, &done);
     if (r) {
       zr::time_collect();
       return r;
     }
     if (done) {
-      if (pinned) {
-        memcpy(counts, c.perft_counts_host, (size_t)n * 8);
-      } else {
-        ZCHECK(hipMemcpyAsync(counts, g_ps.counts.p, (size_t)n * 8, hipMemcpyDeviceToHost, c.stream));
-        ZCHECK(hipStreamSynchronize(c.stream));
-      }
+      if (!pinned) ZCHECK(hipMemcpyAsync(counts, out, (size_t)n * 8, hipMemcpyDeviceToHost, c.stream));
+      if (!pinned || depth == 1) ZCHECK(hipStreamSynchronize(c.stream));
+      if (pinned) memcpy(counts, c.perft_counts_host, (size_t)n * 8);
       zr::time_collect();
       return ZETA_OK;
     }
