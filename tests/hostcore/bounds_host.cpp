@@ -171,3 +171,13 @@ extern "C" void hs_bounds(uint32_t seed, int shared, int64_t *out) {
   out[2] = searches;
   out[3] = off;
 }
+
+// plies that captures from ply sd on a board of `pieces` can reach
+extern "C" int hs_deepest(int sd, int pieces) {
+  while (pieces > 2) {
+    sd++;
+    pieces--;
+  }
+  return sd;
+}
+extern "C" int hs_any_ply(int sd, int pieces, int maxply) { return any_ply(sd, pieces, maxply); }

@@ -35,3 +35,13 @@ def test_stored_bounds_hold(H, shared):
     assert total[0] > 1000000
     assert total[1] == 0
     assert total[3] == 0
+
+
+def test_quiescence_values_out_of_the_ply_limits_reach(H):
+    """A value kept for any ply must not depend on the ply limit (64): at every
+    ply and number of pieces, full boards included."""
+    for sd in range(1, 65):
+        for pieces in range(3, 65):
+            if H.hs_any_ply(sd, pieces, 64):
+                assert H.hs_deepest(sd, pieces) < 64, (sd, pieces)
+    assert H.hs_any_ply(32, 32, 64)  # as deep as any game's board was kept

@@ -36,4 +36,8 @@ ZD uint32_t bound_kind(int sd, int32_t ra, bool raised, int32_t v) {
   return (raised && bound_holds(sd, ra, true, v) ? Q_LOWER : Q_NONE) | (bound_holds(sd, ra, false, v) ? Q_UPPER : Q_NONE);
 }
 
+// Is a quiescence value at ply sd out of the ply limit's reach, whatever the
+// captures below?  Each takes a piece off, and two that are left are a draw.
+ZD bool any_ply(int sd, int pieces, int maxply) { return sd + pieces <= maxply; }
+
 }  // namespace zc

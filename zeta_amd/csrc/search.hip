@@ -1368,8 +1368,7 @@ __device__ __forceinline__ int qsearch(Lds &L, const LaneSq &me, int lane, Pos p
         if (!draw && sd >= MAXPLY) lcount(cvec, C_MAXPLY, 1);
         v = ev;
       }
-      // (no deeper than 32 plies, the ply limit is out of reach below the node)
-      if (TABLE && !leaf && !ep && !draw && sd <= 32) {
+      if (TABLE && !leaf && !ep && !draw && any_ply(sd, popc(p.b1 | p.b2 | p.b3), MAXPLY)) {
         const u64 key = phash ^ (u64)p.stm;
         if (sd == sd0) qe = shared_load(args()->qtt + (key & args()->qmask));
         const u64 e = uf(qe);
