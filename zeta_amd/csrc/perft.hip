@@ -292,7 +292,7 @@ struct Level {
   u64 *b0, *b1, *b2, *b3, *cr;
   u64 *wt;    // paths from the root that the node stands for
   u32 *meta;  // root index << 1 | side to move
-  u32 *mv;    // the move that led to it
+  u32 *mv;    // the move that led to it, where k_spread's list in LDS was full
   u32 *par;   // its parent's index in the level above
   u64 *count; // nodes wanted so far (those past the capacity are not stored)
   u64 cap;
@@ -308,14 +308,13 @@ __device__ __forceinline__ Pos level_pos(const Level &f, size_t i) {
   p.stm = f.meta[i] & 1u;
   return p;
 }
-__device__ __forceinline__ void level_store(const Level &f, size_t i, const Pos &c, u32 root, u32 mv, u32 par, u64 wt) {
+__device__ __forceinline__ void level_store(const Level &f, size_t i, const Pos &c, u32 root, u32 par, u64 wt) {
   f.b0[i] = c.b0;
   f.b1[i] = c.b1;
   f.b2[i] = c.b2;
   f.b3[i] = c.b3;
   f.cr[i] = c.cr;
   f.meta[i] = (root << 1) | c.stm;
-  f.mv[i] = mv;
   f.par[i] = par;
   f.wt[i] = wt;
 }
@@ -414,7 +413,7 @@ __global__ __launch_bounds__(WIDE_TPB) void k_wide(const u64 *__restrict__ in, i
     __syncthreads();
     const u64 base = lbase + before;
     for (int k = lane; k < m; k += 64)
-      if (base + k < g.cap) level_store(g, base + k, apply_count(p, list[w][k]), root, list[w][k], (u32)i, wt);
+      if (base + k < g.cap) level_store(g, base + k, apply_count(p, list[w][k]), root, (u32)i, wt);
     __syncthreads();
   }
 }
@@ -522,7 +521,7 @@ __global__ __launch_bounds__(XTPB) void k_spread(Level f, u64 i0, u64 i1, Level 
         q.b3 = lb3[l];
         q.cr = lcr[l];
         q.stm = lmeta[l] & 1u;
-        level_store(g, base + k, apply_count(q, code), lmeta[l] >> 1, code, (u32)(c0 + l), lwt[l]);
+        level_store(g, base + k, apply_count(q, code), lmeta[l] >> 1, (u32)(c0 + l), lwt[l]);
       }
     }
     __syncthreads();
@@ -667,7 +666,7 @@ __global__ __launch_bounds__(TPB) void k_compact(Level f, Level g) {
     __syncthreads();
     u64 o = base + (u64)popc(b & ((1ULL << lane) - 1));
     for (int k = 0; k < w; k++) o += part[k];
-    if (stay && o < g.cap) level_store(g, o, level_pos(f, i), f.meta[i] >> 1, f.mv[i], f.par[i], f.wt[i]);
+    if (stay && o < g.cap) level_store(g, o, level_pos(f, i), f.meta[i] >> 1, f.par[i], f.wt[i]);
   }
 }
 // the roots as level 0 (many roots)
@@ -675,7 +674,7 @@ __global__ __launch_bounds__(TPB) void k_load_roots(const u64 *__restrict__ in, 
   const int i = blockIdx.x * TPB + threadIdx.x;
   if (i >= n) return;
   if (i == 0) *f.count = (u64)n;
-  level_store(f, i, root_pos(in, i), (u32)i, 0, (u32)i, 1);
+  level_store(f, i, root_pos(in, i), (u32)i, (u32)i, 1);
   counts[i] = 0;
 }
 // The end of a chain: the sizes of its levels to the host's words (and cleared

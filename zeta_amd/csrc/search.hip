@@ -76,7 +76,6 @@ inline int default_split(int workers) { return workers >= 16 ? 1 : 2; }
 constexpr int POLL_EVERY = 64;
 
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));  // one 16-byte TT entry
-typedef u32 u32x2 __attribute__((ext_vector_type(2)));  // one 8-byte quiescence entry
 
 // The quiescence table.  A quiescence node's value is a function of its pieces
 // and side to move alone (captures only, no repetition, no castling), so the
@@ -141,7 +140,7 @@ struct SearchArgs {
   int split_depth;   // ABDADA deferral / busy marking at depth - 1 >= split_depth
   u64 *tt;           // 2 words per entry
   u64 ttmask;        // entries - 1 (0 = no TT)
-  u64 *qtt;          // quiescence table, see QEntry (used where there is a TT)
+  u64 *qtt;          // quiescence table, 8 bytes an entry (qt_store), where there is a TT
   u64 qmask;         // its entries - 1
   const u64 *hint;   // read-only table in the TT's format whose moves go first (null = none)
   u64 *rbound;       // per root (slot): best root score so far, ticket << 32 | iteration << 16 | score + 32768
@@ -249,11 +248,6 @@ __device__ __forceinline__ s32 wave_sum_i(s32 v) {
 }
 __device__ __forceinline__ u32 wave_max_u32(u32 v) {
   return (u32)__builtin_amdgcn_readlane((int)zw::wave_scan_max(v), 63);
-}
-__device__ __forceinline__ int wave_exscan_i(int v, int lane, int &total) {
-  const int x = zw::wave_scan_add(v);
-  total = __builtin_amdgcn_readlane(x, 63);
-  return x - v;
 }
 
 // TT / busy-table key: the reference hash plus the exact castle squares
@@ -732,12 +726,6 @@ __device__ int serve_pick(Args a, int lane, u64 &tk_out) {
       backoff = backoff < 16 ? 2 * backoff : 16;
     }
   }
-}
-
-// serving: abort test at the periodic poll
-__device__ __forceinline__ bool serve_abort(Args a, int r, u64 tk) {
-  const u64 v = ag_load(&a->sw[r]);
-  return sw_tk(v) != tk || sw_st(v) != SV_RUN || ag_load(&a->dcancel[r]) == tk || ag_load(&a->sv->shut) != 0;
 }
 
 // serving: leave the request.  The worker that completes it (or fails it)
@@ -2139,8 +2127,6 @@ int qt_clear(unsigned grid, hipStream_t st, SearchArgs &sa) {
   sa.qmask = entries - 1;
   return 0;
 }
-
-inline unsigned nblocks(size_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
 }  // namespace
 
