@@ -42,8 +42,8 @@ HBM_BYTES_PER_POSITION = 9.80
 # over the depth-6 search leg (profiles/search_c3_pmc.md).  A CU's arbiter
 # issues at most one scalar instruction per cycle (each SIMD's waves get one
 # SALU slot every 4 cycles), so the SALU issue peak is 256 CU x 2.4 GHz.
-VALU_WAVE_INSTS_PER_NODE = 312.8
-SALU_INSTS_PER_NODE = 280.6
+VALU_WAVE_INSTS_PER_NODE = 308.9
+SALU_INSTS_PER_NODE = 275.0
 SALU_PEAK = 256 * 2.4e9
 # the ordering network: 908 -> 256 -> 32 -> 1, dense FLOP of one scored move
 # (2 x (908 x 256 + 256 x 32 + 32)); a training pair scores two moves and its

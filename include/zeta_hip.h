@@ -165,17 +165,18 @@ int zeta_search_batch(const zeta_pos *pos, int n, const zeta_search_opts *opts, 
 /* Abort switch of the search batches.  No counterpart at the reference's
  * boundary (its helpers stop on the kernel's own finito flag and the node
  * budget, src/zeta.cl:1940-1953).  on = 1: a zeta_search_batch running on
- * another host thread stops at its workers' next poll (every 64 nodes), and
- * every batch started while the switch is on returns at once; the roots left
- * unfinished get status ZETA_ECANCELED.  on = 0 re-arms.  The one call that
- * may be made while zeta_search_batch runs; it touches a word in pinned host
- * memory only. */
+ * another host thread stops at its workers' second poll after it (they poll
+ * every 64 nodes), and every batch started while the switch is on returns at
+ * once; the roots left unfinished get status ZETA_ECANCELED.  on = 0 re-arms.
+ * The one call that may be made while zeta_search_batch runs; it touches a
+ * word in pinned host memory only. */
 int zeta_search_abort(int on);
 /* Counters of the last zeta_search_batch: [0] TT probes, [1] TT key hits,
  * [2] TT scores used, [3] TT stores, [4] ABDADA deferrals, [5] MAXPLY cuts,
  * [6] nodes ordered by the network, [7] training pairs logged, [8] nodes
  * made by all workers (after zeta_serve_stop: of the whole serving session).
- * Each probe / store moves one 16-byte entry. */
+ * Each probe / store moves one 16-byte entry, nodes with two plies left or
+ * more a second one where their bounds hold on their path only. */
 int zeta_search_counters(uint64_t *out, int n);
 
 /* ---------------------------------------------------------------- serving

@@ -318,7 +318,7 @@ ZD void many_kings(Legal &L, u64 e, u64 &A, u64 &chkray) {
 // Bound: VALU issue where a lane takes a position (perft).  The three fills of
 // a direction share the doubled empty sets; three-operand logic and the rank
 // carries, here, in apply_v and in count_legal, took a perft leaf from 990 to
-// 880 lane-instructions (130.8 M leaves: 3.42 to 3.25 ms).
+// 865 lane-instructions (128.9 M leaves: 3.41 to 2.9 ms).
 ZD void analyse(const Pos &p, Legal &L) {
   const u64 occ = bop3<(TA | TB | TC)>(p.b1, p.b2, p.b3);
   const u64 black = 0 - (u64)(p.stm & 1u);

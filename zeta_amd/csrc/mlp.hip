@@ -126,11 +126,15 @@ constexpr int S_B1 = 0, S_B2 = NH1, S_W3 = S_B2 + NH2, S_B3 = S_W3 + NH2, S_LOSS
 // weight gradients need goes out as BF16 operands (h1, dz1, dz2) and as the
 // one-hot rows' bits, 1/16 of their BF16 size.  nrec > 0: the step's pairs are
 // drawn here (sample_index); nrec = 0: pair p is record p.
-// Bound: the W1 operand, 464 KB a block at the 64 bytes a cycle a CU loads
-// (3 us), and the record's latency; a third of it is asked for before the
-// records are looked at, a third while the features are taken apart.
-// At 2048 pairs 14.6 us, where features, layer 1, head and layer-1 backward as
-// launches of their own took 39 us; 51 us at 16384 pairs.
+// Bound: latency.  The phases follow one another -- record, features, the W1
+// operand (464 KB a block), a chain of products, the head -- and 0.4 of the
+// wavefronts' cycles wait for memory, 0.35 for an issue slot; the L1 gives
+// 0.36 of its 64 bytes a cycle, the matrix units are busy 0.12 of the time, and
+// at 2048 pairs half of the CUs have no block.  A third of the W1 operand is
+// asked for before the records are looked at, a third while the features are
+// taken apart.
+// At 2048 pairs 14.3 us, where features, layer 1, head and layer-1 backward as
+// launches of their own took 39 us; 50 us at 16384 pairs.
 __global__ __launch_bounds__(TPB) void k_rows(const PairRec *__restrict__ recs, int B, u64 nrec, u64 seed,
                                               const float *__restrict__ prm, const u16 *__restrict__ w1x,
                                               const u16 *__restrict__ w2t, const u16 *__restrict__ w2,
@@ -356,9 +360,12 @@ constexpr int SUM_BLOCKS = (NSUM + 31) / 32;  // 32 sums a block
 // own updates the weights); else the gradient in the ABI's layout.  The last
 // blocks do the same for the biases and the head, whose sums k_rows left.
 // X comes from its bits (a byte is one operand).
-// At 2048 pairs 9.2 us, where the two products (22 us) and the update (6.6 us)
-// were passes of their own; at 16384 pairs 49 us, near the 64 bytes a cycle a
-// CU loads.
+// At 2048 pairs 9.3 us, where the two products (22 us) and the update (6.6 us)
+// were passes of their own; 48 us at 16384 pairs.  Bound: latency, of operands
+// that another chiplet's kernel has just written, and of the table lookups (a
+// tenth of the cycles are bank conflicts) ahead of one chain of products: 0.4 of
+// the cycles wait for memory, the L1 gives 0.36 of its 64 bytes a cycle, the
+// matrix units are busy 0.14 of the time.
 template <bool UPDATE>
 __global__ __launch_bounds__(TPB) void k_weights(int B, const u32 *__restrict__ bits, const u16 *__restrict__ h1x,
                                                  const u16 *__restrict__ dz2x, const u16 *__restrict__ dz1x, const float *__restrict__ sums,

@@ -285,9 +285,10 @@ __global__ __launch_bounds__(TPB) void k_leaf(Front f, const u64 *__restrict__ p
 // Levels 3 and deeper merge transpositions: positions of a root reached by
 // several move orders become one node that carries their number (k_merge).
 // Measured against the chunked driver (host waits for every level, three scan
-// launches each): one position at depth 4 139 -> 47 us, at depth 6 (119 M and
-// 8 G leaves) 2.05 -> 0.39 and 5.8 -> 0.52 ms.  The first of these is launches
-// and the host's one wait; the others are bound by the leaves' VALU issue.
+// launches each): one position at depth 4 146 -> 54 us, at depth 6 (119 M and
+// 8 G leaves) 2.05 -> 0.39 and 5.8 -> 0.52 ms.  Of the first, 46 us are its four
+// kernels (7, 10, 26 and 4), the rest launches and the host's one wait; the
+// others are bound by the leaves' VALU issue.
 struct Level {
   u64 *b0, *b1, *b2, *b3, *cr;
   u64 *wt;    // paths from the root that the node stands for
@@ -419,7 +420,9 @@ __global__ __launch_bounds__(WIDE_TPB) void k_wide(const u64 *__restrict__ in, i
 }
 
 // the last level below few parents: each lane makes a child and counts its
-// moves (nobulk: generates them and counts the child itself)
+// moves (nobulk: generates them and counts the child itself).
+// Bound: latency of one wavefront's work on a parent: 1000 parents are 128 blocks
+// on 256 CUs, and 0.6 of their cycles wait (26 us).
 __global__ __launch_bounds__(WIDE_TPB) void k_wide_leaf(const u64 *__restrict__ in, int nroots, Level f,
                                                         u64 *__restrict__ counts, int nobulk) {
   __shared__ u32 list[WIDE_TPB / 64][MAXMOVES];
@@ -451,7 +454,7 @@ __global__ __launch_bounds__(WIDE_TPB) void k_wide_leaf(const u64 *__restrict__ 
 // the stores are coalesced.  PAIRS: the moves are not made but written as
 // (parent << 32 | move) for the leaf kernel.  Takes the parents [i0, i1).
 // Bound: VALU issue of the move loops, where a wavefront runs as many steps as
-// its busiest lane has of each kind (4.2 M parents, 130 M pairs: 0.54 ms; the
+// its busiest lane has of each kind (3.97 M parents, 128.9 M pairs: 0.57 ms; the
 // stores alone would take 0.22).
 template <bool PAIRS>
 __global__ __launch_bounds__(XTPB) void k_spread(Level f, u64 i0, u64 i1, Level g, u64 *__restrict__ pm) {
@@ -529,11 +532,12 @@ __global__ __launch_bounds__(XTPB) void k_spread(Level f, u64 i0, u64 i1, Level 
 }
 
 // ---- leaf: the children of `f` that the pairs name, counted into their roots.
-// Bound: VALU issue (0.99 of it); a child costs about 850 lane-instructions.
+// Bound: VALU issue (0.97-0.99 of the peak): a child costs 865 lane-instructions,
+// 128.9 M of them 2.85-2.93 ms.
 // A wavefront takes runs of 512 pairs in turn, one atomic a root of the run; of
 // the grid about three blocks a CU are resident, and the rest of its 48 a CU
-// fills the places of those that end first (3.20 ms for 130 M pairs, 3.59 ms
-// with a grid of the resident ones).
+// fills the places of those that end first (a grid of the resident ones took
+// 12 % longer).
 // WT: f is a merged level, whose nodes count as often as they have paths.
 constexpr int LEAF_BLOCKS = 48;
 constexpr u32 LEAF_RUN = 512;

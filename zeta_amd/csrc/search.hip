@@ -217,6 +217,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // quiescence table, no entries by path, full windows.  Its workers make about
 // the nodes they made before all that, so that the same budgets stop the same
 // searches (with it, a root of 30000 nodes over 8 workers ends within 2000 each).
+// The engine's moves, whose clock is a node budget, run this one.
 enum { T_NONE = 0, T_SHARED, T_BUDGET };  // a search's tables
 __device__ __forceinline__ u64 shared_load(const u64 *p) {
   return __hip_atomic_load(glob(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -988,7 +989,9 @@ __device__ __forceinline__ s32 static_eval(const Pos &p, int lane) {
 }
 
 // The periodic test (every POLL_EVERY nodes) looks at words that were loaded at
-// the test before it: the abort word lies in host memory, a read of 2 us.
+// the test before it: the abort word lies in host memory, a read of 2 us.  So
+// what the host or another worker sets is seen at the second test after it, up
+// to 2 * POLL_EVERY nodes later; a node budget at the first.
 struct Poll {
   int count;      // nodes since the last test
   u64 nodes;      // nodes made at this root
