@@ -46,7 +46,10 @@ constexpr int MAXPLY = 64;  // src/types.h:76
 constexpr s32 INF = 32000;
 constexpr s32 MATESCORE = 30000;
 constexpr int MSTACK = 1024;  // move-stack slots per worker (LDS)
-constexpr int MPAD = 48;      // slots past them for captures not yet tested for legality
+// Slots past them for moves not yet tested for legality: a list whose legal moves
+// fit must fit before the test too.  No position of a game has 256 moves, legal or
+// not; eight workers a CU have room for them.
+constexpr int MPAD = 256;
 // A move-list entry is a move code and a key: the ordering score + 32768 in the
 // upper half (0: the move was searched), in the lower half what is known of
 // the child, if it is a quiescence node: KEY_CHECK, KEY_OPEN, or its static
