@@ -1296,7 +1296,8 @@ __device__ __forceinline__ int gen_moves(Lds &L, const LaneSq &me, int lane, con
       if (!QS) known = known && !is_promo(m) && child_hmc(hmc, m) < 100;
       if (known) key = (u32)((p.stm ? e : -e) + 32768);
     }
-    if (king_attacked(c, oq, okb != 0, oknight, opawn, p.stm)) key = KEY_CHECK;
+    // (a captured king is in no check)
+    if (king_attacked(c, oq, okb != 0 && (cap >> 1) != KING, oknight, opawn, p.stm)) key = KEY_CHECK;
     const s32 sc = QS ? piece_value(cap >> 1) * 16 - piece_value(pt >> 1) : plain_score(L.tab, p.stm, m, killer, counter);
     const u64 lm = __ballot(legal);
     const int slot = mbeg + kept + popc(lm & ((1ULL << lane) - 1));
