@@ -33,3 +33,42 @@ def test_search_where_a_king_can_be_taken(zeta, oracle, tt):
     assert (got["score"] == want).all()
     if not tt:
         assert (got["nodes"] == nodes).all()
+
+
+def _board(rng, i):
+    """2-24 pieces anywhere: one king a side, any number, or several; any flags."""
+    b = np.zeros(7, dtype=np.uint64)
+    for j, sq in enumerate(rng.permutation(64)[:int(rng.integers(2, 24))]):
+        piece, black = int(rng.integers(1, 7)), int(rng.integers(0, 2))
+        if i % 4 != 1 and j < (4 if i % 4 == 2 else 2):
+            piece, black = 3, j & 1
+        elif i % 4 == 3:
+            piece = int(rng.choice([1, 5]))
+        for t in range(3):
+            b[1 + t] |= np.uint64((piece >> t & 1) << int(sq))
+        b[0] |= np.uint64(black << int(sq))
+    cr = int(rng.integers(0, 1 << 64, dtype=np.uint64))
+    if i % 3 == 0:
+        cr |= 0xFFFF << 24
+    elif i % 3 == 1:
+        cr = (cr | 0xFFFF << 24) & ~(1 << int(rng.integers(24, 40)))
+    b[4] = np.uint64(cr)
+    return b
+
+
+@pytest.mark.parametrize("depth", [2, 3])
+def test_perft_of_any_board_with_few_and_many_others(zeta, oracle, depth):
+    """Few positions go a wavefront a parent, many a lane a parent: on any board
+    the same tree."""
+    rng = np.random.default_rng(23)
+    n = 600
+    pos = np.zeros(n, dtype=oracle.POS_DTYPE)
+    for i in range(n):
+        pos[i]["b"] = _board(rng, i)
+        pos[i]["stm"] = i & 1
+    few = np.concatenate([zeta.perft(pos[k:k + 15], depth) for k in range(0, n, 15)])
+    many = zeta.perft(np.tile(pos, 34), depth).reshape(34, n)  # past 16384
+    assert (many == many[0]).all()
+    bad = np.nonzero(few != many[0])[0]
+    print("differ", len(bad), [(int(i), int(few[i]), int(many[0][i])) for i in bad[:5]], flush=True)
+    assert not len(bad)

@@ -747,6 +747,20 @@ ZD u64 lane_targets(const Pos &p, const Node0 &B, u64 A, int sq, bool qs) {
   return t & T;
 }
 
+// Do lane_targets, square by square, find the moves that for_each_legal does?
+// The set-wise form takes boards no game reaches in its own way: several kings,
+// and an e.p. flag that is not alone on a pawn that can have stepped two past an
+// empty square, or next to which the kings stand side by side.
+ZD bool lanes_serve(const Pos &p, const Node0 &B) {
+  const u64 okb = B.opp & B.kings, w = ~p.cr & RANKS45;
+  bool serve = (popc(B.kbb) == 1) & ((okb & (okb - 1)) == 0);
+  if (w) {
+    const u64 stepped = B.opp & B.pawns & (p.stm ? RANK4 : RANK5);
+    serve &= !(w & (w - 1)) & ((w & stepped) != 0) & !((p.stm ? w >> 8 : w << 8) & B.occ) & !(king_att(B.kbb) & okb);
+  }
+  return serve;
+}
+
 // ---- lane = square of one position whose king is not in check: what a slider
 // on the lane's square would see
 struct LaneRays {

@@ -347,13 +347,13 @@ __global__ __launch_bounds__(64) void k_count_roots(const u64 *__restrict__ in, 
 }
 
 // ---- wide: the legal moves of one position, spread over a wavefront: lane
-// takes move number `lane` + 64 k of list[0 .. n).  A position without exactly
-// one king of its own is enumerated by one lane (the per-square form below
-// takes each king for itself).
+// takes move number `lane` + 64 k of list[0 .. n).  Boards that the per-square
+// form takes otherwise than the counts do (lanes_serve) are enumerated by one
+// lane.
 __device__ __forceinline__ int wide_moves(const Pos &p, int lane, u32 *list) {
   Node0 B;
   node_basics(p, B);
-  if (popc(B.kbb) != 1) {
+  if (!lanes_serve(p, B)) {
     int n = 0;
     if (lane == 0) {
       Legal L;
