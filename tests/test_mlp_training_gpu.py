@@ -103,3 +103,22 @@ def test_training_repeats_itself(zeta, pairs, npairs):
     assert np.array_equal(runs[0][0].view(np.uint32), runs[1][0].view(np.uint32))
     assert np.array_equal(runs[0][1].view(np.uint32), runs[1][1].view(np.uint32))
     zeta.records_clear()
+
+
+def test_training_after_a_batch_that_does_not_fit(zeta, pairs):
+    """A batch of 400 GB of activations is refused, and what ran before runs on."""
+    w = np.random.default_rng(13).normal(0, 0.06, M.NPARAMS).astype(np.float32)
+    zeta.records_reserve(LOGGED)
+
+    def train():
+        zeta.records_clear()
+        zeta.records_put(pairs)
+        zeta.mlp_set(w)
+        return zeta.mlp_train(3, 256, 1e-3, 3), zeta.mlp_get(), zeta.mlp_grad(pairs[:64])[1]
+
+    before = train()
+    with pytest.raises(zeta.ZetaError):
+        zeta.mlp_train(1, 400_000_000, 1e-3, 3)
+    for a, b in zip(before, train()):
+        assert np.array_equal(a, b)
+    zeta.records_clear()

@@ -618,12 +618,15 @@ int ensure_weights() {
 }
 
 int ensure_batch(int P) {
+  int r;
+  if ((r = zr::ensure(g_ms.loss, 64))) return r;  // (training grows it by itself)
   if (g_ms.cap_pairs >= P) return ZETA_OK;
   const size_t B = 2 * (size_t)P;
-  int r;
-  if ((r = zr::ensure(g_ms.bits, B / 32 * NINP * 4)) || (r = zr::ensure(g_ms.h1x, B * NH1 * 2)) ||
-      (r = zr::ensure(g_ms.dz2x, B * NH2 * 2)) || (r = zr::ensure(g_ms.dz1x, B * NH1 * 2)) ||
-      (r = zr::ensure(g_ms.sums, B / 32 * NSUM * 4)) || (r = zr::ensure(g_ms.loss, 64)))
+  // none until all are there: one that cannot grow is gone
+  g_ms.cap_pairs = 0;
+  if ((r = zr::ensure(g_ms.h1x, B * NH1 * 2)) || (r = zr::ensure(g_ms.dz1x, B * NH1 * 2)) ||
+      (r = zr::ensure(g_ms.bits, B / 32 * NINP * 4)) || (r = zr::ensure(g_ms.dz2x, B * NH2 * 2)) ||
+      (r = zr::ensure(g_ms.sums, B / 32 * NSUM * 4)))
     return r;
   g_ms.cap_pairs = P;
   return ZETA_OK;

@@ -893,6 +893,7 @@ int ensure_level(int L, size_t n) {
     return zr::fail(ZETA_ENOMEM, "perft scratch: level %d needs %zu positions, holds %zu", L, n, b.cap);
   size_t cap = n + n / 4 + 1024;
   int r;
+  b.cap = 0;  // none until all are there: one that cannot grow is gone
   if ((r = zr::ensure(b.b0, cap * 8)) || (r = zr::ensure(b.b1, cap * 8)) || (r = zr::ensure(b.b2, cap * 8)) ||
       (r = zr::ensure(b.b3, cap * 8)) || (r = zr::ensure(b.cr, cap * 8)) || (r = zr::ensure(b.meta, cap * 4)) ||
       (r = zr::ensure(b.cnt, cap * 4)) || (r = zr::ensure(b.off, (cap + 1) * 8)) ||
@@ -909,6 +910,7 @@ int ensure_pairs(int L, size_t m) {
     return zr::fail(ZETA_ENOMEM, "perft scratch: level %d needs %zu pairs, holds %zu", L, m, b.paircap);
   size_t cap = m + m / 8 + 1024;
   int r;
+  b.paircap = 0;
   if ((r = zr::ensure(b.pm, cap * 8))) return r;
   b.paircap = cap;
   return ZETA_OK;
